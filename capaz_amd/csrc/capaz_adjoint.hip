@@ -120,9 +120,13 @@ __global__ void k_obs_adjoint(double* lSw, double* lSn, const int64_t* cells, in
 template <int IT>
 struct AdjNewtonStore {
     AdjIO a;
-    __device__ __forceinline__ void operator()(const DevParams& p, int i, int j, int k, int64_t l, const CoefT<3>& c,
-                                               const double* div) const {
-        adj_newton_tail<IT>(p, a, i, j, k, l, c.ro, c.P[0], c.Sw, c.Sn, div);
+    template <class At>
+    __device__ __forceinline__ int prefetch(const At&) const { return 0; }
+    template <bool GENERAL, class At>
+    __device__ __forceinline__ bool cell(const DevParams& p, const DevParams&, int i, int j, int k, const At& at,
+                                         const CellState<3>& s, const double* div, int) const {
+        adj_newton_tail<IT>(p, a, i, j, k, at.l(), s.ro, s.P, s.Sw, s.Sn, div);
+        return true;
     }
 };
 
@@ -130,9 +134,9 @@ constexpr int kTX = 64, kTY = 8;
 
 template <int CLOSURE, int IT>
 __global__ void __launch_bounds__(kTX * kTY) k_adj_newton_z(DevParams p, StepIO io, AdjIO a, int kchunk) {
-    __shared__ FusedLds<9, kTX, kTY> lds;
-    fused_z_tile<3, CLOSURE, kTX, kTY, true>(p, io, kchunk, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, lds,
-                                             AdjNewtonStore<IT>{a});
+    __shared__ FusedLds<3, CLOSURE, kTX, kTY> lds;
+    fused_z_tile<3, CLOSURE, kTX, kTY, false>(p, kernel_params(), io, kchunk, (int)blockIdx.x, (int)blockIdx.y,
+                                              (int)blockIdx.z, lds, AdjNewtonStore<IT>{a});
 }
 
 // Pass 2 over tiles of kTX x kTY columns (every cell, boundary included)

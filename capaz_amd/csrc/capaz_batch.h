@@ -23,8 +23,10 @@ struct BatchDomain {
 // Tile shape of the batch kernels: TX x TY columns, kchunk planes per tile;
 // persistent 1: a grid that fills the GPU once and takes tiles from a queue
 // (one atomic counter per step), 0: one workgroup per tile.
+// full: every realization has Nx, Nz >= 3 (set by the batch, not by a caller).
 struct BatchShape {
     int tx = 64, ty = 8, kchunk = 16, persistent = 1;
+    bool full = false;
 };
 
 bool batch_shape_supported(int tx, int ty);

@@ -20,23 +20,21 @@ namespace capaz {
 namespace {
 
 // Occupancy bounds: the two-phase Corey-2 tiles of 256 threads (the 32 x 8
-// and 64 x 4 shapes) fit in 94 VGPRs without a spill, 5 waves per SIMD
-// against 4 at the compiler's own 106-108: the 64-realization ensemble went
-// from 46.4 to 50.2 Gcell-steps/s; bound to 6 waves (80 VGPRs, 17 spilled)
-// it ran at 44.5.  The three-phase Corey-2 tiles fit in 128 VGPRs without a
-// spill against the compiler's own 129-131, 4 waves per SIMD against 3 (one
-// 512-thread workgroup per CU for 64 x 8): a 24-realization three-phase
-// batch (edges 32-96) 0.331 -> 0.305 ms per step on 32 x 8 tiles, 0.524 ->
-// 0.376 ms on 64 x 8.
+// and 64 x 4 shapes) at 5 waves per SIMD (96 VGPRs, few spilled), the
+// three-phase Corey-2 ones at 4 (128 VGPRs).  32 two-phase realizations of edges
+// 32-96 step in 186 us on 32 x 8 tiles of 8 planes, one workgroup each,
+// against 218 with the tiles before (capaz_fused.h).
 template <int MODEL, int CLOSURE, int TX, int TY>
 constexpr int kBatchWaves =
     MODEL == 2 && CLOSURE == 2 && TX * TY == 256 ? 5 : (MODEL == 3 && CLOSURE == 2 ? 4 : 1);
 
-template <int MODEL, int CLOSURE, int TX, int TY>
+using ConstDomain = const __attribute__((address_space(4))) BatchDomain;
+
+template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(kBatchWaves<MODEL, CLOSURE, TX, TY>)))
     k_batch_z(const BatchDomain* __restrict__ doms, const int* __restrict__ owner, int ntiles, int parity,
               int kchunk, int* counter) {
-    __shared__ FusedLds<3 * MODEL, TX, TY> lds;
+    __shared__ FusedLds<MODEL, CLOSURE, TX, TY> lds;
     __shared__ int claimed;
     // one workgroup per tile: each XCD (workgroups go to the 8 XCDs round
     // robin) takes a contiguous run of the tile list, so a realization's
@@ -51,11 +49,14 @@ __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(kB
             __syncthreads();  // all have read `claimed` before it is overwritten
         }
         if (t < 0 || t >= ntiles) return;
-        const BatchDomain* d = doms + owner[t];
+        // the realization's entry, wave-uniform and read-only while the kernel runs: scalar loads
+        ConstDomain* d = (ConstDomain*)(uintptr_t)doms + __builtin_amdgcn_readfirstlane(owner[t]);
+        const DevParams p = *(const DevParams*)&d->p;
+        const StepIO io = *(const StepIO*)&d->io[parity];
         const int lt = t - d->tile_begin;
         const int bx = lt % d->tiles_x, r = lt / d->tiles_x;
-        fused_z_tile<MODEL, CLOSURE, TX, TY, true>(d->p, d->io[parity], kchunk, bx, r % d->tiles_y, r / d->tiles_y,
-                                                   lds, FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE>{d->io[parity]});
+        fused_z_tile<MODEL, CLOSURE, TX, TY, FULL>(p, &d->p, io, kchunk, bx, r % d->tiles_y, r / d->tiles_y, lds,
+                                                    FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE>{io});
         if (!counter) return;
     }
 }
@@ -67,20 +68,23 @@ __global__ void __launch_bounds__(256)
     fused_face<MODEL, CLOSURE>(d->p, d->io[parity], (int64_t)((int)blockIdx.x - d->face_block_begin) * 256 + threadIdx.x);
 }
 
+// Planes per tile (the tile body's limit).
+int tile_planes(const BatchShape& sh) { return sh.kchunk < kMaxPlanes ? sh.kchunk : kMaxPlanes; }
+
 __global__ void k_zero_ints(int* p, int n) {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (i < n) p[i] = 0;
 }
 
-template <int MODEL, int CLOSURE, int TX, int TY>
-hipError_t step_shape(const BatchShape& sh, const BatchDomain* doms, const int* tile_owner, int ntiles,
+template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
+hipError_t step_full(const BatchShape& sh, const BatchDomain* doms, const int* tile_owner, int ntiles,
                       const int* face_owner, int nface_blocks, int parity, int* counter, int grid, hipStream_t s) {
     if (ntiles > 0) {
         // (the one-per-tile grid is rounded up to a multiple of the 8 XCDs;
         // the extra workgroups find no tile and exit)
         const int g = sh.persistent ? grid : (ntiles + 7) / 8 * 8;
-        hipLaunchKernelGGL((k_batch_z<MODEL, CLOSURE, TX, TY>), dim3(g), dim3(TX, TY), 0, s, doms, tile_owner, ntiles,
-                           parity, sh.kchunk, sh.persistent ? counter : nullptr);
+        hipLaunchKernelGGL((k_batch_z<MODEL, CLOSURE, TX, TY, FULL>), dim3(g), dim3(TX, TY), 0, s, doms, tile_owner, ntiles,
+                           parity, tile_planes(sh), sh.persistent ? counter : nullptr);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
@@ -89,6 +93,15 @@ hipError_t step_shape(const BatchShape& sh, const BatchDomain* doms, const int* 
         hipLaunchKernelGGL((k_batch_faces<MODEL, CLOSURE>), dim3(nface_blocks), dim3(256), 0, s, doms, face_owner,
                            parity);
     return hipGetLastError();
+}
+
+template <int MODEL, int CLOSURE, int TX, int TY>
+hipError_t step_shape(const BatchShape& sh, const BatchDomain* doms, const int* tile_owner, int ntiles,
+                      const int* face_owner, int nface_blocks, int parity, int* counter, int grid, hipStream_t s) {
+    return sh.full ? step_full<MODEL, CLOSURE, TX, TY, true>(sh, doms, tile_owner, ntiles, face_owner, nface_blocks,
+                                                             parity, counter, grid, s)
+                   : step_full<MODEL, CLOSURE, TX, TY, false>(sh, doms, tile_owner, ntiles, face_owner, nface_blocks,
+                                                              parity, counter, grid, s);
 }
 
 template <int MODEL, int CLOSURE>
@@ -104,13 +117,17 @@ hipError_t step_closure(const BatchShape& sh, const BatchDomain* doms, const int
                                              grid, s);
 }
 
+template <int MODEL, int CLOSURE, bool FULL>
+hipError_t occupancy_full(const BatchShape& sh, int* n) {
+    if (sh.tx == 64 && sh.ty == 8)
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, k_batch_z<MODEL, CLOSURE, 64, 8, FULL>, 512, 0);
+    if (sh.tx == 64 && sh.ty == 4)
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, k_batch_z<MODEL, CLOSURE, 64, 4, FULL>, 256, 0);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, k_batch_z<MODEL, CLOSURE, 32, 8, FULL>, 256, 0);
+}
 template <int MODEL, int CLOSURE>
 hipError_t occupancy_closure(const BatchShape& sh, int* n) {
-    if (sh.tx == 64 && sh.ty == 8)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, k_batch_z<MODEL, CLOSURE, 64, 8>, 512, 0);
-    if (sh.tx == 64 && sh.ty == 4)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, k_batch_z<MODEL, CLOSURE, 64, 4>, 256, 0);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, k_batch_z<MODEL, CLOSURE, 32, 8>, 256, 0);
+    return sh.full ? occupancy_full<MODEL, CLOSURE, true>(sh, n) : occupancy_full<MODEL, CLOSURE, false>(sh, n);
 }
 
 }  // namespace
@@ -123,7 +140,8 @@ void batch_tiles(const DevParams& p, const BatchShape& sh, int* nx, int* ny, int
     const int ix = p.Nx >= 3 ? p.Nx - 2 : 1, iy = p.Ny - 2, iz = p.Nz >= 3 ? p.Nz - 2 : 1;
     *nx = (ix + sh.tx - 1) / sh.tx;
     *ny = (iy + sh.ty - 1) / sh.ty;
-    *nz = (iz + sh.kchunk - 1) / sh.kchunk;
+    const int planes = tile_planes(sh);
+    *nz = (iz + planes - 1) / planes;
 }
 
 hipError_t batch_occupancy(int model, int closure, const BatchShape& sh, int* n) {

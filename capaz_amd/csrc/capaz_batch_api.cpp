@@ -289,6 +289,8 @@ int capaz_batch_create(const capaz_params* base, int count, const int* dims, cap
     std::memset(b->h_doms, 0, count * sizeof(capaz::BatchDomain));
     if ((e = hipMalloc(&b->d_doms, count * sizeof(capaz::BatchDomain))) != hipSuccess)
         return bail(CAPAZ_ERR_NOMEM, "hipMalloc");
+    b->shape.full = std::all_of(b->dom.begin(), b->dom.end(),
+                                [](const capaz_ctx* c) { return c->p.Nx >= 3 && c->p.Nz >= 3; });
     b->order.resize(count);
     std::iota(b->order.begin(), b->order.end(), 0);
     std::stable_sort(b->order.begin(), b->order.end(), [&](int x, int y) {
@@ -433,7 +435,7 @@ int capaz_batch_autotune(capaz_batch* b, int steps, double* best_ms) {
         for (const auto& s : shapes) {
             if (rc) break;
             for (int kc : kchunks) {
-                b->shape = BatchShape{s[0], s[1], kc, persistent};
+                b->shape = BatchShape{s[0], s[1], kc, persistent, keep.full};
                 if ((rc = run_steps(b, 2, false))) break;  // warm-up
                 if ((rc = prepare(b))) break;
                 if ((rc = ensure_counters(b, steps))) break;

@@ -21,6 +21,7 @@
 
 #include <math.h>
 #include <stdint.h>
+#include <string.h>
 
 #include "capaz_params.h"
 
@@ -88,6 +89,47 @@ CAPAZ_HD double rcp_rn_pivot(double b) {
     return 1. / b;
 #endif
 }
+
+// RN(1/b) for |b| in [2^-1000, 2^1000] (anything else: any value).  The
+// estimate's relative error e is below 2^-20, so y (1 + e + e^2) is within
+// e^3 < 2^-60 of 1/b before its rounding: one step in place of the two
+// Newton-Raphson steps of rcp_rn, then the same final correction.
+CAPAZ_HD double rcp_in_range(double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double y = __builtin_amdgcn_rcp(b);
+    double e = fma(-b, y, 1.);
+    y = fma(fma(e, e, e), y, y);
+    e = fma(-b, y, 1.);
+    return fma(e, y, y);
+#else
+    return 1. / b;
+#endif
+}
+
+// Collects whether the divisors seen so far all lie in [1e-8, 2^1000] in
+// magnitude (no branch per divisor): the largest of their high words'
+// distances above 1e-8's, the sign shifted out; a smaller magnitude wraps to a
+// large value.  A divisor whose high word equals 1e-8's counts as outside.
+struct DivisorRange {
+    uint32_t worst = 0;
+    CAPAZ_HD void see(double b) {
+        struct Words {
+            uint32_t lo, hi;
+        };
+        Words w;
+        memcpy(&w, &b, sizeof(w));
+        const uint32_t c = 0u - 2u * (0x3E45798Eu + 1u);  // 1e-8 = 0x3E45798EE2308C3A
+        uint32_t d;
+#if defined(__HIP_DEVICE_COMPILE__)
+        // 2 * hi + c, which the compiler makes of a 64-bit shift, an and and an add
+        asm("v_lshl_add_u32 %0, %1, 1, %2" : "=v"(d) : "v"(w.hi), "s"(c));
+#else
+        d = 2u * w.hi + c;
+#endif
+        worst = d > worst ? d : worst;
+    }
+    CAPAZ_HD bool ok() const { return worst <= 2u * (0x7E700000u - (0x3E45798Eu + 1u)); }  // 2^1000 = 0x7E70...
+};
 
 CAPAZ_HD double half(double x) { return x * 0.5; }
 // x clipped to [0, 1]; a NaN passes through (so a non-finite state spreads
@@ -513,6 +555,38 @@ CAPAZ_HD bool reverse3_nopivot_a02zero(double* a) {
     return true;
 }
 
+// reverse3_nopivot_a02zero without its tests: the pivots are noted in `range`
+// instead, and the result means nothing if range.ok() is false.
+CAPAZ_HD void reverse3_a02zero(double* a, DivisorRange& range) {
+    double f = a[0];
+    range.see(f);
+    double rf = rcp_in_range(f);
+    double r01 = exact_div(a[1], f, rf), r03 = rf;
+    double f1 = a[3];
+    double b11 = a[4] - r01 * f1, b12 = a[5], b13 = -(r03 * f1);
+    double f2 = a[6];
+    double b21 = a[7] - r01 * f2, b22 = a[8], b23 = -(r03 * f2);
+    f = b11;
+    range.see(f);
+    rf = rcp_in_range(f);
+    double s12 = exact_div(b12, f, rf), s13 = exact_div(b13, f, rf), s14 = rf;
+    f1 = r01;
+    double c02 = -(s12 * f1), c03 = r03 - s13 * f1, c04 = -(s14 * f1);
+    f2 = b21;
+    double c22 = b22 - s12 * f2, c23 = b23 - s13 * f2, c24 = -(s14 * f2);
+    f = c22;
+    range.see(f);
+    rf = rcp_in_range(f);
+    double t23 = exact_div(c23, f, rf), t24 = exact_div(c24, f, rf), t25 = rf;
+    f1 = c02;
+    double o03 = c03 - t23 * f1, o04 = c04 - t24 * f1, o05 = -(t25 * f1);
+    f2 = s12;
+    double o13 = s13 - t23 * f2, o14 = s14 - t24 * f2, o15 = -(t25 * f2);
+    a[0] = o03; a[1] = o04; a[2] = o05;
+    a[3] = o13; a[4] = o14; a[5] = o15;
+    a[6] = t23; a[7] = t24; a[8] = t25;
+}
+
 // reverse_matrix<3> with the no-pivot path first.  `a` stays in registers;
 // only the rare fallback copies it to a stack buffer for the out-of-line call
 // (reverse3_nopivot leaves `a` unchanged when it fails).
@@ -532,9 +606,9 @@ CAPAZ_HD int reverse3(double* a) {
 
 // Two-phase fixed-iteration 2x2 Newton by Cramer's rule (two-phase.cpp:25-56).
 // CL: the fused kernels' closure id (0 the reference's Brooks-Corey, 1 and 2
-// Corey), or -1 for p.closure at run time.
-template <int CL = -1>
-CAPAZ_HD void newton2(const DevParams& p, double& P, double& Sn, double roS_w, double roS_n) {
+// Corey), or -1 for p.closure at run time.  rcp(det): RN(1 / det).
+template <int CL, class Rcp>
+CAPAZ_HD void newton2_with(const DevParams& p, double& P, double& Sn, double roS_w, double roS_n, Rcp&& rcp) {
     for (int w = 1; w <= p.iterations; w++) {
         double P_k, PkS;
         if (CL >= 1 || (CL < 0 && p.closure == 1)) {
@@ -554,17 +628,41 @@ CAPAZ_HD void newton2(const DevParams& p, double& P, double& Sn, double roS_w, d
         double F1S = (-1) * p.ro0_w * (1 + p.beta_w * (P - p.P_atm));
         double F2S = p.ro0_n * (1 + p.beta_n * (P + P_k - p.P_atm + (Sn * PkS)));
         double det = F1P * F2S - F1S * F2P;
-        double rdet = rcp_rn(det);  // 1 / det
+        double rdet = rcp(det);  // 1 / det
         P = P - rdet * (F2S * F1 - F1S * F2);
         Sn = Sn - rdet * (F1P * F2 - F2P * F1);
     }
+}
+template <int CL = -1>
+CAPAZ_HD void newton2(const DevParams& p, double& P, double& Sn, double roS_w, double roS_n) {
+    newton2_with<CL>(p, P, Sn, roS_w, roS_n, [](double det) { return rcp_rn(det); });
+}
+// newton2 for a kernel's hot path, with no call and no branch per iteration:
+// false (and any values) if some determinant lay outside the fast
+// reciprocal's range; newton2_ieee (an IEEE division, inline) then redoes the
+// cell.  RN(1 / det) either way, so the same bits.
+template <int CL>
+CAPAZ_HD bool newton2_fast(const DevParams& p, double& P, double& Sn, double roS_w, double roS_n) {
+    double lo = 0x1p0, hi = 0x1p0;
+    newton2_with<CL>(p, P, Sn, roS_w, roS_n, [&](double det) {
+        lo = fmin(lo, fabs(det));
+        hi = fmax(hi, fabs(det));
+        return rcp_in_range(det);
+    });
+    return lo >= 0x1p-1000 && hi <= 0x1p1000;
+}
+template <int CL>
+CAPAZ_HD void newton2_ieee(const DevParams& p, double& P, double& Sn, double roS_w, double roS_n) {
+    newton2_with<CL>(p, P, Sn, roS_w, roS_n, [](double det) { return 1. / det; });
 }
 
 // Three-phase fixed-iteration 3x3 Newton (three-phase.cpp:286-339) with the
 // CPU path's zero capillary pressures folded; dF[4] = ro0_n*S_n keeps the
 // reference's Jacobian entry (three-phase.cpp:319).
-CAPAZ_HD void newton3(const DevParams& p, double& P, double& Sw, double& Sn, double roS_w, double roS_n,
-                      double roS_g) {
+// inverse(dF): the inverse in place, as reverse_matrix; dF[2] is +0.
+template <class Inverse>
+CAPAZ_HD void newton3_with(const DevParams& p, double& P, double& Sw, double& Sn, double roS_w, double roS_n,
+                           double roS_g, Inverse&& inverse) {
     for (int w = 1; w <= p.iterations; w++) {
         double Sg = 1. - Sw - Sn;
         double rw = p.ro0_w * (1. + p.beta_w * (P - p.P_atm));  // dF[1]
@@ -583,11 +681,29 @@ CAPAZ_HD void newton3(const DevParams& p, double& P, double& Sw, double& Sn, dou
         dF[6] = exact_div(p.ro0_g * Sg, p.P_atm, p.r_P_atm);
         dF[7] = -gP;
         dF[8] = -gP;
-        reverse3<true>(dF);
+        inverse(dF);
         P = P - (dF[0] * F1 + dF[1] * F2 + dF[2] * F3);
         Sw = Sw - (dF[3] * F1 + dF[4] * F2 + dF[5] * F3);
         Sn = Sn - (dF[6] * F1 + dF[7] * F2 + dF[8] * F3);
     }
+}
+CAPAZ_HD void newton3(const DevParams& p, double& P, double& Sw, double& Sn, double roS_w, double roS_n,
+                      double roS_g) {
+    newton3_with(p, P, Sw, Sn, roS_w, roS_n, roS_g, [](double* dF) { reverse3<true>(dF); });
+}
+// newton3 for a kernel's hot path, with no call and no branch per iteration:
+// false (and any values) if some pivot needed the pivot search or lay outside
+// the fast reciprocal's range; newton3_general (gauss.cpp's routine, inline)
+// then redoes the cell.  The same bits either way.
+CAPAZ_HD bool newton3_fast(const DevParams& p, double& P, double& Sw, double& Sn, double roS_w, double roS_n,
+                           double roS_g) {
+    DivisorRange range;
+    newton3_with(p, P, Sw, Sn, roS_w, roS_n, roS_g, [&](double* dF) { reverse3_a02zero(dF, range); });
+    return range.ok();
+}
+CAPAZ_HD void newton3_general(const DevParams& p, double& P, double& Sw, double& Sn, double roS_w, double roS_n,
+                              double roS_g) {
+    newton3_with(p, P, Sw, Sn, roS_w, roS_n, roS_g, [](double* dF) { reverse_matrix<3>(dF); });
 }
 
 // ---- energy closures (energy.cpp:4-143) ---------------------------------------------------

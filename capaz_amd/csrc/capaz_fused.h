@@ -35,7 +35,20 @@ struct CoefT {
     double Sw, Sn;  // the cell's saturations, as read
 };
 
-// Corey k_r with the exponent fixed at 2 (CLOSURE 2) or read from p (1).
+// -K k_r of a phase with the Corey closure: exponent 2 (CLOSURE 2) or read
+// from p (1).  For exponent 2 the clip to [0, 1] is one instruction (the clamp
+// modifier, which makes a NaN 0), and a NaN s comes back through K: 0 * s + K
+// is K for every finite s, and the quotient s is finite or NaN.
+template <int CLOSURE>
+__device__ __forceinline__ double corey_mK(const DevParams& p, double K, double s) {
+    if constexpr (CLOSURE == 2) {
+        const double c = fmin(fmax(s, 0.), 1.);
+        return (-1.) * fma(0., s, K) * (c * c);
+    } else {
+        return (-1.) * K * corey_kr(p, s);
+    }
+}
+
 template <int CLOSURE>
 __device__ __forceinline__ double corey_t(const DevParams& p, double s) {
     if constexpr (CLOSURE == 2) {
@@ -194,38 +207,342 @@ struct EpiWantsU : std::false_type {};
 template <class E>
 struct EpiWantsU<E, std::void_t<decltype(E::kWantsU)>> : std::bool_constant<E::kWantsU> {};
 
-template <int NV, int TX, int TY>
+// Pressures staged per cell: the phases' pressures are one value except where
+// a closure has a capillary pressure (two phases, Brooks-Corey).  Three
+// phases: P_n = P_g = P_w in the interior and, once Border_P has run, on the
+// x and z faces; the top and bottom rows' own P_n and P_g are staged apart.
+template <int MODEL, int CLOSURE>
+constexpr int kStagedP = MODEL == 2 && CLOSURE == 0 ? 2 : 1;
+
+// LDS of a tile: two planes' coefficients (P, Xi, ro) of the tile and its
+// one-cell ring, the plane being read and the one being staged.  A cell's
+// values lie together, so that a neighbour's are one address and constant
+// offsets that a paired read reaches (an array per value needed ~20 address
+// additions per cell); their number is odd, which puts 64 lanes' reads of one
+// value on distinct banks.  Three phases: edge[.][0 / 1] = P_n, P_g of the top / bottom row (j = 0 / Ny - 1)
+// where the tile touches it, odd[.][row] = the plane k in which a staged x
+// face cell of that row has a P_n or P_g of its own (any other value: none).
+template <int MODEL, int CLOSURE, int TX, int TY>
 struct FusedLds {
-    double v[NV][TY + 2][TX + 2];
+    static constexpr int kNV = (kStagedP<MODEL, CLOSURE> + 2 * MODEL) | 1;
+    double v[2][TY + 2][TX + 2][kNV];
+    double edge[2][MODEL == 3 ? 2 : 0][2][TX + 2];
+    int odd[2][MODEL == 3 ? TY + 2 : 0];
+};
+
+// A cell of a field array: a wave-uniform index (scalar registers) and the
+// lane's own offset in bytes, which a load or store then takes as they are.
+struct CellAt {
+    int64_t base;
+    uint32_t off;
+    __device__ __forceinline__ int64_t l() const { return base + off / 8u; }
+};
+// The row's address in a scalar register pair and the lane's offset in one
+// vector register, the two operands of a global access: left to itself the
+// compiler adds the lane's offset to the field's address outside the plane
+// loop (two vector registers per field) and the row to that for every access
+// (a 64-bit add).  renew(): to be called in each block of code that accesses
+// the cell, so that the offset is known to be a 32-bit value there.
+__device__ __forceinline__ __attribute__((address_space(1))) char* row_of(const double* f, int64_t base) {
+    auto* r = (__attribute__((address_space(1))) char*)(f + base);
+    asm("" : "+s"(r));
+    return r;
+}
+__device__ __forceinline__ void renew(CellAt& a) { asm volatile("" : "+v"(a.off)); }
+__device__ __forceinline__ double ld(const double* f, const CellAt& a) {
+    return *(__attribute__((address_space(1))) const double*)(row_of(f, a.base) + a.off);
+}
+// A cell by its own index alone.
+struct CellIndex {
+    int64_t i;
+    __device__ __forceinline__ int64_t l() const { return i; }
+};
+__device__ __forceinline__ void renew(CellIndex&) {}
+__device__ __forceinline__ double ld(const double* f, const CellIndex& a) { return f[a.i]; }
+__device__ __forceinline__ void st(double* f, const CellIndex& a, double v) { f[a.i] = v; }
+__device__ __forceinline__ void st(double* f, const CellAt& a, double v) {
+    *(__attribute__((address_space(1))) double*)(row_of(f, a.base) + a.off) = v;
+}
+
+// The parameter block in constant memory.  The tiles hold more parameters
+// than there are scalar registers; kept across the plane loop, the rest lived
+// in lanes of vector registers, one v_readlane (a VALU slot) per word and use:
+// some 45 per cell of the 256^3 Corey-2 step's 795.  fresh() makes the compiler
+// read the ones a part of a plane's work needs where it begins (scalar loads).
+using ConstParams = const __attribute__((address_space(4))) DevParams;
+__device__ __forceinline__ ConstParams* fresh(ConstParams* p) {
+    asm volatile("" : "+s"(p));
+    return p;
+}
+// The kernel's first argument.
+__device__ __forceinline__ ConstParams* kernel_params() {
+    return (ConstParams*)__builtin_amdgcn_kernarg_segment_ptr();
+}
+// The parameters that coef_of / the fluxes / the Newton solves read.
+template <int MODEL, int CLOSURE>
+__device__ __forceinline__ DevParams coef_params(ConstParams* q) {
+    DevParams p;
+    if constexpr (CLOSURE == 3) return p;
+    p.closure = CLOSURE == 0 ? 0 : 1;
+    p.P_atm = q->P_atm;
+    p.mu_w = q->mu_w, p.r_mu_w = q->r_mu_w;
+    p.mu_n = q->mu_n, p.r_mu_n = q->r_mu_n;
+    p.ro0_w = q->ro0_w, p.beta_w = q->beta_w;
+    p.ro0_n = q->ro0_n, p.beta_n = q->beta_n;
+    p.S_wr = q->S_wr;
+    if constexpr (CLOSURE == 1) p.corey_n = q->corey_n;
+    if constexpr (MODEL == 2) {
+        if constexpr (CLOSURE == 0) {
+            p.den2 = q->den2, p.r_den2 = q->r_den2;
+            p.bc_ew = q->bc_ew, p.bc_en = q->bc_en, p.bc_epk = q->bc_epk, p.P_d = q->P_d;
+        } else {
+            p.den2c = q->den2c, p.r_den2c = q->r_den2c;
+        }
+    } else {
+        p.S_nr = q->S_nr, p.den3 = q->den3, p.r_den3 = q->r_den3;
+        p.mu_g = q->mu_g, p.r_mu_g = q->r_mu_g;
+        p.ro0_g = q->ro0_g, p.r_P_atm = q->r_P_atm;
+        if constexpr (CLOSURE == 0) p.vg_a = q->vg_a, p.vg_b = q->vg_b, p.vg_c = q->vg_c;
+    }
+    return p;
+}
+__device__ __forceinline__ DevParams flux_params(ConstParams* q) {
+    DevParams p;
+    p.hx = q->hx, p.r_hx = q->r_hx, p.hy = q->hy, p.r_hy = q->r_hy, p.hz = q->hz, p.r_hz = q->r_hz, p.g = q->g;
+    p.two_hx = q->two_hx, p.r_two_hx = q->r_two_hx, p.two_hy = q->two_hy, p.r_two_hy = q->r_two_hy;
+    p.two_hz = q->two_hz, p.r_two_hz = q->r_two_hz;
+    return p;
+}
+template <int MODEL, int CLOSURE>
+__device__ __forceinline__ DevParams newton_params(ConstParams* q) {
+    DevParams p;
+    p.closure = CLOSURE == 0 ? 0 : 1;
+    p.iterations = q->iterations;
+    p.P_atm = q->P_atm;
+    p.ro0_w = q->ro0_w, p.beta_w = q->beta_w;
+    p.ro0_n = q->ro0_n, p.beta_n = q->beta_n;
+    if constexpr (MODEL == 3) {
+        p.ro0_g = q->ro0_g, p.r_P_atm = q->r_P_atm;
+        p.c_wb = q->c_wb, p.c_nb = q->c_nb;
+    } else if constexpr (CLOSURE == 0) {
+        p.S_wr = q->S_wr, p.den2 = q->den2, p.r_den2 = q->r_den2, p.P_d = q->P_d;
+        p.bc_epk = q->bc_epk, p.bc_eaaa = q->bc_eaaa, p.bc_pks_den = q->bc_pks_den, p.r_bc_pks_den = q->r_bc_pks_den;
+    }
+    return p;
+}
+
+// The values of a cell that its coefficients are made of, as read (loaded
+// ahead of their use), and the coefficients themselves.
+template <int MODEL, int CLOSURE>
+struct CellRaw {
+    double Pw, Sw, Sn, K, Pn, Pg, Xi[MODEL], ro[MODEL];
+};
+template <int MODEL, int CLOSURE>
+struct CellCoef {
+    double P[kStagedP<MODEL, CLOSURE>], Xi[MODEL], ro[MODEL];
+};
+
+template <int MODEL, int CLOSURE, class At>
+__device__ __forceinline__ void load_raw(const StepIO& io, const At& at, bool inner, CellRaw<MODEL, CLOSURE>& r) {
+    r.Pw = ld(io.Pw, at);
+    r.Sn = ld(io.Sn, at);
+    if constexpr (MODEL == 3) r.Sw = ld(io.Sw, at);
+    if constexpr (CLOSURE == 3) {
+#pragma unroll
+        for (int a = 0; a < MODEL; ++a) {
+            r.Xi[a] = ld(io.Xi[a], at);
+            r.ro[a] = ld(io.ro[a], at);
+        }
+    } else {
+        r.K = ld(io.K, at);
+    }
+    if constexpr (MODEL == 3) {
+        if (!inner) {
+            r.Pn = ld(io.Pn, at);
+            r.Pg = ld(io.Pg, at);
+        }
+    }
+}
+
+// coef_at's values from what load_raw read; the return value tells a cell
+// whose P_n or P_g is not its P_w (three phases, boundary cells).
+template <int MODEL, int CLOSURE>
+__device__ __forceinline__ bool coef_of(const DevParams& p, const CellRaw<MODEL, CLOSURE>& r, bool inner,
+                                        CellCoef<MODEL, CLOSURE>& c) {
+    c.P[0] = r.Pw;
+    if constexpr (CLOSURE == 3) {
+#pragma unroll
+        for (int a = 0; a < MODEL; ++a) {
+            c.Xi[a] = r.Xi[a];
+            c.ro[a] = r.ro[a];
+        }
+    } else if constexpr (MODEL == 2) {
+        double mKw, mKn;  // -K k_r
+        if constexpr (CLOSURE >= 1) {
+            const double se = exact_div(1. - r.Sn - p.S_wr, p.den2c, p.r_den2c);
+            mKw = corey_mK<CLOSURE>(p, r.K, se);
+            mKn = corey_mK<CLOSURE>(p, r.K, 1. - se);
+        } else {
+            double kw, kn, Pk;
+            relperm2(p, r.Sn, kw, kn, Pk);
+            mKw = (-1.) * r.K * kw;
+            mKn = (-1.) * r.K * kn;
+            c.P[1] = r.Pw + Pk;
+        }
+        c.Xi[0] = exact_div(mKw, p.mu_w, p.r_mu_w);
+        c.Xi[1] = exact_div(mKn, p.mu_n, p.r_mu_n);
+        c.ro[0] = ro_w_of(p, r.Pw);
+        c.ro[1] = ro_n_of(p, CLOSURE >= 1 ? r.Pw : c.P[kStagedP<MODEL, CLOSURE> - 1]);
+    } else {
+        double mKw, mKn, mKg;  // -K k_r
+        if constexpr (CLOSURE >= 1) {
+            const double Swe = exact_div(r.Sw - p.S_wr, p.den3, p.r_den3);
+            const double Sne = exact_div(r.Sn - p.S_nr, p.den3, p.r_den3);
+            const double Sge = 1. - Swe - Sne;
+            mKw = corey_mK<CLOSURE>(p, r.K, Swe);
+            mKn = corey_mK<CLOSURE>(p, r.K, Sne);
+            mKg = corey_mK<CLOSURE>(p, r.K, Sge);
+        } else {
+            double kw, kn, kg;
+            relperm3(p, r.Sw, r.Sn, kw, kn, kg);
+            mKw = (-1.) * r.K * kw;
+            mKn = (-1.) * r.K * kn;
+            mKg = (-1.) * r.K * kg;
+        }
+        c.Xi[0] = exact_div(mKw, p.mu_w, p.r_mu_w);
+        c.Xi[1] = exact_div(mKn, p.mu_n, p.r_mu_n);
+        c.Xi[2] = exact_div(mKg, p.mu_g, p.r_mu_g);
+        c.ro[0] = ro_w_of(p, r.Pw);
+        c.ro[1] = ro_n_of(p, r.Pw);
+        c.ro[2] = ro_g_of(p, r.Pw);
+    }
+    if constexpr (MODEL == 3) {
+        if (!inner) {
+            if constexpr (CLOSURE != 3) {
+                c.ro[1] = ro_n_of(p, r.Pn);
+                c.ro[2] = ro_g_of(p, r.Pg);
+            }
+            return r.Pn != r.Pw || r.Pg != r.Pw;
+        }
+    }
+    return false;
+}
+
+// The state, the divergence (and, for U, the velocities u[phase][axis]) of an
+// interior cell from memory, every neighbour with its own phase pressures;
+// one axis at a time, for few registers.
+template <int MODEL, int CLOSURE, bool U>
+__device__ __forceinline__ void general_cell(const DevParams& p, const StepIO& io, int i, int j, int k, double* ro,
+                                             double* div, double (&u)[MODEL][3]) {
+    auto at = [&](int ii, int jj, int kk) {
+        return coef_at<MODEL, CLOSURE>(p, io, (int64_t)ii + (int64_t)jj * p.sy + (int64_t)kk * p.sz,
+                                       inner_cell<MODEL>(p, ii, jj, kk));
+    };
+    const CoefT<MODEL> c = at(i, j, k);
+#pragma unroll
+    for (int a = 0; a < MODEL; ++a) ro[a] = c.ro[a];
+    auto axis = [&](bool has, int dx, int dy, int dz, int x, double h, double rh, double h2, double rh2) {
+        if (!has) {
+#pragma unroll
+            for (int a = 0; a < MODEL; ++a) {
+                if (x != 0) div[a] = div[a] + 0.;
+                else div[a] = 0.;
+                u[a][x] = 0.;
+            }
+            return;
+        }
+        const CoefT<MODEL> m = at(i - dx, j - dy, k - dz), q = at(i + dx, j + dy, k + dz);
+#pragma unroll
+        for (int a = 0; a < MODEL; ++a) {
+            double x1 = -1. * exact_div(c.P[a] - m.P[a], h, rh), x2 = -1. * exact_div(q.P[a] - c.P[a], h, rh);
+            if (x == 1) {
+                x1 = x1 + p.g * c.ro[a];
+                x2 = x2 + p.g * c.ro[a];
+            }
+            const double f = directed(x1, x2, c.Xi[a], c.ro[a], m.Xi[a], m.ro[a], q.Xi[a], q.ro[a], h, rh);
+            div[a] = x == 0 ? (a == 2 ? 0. + f : f) : div[a] + f;
+            if (U) {
+                const double d = exact_div(q.P[a] - m.P[a], h2, rh2);
+                u[a][x] = c.Xi[a] * (x == 1 ? d - c.ro[a] * p.g : d);
+            }
+        }
+    };
+    // x, y, z in turn: the order of the sum (cpu.cpp:707-708)
+    axis(p.Nx >= 3, 1, 0, 0, 0, p.hx, p.r_hx, p.two_hx, p.r_two_hx);
+    axis(true, 0, 1, 0, 1, p.hy, p.r_hy, p.two_hy, p.r_two_hy);
+    axis(p.Nz >= 3, 0, 0, 1, 2, p.hz, p.r_hz, p.two_hz, p.r_two_hz);
+}
+
+using LdsDouble = __attribute__((address_space(3))) double*;
+
+// What an epilogue reads of the cell it finishes.
+template <int MODEL>
+struct CellState {
+    double P, Sw, Sn, ro[MODEL];
 };
 
 // One tile of the fused step: interior columns i0 .. i0+TX-1 (i0 = first
 // interior i + TX*bx), j0 .. j0+TY-1 (j0 = 1 + TY*by), planes k0 .. k0+kchunk-1
 // (k0 = first interior k + kchunk*bz), on a TX x TY workgroup (TY >= 3,
-// TX >= 2*TY: rows 0-2 of the workgroup also load the halo ring).
+// TX >= 2*TY: rows 0-2 of the workgroup also load the halo ring; TX 32 or 64,
+// so that a wavefront holds whole rows).
 //
-// CARRY: keep the next plane's coefficients of the own column in registers
-// (computed for the z flux) as the next centre, or recompute the centre at
-// the top of every plane (fewer live registers across the Newton solve).
-// Epi: what happens at an interior cell once its coefficients c and flux
-// divergence div are known -- the Newton solve and store of the step
-// (FusedStore) or the adjoint's backward Newton (AdjNewtonStore).
-template <int MODEL, int CLOSURE, int TX, int TY, bool CARRY, class Epi>
-__device__ __forceinline__ void fused_z_tile(const DevParams& p, const StepIO& io, int kchunk, int bx, int by, int bz,
-                                             FusedLds<3 * MODEL, TX, TY>& lds, const Epi& epi) {
+// What bounds it: VALU issue (FP64).  The 256^3 three-phase Corey-2 step went
+// from 850 to some 660 VALU instructions per cell and from 571 to 488 us, the
+// two-phase one from 336 to 285 us, against the tiles before (two barriers
+// and one LDS buffer per plane, every phase's pressure staged, calls and
+// branches in the Newton, parameters in vector-register lanes).
+//
+// A plane's turn: issue the loads of the next plane (own cell and ring) and
+// of what the epilogue reads; the x and y fluxes of this plane from LDS,
+// which cover those loads; the next plane's coefficients, staged in the
+// other LDS buffer; the z flux; the epilogue; one barrier.  The closures that
+// raise powers (EARLY) take the coefficients first, while few values are
+// live, and read the own ones back from LDS for the z flux.  Across planes a
+// thread keeps two pressure parts, the minus z face's flux terms and its
+// saturations; its own coefficients come back from LDS.
+//
+// FULL: Nx, Ny, Nz >= 3 (no axis tests in the plane's code).
+// Epi: what happens at an interior cell once its state and flux divergence
+// are known -- the Newton solve and store of the step (FusedStore) or the
+// adjoint's backward Newton (AdjNewtonStore).  prefetch() loads what it needs;
+// epi.cell<false> may leave the cell undone and say so (false), epi.cell<true>
+// does every cell.
+//
+// Cells that the planes' code does not cover -- the epilogue left it undone (a
+// pivot search), or an x or z face neighbour has a P_n or P_g that is not its
+// P_w (values a caller set; Border_P gives those faces P_n = P_g = P_w) -- are
+// marked and done after the last plane from the state the step reads, which
+// it does not write: the planes' code then holds no call and no registers for
+// them (kchunk <= kMaxPlanes, one mark per plane).
+// cp: p in constant memory (fresh()).
+constexpr int kMaxPlanes = 32;
+template <int MODEL, int CLOSURE, int TX, int TY, bool FULL, class Epi>
+__device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp, const StepIO& io, int kchunk, int bx, int by, int bz,
+                                             FusedLds<MODEL, CLOSURE, TX, TY>& lds, const Epi& epi) {
     static_assert(TY >= 3 && TX >= 2 * TY, "halo ring needs TY >= 3 and TX >= 2*TY");
-    constexpr int NPH = MODEL;
+    static_assert(TX == 32 || TX == 64, "whole rows per wavefront");
+    constexpr int NPH = MODEL, NPR = kStagedP<MODEL, CLOSURE>, NV = FusedLds<MODEL, CLOSURE, TX, TY>::kNV;
+    constexpr int ROW = (TX + 2) * NV, PLANE = (TY + 2) * ROW;  // LDS pitch of a row, of a plane
+    constexpr bool U = EpiWantsU<Epi>::value;
+    constexpr bool EARLY = CLOSURE == 0 || CLOSURE == 1;
 
     const int tx = threadIdx.x, ty = threadIdx.y;
-    const bool hasx = p.Nx >= 3, hasz = p.Nz >= 3;
+    const bool hasx = FULL || p.Nx >= 3, hasz = FULL || p.Nz >= 3;
     const int ilo = hasx ? 1 : 0, ihi = hasx ? p.Nx - 2 : 0;
     const int klo = hasz ? 1 : 0, khi = hasz ? p.Nz - 2 : 0;
     const int i0 = ilo + TX * bx, j0 = 1 + TY * by;
     const int k0 = klo + kchunk * bz;
     const int k1 = min(khi, k0 + kchunk - 1);
     const int i = i0 + tx, j = j0 + ty;
-    const bool own_in_grid = i < p.Nx && j < p.Ny;
     const bool active = i <= ihi && j <= p.Ny - 2;
+    // the own column, clamped into the grid (lanes past it stage values that
+    // no active lane reads); jw: the wavefront's first row
+    const int ic = min(i, p.Nx - 1), jc = min(j, p.Ny - 1);
+    const int jw = __builtin_amdgcn_readfirstlane(jc);
+    const bool own_ij = inner_ij<MODEL>(p, ic, jc);
+    CellAt own{(int64_t)i0 + (int64_t)jw * p.sy + (int64_t)k0 * p.sz, 8u * (uint32_t)(ic - i0)};
+    if (TX < 64) own.off += 8u * (uint32_t)(jc - jw) * (uint32_t)p.sy;
 
     // This thread's halo cell of each plane, if any (ty 0 / 1: the y rows
     // below / above the block, ty 2: the x columns left / right of it).
@@ -234,141 +551,256 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, const StepIO& i
     else if (ty == 1) { hi = i; hj = j0 + TY; hx = tx + 1; hy = TY + 1; }
     else if (ty == 2 && tx < TY) { hi = i0 - 1; hj = j0 + tx; hx = 0; hy = tx + 1; }
     else if (ty == 2 && tx >= TY && tx < 2 * TY) { hi = i0 + TX; hj = j0 + tx - TY; hx = TX + 1; hy = tx - TY + 1; }
-    const bool halo_in_grid = hi >= 0 && hi < p.Nx && hj >= 0 && hj < p.Ny && (hasx || hi == i0 + tx);
+    const bool halo = hi >= 0 && hi < p.Nx && hj >= 0 && hj < p.Ny && (hasx || hi == i0 + tx);
+    const bool halo_ij = inner_ij<MODEL>(p, hi, hj);
+    int64_t hl = (int64_t)hi + (int64_t)hj * p.sy + (int64_t)k0 * p.sz;
 
-    const int64_t col = (int64_t)i + (int64_t)j * p.sy;
-    const int64_t hcol = (int64_t)hi + (int64_t)hj * p.sy;
-    const bool own_ij = inner_ij<MODEL>(p, i, j), halo_ij = inner_ij<MODEL>(p, hi, hj);
-
-    // The z window: with ZPARTS the minus z face is carried between planes
-    // as its two parts of directed(), zneg = neg_part(x1) and zt2 = t2 (x1 =
-    // -dz; computed from the same operands as at the plane itself, one plane
-    // earlier): two values per phase instead of dz and the plane below's Xi
-    // and ro, and no register copies of those.  That frees registers in the
-    // Corey-2 kernels (the headline's: 543 -> 536 us at 256^3), but adds
-    // spill to the kernels already held to 128 VGPRs (the closures with
-    // powers), which keep dz, Xi and ro.
-    constexpr bool ZPARTS = CLOSURE == 2;
-    CoefT<NPH> zm{}, c{}, zp{};
-    double zneg[NPH], zt2[NPH], dz[NPH];
+    // LDS places in the buffer of plane 0: the own and the halo cell
+    auto buffer = [](int k) { return (k & 1) * PLANE; };
+    const LdsDouble v0 = (LdsDouble)&lds.v[0][ty + 1][tx + 1][0], vh = (LdsDouble)&lds.v[0][hy][hx][0];
+    auto stage = [&](int k, LdsDouble w, int row, int x, int jj, const CellRaw<MODEL, CLOSURE>& r, bool inner,
+                     const CellCoef<MODEL, CLOSURE>& c, bool odd) {
 #pragma unroll
-    for (int a = 0; a < NPH; ++a) zneg[a] = zt2[a] = dz[a] = 0.;
-    if (own_in_grid) {
-        c = coef_at<MODEL, CLOSURE>(p, io, col + (int64_t)k0 * p.sz, own_ij && inner_k(p, k0));
-        if (hasz) {
-            zm = coef_at<MODEL, CLOSURE>(p, io, col + (int64_t)(k0 - 1) * p.sz, own_ij && inner_k(p, k0 - 1));
+        for (int a = 0; a < NPR; ++a) w[a] = c.P[a];
 #pragma unroll
-            for (int a = 0; a < NPH; ++a) {
-                const double d = exact_div(c.P[a] - zm.P[a], p.hz, p.r_hz);
-                if constexpr (ZPARTS) {
-                    zneg[a] = neg_part(-1. * d);
-                    zt2[a] = directed_t2(-1. * d, zm.Xi[a], zm.ro[a]);
-                } else {
-                    dz[a] = d;
+        for (int a = 0; a < NPH; ++a) {
+            w[NPR + a] = c.Xi[a];
+            w[NPR + NPH + a] = c.ro[a];
+        }
+        if constexpr (MODEL == 3) {
+            if (!inner) {
+                if (jj == 0 || jj == p.Ny - 1) {
+                    lds.edge[k & 1][jj == 0 ? 0 : 1][0][x] = r.Pn;
+                    lds.edge[k & 1][jj == 0 ? 0 : 1][1][x] = r.Pg;
+                } else if (odd) {
+                    lds.odd[k & 1][row] = k;
                 }
             }
+        }
+    };
+
+    // the minus z face (directed()'s neg_part(x1) and t2) and the own
+    // saturations, carried from plane to plane
+    double zneg[NPR], zt2[NPH], zmP[NPR], Sw = 0., Sn = 0.;
+    uint64_t zodd = 0;  // the lanes whose cell below (k - 1) has a P_n or P_g of its own
+    uint32_t undone = 0;
+#pragma unroll
+    for (int a = 0; a < NPR; ++a) zneg[a] = zmP[a] = 0.;
+#pragma unroll
+    for (int a = 0; a < NPH; ++a) zt2[a] = 0.;
+    {
+        CellRaw<MODEL, CLOSURE> r, rm, rh;
+        const bool inner = own_ij && inner_k(p, k0), inner_m = own_ij && inner_k(p, k0 - 1);
+        const bool inner_h = halo_ij && inner_k(p, k0);
+        load_raw(io, own, inner, r);
+        if (hasz) load_raw(io, CellAt{own.base - p.sz, own.off}, inner_m, rm);
+        if (halo) load_raw(io, CellIndex{hl}, inner_h, rh);
+        CellCoef<MODEL, CLOSURE> c, m;
+        const DevParams pc = coef_params<MODEL, CLOSURE>(cp);
+        const bool odd = coef_of(pc, r, inner, c);
+        stage(k0, v0 + buffer(k0), ty + 1, tx + 1, jc, r, inner, c, odd);
+        Sn = r.Sn;
+        if constexpr (MODEL == 3) Sw = r.Sw;
+        if (hasz) {
+            zodd = __ballot(coef_of(pc, rm, inner_m, m));
+#pragma unroll
+            for (int a = 0; a < NPR; ++a) {
+                zmP[a] = m.P[a];
+                const double d = exact_div(c.P[a] - m.P[a], p.hz, p.r_hz);
+                zneg[a] = neg_part(-1. * d);
+#pragma unroll
+                for (int b = a; b < (NPR == 1 ? NPH : a + 1); ++b) zt2[b] = directed_t2(-1. * d, m.Xi[b], m.ro[b]);
+            }
+        }
+        if (halo) {
+            const bool oddh = coef_of(pc, rh, inner_h, c);
+            stage(k0, vh + buffer(k0), hy, hx, hj, rh, inner_h, c, oddh);
+        }
+    }
+    __syncthreads();
+
+    for (int k = k0; k <= k1; ++k) {
+        const bool next = k < k1;  // another plane follows in this tile
+        renew(own);
+        CellRaw<MODEL, CLOSURE> r, rh;
+        const bool inner = own_ij && inner_k(p, k + 1), inner_h = halo_ij && inner_k(p, k + 1);
+        if (hasz) load_raw(io, CellAt{own.base + p.sz, own.off}, inner, r);
+        if (next && halo) load_raw(io, CellIndex{hl + p.sz}, inner_h, rh);
+        const auto pre = epi.prefetch(own);
+        // the next plane: coefficients, staged in the other buffer
+        CellCoef<MODEL, CLOSURE> zp;
+        uint64_t odd = 0;
+        auto next_plane = [&]() {
+            const DevParams pc = coef_params<MODEL, CLOSURE>(fresh(cp));
+            if (hasz) {
+                const bool mine = coef_of(pc, r, inner, zp);
+                if constexpr (MODEL == 3) odd = __ballot(mine);
+                if (next || EARLY) stage(k + 1, v0 + buffer(k + 1), ty + 1, tx + 1, jc, r, inner, zp, mine);
+            }
+            if (next && halo) {
+                CellCoef<MODEL, CLOSURE> h;
+                const bool oddh = coef_of(pc, rh, inner_h, h);
+                stage(k + 1, vh + buffer(k + 1), hy, hx, hj, rh, inner_h, h, oddh);
+            }
+        };
+        if constexpr (EARLY) next_plane();
+
+        // the own cell's row and the rows below and above it, from the cell at
+        // x - 1 on; one register each, every value a constant offset away
+        LdsDouble row[3];
+#pragma unroll
+        for (int y = 0; y < 3; ++y) {
+            row[y] = v0 + buffer(k) + (y - 1) * ROW - NV;
+            asm("" : "+v"(row[y]));
+        }
+        auto P_at = [&](int a, int y, int x) { return row[y][x * NV + a]; };
+        auto Xi_at = [&](int a, int y, int x) { return row[y][x * NV + NPR + a]; };
+        auto ro_at = [&](int a, int y, int x) { return row[y][x * NV + NPR + NPH + a]; };
+        double div[NPH], u[NPH][3];
+        CellCoef<MODEL, CLOSURE> c;
+        const DevParams pf = flux_params(fresh(cp));
+        if (active) {
+            // order as cpu.cpp:651-708: z, x, y, then (-q + fx + fy + fz)
+#pragma unroll
+            for (int a = 0; a < NPR; ++a) c.P[a] = P_at(a, 1, 1);
+#pragma unroll
+            for (int a = 0; a < NPH; ++a) {
+                c.Xi[a] = Xi_at(a, 1, 1);
+                c.ro[a] = ro_at(a, 1, 1);
+                div[a] = 0.;
+            }
+            if (hasx) {
+#pragma unroll
+                for (int q = 0; q < NPR; ++q) {
+                    const double Pm = P_at(q, 1, 0), Pp = P_at(q, 1, 2);
+                    const double x1 = -1. * exact_div(c.P[q] - Pm, pf.hx, pf.r_hx);
+                    const double x2 = -1. * exact_div(Pp - c.P[q], pf.hx, pf.r_hx);
+                    const double s1 = (pos_part(x2) - neg_part(x1)) * (-1.), s2 = pos_part(x1) * (-1.),
+                                 s3 = neg_part(x2) * (-1.);
+#pragma unroll
+                    for (int a = q; a < (NPR == 1 ? NPH : q + 1); ++a) {
+                        const double t1 = s1 * c.Xi[a] * c.ro[a];
+                        const double t2 = s2 * Xi_at(a, 1, 0) * ro_at(a, 1, 0);
+                        const double t3 = s3 * Xi_at(a, 1, 2) * ro_at(a, 1, 2);
+                        const double fx = exact_div(t1 - t2 + t3, pf.hx, pf.r_hx);
+                        div[a] = a == 2 ? 0. + fx : fx;
+                        if constexpr (U) u[a][0] = c.Xi[a] * exact_div(Pp - Pm, pf.two_hx, pf.r_two_hx);
+                    }
+                }
+            } else if constexpr (U) {
+#pragma unroll
+                for (int a = 0; a < NPH; ++a) u[a][0] = 0.;
+            }
+            // the x neighbours' values are done with before the y ones are read
+            asm volatile("" ::: "memory");
+            // the face differences dm, dp and their sum's dd of phase a's pressure
+            auto y_flux = [&](int a, double dm, double dp, double dd) {
+                div[a] = div[a] + flux_y(pf, dm, dp, c.Xi[a], c.ro[a], Xi_at(a, 0, 1), ro_at(a, 0, 1), Xi_at(a, 2, 1),
+                                         ro_at(a, 2, 1));
+                if constexpr (U) u[a][1] = c.Xi[a] * (exact_div(dd, pf.two_hy, pf.r_two_hy) - c.ro[a] * pf.g);
+            };
+            // three phases, next to the top and bottom rows: their own P_n and P_g
+            const int jr = TX == 64 ? jw : j;
+            if (MODEL == 3 && (jr == 1 || jr == p.Ny - 2)) {
+#pragma unroll
+                for (int a = 0; a < NPH; ++a) {
+                    double Pm = P_at(0, 0, 1), Pp = P_at(0, 2, 1);
+                    if constexpr (MODEL == 3) {
+                        if (a > 0 && jr == 1) Pm = lds.edge[k & 1][0][a - 1][tx + 1];
+                        if (a > 0 && jr == p.Ny - 2) Pp = lds.edge[k & 1][1][a - 1][tx + 1];
+                    }
+                    y_flux(a, exact_div(c.P[0] - Pm, pf.hy, pf.r_hy), exact_div(Pp - c.P[0], pf.hy, pf.r_hy), Pp - Pm);
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < NPR; ++q) {
+                    const double Pm = P_at(q, 0, 1), Pp = P_at(q, 2, 1);
+                    const double dm = exact_div(c.P[q] - Pm, pf.hy, pf.r_hy), dp = exact_div(Pp - c.P[q], pf.hy, pf.r_hy);
+#pragma unroll
+                    for (int a = q; a < (NPR == 1 ? NPH : q + 1); ++a) y_flux(a, dm, dp, Pp - Pm);
+                }
+            }
+        }
+        if constexpr (!EARLY) next_plane();
+        if constexpr (EARLY) {
+            // own values staged above, read back where they are used
+            const LdsDouble w = v0 + buffer(k + 1);
+#pragma unroll
+            for (int a = 0; a < NPR; ++a) zp.P[a] = w[a];
+#pragma unroll
+            for (int a = 0; a < NPH; ++a) {
+                zp.Xi[a] = w[NPR + a];
+                zp.ro[a] = w[NPR + NPH + a];
+            }
+        }
+        if (active) {
+            if (hasz) {
+#pragma unroll
+                for (int q = 0; q < NPR; ++q) {
+                    const double x2 = -1. * exact_div(zp.P[q] - c.P[q], pf.hz, pf.r_hz);
+                    const double n2 = neg_part(x2), p2 = pos_part(x2);
+                    const double s1 = (p2 - zneg[q]) * (-1.), s3 = n2 * (-1.), s2 = p2 * (-1.);
+#pragma unroll
+                    for (int a = q; a < (NPR == 1 ? NPH : q + 1); ++a) {
+                        const double t1 = s1 * c.Xi[a] * c.ro[a];
+                        const double t3 = s3 * zp.Xi[a] * zp.ro[a];
+                        div[a] = div[a] + exact_div(t1 - zt2[a] + t3, pf.hz, pf.r_hz);
+                        zt2[a] = s2 * c.Xi[a] * c.ro[a];  // the next plane's minus face
+                        if constexpr (U) u[a][2] = c.Xi[a] * exact_div(zp.P[q] - zmP[q], pf.two_hz, pf.r_two_hz);
+                    }
+                    zneg[q] = n2;
+                    if constexpr (U) zmP[q] = c.P[q];
+                }
+            } else {
+#pragma unroll
+                for (int a = 0; a < NPH; ++a) {
+                    div[a] = div[a] + 0.;
+                    if constexpr (U) u[a][2] = 0.;
+                }
+            }
+            CellState<MODEL> s;
+            s.P = c.P[0];
+            s.Sw = Sw;
+            s.Sn = Sn;
+#pragma unroll
+            for (int a = 0; a < NPH; ++a) s.ro[a] = c.ro[a];
+            bool done = true;
+            if constexpr (MODEL == 3) {
+                const uint64_t lane = 1ull << ((ty * TX + tx) & 63);
+                const bool row_odd = lds.odd[k & 1][ty + 1] == k;
+                if (__builtin_expect((zodd | odd) != 0 || __ballot(row_odd) != 0, 0))
+                    done = !row_odd && ((zodd | odd) & lane) == 0;
+            }
+            if (done) {
+                if constexpr (U) epi.store_u(own, u);
+                done = epi.template cell<false>(p, newton_params<MODEL, CLOSURE>(fresh(cp)), i, j, k, own, s, div, pre);
+            }
+            if (__builtin_expect(__ballot(!done) != 0, 0)) {
+                if (!done) undone |= 1u << (k - k0);
+            }
+        }
+        if (next) {
+            zodd = odd;
+            Sn = r.Sn;
+            if constexpr (MODEL == 3) Sw = r.Sw;
+            own.base += p.sz;
+            hl += p.sz;
+            __syncthreads();
         }
     }
 
-    for (int k = k0; k <= k1; ++k) {
-        if (!CARRY && own_in_grid && k != k0)
-            c = coef_at<MODEL, CLOSURE>(p, io, col + (int64_t)k * p.sz, own_ij && inner_k(p, k));
-        // stage plane k: own cell and halo cell
-        if (own_in_grid) {
-#pragma unroll
-            for (int a = 0; a < NPH; ++a) {
-                lds.v[a][ty + 1][tx + 1] = c.P[a];
-                lds.v[NPH + a][ty + 1][tx + 1] = c.Xi[a];
-                lds.v[2 * NPH + a][ty + 1][tx + 1] = c.ro[a];
-            }
-        }
-        if (hi >= 0 && halo_in_grid) {
-            CoefT<NPH> h = coef_at<MODEL, CLOSURE>(p, io, hcol + (int64_t)k * p.sz, halo_ij && inner_k(p, k));
-#pragma unroll
-            for (int a = 0; a < NPH; ++a) {
-                lds.v[a][hy][hx] = h.P[a];
-                lds.v[NPH + a][hy][hx] = h.Xi[a];
-                lds.v[2 * NPH + a][hy][hx] = h.ro[a];
-            }
-        }
-        __syncthreads();
-
-        if (own_in_grid && hasz)
-            zp = coef_at<MODEL, CLOSURE>(p, io, col + (int64_t)(k + 1) * p.sz, own_ij && inner_k(p, k + 1));
-        // the plus z face's difference; the next plane's dz
-        double zd[NPH];
-#pragma unroll
-        for (int a = 0; a < NPH; ++a) zd[a] = hasz ? exact_div(zp.P[a] - c.P[a], p.hz, p.r_hz) : 0.;
-
-        if (active) {
-            const int64_t l = col + (int64_t)k * p.sz;
-            double div[NPH];
-#pragma unroll
-            for (int a = 0; a < NPH; ++a) {
-                // order as cpu.cpp:651-708: z, x, y, then (-q + fx + fy + fz)
-                double fz = 0., fx = 0.;
-                if (hasz) {
-                    if constexpr (ZPARTS)
-                        fz = directed_parts(zneg[a], zt2[a], -1. * zd[a], c.Xi[a], c.ro[a], zp.Xi[a], zp.ro[a], p.hz,
-                                            p.r_hz);
-                    else
-                        fz = flux_x(dz[a], zd[a], c.Xi[a], c.ro[a], zm.Xi[a], zm.ro[a], zp.Xi[a], zp.ro[a], p.hz,
-                                    p.r_hz);
-                }
-                if (hasx) {
-                    const double Pm = lds.v[a][ty + 1][tx], Pp = lds.v[a][ty + 1][tx + 2];
-                    const double dm = exact_div(c.P[a] - Pm, p.hx, p.r_hx);
-                    const double dp = exact_div(Pp - c.P[a], p.hx, p.r_hx);
-                    fx = flux_x(dm, dp, c.Xi[a], c.ro[a], lds.v[NPH + a][ty + 1][tx], lds.v[2 * NPH + a][ty + 1][tx],
-                                lds.v[NPH + a][ty + 1][tx + 2], lds.v[2 * NPH + a][ty + 1][tx + 2], p.hx, p.r_hx);
-                }
-                const double Pm = lds.v[a][ty][tx + 1], Pp = lds.v[a][ty + 2][tx + 1];
-                const double dm = exact_div(c.P[a] - Pm, p.hy, p.r_hy);
-                const double dp = exact_div(Pp - c.P[a], p.hy, p.r_hy);
-                const double fy = flux_y(p, dm, dp, c.Xi[a], c.ro[a], lds.v[NPH + a][ty][tx + 1],
-                                         lds.v[2 * NPH + a][ty][tx + 1], lds.v[NPH + a][ty + 2][tx + 1],
-                                         lds.v[2 * NPH + a][ty + 2][tx + 1]);
-                double s = (a == 2 ? 0. + fx : fx) + fy;
-                div[a] = s + fz;
-            }
-            // the plus z face's parts, the next plane's minus face's (only
-            // active cells read them)
-            if constexpr (ZPARTS) {
-#pragma unroll
-                for (int a = 0; a < NPH; ++a) {
-                    zneg[a] = neg_part(-1. * zd[a]);
-                    zt2[a] = directed_t2(-1. * zd[a], c.Xi[a], c.ro[a]);
-                }
-            }
-            if constexpr (EpiWantsU<Epi>::value) {
-                // interior cell: central differences on every axis longer than 2
-                double u[NPH][3];
-#pragma unroll
-                for (int a = 0; a < NPH; ++a) {
-                    u[a][0] = hasx ? c.Xi[a] * exact_div(lds.v[a][ty + 1][tx + 2] - lds.v[a][ty + 1][tx], p.two_hx,
-                                                         p.r_two_hx)
-                                   : 0.;
-                    u[a][1] = c.Xi[a] * (exact_div(lds.v[a][ty + 2][tx + 1] - lds.v[a][ty][tx + 1], p.two_hy,
-                                                   p.r_two_hy) -
-                                         c.ro[a] * p.g);
-                    u[a][2] = hasz ? c.Xi[a] * exact_div(zp.P[a] - zm.P[a], p.two_hz, p.r_two_hz) : 0.;
-                }
-                epi.store_u(l, u);
-            }
-            epi(p, i, j, k, l, c, div);
-        }
-        __syncthreads();
-        // roll the z window
-#pragma unroll
-        for (int a = 0; a < NPH; ++a) {
-            if constexpr (!ZPARTS) {
-                dz[a] = zd[a];
-                zm.Xi[a] = c.Xi[a];
-                zm.ro[a] = c.ro[a];
-            }
-            if constexpr (EpiWantsU<Epi>::value) zm.P[a] = c.P[a];
-        }
-        if (CARRY) c = zp;
+    while (__builtin_expect(undone != 0, 0)) {
+        const int k = k0 + __ffs(undone) - 1;
+        undone &= undone - 1;
+        const CellIndex at{(int64_t)i + (int64_t)j * p.sy + (int64_t)k * p.sz};
+        CellState<MODEL> s;
+        s.P = ld(io.Pw, at);
+        s.Sn = ld(io.Sn, at);
+        s.Sw = MODEL == 3 ? ld(io.Sw, at) : 0.;
+        double div[NPH], u[NPH][3];
+        general_cell<MODEL, CLOSURE, U>(p, io, i, j, k, s.ro, div, u);
+        if constexpr (U) epi.store_u(at, u);
+        epi.template cell<true>(p, p, i, j, k, at, s, div, epi.prefetch(at));
     }
 }
 
@@ -394,7 +826,7 @@ __device__ __forceinline__ void xcd_tile(int& bx, int& by, int& bz) {
 // values k_fused_faces would write.
 template <int MODEL>
 __device__ __forceinline__ void store_faces(const DevParams& p, const StepIO& io, int i, int j, int k, int64_t l,
-                                            const CoefT<MODEL>& c, double Pw, double Sw, double Sn) {
+                                            const double* ro, double Pw, double Sw, double Sn) {
     const bool hasx = p.Nx >= 3, hasz = p.Nz >= 3;
     const bool xl = hasx && i == 1, xh = hasx && i == p.Nx - 2;
     const bool yl = j == 1, yh = j == p.Ny - 2;
@@ -404,7 +836,7 @@ __device__ __forceinline__ void store_faces(const DevParams& p, const StepIO& io
     if constexpr (MODEL == 2) {
         // ro_eff_gdy (main.cpp:255-267) for the bottom face: this step's
         // densities of the cell (from its previous state), its new saturation
-        if (yh) ro_eff = (c.ro[1] * Sn + c.ro[0] * (1 - Sn)) * io.m[l] * p.g * p.hy;
+        if (yh) ro_eff = (ro[1] * Sn + ro[0] * (1 - Sn)) * io.m[l] * p.g * p.hy;
     }
     int xo[3] = {0, 0, 0}, yo[3] = {0, 0, 0}, zo[3] = {0, 0, 0};
     int nx = 1, ny = 1, nz = 1;
@@ -430,28 +862,42 @@ __device__ __forceinline__ void store_faces(const DevParams& p, const StepIO& io
 template <int MODEL, bool FACES = false, int CLOSURE = -1>
 struct FusedStore {
     StepIO io;
-    __device__ __forceinline__ void operator()(const DevParams& p, int i, int j, int k, int64_t l,
-                                               const CoefT<MODEL>& c, const double* div) const {
+    // dt / m, computed once per porosity field
+    template <class At>
+    __device__ __forceinline__ double prefetch(const At& at) const { return ld(io.dtm, at); }
+    template <bool GENERAL, class At>
+    __device__ __forceinline__ bool cell(const DevParams& p, const DevParams& pn, int i, int j, int k, const At& at,
+                                         const CellState<MODEL>& s, const double* div, double dtm) const {
         (void)i; (void)j; (void)k;
-        const double dtm = io.dtm[l];  // dt / m, computed once per porosity field
-        double Pw = c.P[0], Sn = c.Sn, Sw = c.Sw;
+        double Pw = s.P, Sn = s.Sn, Sw = s.Sw;
         if constexpr (MODEL == 2) {
-            const double A1 = c.ro[0] * (1. - Sn) - dtm * div[0];
-            const double A2 = c.ro[1] * Sn - dtm * div[1];
-            newton2<CLOSURE>(p, Pw, Sn, A1, A2);
-            io.Pw1[l] = Pw;
-            io.Sn1[l] = Sn;
-            if constexpr (FACES) store_faces<2>(p, io, i, j, k, l, c, Pw, 0., Sn);
+            const double A1 = s.ro[0] * (1. - Sn) - dtm * div[0];
+            const double A2 = s.ro[1] * Sn - dtm * div[1];
+            if constexpr (GENERAL)
+                newton2_ieee<CLOSURE>(pn, Pw, Sn, A1, A2);
+            else if (!newton2_fast<CLOSURE>(pn, Pw, Sn, A1, A2))
+                return false;
+            At to = at;
+            renew(to);
+            st(io.Pw1, to, Pw);
+            st(io.Sn1, to, Sn);
+            if constexpr (FACES) store_faces<2>(p, io, i, j, k, at.l(), s.ro, Pw, 0., Sn);
         } else {
-            const double A1 = c.ro[0] * Sw - dtm * div[0];
-            const double A2 = c.ro[1] * Sn - dtm * div[1];
-            const double A3 = c.ro[2] * (1. - Sw - Sn) - dtm * div[2];
-            newton3(p, Pw, Sw, Sn, A1, A2, A3);
-            io.Pw1[l] = Pw;
-            io.Sw1[l] = Sw;
-            io.Sn1[l] = Sn;
-            if constexpr (FACES) store_faces<3>(p, io, i, j, k, l, c, Pw, Sw, Sn);
+            const double A1 = s.ro[0] * Sw - dtm * div[0];
+            const double A2 = s.ro[1] * Sn - dtm * div[1];
+            const double A3 = s.ro[2] * (1. - Sw - Sn) - dtm * div[2];
+            if constexpr (GENERAL)
+                newton3_general(pn, Pw, Sw, Sn, A1, A2, A3);
+            else if (!newton3_fast(pn, Pw, Sw, Sn, A1, A2, A3))
+                return false;
+            At to = at;
+            renew(to);
+            st(io.Pw1, to, Pw);
+            st(io.Sw1, to, Sw);
+            st(io.Sn1, to, Sn);
+            if constexpr (FACES) store_faces<3>(p, io, i, j, k, at.l(), s.ro, Pw, Sw, Sn);
         }
+        return true;
     }
 };
 
@@ -467,11 +913,16 @@ struct FusedStoreRecord {
     FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE> step;
     double* div;
     int64_t stride;
-    __device__ __forceinline__ void operator()(const DevParams& p, int i, int j, int k, int64_t l,
-                                               const CoefT<MODEL>& c, const double* d) const {
+    template <class At>
+    __device__ __forceinline__ double prefetch(const At& at) const { return step.prefetch(at); }
+    template <bool GENERAL, class At>
+    __device__ __forceinline__ bool cell(const DevParams& p, const DevParams& pn, int i, int j, int k, const At& at,
+                                         const CellState<MODEL>& s, const double* d, double dtm) const {
+        At to = at;
+        renew(to);
 #pragma unroll
-        for (int a = 0; a < MODEL; ++a) div[a * stride + l] = d[a];
-        step(p, i, j, k, l, c, d);
+        for (int a = 0; a < MODEL; ++a) st(div + a * stride, to, d[a]);
+        return step.template cell<GENERAL>(p, pn, i, j, k, at, s, d, dtm);
     }
 };
 
@@ -485,31 +936,39 @@ struct RoSStore {
     const double* dtm;
     double *roS[3], *roS_old[3];
     double* u[3][3];  // [phase][axis]: ux_w, uy_w, uz_w, ux_n, ... (U only)
-    __device__ __forceinline__ void store_u(int64_t l, const double (&v)[3][3]) const {
+    template <class At>
+    __device__ __forceinline__ double prefetch(const At& at) const { return ld(dtm, at); }
+    template <class At>
+    __device__ __forceinline__ void store_u(const At& at, const double (&v)[3][3]) const {
+        At to = at;
+        renew(to);
 #pragma unroll
         for (int a = 0; a < 3; ++a)
 #pragma unroll
-            for (int x = 0; x < 3; ++x) u[a][x][l] = v[a][x];
+            for (int x = 0; x < 3; ++x) st(u[a][x], to, v[a][x]);
     }
-    __device__ __forceinline__ void operator()(const DevParams& p, int i, int j, int k, int64_t l,
-                                               const CoefT<3>& c, const double* div) const {
-        (void)p; (void)i; (void)j; (void)k;
-        const double old[3] = {c.ro[0] * c.Sw, c.ro[1] * c.Sn, c.ro[2] * (1. - c.Sw - c.Sn)};
-        const double d = dtm[l];
+    template <bool GENERAL, class At>
+    __device__ __forceinline__ bool cell(const DevParams& p, const DevParams& pn, int i, int j, int k, const At& at,
+                                         const CellState<3>& s, const double* div, double d) const {
+        (void)p; (void)pn; (void)i; (void)j; (void)k;
+        const double old[3] = {s.ro[0] * s.Sw, s.ro[1] * s.Sn, s.ro[2] * (1. - s.Sw - s.Sn)};
+        At to = at;
+        renew(to);
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            roS_old[a][l] = old[a];
-            roS[a][l] = old[a] - d * div[a];
+            st(roS_old[a], to, old[a]);
+            st(roS[a], to, old[a] - d * div[a]);
         }
+        return true;
     }
 };
 
-template <int TX, int TY, bool CARRY, bool U>
+template <int TX, int TY, bool FULL, bool U>
 __global__ void __launch_bounds__(TX * TY) k_roS_z(DevParams p, StepIO io, int kchunk, RoSStore<U> st) {
-    __shared__ FusedLds<9, TX, TY> lds;
+    __shared__ FusedLds<3, 3, TX, TY> lds;
     int bx, by, bz;
     xcd_tile(bx, by, bz);
-    fused_z_tile<3, 3, TX, TY, CARRY>(p, io, kchunk, bx, by, bz, lds, st);
+    fused_z_tile<3, 3, TX, TY, FULL>(p, kernel_params(), io, kchunk, bx, by, bz, lds, st);
 }
 
 // The energy step's E pass (assign_E_new, energy.cpp:235-340, as body_E_with)
@@ -644,41 +1103,37 @@ __global__ void __launch_bounds__(TX * TY) k_energy_e_z(DevParams p, EnergyEIO a
     }
 }
 
-template <int MODEL, int CLOSURE, int TX, int TY, bool CARRY>
+template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
 __global__ void __launch_bounds__(TX * TY) k_fused_z_record(DevParams p, StepIO io, int kchunk, double* div,
                                                            int64_t stride) {
-    __shared__ FusedLds<3 * MODEL, TX, TY> lds;
+    __shared__ FusedLds<MODEL, CLOSURE, TX, TY> lds;
     int bx, by, bz;
     xcd_tile(bx, by, bz);
-    fused_z_tile<MODEL, CLOSURE, TX, TY, CARRY>(p, io, kchunk, bx, by, bz, lds,
-                                                FusedStoreRecord<MODEL, CLOSURE>{
-                                                    FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE>{io}, div, stride});
+    fused_z_tile<MODEL, CLOSURE, TX, TY, FULL>(p, kernel_params(), io, kchunk, bx, by, bz, lds,
+                                               FusedStoreRecord<MODEL, CLOSURE>{
+                                                   FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE>{io}, div, stride});
 }
 
-
-// Occupancy bound: the kernels with a closure that raises powers (the
-// reference's van Genuchten or Brooks-Corey k_r, a Corey exponent read at run
-// time) need 130-160 VGPRs, which leaves one 512-thread workgroup per CU; held
-// to 128 (4 waves per SIMD) they spill at most some 32 VGPRs and still run
-// faster (the reference's three-phase deck at 256^3: 1.76 against 1.84 ms per
-// step).
-template <int MODEL, int CLOSURE>
-constexpr int kFusedWaves = CLOSURE == 0 || CLOSURE == 1 ? 4 : 1;
-// The two-phase Corey-2 tiles of 64 x 4 (256 threads) fit in 94 VGPRs
-// without a spill at 5 waves per SIMD: 330 us per step at 256^3 against 374
-// for 64 x 8 tiles at 4 (the automatic tile_y of that step).  The
-// three-phase ones would spill 28 VGPRs there and take 871 us against 543.
+// Waves per SIMD and the automatic tile height.  Measured on one MI355X, us per
+// step: three-phase Corey-2 (256^3) 64 x 8 at 4 waves (128 VGPRs, a few spilled)
+// 488, 64 x 4 (whose two LDS buffers leave 3 workgroups per CU) 515; two-phase
+// Corey-2 (256^3) 64 x 4 at 5 waves (95 VGPRs) 285, 64 x 8 at 4 296; the
+// closures that raise powers want registers more than waves: van Genuchten
+// (160 x 144 x 130) 64 x 4 at 3 waves (168 VGPRs) 322, 64 x 8 at 4 waves
+// (128, ~90 spilled) 400; Brooks-Corey (190 x 150 x 110) 235 against 267.
 template <int MODEL, int CLOSURE, int TY>
-constexpr int kFusedWavesTY = MODEL == 2 && CLOSURE == 2 && TY == 4 ? 5 : kFusedWaves<MODEL, CLOSURE>;
+constexpr int kFusedWaves = CLOSURE == 2 ? (MODEL == 2 ? (TY == 4 ? 5 : 4) : (TY == 4 ? 3 : 4)) : (TY == 4 ? 3 : 4);
+template <int MODEL, int CLOSURE>
+constexpr int kFusedTileY = MODEL == 3 && CLOSURE == 2 ? 8 : 4;
 
-template <int MODEL, int CLOSURE, int TX, int TY, bool CARRY>
-__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(kFusedWavesTY<MODEL, CLOSURE, TY>)))
+template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
+__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(kFusedWaves<MODEL, CLOSURE, TY>)))
 k_fused_z(DevParams p, StepIO io, int kchunk) {
-    __shared__ FusedLds<3 * MODEL, TX, TY> lds;
+    __shared__ FusedLds<MODEL, CLOSURE, TX, TY> lds;
     int bx, by, bz;
     xcd_tile(bx, by, bz);
-    fused_z_tile<MODEL, CLOSURE, TX, TY, CARRY>(p, io, kchunk, bx, by, bz, lds,
-                                                FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE>{io});
+    fused_z_tile<MODEL, CLOSURE, TX, TY, FULL>(p, kernel_params(), io, kchunk, bx, by, bz, lds,
+                                               FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE>{io});
 }
 
 // Cell number t of a box of ni x nj cells per plane starting at (i0, j0, k0),

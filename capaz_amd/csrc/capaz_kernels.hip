@@ -286,14 +286,17 @@ int resident_groups(int threads) {
 }
 
 int fused_kchunk(const DevParams& p, int kchunk, int ty, int resident) {
-    if (kchunk >= 1) return kchunk;
+    if (kchunk >= 1) return std::min(kchunk, kMaxPlanes);
     // automatic: the planes per tile that minimise (rounds of resident
-    // workgroups) x (planes per tile + the tile's extra coefficient planes)
+    // workgroups) x (planes per tile + the tile's extra coefficient planes).
+    // One plane is worth it where the workgroups then still fit at once: a
+    // 24^3 three-phase step takes 12.7 us against 15.9 with two (40^3 two
+    // phases: 7.4 against 8.5), each plane's latency being a quarter of that.
     const int64_t nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
     const int64_t txy = ((nx + 63) / 64) * ((ny + ty - 1) / ty);
     int best = 16;
     double best_cost = -1.;
-    for (int kc = 2; kc <= 16; ++kc) {
+    for (int kc = 1; kc <= 16; ++kc) {
         const int64_t groups = txy * ((nz + kc - 1) / kc);
         const int64_t rounds = (groups + resident - 1) / resident;
         const double cost = (double)rounds * (std::min<int64_t>(kc, nz) + 0.5);
@@ -324,10 +327,10 @@ hipError_t launch_pack_model(const DevParams& p, const StepIO& io, hipStream_t s
     return launch_pack<MODEL, 1>(p, io, s);
 }
 
-template <int MODEL, int CLOSURE, int TY, bool CARRY>
+template <int MODEL, int CLOSURE, int TY, bool FULL>
 hipError_t launch_z(const DevParams& p, const StepIO& io, int kchunk, hipStream_t s, const KernelEvents* ev) {
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
-    constexpr auto kernel = k_fused_z<MODEL, CLOSURE, 64, TY, CARRY>;
+    constexpr auto kernel = k_fused_z<MODEL, CLOSURE, 64, TY, FULL>;
     kchunk = fused_kchunk(p, kchunk, TY, resident_groups<kernel>(64 * TY));
     dim3 grid((nx + 63) / 64, (ny + TY - 1) / TY, (nz + kchunk - 1) / kchunk);
     hipError_t e;
@@ -349,14 +352,13 @@ hipError_t launch_z(const DevParams& p, const StepIO& io, int kchunk, hipStream_
 
 template <int MODEL, int CLOSURE>
 hipError_t launch_z_ty(const DevParams& p, const StepIO& io, const Tuning& t, hipStream_t s, const KernelEvents* ev) {
-    const bool carry = t.fused_kernel == 1;
-    // tile_y 0: 64 x 4 tiles for the two-phase Corey-2 step, 64 x 8 otherwise
-    const int ty = t.tile_y ? t.tile_y : (MODEL == 2 && CLOSURE == 2 ? 4 : 8);
+    const bool full = p.Nx >= 3 && p.Nz >= 3;
+    const int ty = t.tile_y ? t.tile_y : kFusedTileY<MODEL, CLOSURE>;
     if (ty == 8)
-        return carry ? launch_z<MODEL, CLOSURE, 8, true>(p, io, t.kchunk, s, ev)
-                     : launch_z<MODEL, CLOSURE, 8, false>(p, io, t.kchunk, s, ev);
-    return carry ? launch_z<MODEL, CLOSURE, 4, true>(p, io, t.kchunk, s, ev)
-                 : launch_z<MODEL, CLOSURE, 4, false>(p, io, t.kchunk, s, ev);
+        return full ? launch_z<MODEL, CLOSURE, 8, true>(p, io, t.kchunk, s, ev)
+                    : launch_z<MODEL, CLOSURE, 8, false>(p, io, t.kchunk, s, ev);
+    return full ? launch_z<MODEL, CLOSURE, 4, true>(p, io, t.kchunk, s, ev)
+                : launch_z<MODEL, CLOSURE, 4, false>(p, io, t.kchunk, s, ev);
 }
 
 // CLOSURE ids of the fused kernels: 0 reference, 1 Corey with a run-time
@@ -379,42 +381,37 @@ hipError_t launch_fused(const DevParams& p, const StepIO& io, const Tuning& t, h
     return p.model == 3 ? launch_z_model<3>(p, io, t, s, ev) : launch_z_model<2>(p, io, t, s, ev);
 }
 
+template <int MODEL, int CLOSURE, bool FULL>
+hipError_t launch_record(const DevParams& p, const StepIO& io, int kchunk, double* div, int64_t stride,
+                         hipStream_t s) {
+    const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
+    constexpr auto kernel = k_fused_z_record<MODEL, CLOSURE, 64, 8, FULL>;
+    kchunk = fused_kchunk(p, kchunk, 8, resident_groups<kernel>(512));
+    dim3 grid((nx + 63) / 64, (ny + 7) / 8, (nz + kchunk - 1) / kchunk);
+    hipLaunchKernelGGL(kernel, grid, dim3(64, 8), 0, s, p, io, kchunk, div, stride);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || kFusedFaces<MODEL>) return e;  // two phases: the tiles write the boundary cells
+    hipLaunchKernelGGL((k_fused_faces<MODEL, CLOSURE>), grid_for(fused_face_cells(p)), dim3(256), 0, s, p, io);
+    return hipGetLastError();
+}
+template <int MODEL, int CLOSURE>
+hipError_t launch_record_full(const DevParams& p, const StepIO& io, int kchunk, double* div, int64_t stride,
+                              hipStream_t s) {
+    return p.Nx >= 3 && p.Nz >= 3 ? launch_record<MODEL, CLOSURE, true>(p, io, kchunk, div, stride, s)
+                                  : launch_record<MODEL, CLOSURE, false>(p, io, kchunk, div, stride, s);
+}
+
 hipError_t launch_fused_record(const DevParams& p, const StepIO& io, int kchunk, double* div, int64_t stride,
                                hipStream_t s) {
-    const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
     if (p.model == 2) {
-        // the Corey closures; the tiles write the boundary cells
-        if (p.closure == 0) return hipErrorInvalidValue;
-        kchunk = fused_kchunk(p, kchunk, 8, resident_groups<k_fused_z_record<2, 2, 64, 8, true>>(512));
-        dim3 grid2((nx + 63) / 64, (ny + 7) / 8, (nz + kchunk - 1) / kchunk);
-        if (p.corey_n == 2.)
-            hipLaunchKernelGGL((k_fused_z_record<2, 2, 64, 8, true>), grid2, dim3(64, 8), 0, s, p, io, kchunk, div,
-                               stride);
-        else
-            hipLaunchKernelGGL((k_fused_z_record<2, 1, 64, 8, true>), grid2, dim3(64, 8), 0, s, p, io, kchunk, div,
-                               stride);
-        return hipGetLastError();
+        if (p.closure == 0) return hipErrorInvalidValue;  // the Corey closures
+        return p.corey_n == 2. ? launch_record_full<2, 2>(p, io, kchunk, div, stride, s)
+                               : launch_record_full<2, 1>(p, io, kchunk, div, stride, s);
     }
     if (p.model != 3) return hipErrorInvalidValue;
-    kchunk = fused_kchunk(p, kchunk, 8, resident_groups<k_fused_z_record<3, 2, 64, 8, true>>(512));
-    dim3 grid((nx + 63) / 64, (ny + 7) / 8, (nz + kchunk - 1) / kchunk);
-    if (p.closure == 0) {
-        hipLaunchKernelGGL((k_fused_z_record<3, 0, 64, 8, true>), grid, dim3(64, 8), 0, s, p, io, kchunk, div, stride);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((k_fused_faces<3, 0>), grid_for(fused_face_cells(p)), dim3(256), 0, s, p, io);
-    } else if (p.corey_n == 2.) {
-        hipLaunchKernelGGL((k_fused_z_record<3, 2, 64, 8, true>), grid, dim3(64, 8), 0, s, p, io, kchunk, div, stride);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((k_fused_faces<3, 2>), grid_for(fused_face_cells(p)), dim3(256), 0, s, p, io);
-    } else {
-        hipLaunchKernelGGL((k_fused_z_record<3, 1, 64, 8, true>), grid, dim3(64, 8), 0, s, p, io, kchunk, div, stride);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((k_fused_faces<3, 1>), grid_for(fused_face_cells(p)), dim3(256), 0, s, p, io);
-    }
-    return hipGetLastError();
+    if (p.closure == 0) return launch_record_full<3, 0>(p, io, kchunk, div, stride, s);
+    return p.corey_n == 2. ? launch_record_full<3, 2>(p, io, kchunk, div, stride, s)
+                           : launch_record_full<3, 1>(p, io, kchunk, div, stride, s);
 }
 
 // roS (and, with U, u) of the interior cells on the z tiles, from the P, Xi
@@ -443,10 +440,14 @@ hipError_t launch_roS_tiles(const DevParams& p, const DevFields& F, const double
         for (int x = 0; x < 3; ++x) st.u[a][x] = U ? F.f[uf[a][x]] : nullptr;
     }
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
-    const int kchunk = fused_kchunk(p, 0, 8, resident_groups<k_roS_z<64, 8, true, U>>(512));
-    dim3 grid((nx + 63) / 64, (ny + 7) / 8, (nz + kchunk - 1) / kchunk);
-    hipLaunchKernelGGL((k_roS_z<64, 8, true, U>), grid, dim3(64, 8), 0, s, p, io, kchunk, st);
-    return hipGetLastError();
+    auto launch = [&](auto full) {
+        constexpr auto kernel = k_roS_z<64, 8, decltype(full)::value, U>;
+        const int kchunk = fused_kchunk(p, 0, 8, resident_groups<kernel>(512));
+        dim3 grid((nx + 63) / 64, (ny + 7) / 8, (nz + kchunk - 1) / kchunk);
+        hipLaunchKernelGGL(kernel, grid, dim3(64, 8), 0, s, p, io, kchunk, st);
+        return hipGetLastError();
+    };
+    return p.Nx >= 3 && p.Nz >= 3 ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
 // E_new of the interior cells on the z tiles; lam: the step's stored

@@ -10,10 +10,8 @@ namespace capaz {
 enum class Entry { S, P_Xi_ro, U, RoS, HE, E, Newton, Boundary };
 
 // Launch shape of the fused step: fused_kernel 0 = one thread per cell
-// (k_fused_step), 1 = z-marching tiles (k_fused_z) of 64 x tile_y columns
-// and kchunk planes per workgroup (0: chosen from the grid) that carry the
-// next plane's coefficients in registers, 2 = the same tiles recomputing
-// them per plane.
+// (k_fused_step), 1 and 2 = z-marching tiles (k_fused_z) of 64 x tile_y
+// columns and kchunk planes per workgroup (0: chosen from the grid).
 // adjoint_kernel: 2 = the backward Newton per cell from the flux divergence
 // recorded by the segment's forward recompute, then the coefficient pass per
 // cell; 1 = both passes on the z-marching LDS tiles; 0 = both per cell,
@@ -32,7 +30,7 @@ enum class Entry { S, P_Xi_ro, U, RoS, HE, E, Newton, Boundary };
 struct Tuning {
     int check_every = 0;  // non-finite sentinel after every check_every-th step (0: off)
     int fused_kernel = 1;
-    int tile_y = 0;  // 0: automatic (4 for the two-phase Corey-2 step, else 8)
+    int tile_y = 0;  // 0: automatic (kFusedTileY: 8 for the three-phase Corey-2 step, else 4)
     int kchunk = 0;
     int adjoint_kernel = 2;
     int adjoint_streams = 2;

@@ -187,11 +187,12 @@ int capaz_step(capaz_ctx* ctx, long first_step, long nsteps);
 
 /* Launch shape of capaz_step's kernels (does not change results):
  *   "fused_kernel"  0: one thread per cell; 1: z-marching 64 x tile_y tiles
- *                   with the plane's coefficients staged in LDS (default);
- *                   2: as 1, recomputing the centre coefficients per plane
- *   "tile_y"        0, 4 or 8 (default 0: 4 for the two-phase Corey-2 step, 8 otherwise)
- *   "kchunk"        planes per workgroup along z; 0 (default): chosen from
- *                   the grid (16 on large grids, fewer on small ones)
+ *                   with two planes' coefficients staged in LDS (default);
+ *                   2: as 1
+ *   "tile_y"        0, 4 or 8 (default 0: 8 for the three-phase Corey-2 step, 4 otherwise)
+ *   "kchunk"        planes per workgroup along z (above 32: 32); 0 (default):
+ *                   chosen from the grid (16 on large grids, fewer on small
+ *                   ones)
  *   "adjoint_kernel" capaz_adjoint's passes: 2 (default) the backward
  *                   Newton from the flux divergence recorded while each
  *                   segment is recomputed; 1 both passes on z-marching LDS
@@ -406,7 +407,7 @@ int capaz_batch_domain(capaz_batch* b, int r, capaz_ctx** ctx);
 int capaz_batch_step(capaz_batch* b, long first_step, long nsteps);
 /* Launch shape (results do not change):
  *   "tile_x", "tile_y"  interior tile: 64x8 (default), 64x4 or 32x8 columns
- *   "kchunk"            planes per tile (default 16)
+ *   "kchunk"            planes per tile (default 16; above 32: 32)
  *   "persistent"        1: a resident grid taking tiles from a queue
  *                       (default); 0: one workgroup per tile
  *   "graph"             1: capture each run of steps as a HIP graph (default) */

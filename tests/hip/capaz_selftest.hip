@@ -42,6 +42,18 @@ __global__ void k_rcp(uint64_t n, uint64_t seed, int emin, int emax, unsigned lo
     if (local) atomicAdd(bad, local);
 }
 
+__global__ void k_rcp_in_range(uint64_t n, uint64_t seed, int emin, int emax, unsigned long long* bad) {
+    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    unsigned long long local = 0;
+    for (; i < n; i += stride) {
+        double b = draw(seed, i, emin, emax);
+        double want = 1. / b, got = capaz::rcp_in_range(b);
+        if (__double_as_longlong(want) != __double_as_longlong(got)) ++local;
+    }
+    if (local) atomicAdd(bad, local);
+}
+
 __global__ void k_div(uint64_t n, uint64_t seed, int emin, int emax, unsigned long long* bad) {
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -127,14 +139,17 @@ int capaz_selftest_pow(const double* x, double e, double* y, unsigned long long 
     return rc;
 }
 
-// Number of draws where rcp_rn(b) != 1.0/b (which = 0) or
-// exact_div(a, b, rcp_rn(b)) != a/b (which = 1); -1 on a HIP error.
+// Number of draws where rcp_rn(b) != 1.0/b (which = 0),
+// exact_div(a, b, rcp_rn(b)) != a/b (which = 1) or rcp_in_range(b) != 1.0/b
+// (which = 2); -1 on a HIP error.
 long long capaz_selftest(int which, unsigned long long n, unsigned long long seed, int emin, int emax) {
     unsigned long long* d = nullptr;
     if (hipMalloc(&d, sizeof(*d)) != hipSuccess) return -1;
     if (hipMemset(d, 0, sizeof(*d)) != hipSuccess) return -1;
     if (which == 0)
         hipLaunchKernelGGL(k_rcp, dim3(4096), dim3(256), 0, 0, (uint64_t)n, (uint64_t)seed, emin, emax, d);
+    else if (which == 2)
+        hipLaunchKernelGGL(k_rcp_in_range, dim3(4096), dim3(256), 0, 0, (uint64_t)n, (uint64_t)seed, emin, emax, d);
     else
         hipLaunchKernelGGL(k_div, dim3(4096), dim3(256), 0, 0, (uint64_t)n, (uint64_t)seed, emin, emax, d);
     unsigned long long h = 0;

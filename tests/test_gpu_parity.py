@@ -191,6 +191,42 @@ def test_every_launch_shape_gives_the_same_bits(model, over):
             assert bit_equal(base[f], want[f]), f"{f}: max rel {max_rel(base[f], want[f]):.3e} against the oracle"
 
 
+@pytest.mark.parametrize("dims,tune", [((70, 13, 11), dict()), ((64, 10, 3), dict(tile_y=8)), ((3, 3, 3), dict()),
+                                       ((66, 9, 50), dict(kchunk=64)), ((129, 11, 6), dict(tile_y=4, kchunk=2)),
+                                       ((1, 21, 9), dict()), ((68, 6, 1), dict())])
+@pytest.mark.parametrize("closure", ["corey", "reference"])
+def test_tile_cells_done_after_the_planes(dims, tune, closure):
+    """The cells that a tile leaves for after its planes: next to x and z faces
+    whose P_n and P_g are not their P_w (in a part of the faces only), and
+    where the Newton needs the pivot search (S_w near zero in some cells).
+    Every field as from the kernel with one thread per cell, after 1 and 3
+    steps."""
+    keys = case("3ph", *dims, DT=1e-5, SOURCE=1, CLOSURE=closure)
+    if closure == "corey":
+        keys.update(BETA_W=4.5e-10, S_WR_0=0.0, S_NR_0=0.0)
+    st = random_state(keys, seed=sum(dims))
+    nz, ny, nx = st["P_w"].shape
+    rng = np.random.default_rng(sum(dims) + 1)
+    own = rng.random((nz, ny, nx)) < 0.3
+    for f in ("P_n", "P_g"):
+        st[f] = np.where(own, st["P_w"] + rng.uniform(-20, 20, own.shape), st["P_w"])
+    if closure == "corey":
+        st["S_w"] = np.where(rng.random(own.shape) < 0.2, 0.01, st["S_w"])
+    got = []
+    for t in (tune, dict(fused_kernel=0)):
+        d = capaz.Domain(keys, st)
+        d.tune(**t)
+        d.run(1)
+        one = d.fields()
+        d.run(2, first_step=2)
+        got.append((one, d.fields()))
+        d.close()
+    for a, b in zip(*got):
+        for f in b:
+            assert bit_equal(a[f], b[f]), f
+        assert np.isfinite(b["P_w"]).all()
+
+
 def test_headline_physics_bitwise_at_96():
     """The benchmark physics (three-phase, Corey-2, lognormal K, top
     injection) at 96^3: one and three fused steps equal the oracle bit for bit."""

@@ -30,6 +30,12 @@ def test_rcp_rn_is_correctly_rounded(emin, emax):
     assert selftest(0, 1 << 30, 12345 + emin, emin, emax) == 0
 
 
+@pytest.mark.parametrize("emin,emax", [(-27, 999), (-1000, 999), (-3, 3)])
+def test_rcp_in_range_is_correctly_rounded(emin, emax):
+    """The hot Newton's reciprocal, one cubic step after the hardware's estimate."""
+    assert selftest(2, 1 << 30, 4321 + emin, emin, emax) == 0
+
+
 @pytest.mark.parametrize("emin,emax", [(-60, 60), (-400, 400)])
 def test_exact_div_with_rcp_rn_is_ieee_division(emin, emax):
     assert selftest(1, 1 << 29, 777 + emin, emin, emax) == 0
