@@ -264,6 +264,31 @@ __device__ __forceinline__ void st(double* f, const CellAt& a, double v) {
     *(__attribute__((address_space(1))) double*)(row_of(f, a.base) + a.off) = v;
 }
 
+// A tile's halo cell (hi, hj) of a plane: from the cell below and left of the
+// tile's first (i0, j0), whose index is uniform, a lane offset of up to 9 rows,
+// below 2^32 bytes for rows of at most kMaxRow32 cells (which leaves a factor
+// of 50); with(k, f) calls f with the cell of plane k, by its own 64-bit index
+// in wider grids.
+constexpr int kMaxRow32 = 1 << 20;
+struct HaloAt {
+    int64_t base;
+    uint32_t off;
+    int i, j;
+    __device__ __forceinline__ HaloAt(const DevParams& p, int i0, int j0, int hi, int hj)
+        : base((int64_t)(i0 - 1) + (int64_t)(j0 - 1) * p.sy),
+          off(8u * ((uint32_t)(hi - i0 + 1) + (uint32_t)(hj - j0 + 1) * (uint32_t)p.Nx)), i(hi), j(hj) {}
+    template <class F>
+    __device__ __forceinline__ void with(const DevParams& p, int k, const F& f) const {
+        if (__builtin_expect(p.Nx <= kMaxRow32, 1)) {
+            CellAt at{base + (int64_t)k * p.sz, off};
+            renew(at);
+            f(at);
+        } else {
+            f(CellIndex{(int64_t)i + (int64_t)j * p.sy + (int64_t)k * p.sz});
+        }
+    }
+};
+
 // The parameter block in constant memory.  The tiles hold more parameters
 // than there are scalar registers; kept across the plane loop, the rest lived
 // in lanes of vector registers, one v_readlane (a VALU slot) per word and use:
@@ -553,7 +578,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
     else if (ty == 2 && tx >= TY && tx < 2 * TY) { hi = i0 + TX; hj = j0 + tx - TY; hx = TX + 1; hy = tx - TY + 1; }
     const bool halo = hi >= 0 && hi < p.Nx && hj >= 0 && hj < p.Ny && (hasx || hi == i0 + tx);
     const bool halo_ij = inner_ij<MODEL>(p, hi, hj);
-    int64_t hl = (int64_t)hi + (int64_t)hj * p.sy + (int64_t)k0 * p.sz;
+    const HaloAt hat(p, i0, j0, hi, hj);
 
     // LDS places in the buffer of plane 0: the own and the halo cell
     auto buffer = [](int k) { return (k & 1) * PLANE; };
@@ -594,7 +619,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
         const bool inner_h = halo_ij && inner_k(p, k0);
         load_raw(io, own, inner, r);
         if (hasz) load_raw(io, CellAt{own.base - p.sz, own.off}, inner_m, rm);
-        if (halo) load_raw(io, CellIndex{hl}, inner_h, rh);
+        if (halo) hat.with(p, k0, [&](const auto& at) { load_raw(io, at, inner_h, rh); });
         CellCoef<MODEL, CLOSURE> c, m;
         const DevParams pc = coef_params<MODEL, CLOSURE>(cp);
         const bool odd = coef_of(pc, r, inner, c);
@@ -625,7 +650,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
         CellRaw<MODEL, CLOSURE> r, rh;
         const bool inner = own_ij && inner_k(p, k + 1), inner_h = halo_ij && inner_k(p, k + 1);
         if (hasz) load_raw(io, CellAt{own.base + p.sz, own.off}, inner, r);
-        if (next && halo) load_raw(io, CellIndex{hl + p.sz}, inner_h, rh);
+        if (next && halo) hat.with(p, k + 1, [&](const auto& at) { load_raw(io, at, inner_h, rh); });
         const auto pre = epi.prefetch(own);
         // the next plane: coefficients, staged in the other buffer
         CellCoef<MODEL, CLOSURE> zp;
@@ -784,7 +809,6 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
             Sn = r.Sn;
             if constexpr (MODEL == 3) Sw = r.Sw;
             own.base += p.sz;
-            hl += p.sz;
             __syncthreads();
         }
     }
@@ -972,46 +996,70 @@ __global__ void __launch_bounds__(TX * TY) k_roS_z(DevParams p, StepIO io, int k
 }
 
 // The energy step's E pass (assign_E_new, energy.cpp:235-340, as body_E_with)
-// on z-marching TX x TY tiles: per plane, each cell's lambda_eff * T and its
-// advected products (ro_a * H_a) * ux_a and (ro_a * H_a) * uy_a are staged in
-// LDS with a one-cell halo ring; the z neighbours' lambda_eff * T and
-// (ro_a * H_a) * uy_a (the z term advects with uy, energy.cpp:300-305) are
-// computed per column.  Each term is the product the per-cell body forms, so
-// E_new has its bits.
-// lam: lambda_eff per cell as the step's first pass stored it, or NULL (the
-// entry point) to evaluate it from m, S_w, S_n, S_g and T.
-// uzz: the velocities the z term advects with -- uy (energy.cpp:300-305), or
-// uz in the configurations' energy closure (p.ecfg), whose conductivity is
-// the constant p.lam_eff and whose z conduction adds to the x and y terms.
+// on z-marching TX x TY tiles: each cell's lambda_eff * T and its advected
+// products (ro_a * H_a) * u_a are formed once (and once more where another
+// tile's ring holds the cell), staged in LDS with a one-cell halo ring for the
+// x and y neighbours and carried in registers for the z ones.  Each term is
+// the product the per-cell body forms, so E_new has its bits.
+//
+// Bound by memory (14 fields read and one written per cell): the next plane's
+// loads are issued before this plane's sums and one barrier ends a plane (two
+// LDS buffers).  160 x 128 x 96: 92 us against 115 for tiles that read the
+// fields again for the z neighbours.
+//
+// LAM, where lambda_eff comes from: kLamStored, lam as the step's first pass
+// stored it; kLamEvaluated (the entry point), from m, S_w, S_n, S_g and T;
+// kLamConstant, lam_cfg: the configurations' energy closure, whose z term
+// advects with uz (the reference's with uy, energy.cpp:300-305) and whose z
+// conduction adds to the x and y terms.
+enum { kLamStored, kLamEvaluated, kLamConstant };
 struct EnergyEIO {
     const double *lam, *T, *E;
     const double *m, *Sw, *Sn, *Sg;
-    const double *ro[3], *H[3], *ux[3], *uy[3], *uzz[3];
+    const double *ro[3], *H[3], *ux[3], *uy[3], *uz[3];
     double* E_new;
-    double lam_cfg;  // > 0: the constant conductivity of p.ecfg
+    double lam_cfg;
 };
 
-__device__ __forceinline__ double energy_lam(const EnergyEIO& a, int64_t l) {
-    if (a.lam_cfg > 0) return a.lam_cfg;
-    return a.lam ? a.lam[l] : lambda_eff(a.m[l], a.Sw[l], a.Sn[l], a.Sg[l], a.T[l]);
-}
-
-// v[0] = lambda_eff * T, v[1 + a] = (ro_a H_a) ux_a, v[4 + a] = (ro_a H_a) uy_a
-__device__ __forceinline__ void energy_e_vals(const EnergyEIO& a, int64_t l, double* v) {
-    v[0] = energy_lam(a, l) * a.T[l];
+template <int LAM>
+struct EnergyRaw {
+    double lam, m, Sw, Sn, Sg, T, ro[3], H[3], ux[3], uy[3], uz[3];
+};
+template <int LAM, class At>
+__device__ __forceinline__ void load_energy(const EnergyEIO& a, const At& at, EnergyRaw<LAM>& r) {
+    r.T = ld(a.T, at);
+    if constexpr (LAM == kLamStored) r.lam = ld(a.lam, at);
+    if constexpr (LAM == kLamEvaluated) {
+        r.m = ld(a.m, at);
+        r.Sw = ld(a.Sw, at);
+        r.Sn = ld(a.Sn, at);
+        r.Sg = ld(a.Sg, at);
+    }
 #pragma unroll
-    for (int ph = 0; ph < 3; ++ph) {
-        const double rh = a.ro[ph][l] * a.H[ph][l];
-        v[1 + ph] = rh * a.ux[ph][l];
-        v[4 + ph] = rh * a.uy[ph][l];
+    for (int q = 0; q < 3; ++q) {
+        r.ro[q] = ld(a.ro[q], at);
+        r.H[q] = ld(a.H[q], at);
+        r.ux[q] = ld(a.ux[q], at);
+        r.uy[q] = ld(a.uy[q], at);
+        if constexpr (LAM == kLamConstant) r.uz[q] = ld(a.uz[q], at);
     }
 }
-
-// lambda_eff * T and the uzz products of a z neighbour: w[0], w[1 + a]
-__device__ __forceinline__ void energy_e_zvals(const EnergyEIO& a, int64_t l, double* w) {
-    w[0] = energy_lam(a, l) * a.T[l];
+// v[0] = lambda_eff * T, v[1 + a] = (ro_a H_a) ux_a, v[4 + a] = (ro_a H_a) uy_a;
+// z[a]: the product that the z term advects
+template <int LAM>
+__device__ __forceinline__ void energy_vals(const EnergyEIO& a, const EnergyRaw<LAM>& r, double* v, double* z) {
+    double lam;
+    if constexpr (LAM == kLamStored) lam = r.lam;
+    if constexpr (LAM == kLamEvaluated) lam = lambda_eff(r.m, r.Sw, r.Sn, r.Sg, r.T);
+    if constexpr (LAM == kLamConstant) lam = a.lam_cfg;
+    v[0] = lam * r.T;
 #pragma unroll
-    for (int ph = 0; ph < 3; ++ph) w[1 + ph] = a.ro[ph][l] * a.H[ph][l] * a.uzz[ph][l];
+    for (int q = 0; q < 3; ++q) {
+        const double rh = r.ro[q] * r.H[q];
+        v[1 + q] = rh * r.ux[q];
+        v[4 + q] = rh * r.uy[q];
+        z[q] = LAM == kLamConstant ? rh * r.uz[q] : v[4 + q];
+    }
 }
 
 // advection's (((X_w+ - X_w-) + X_n+) - X_n-) + X_g+) - X_g- (the body's order)
@@ -1019,10 +1067,12 @@ __device__ __forceinline__ double energy_adv(double wp, double wm, double np_, d
     return wp - wm + np_ - nm + gp - gm;
 }
 
-template <int TX, int TY>
-__global__ void __launch_bounds__(TX * TY) k_energy_e_z(DevParams p, EnergyEIO a, int kchunk) {
-    static_assert(TY >= 3 && TX >= 2 * TY, "halo ring needs TY >= 3 and TX >= 2*TY");
-    __shared__ double lds[7][TY + 2][TX + 2];
+template <int LAM, int TX, int TY>
+__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(4)))
+k_energy_e_z(DevParams p, EnergyEIO a, int kchunk) {
+    static_assert(TY >= 3 && TX == 64, "halo ring and whole rows per wavefront");
+    constexpr int NV = 7, ROW = (TX + 2) * NV, PLANE = (TY + 2) * ROW;
+    __shared__ double lds[2][TY + 2][TX + 2][NV];
     int bx, by, bz;
     xcd_tile(bx, by, bz);
     const int tx = threadIdx.x, ty = threadIdx.y;
@@ -1033,72 +1083,100 @@ __global__ void __launch_bounds__(TX * TY) k_energy_e_z(DevParams p, EnergyEIO a
     const int k0 = klo + kchunk * bz;
     const int k1 = min(khi, k0 + kchunk - 1);
     const int i = i0 + tx, j = j0 + ty;
-    const bool own_in_grid = i < p.Nx && j < p.Ny;
     const bool active = i <= ihi && j <= p.Ny - 2;
-    // halo cell of this thread, as in fused_z_tile
+    // the own column, clamped into the grid, and the halo cell, as in fused_z_tile
+    const int ic = min(i, p.Nx - 1), jw = __builtin_amdgcn_readfirstlane(min(j, p.Ny - 1));
+    CellAt own{(int64_t)i0 + (int64_t)jw * p.sy + (int64_t)k0 * p.sz, 8u * (uint32_t)(ic - i0)};
     int hi = -1, hj = -1, hx = 0, hy = 0;
     if (ty == 0) { hi = i; hj = j0 - 1; hx = tx + 1; hy = 0; }
     else if (ty == 1) { hi = i; hj = j0 + TY; hx = tx + 1; hy = TY + 1; }
     else if (ty == 2 && tx < TY) { hi = i0 - 1; hj = j0 + tx; hx = 0; hy = tx + 1; }
     else if (ty == 2 && tx >= TY && tx < 2 * TY) { hi = i0 + TX; hj = j0 + tx - TY; hx = TX + 1; hy = tx - TY + 1; }
-    const bool halo_in_grid = hi >= 0 && hi < p.Nx && hj >= 0 && hj < p.Ny && (hasx || hi == i0 + tx);
-    const int64_t col = (int64_t)i + (int64_t)j * p.sy;
-    const int64_t hcol = (int64_t)hi + (int64_t)hj * p.sy;
+    const bool halo = hi >= 0 && hi < p.Nx && hj >= 0 && hj < p.Ny && (hasx || hi == i0 + tx);
+    const HaloAt hat(p, i0, j0, hi, hj);
+    const LdsDouble v0 = (LdsDouble)&lds[0][ty + 1][tx + 1][0], vh = (LdsDouble)&lds[0][hy][hx][0];
+    auto stage = [&](LdsDouble w, const double* v) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) w[q] = v[q];
+    };
 
-    double zm[4] = {}, zp[4] = {};
-    if (own_in_grid && hasz) energy_e_zvals(a, col + (int64_t)(k0 - 1) * p.sz, zm);
+    // lambda_eff * T and the z products of the planes k - 1 and k
+    double lm = 0., zm[3] = {}, lc, zc[3];
+    {
+        EnergyRaw<LAM> r, rh;
+        double v[NV], z[3];
+        if (hasz) {
+            load_energy(a, CellAt{own.base - p.sz, own.off}, r);
+            energy_vals(a, r, v, zm);
+            lm = v[0];
+        }
+        asm volatile("" ::: "memory");  // one plane's values in registers at a time
+        load_energy(a, own, r);
+        if (halo) hat.with(p, k0, [&](const auto& at) { load_energy(a, at, rh); });
+        energy_vals(a, r, v, zc);
+        lc = v[0];
+        stage(v0 + (k0 & 1) * PLANE, v);
+        if (halo) {
+            energy_vals(a, rh, v, z);
+            stage(vh + (k0 & 1) * PLANE, v);
+        }
+    }
+    __syncthreads();
     for (int k = k0; k <= k1; ++k) {
-        const int64_t l = col + (int64_t)k * p.sz;
-        double v[7] = {};
-        if (own_in_grid) {
-            energy_e_vals(a, l, v);
-#pragma unroll
-            for (int q = 0; q < 7; ++q) lds[q][ty + 1][tx + 1] = v[q];
+        const bool next = k < k1;
+        renew(own);
+        EnergyRaw<LAM> r, rh;
+        if (hasz) load_energy(a, CellAt{own.base + p.sz, own.off}, r);
+        if (next && halo) hat.with(p, k + 1, [&](const auto& at) { load_energy(a, at, rh); });
+        const double E = ld(a.E, own);
+        const LdsDouble c = v0 + (k & 1) * PLANE;
+        double T_flow = 0, E_flow = 0;
+        if (p.Nx > 2) {
+            const LdsDouble m = c - NV, q = c + NV;
+            T_flow += exact_div(q[0] - 2 * lc + m[0], p.hx2, p.r_hx2);
+            E_flow += exact_div(energy_adv(q[1], m[1], q[2], m[2], q[3], m[3]), p.two_hx, p.r_two_hx);
         }
-        if (hi >= 0 && halo_in_grid) {
-            double h[7];
-            energy_e_vals(a, hcol + (int64_t)k * p.sz, h);
-#pragma unroll
-            for (int q = 0; q < 7; ++q) lds[q][hy][hx] = h[q];
+        {
+            const LdsDouble m = c - ROW, q = c + ROW;
+            T_flow += exact_div(q[0] - 2 * lc + m[0], p.hy2, p.r_hy2);
+            E_flow += exact_div(energy_adv(q[4], m[4], q[5], m[5], q[6], m[6]), p.two_hy, p.r_two_hy);
         }
-        __syncthreads();
-        if (own_in_grid && hasz) energy_e_zvals(a, l + p.sz, zp);
+        double zp[3], lp = 0.;
+        if (hasz) {
+            double v[NV];
+            energy_vals(a, r, v, zp);
+            lp = v[0];
+            if (next) stage(v0 + ((k + 1) & 1) * PLANE, v);
+        }
+        if (next && halo) {
+            double v[NV], z[3];
+            energy_vals(a, rh, v, z);
+            stage(vh + ((k + 1) & 1) * PLANE, v);
+        }
+        if (hasz) {
+            const double tz = exact_div(lp - 2 * lc + lm, p.hz2, p.r_hz2);
+            if constexpr (LAM == kLamConstant)
+                T_flow += tz;
+            else
+                T_flow = tz;  // '=' as energy.cpp:257
+            E_flow += exact_div(energy_adv(zp[0], zm[0], zp[1], zm[1], zp[2], zm[2]), p.two_hz, p.r_two_hz);
+        }
         if (active) {
-            const double lc = energy_lam(a, l), Tc = a.T[l];
-            double T_flow = 0;
-            if (p.Nx > 2)
-                T_flow += exact_div(lds[0][ty + 1][tx + 2] - 2 * lc * Tc + lds[0][ty + 1][tx], p.hx2, p.r_hx2);
-            if (p.Ny > 2)
-                T_flow += exact_div(lds[0][ty + 2][tx + 1] - 2 * lc * Tc + lds[0][ty][tx + 1], p.hy2, p.r_hy2);
-            if (p.Nz > 2) {
-                const double tz = exact_div(zp[0] - 2 * lc * Tc + zm[0], p.hz2, p.r_hz2);
-                if (p.ecfg)
-                    T_flow += tz;
-                else
-                    T_flow = tz;  // '=' as energy.cpp:257
-            }
-            double E_flow = 0;
-            if (p.Nx > 2)
-                E_flow += exact_div(energy_adv(lds[1][ty + 1][tx + 2], lds[1][ty + 1][tx], lds[2][ty + 1][tx + 2],
-                                               lds[2][ty + 1][tx], lds[3][ty + 1][tx + 2], lds[3][ty + 1][tx]),
-                                    p.two_hx, p.r_two_hx);
-            if (p.Ny > 2)
-                E_flow += exact_div(energy_adv(lds[4][ty + 2][tx + 1], lds[4][ty][tx + 1], lds[5][ty + 2][tx + 1],
-                                               lds[5][ty][tx + 1], lds[6][ty + 2][tx + 1], lds[6][ty][tx + 1]),
-                                    p.two_hy, p.r_two_hy);
-            if (p.Nz > 2)
-                E_flow += exact_div(energy_adv(zp[1], zm[1], zp[2], zm[2], zp[3], zm[3]), p.two_hz, p.r_two_hz);
             double Q_hw = 0, Q_hr = 0;
-            a.E_new[l] = a.E[l] + p.dt * (T_flow + Q_hw + Q_hr - E_flow);
+            CellAt to = own;
+            renew(to);
+            st(a.E_new, to, E + p.dt * (T_flow + Q_hw + Q_hr - E_flow));
         }
-        __syncthreads();
-        // roll the z window: the centre's lambda_eff * T and uzz products
-        if (p.ecfg) {
-            if (own_in_grid) energy_e_zvals(a, l, zm);
-        } else {
-            zm[0] = v[0];
+        if (next) {
+            lm = lc;
+            lc = lp;
 #pragma unroll
-            for (int ph = 0; ph < 3; ++ph) zm[1 + ph] = v[4 + ph];
+            for (int q = 0; q < 3; ++q) {
+                zm[q] = zc[q];
+                zc[q] = zp[q];
+            }
+            own.base += p.sz;
+            __syncthreads();
         }
     }
 }

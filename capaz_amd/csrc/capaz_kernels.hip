@@ -469,14 +469,19 @@ hipError_t launch_energy_e_tiles(const DevParams& p, const DevFields& F, const d
         ea.H[a] = F.f[H[a]];
         ea.ux[a] = F.f[ux[a]];
         ea.uy[a] = F.f[uy[a]];
-        ea.uzz[a] = F.f[p.ecfg ? uz[a] : uy[a]];
+        ea.uz[a] = F.f[uz[a]];
     }
-    ea.lam_cfg = p.ecfg ? p.lam_eff : 0.;
+    ea.lam_cfg = p.lam_eff;
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
-    const int kc = fused_kchunk(p, 0, 8, resident_groups<k_energy_e_z<64, 8>>(512));
-    dim3 ge((nx + 63) / 64, (ny + 7) / 8, (nz + kc - 1) / kc);
-    hipLaunchKernelGGL((k_energy_e_z<64, 8>), ge, dim3(64, 8), 0, s, p, ea, kc);
-    return hipGetLastError();
+    auto launch = [&](auto lam_id) {
+        constexpr auto kernel = k_energy_e_z<decltype(lam_id)::value, 64, 8>;
+        const int kc = fused_kchunk(p, 0, 8, resident_groups<kernel>(512));
+        dim3 ge((nx + 63) / 64, (ny + 7) / 8, (nz + kc - 1) / kc);
+        hipLaunchKernelGGL(kernel, ge, dim3(64, 8), 0, s, p, ea, kc);
+        return hipGetLastError();
+    };
+    if (p.ecfg) return launch(std::integral_constant<int, kLamConstant>{});
+    return lam ? launch(std::integral_constant<int, kLamStored>{}) : launch(std::integral_constant<int, kLamEvaluated>{});
 }
 
 hipError_t launch_newton_energy(const DevParams& p, const DevFields& F, unsigned char* redo, hipStream_t s) {

@@ -227,6 +227,28 @@ def test_tile_cells_done_after_the_planes(dims, tune, closure):
         assert np.isfinite(b["P_w"]).all()
 
 
+@pytest.mark.parametrize("model,tune", [("3ph", dict(tile_y=8)), ("3ph", dict(tile_y=4)), ("3phe", dict()),
+                                        ("3phe", dict(energy_kernel=0))])
+@pytest.mark.parametrize("nx", [1 << 20, (1 << 20) + 1024])
+def test_rows_at_the_halo_offset_limit(model, tune, nx):
+    """Rows of 2^20 cells, whose halo cells a tile addresses by a 32-bit lane
+    offset, and longer ones (64-bit indexes): a state that repeats every 1024
+    columns gives, at both ends, the same bits in rows of 4096 cells."""
+    col = random_state(case(model, 1024, 4, 1), seed=5)
+    got = []
+    for n in (nx, 4096):
+        d = capaz.Domain(case(model, n, 4, 1, DT=1e-5, SOURCE=0, CLOSURE="corey"),
+                         {f: np.tile(a, (1, 1, n // 1024)) for f, a in col.items()})
+        d.tune(**tune)
+        d.run(2)
+        got.append({f: d.field(f) for f in ("P_w", "S_w", "S_n") + (("T", "E") if model == "3phe" else ())})
+        d.close()
+    for f, a in got[0].items():
+        assert bit_equal(np.ascontiguousarray(a[..., :2048]), np.ascontiguousarray(got[1][f][..., :2048])), f
+        assert bit_equal(np.ascontiguousarray(a[..., -2048:]), np.ascontiguousarray(got[1][f][..., -2048:])), f
+        assert np.isfinite(a).all()
+
+
 def test_headline_physics_bitwise_at_96():
     """The benchmark physics (three-phase, Corey-2, lognormal K, top
     injection) at 96^3: one and three fused steps equal the oracle bit for bit."""
