@@ -71,7 +71,7 @@ CAPAZ_HD void corey_d(const DevParams& p, double s, double& kr, double& dkr) {
 // vg_k_n and vg_k_g evaluate them) and their partial derivatives in the
 // effective saturations x = Swe, y = Sne (z = Sge = 1 - x - y), by the chain
 // rule on each power (a = p.vg_a, b = p.vg_b, c = p.vg_c; the powers are the
-// forward step's pow_cl, whose log of a base the compiler computes once):
+// forward step's, a base's log taken once):
 //   k_w = x^(1/2) t^2,           t = 1 - (1 - x^a)^b        (x >= 1e-3)
 //   k_g = z^(1/2) v^c,           v = 1 - (1 - z)^a          (z >= 1e-3)
 //   k_n = y k_nw k_ng / D,       D = (1 - x)(x + y)         (y >= 1e-3)
@@ -82,25 +82,36 @@ CAPAZ_HD void vg_d(const DevParams& p, double x, double y, double& kw, double& k
     const double z = 1. - x - y;
     kw = kn = kg = dkw_dx = dkn_dx = dkn_dy = dkg_dz = 0.;
     if (x >= 1e-3) {
-        const double u = 1. - pow_cl(x, a), t = 1. - pow_cl(u, b);
-        const double dt = b * pow_cl(u, b - 1.) * a * pow_cl(x, a - 1.);
+        const PowBase bx = pow_base(x);
+        const double u = 1. - pow_of(bx, a);
+        const PowBase bu = pow_base(u);
+        const double t = 1. - pow_of(bu, b);
+        const double dt = b * pow_of(bu, b - 1.) * a * pow_of(bx, a - 1.);
         const double sx = sqrt(x);
         kw = sx * t * t;
         dkw_dx = 0.5 / sx * t * t + 2. * sx * t * dt;
     }
     if (z >= 1e-3) {
-        const double v = 1. - pow_cl(1. - z, a), vc = pow_cl(v, c);
-        const double dv = a * pow_cl(1. - z, a - 1.);
+        const PowBase bz = pow_base(1. - z);
+        const double v = 1. - pow_of(bz, a);
+        const PowBase bv = pow_base(v);
+        const double vc = pow_of(bv, c);
+        const double dv = a * pow_of(bz, a - 1.);
         const double sz = sqrt(z);
         kg = sz * vc;
-        dkg_dz = 0.5 / sz * vc + sz * c * pow_cl(v, c - 1.) * dv;
+        dkg_dz = 0.5 / sz * vc + sz * c * pow_of(bv, c - 1.) * dv;
     }
     if (y >= 1e-3) {
-        const double w = 1. - pow_cl(x, a), sw = sqrt(1. - x);
-        const double knw = sw * pow_cl(w, c);
-        const double dknw = -0.5 / sw * pow_cl(w, c) - sw * c * pow_cl(w, c - 1.) * a * pow_cl(x, a - 1.);
-        const double q = 1. - pow_cl(y, a), s = 1. - pow_cl(q, b);
-        const double ds = b * pow_cl(q, b - 1.) * a * pow_cl(y, a - 1.);
+        const PowBase bx = pow_base(x), by = pow_base(y);
+        const double w = 1. - pow_of(bx, a), sw = sqrt(1. - x);
+        const PowBase bw = pow_base(w);
+        const double wc = pow_of(bw, c);
+        const double knw = sw * wc;
+        const double dknw = -0.5 / sw * wc - sw * c * pow_of(bw, c - 1.) * a * pow_of(bx, a - 1.);
+        const double q = 1. - pow_of(by, a);
+        const PowBase bq = pow_base(q);
+        const double s = 1. - pow_of(bq, b);
+        const double ds = b * pow_of(bq, b - 1.) * a * pow_of(by, a - 1.);
         const double sy = sqrt(y);
         const double kng = sy * s * s;
         const double dkng = 0.5 / sy * s * s + 2. * sy * s * ds;

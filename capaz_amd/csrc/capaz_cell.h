@@ -172,55 +172,95 @@ CAPAZ_HD int64_t inward(const DevParams& p, int i, int j, int k) {
 
 // x^y in the reference closures (the van Genuchten and Brooks-Corey k_r, the
 // energy model's mu_g(T) and lambda_g(T), a Corey exponent read at run time).
-// On the device: exp(y * log|x|) from the device library's log and exp, about
-// 130 VALU instructions against some 215 for its pow, with the log computed
-// once where powers share a base (pow_base / pow_of).  The roundings of log x
-// and of y * log x put up to 2 |y ln x| ulp into the result (tens of ulp for
-// the closures' bases, x >= 1e-15), within the tolerance the reference
-// closures are held to, since the device library's pow is not glibc's either.  pow's other
-// cases, which the closures reach only for states outside their range, by
-// selects (no call, which would cost registers in every kernel that holds a
-// closure's code): a zero exponent gives 1, a negative finite base gives
+// On the device: exp_in(y * log_pos(x)) for a positive normal base, 48 VALU
+// instructions (123 with the device library's exp and constants moved to
+// vector registers, some 215 for its pow), with the log computed once where
+// powers share a base.  The roundings of log x and of y * log x put up to
+// 2 |y ln x| ulp into the result (tens of ulp for the closures' bases,
+// x >= 1e-15), within the tolerance the reference closures are held to, since
+// the device library's pow is not glibc's either.  pow's other cases, which
+// the closures reach only for states outside their range, by selects (pow_of)
+// on the same values: a zero exponent gives 1, a negative finite base gives
 // +-|x|^y for an integer exponent and NaN otherwise.  The host build keeps
 // glibc's pow, whose bits the reference's golden vectors hold.
 #if defined(__HIP_DEVICE_COMPILE__)
-// ln x for x > 0 (pow_base's log|x|): x = 2^k m with m in [sqrt(1/2),
-// sqrt(2)) by the hardware's frexp (subnormals included), then
-// ln m = 2 atanh(s), s = (m - 1) / (m + 1) (|s| <= 0.1716; m - 1 is exact),
-// by the series 2 s (1 + s^2/3 + s^4/5 + ... + s^20/21), whose next term is
-// below 1e-17 of the sum, and k ln 2 with ln 2 split so that k * LN2_HI is
-// exact.  s carries ~2^-52 relative error (the rounded m + 1 and a reciprocal
-// with two Newton steps), which the result keeps for x near 1; for other x
-// the final additions' rounding dominates, as in a correctly rounded log.
-// 0 gives -inf, +inf gives +inf, NaN and negative x give NaN.
-__device__ __forceinline__ double log_cl(double x) {
-    constexpr double kLn2Hi = 0x1.62e42fefa3800p-1, kLn2Lo = 0x1.ef35793c76730p-45;
-    double m = __builtin_amdgcn_frexp_mant(x);  // [0.5, 1) for finite x > 0
+// a * b + k and a * k + b with the constant k in scalar registers: for a
+// polynomial the compiler moves each constant to vector registers first (the
+// accumulating FMA's addend), a second VALU instruction per term.
+__device__ __forceinline__ double fma_add_k(double a, double b, double k) {
+    double r;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(k));
+    return r;
+}
+__device__ __forceinline__ double fma_mul_k(double a, double k, double b) {
+    double r;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(k), "v"(b));
+    return r;
+}
+constexpr double kLn2Hi = 0x1.62e42fefa3800p-1, kLn2Lo = 0x1.ef35793c76730p-45;  // 11 trailing zero bits in hi
+
+// ln x for finite x > 0: x = 2^k m with m in [sqrt(1/2), sqrt(2)) by the
+// hardware's frexp (subnormals included), then ln m = 2 atanh(s),
+// s = (m - 1) / (m + 1) (|s| <= 0.1716; m - 1 is exact) = 2 s + s^3 p(s^2),
+// p the interpolation of that function at 8 Chebyshev nodes (within 6e-19 of
+// ln m relatively), and k ln 2 with ln 2 split so that k * hi is exact.  s
+// carries ~2^-52 relative error (the rounded m + 1 and its reciprocal), which
+// the result keeps for x near 1; for other x the final additions' rounding
+// dominates, as in a correctly rounded log.
+__device__ __forceinline__ double log_pos(double x) {
+    double m = __builtin_amdgcn_frexp_mant(x);  // [0.5, 1)
     int k = __builtin_amdgcn_frexp_exp(x);
-    const bool low = m < 0x1.6a09e667f3bcdp-1;  // sqrt(1/2)
-    m = low ? 2. * m : m;
-    k = low ? k - 1 : k;
+    const int low = m < 0x1.6a09e667f3bcdp-1 ? 1 : 0;  // sqrt(1/2)
+    m = __builtin_amdgcn_ldexp(m, low);
+    k -= low;
     const double q = m + 1.;
     double r = __builtin_amdgcn_rcp(q);
-    r = fma(fma(-q, r, 1.), r, r);
-    r = fma(fma(-q, r, 1.), r, r);
+    const double e = fma(-q, r, 1.);
+    r = fma(fma(e, e, e), r, r);
     const double s = (m - 1.) * r, z = s * s;
-    double poly = 1. / 21.;
-    poly = fma(poly, z, 1. / 19.);
-    poly = fma(poly, z, 1. / 17.);
-    poly = fma(poly, z, 1. / 15.);
-    poly = fma(poly, z, 1. / 13.);
-    poly = fma(poly, z, 1. / 11.);
-    poly = fma(poly, z, 1. / 9.);
-    poly = fma(poly, z, 1. / 7.);
-    poly = fma(poly, z, 1. / 5.);
-    poly = fma(poly, z, 1. / 3.);
-    const double lm = 2. * fma(s * z, poly, s);  // ln m
-    const double kd = (double)k;
-    double l = fma(kd, kLn2Hi, fma(kd, kLn2Lo, lm));
+    double p = fma_add_k(z, 0x1.0c04595972ab8p-3, 0x1.0fbe83c2cbcf3p-3);
+    p = fma_add_k(p, z, 0x1.3b1c360763b8ap-3);
+    p = fma_add_k(p, z, 0x1.745cf901605f7p-3);
+    p = fma_add_k(p, z, 0x1.c71c720160b47p-3);
+    p = fma_add_k(p, z, 0x1.2492492476c87p-2);
+    p = fma_add_k(p, z, 0x1.9999999999a38p-2);
+    p = fma_add_k(p, z, 0x1.5555555555555p-1);
+    const double lm = fma(s * z, p, s + s), kd = (double)k;
+    return fma_mul_k(kd, kLn2Hi, fma_mul_k(kd, kLn2Lo, lm));
+}
+
+// e^t for |t| < 1e8: t = k ln 2 + r, |r| <= ln(2) / 2, e^r = 1 + r + r^2 p(r), p
+// the interpolation of that function at 11 Chebyshev nodes (within 4e-19 of
+// e^r relatively); 2^k by ldexp, which overflows and underflows as e^t does.
+__device__ __forceinline__ double exp_in(double t) {
+    const double k = rint(t * 0x1.71547652b82fep+0);
+    double r = fma_mul_k(-k, kLn2Hi, t);
+    r = fma_mul_k(-k, kLn2Lo, r);
+    double p = fma_add_k(r, 0x1.1f730349868cep-29, 0x1.af4de97ca4194p-26);
+    p = fma_add_k(p, r, 0x1.27e4db646b17ep-22);
+    p = fma_add_k(p, r, 0x1.71de0231960ebp-19);
+    p = fma_add_k(p, r, 0x1.a01a01a6d889cp-16);
+    p = fma_add_k(p, r, 0x1.a01a01abe7fe1p-13);
+    p = fma_add_k(p, r, 0x1.6c16c16c162d4p-10);
+    p = fma_add_k(p, r, 0x1.11111111100dcp-7);
+    p = fma_add_k(p, r, 0x1.5555555555556p-5);
+    p = fma_add_k(p, r, 0x1.5555555555557p-3);
+    p = fma_add_k(p, r, 0.5);
+    return __builtin_amdgcn_ldexp(fma(p, r * r, r) + 1., (int)k);
+}
+
+// log_pos with the other arguments: 0 gives -inf, +inf gives +inf, NaN and
+// negative x give NaN.
+__device__ __forceinline__ double log_cl(double x) {
+    double l = log_pos(x);
     l = x == 0. ? -__builtin_inf() : l;
     l = x == __builtin_inf() ? __builtin_inf() : l;
     return x > 0. || x == 0. ? l : __builtin_nan("");  // NaN and x < 0: NaN
+}
+// exp_in with the other arguments.
+__device__ __forceinline__ double exp_cl(double t) {
+    const double e = exp_in(t);
+    return fabs(t) < 1e8 ? e : (t > 0. ? __builtin_inf() : (t < 0. ? 0. : t));
 }
 #endif
 
@@ -236,7 +276,7 @@ CAPAZ_HD PowBase pow_base(double x) {
 }
 CAPAZ_HD double pow_of(const PowBase& b, double y) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    double r = exp(y * b.lx);
+    double r = exp_cl(y * b.lx);
     const bool integer = y == trunc(y), odd = integer && 0.5 * y != trunc(0.5 * y);
     r = b.x < 0. ? (integer ? (odd ? -r : r) : __builtin_nan("")) : r;
     return y == 0. ? 1. : r;
@@ -244,7 +284,22 @@ CAPAZ_HD double pow_of(const PowBase& b, double y) {
     return pow(b.x, y);
 #endif
 }
-CAPAZ_HD double pow_cl(double x, double y) { return pow_of(pow_base(x), y); }
+// On the device the powers of a positive normal base in a moderate exponent
+// without the selects (the same bits), under a test that such lanes all pass.
+CAPAZ_HD double pow_cl(double x, double y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (__builtin_expect(x >= 0x1p-1000 && x <= 0x1p1000 && fabs(y) <= 1e4, 1)) return exp_in(y * log_pos(x));
+#endif
+    return pow_of(pow_base(x), y);
+}
+// e^t (mu(T)).
+CAPAZ_HD double exp_t(double t) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return exp_cl(t);
+#else
+    return exp(t);
+#endif
+}
 
 CAPAZ_HD double corey_kr(const DevParams& p, double s) {
     s = clamp01(s);
@@ -299,6 +354,31 @@ CAPAZ_HD double vg_k_n(const DevParams& p, double Swe, double Sne, const PowBase
     return 0;
 }
 
+#if defined(__HIP_DEVICE_COMPILE__)
+// relperm3's van Genuchten values for Swe in [0, 1] and Sne, Sge <= 1 under
+// p.pow_fast, without a test per power: bases that may be 0 are raised to the
+// smallest normal number, whose powers in vg_a and vg_b vanish beside 1 and in
+// vg_c >= 1.1 are 0.  The same bits as vg_k_w, vg_k_g and vg_k_n.
+__device__ __forceinline__ void vg_fast(const DevParams& p, double Swe, double Sne, double Sge, double& kw, double& kn,
+                                        double& kg) {
+    constexpr double tiny = 0x1p-1022;
+    auto lg = [](double x) { return log_pos(fmax(x, tiny)); };
+    const double lb1 = lg(1. - exp_in(p.vg_a * lg(Swe)));
+    const double tw = 1. - exp_in(p.vg_b * lb1);
+    kw = pow_half(Swe) * pow_two(tw);
+    kw = Swe >= 1e-3 ? kw : 0.;
+    const double lg1 = lg(1. - exp_in(p.vg_a * lg(1. - Sge)));
+    kg = pow_half(Sge) * exp_in(p.vg_c * lg1);
+    kg = Sge >= 1e-3 ? kg : 0.;
+    const double ln1 = lg(1. - exp_in(p.vg_a * lg(Sne)));
+    const double knw = pow_half(1. - Swe) * exp_in(p.vg_c * lb1);
+    const double kng = pow_half(Sne) * pow_two(1. - exp_in(p.vg_b * ln1));
+    const double Sg = 1. - Swe - Sne;
+    kn = Sne * knw * kng / (1 - Swe) / (1 - Sg);
+    kn = Sne >= 1e-3 ? kn : 0.;
+}
+#endif
+
 // Three-phase relative permeabilities k_w, k_n, k_g of a cell
 // (three-phase.cpp:202-208).
 CAPAZ_HD void relperm3(const DevParams& p, double S_w, double S_n, double& kw, double& kn, double& kg) {
@@ -310,6 +390,12 @@ CAPAZ_HD void relperm3(const DevParams& p, double S_w, double S_n, double& kw, d
         kn = corey_kr(p, Sne);
         kg = corey_kr(p, Sge);
     } else {
+#if defined(__HIP_DEVICE_COMPILE__)
+        if (__builtin_expect(p.pow_fast && Swe >= 0. && Swe <= 1. && Sne <= 1. && Sge <= 1., 1)) {
+            vg_fast(p, Swe, Sne, Sge, kw, kn, kg);
+            return;
+        }
+#endif
         const double pSwe = Swe >= 1e-3 || Sne >= 1e-3 ? pow_cl(Swe, p.vg_a) : 0.;
         const PowBase b1 = pow_base(1. - pSwe);
         kw = vg_k_w(p, Swe, b1);
@@ -327,6 +413,15 @@ CAPAZ_HD void relperm2(const DevParams& p, double S_n, double& kw, double& kn, d
         Pk = 0.;
     } else {
         double se = exact_div(1. - S_n - p.S_wr, p.den2, p.r_den2);
+#if defined(__HIP_DEVICE_COMPILE__)
+        if (__builtin_expect(p.pow_fast && se >= 0x1p-1000 && se <= 0x1p1000, 1)) {
+            const double lx = log_pos(se);  // the same bits without the selects
+            kw = exp_in(p.bc_ew * lx);
+            kn = (1. - se) * (1. - se) * (1 - exp_in(p.bc_en * lx));
+            Pk = p.P_d * exp_in(p.bc_epk * lx);
+            return;
+        }
+#endif
         const PowBase b = pow_base(se);
         kw = pow_of(b, p.bc_ew);
         kn = (1. - se) * (1. - se) * (1 - pow_of(b, p.bc_en));
@@ -337,7 +432,7 @@ CAPAZ_HD void relperm2(const DevParams& p, double S_n, double& kw, double& kn, d
 // Energy-model viscosities mu(T) (three-phase.cpp:212-214).
 CAPAZ_HD void mu_of_T(double T, double& mw, double& mn, double& mg) {
     mw = 1. / (29.21 * T - 7506.64);
-    mn = 7.256E-10 * exp(4141.9 / T);
+    mn = 7.256E-10 * exp_t(4141.9 / T);
     mg = 1.717E-5 * pow_cl(exact_div(T, 273., 1. / 273.), 0.683);
 }
 
@@ -606,9 +701,11 @@ CAPAZ_HD int reverse3(double* a) {
 
 // Two-phase fixed-iteration 2x2 Newton by Cramer's rule (two-phase.cpp:25-56).
 // CL: the fused kernels' closure id (0 the reference's Brooks-Corey, 1 and 2
-// Corey), or -1 for p.closure at run time.  rcp(det): RN(1 / det).
-template <int CL, class Rcp>
-CAPAZ_HD void newton2_with(const DevParams& p, double& P, double& Sn, double roS_w, double roS_n, Rcp&& rcp) {
+// Corey), or -1 for p.closure at run time.  rcp(det): RN(1 / det);
+// powers(S_e, P_k, AAA): the Brooks-Corey P_d S_e^(-1/lambda) and S_e^(-1/lambda - 1).
+template <int CL, class Rcp, class Powers>
+CAPAZ_HD void newton2_with(const DevParams& p, double& P, double& Sn, double roS_w, double roS_n, Rcp&& rcp,
+                           Powers&& powers) {
     for (int w = 1; w <= p.iterations; w++) {
         double P_k, PkS;
         if (CL >= 1 || (CL < 0 && p.closure == 1)) {
@@ -616,9 +713,8 @@ CAPAZ_HD void newton2_with(const DevParams& p, double& P, double& Sn, double roS
             PkS = 0.;
         } else {
             double S_e = exact_div(1 - Sn - p.S_wr, p.den2, p.r_den2);
-            const PowBase b = pow_base(S_e);
-            P_k = p.P_d * pow_of(b, p.bc_epk);
-            double AAA = pow_of(b, p.bc_eaaa);
+            double AAA;
+            powers(S_e, P_k, AAA);
             PkS = exact_div(AAA * p.P_d, p.bc_pks_den, p.r_bc_pks_den);
         }
         double F1 = p.ro0_w * (1. + p.beta_w * (P - p.P_atm)) * (1. - Sn) - roS_w;
@@ -633,27 +729,50 @@ CAPAZ_HD void newton2_with(const DevParams& p, double& P, double& Sn, double roS
         Sn = Sn - rdet * (F1P * F2 - F2P * F1);
     }
 }
+CAPAZ_HD void bc_powers(const DevParams& p, double S_e, double& P_k, double& AAA) {
+    const PowBase b = pow_base(S_e);
+    P_k = p.P_d * pow_of(b, p.bc_epk);
+    AAA = pow_of(b, p.bc_eaaa);
+}
 template <int CL = -1>
 CAPAZ_HD void newton2(const DevParams& p, double& P, double& Sn, double roS_w, double roS_n) {
-    newton2_with<CL>(p, P, Sn, roS_w, roS_n, [](double det) { return rcp_rn(det); });
+    newton2_with<CL>(
+        p, P, Sn, roS_w, roS_n, [](double det) { return rcp_rn(det); },
+        [&](double S_e, double& P_k, double& AAA) { bc_powers(p, S_e, P_k, AAA); });
 }
 // newton2 for a kernel's hot path, with no call and no branch per iteration:
 // false (and any values) if some determinant lay outside the fast
-// reciprocal's range; newton2_ieee (an IEEE division, inline) then redoes the
-// cell.  RN(1 / det) either way, so the same bits.
+// reciprocal's range or some S_e outside that of the powers without selects;
+// newton2_ieee (an IEEE division and the general powers, inline) then redoes
+// the cell.  The same bits either way.
 template <int CL>
 CAPAZ_HD bool newton2_fast(const DevParams& p, double& P, double& Sn, double roS_w, double roS_n) {
     double lo = 0x1p0, hi = 0x1p0;
-    newton2_with<CL>(p, P, Sn, roS_w, roS_n, [&](double det) {
-        lo = fmin(lo, fabs(det));
-        hi = fmax(hi, fabs(det));
-        return rcp_in_range(det);
-    });
-    return lo >= 0x1p-1000 && hi <= 0x1p1000;
+    bool ok = CL >= 1 || p.pow_fast;
+    newton2_with<CL>(
+        p, P, Sn, roS_w, roS_n,
+        [&](double det) {
+            lo = fmin(lo, fabs(det));
+            hi = fmax(hi, fabs(det));
+            return rcp_in_range(det);
+        },
+        [&](double S_e, double& P_k, double& AAA) {
+#if defined(__HIP_DEVICE_COMPILE__)
+            ok = ok && S_e >= 0x1p-1000 && S_e <= 0x1p1000;
+            const double lx = log_pos(S_e);
+            P_k = p.P_d * exp_in(p.bc_epk * lx);
+            AAA = exp_in(p.bc_eaaa * lx);
+#else
+            bc_powers(p, S_e, P_k, AAA);
+#endif
+        });
+    return ok && lo >= 0x1p-1000 && hi <= 0x1p1000;
 }
 template <int CL>
 CAPAZ_HD void newton2_ieee(const DevParams& p, double& P, double& Sn, double roS_w, double roS_n) {
-    newton2_with<CL>(p, P, Sn, roS_w, roS_n, [](double det) { return 1. / det; });
+    newton2_with<CL>(
+        p, P, Sn, roS_w, roS_n, [](double det) { return 1. / det; },
+        [&](double S_e, double& P_k, double& AAA) { bc_powers(p, S_e, P_k, AAA); });
 }
 
 // Three-phase fixed-iteration 3x3 Newton (three-phase.cpp:286-339) with the
@@ -738,7 +857,7 @@ CAPAZ_HD double H_r_T(const DevParams& p, double T) { return p.H0_r + (T - kT0) 
 // capacity, mu0 * exp(-a (T - T_ref)), and the water enthalpy as the integral
 // of c_w (energy.cpp:114's cubic term has the opposite sign).
 
-CAPAZ_HD double mu_cfg(const DevParams& p, double mu0, double T) { return mu0 * exp(-p.mu_T_a * (T - p.mu_T_ref)); }
+CAPAZ_HD double mu_cfg(const DevParams& p, double mu0, double T) { return mu0 * exp_t(-p.mu_T_a * (T - p.mu_T_ref)); }
 
 CAPAZ_HD double H_w_of(const DevParams& p, double T) {
     if (p.ecfg)

@@ -119,6 +119,9 @@ inline DevParams derive(const capaz_params& u) {
     p.vg_a = A / (A - 1.);
     p.vg_b = (A - 1.) / A;
     p.vg_c = 2. * (A - 1.) / A;
+    auto moderate = [](double y) { return y >= -1e4 && y <= 1e4; };
+    p.pow_fast = u.model == 3 ? p.vg_c >= 1.1 && p.vg_c <= 1e4 && p.vg_a >= 0.5 && p.vg_a <= 1e4
+                              : moderate(p.bc_ew) && moderate(p.bc_en) && moderate(p.bc_epk) && moderate(p.bc_eaaa);
     // three-phase.cpp:315-316
     p.c_wb = u.ro0_w * u.beta_w;
     p.c_nb = u.ro0_n * u.beta_n;

@@ -309,6 +309,7 @@ __device__ __forceinline__ DevParams coef_params(ConstParams* q) {
     DevParams p;
     if constexpr (CLOSURE == 3) return p;
     p.closure = CLOSURE == 0 ? 0 : 1;
+    if constexpr (CLOSURE == 0) p.pow_fast = q->pow_fast;
     p.P_atm = q->P_atm;
     p.mu_w = q->mu_w, p.r_mu_w = q->r_mu_w;
     p.mu_n = q->mu_n, p.r_mu_n = q->r_mu_n;
@@ -350,6 +351,7 @@ __device__ __forceinline__ DevParams newton_params(ConstParams* q) {
         p.ro0_g = q->ro0_g, p.r_P_atm = q->r_P_atm;
         p.c_wb = q->c_wb, p.c_nb = q->c_nb;
     } else if constexpr (CLOSURE == 0) {
+        p.pow_fast = q->pow_fast;
         p.S_wr = q->S_wr, p.den2 = q->den2, p.r_den2 = q->r_den2, p.P_d = q->P_d;
         p.bc_epk = q->bc_epk, p.bc_eaaa = q->bc_eaaa, p.bc_pks_den = q->bc_pks_den, p.r_bc_pks_den = q->r_bc_pks_den;
     }
@@ -1196,13 +1198,15 @@ __global__ void __launch_bounds__(TX * TY) k_fused_z_record(DevParams p, StepIO 
 // step: three-phase Corey-2 (256^3) 64 x 8 at 4 waves (128 VGPRs, a few spilled)
 // 488, 64 x 4 (whose two LDS buffers leave 3 workgroups per CU) 515; two-phase
 // Corey-2 (256^3) 64 x 4 at 5 waves (95 VGPRs) 285, 64 x 8 at 4 296; the
-// closures that raise powers want registers more than waves: van Genuchten
-// (160 x 144 x 130) 64 x 4 at 3 waves (168 VGPRs) 322, 64 x 8 at 4 waves
-// (128, ~90 spilled) 400; Brooks-Corey (190 x 150 x 110) 235 against 267.
+// closures that raise powers: van Genuchten (160 x 144 x 130) 64 x 8 at 4 waves
+// 241, 64 x 4 at 3 (whose ring re-evaluates 55% of the cells, not 29%) 269;
+// Brooks-Corey (190 x 150 x 110) 213 and 190, its Newton's powers outweighing the
+// ring's; a run-time Corey exponent, three phases (160 x 144 x 130) 187 and 198,
+// two (256^3) 394 and 400.
 template <int MODEL, int CLOSURE, int TY>
-constexpr int kFusedWaves = CLOSURE == 2 ? (MODEL == 2 ? (TY == 4 ? 5 : 4) : (TY == 4 ? 3 : 4)) : (TY == 4 ? 3 : 4);
+constexpr int kFusedWaves = TY == 8 ? 4 : (MODEL == 2 && CLOSURE == 2 ? 5 : 3);
 template <int MODEL, int CLOSURE>
-constexpr int kFusedTileY = MODEL == 3 && CLOSURE == 2 ? 8 : 4;
+constexpr int kFusedTileY = MODEL == 2 && CLOSURE != 1 ? 4 : 8;
 
 template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(kFusedWaves<MODEL, CLOSURE, TY>)))

@@ -39,6 +39,9 @@ struct DevParams {
     double bc_ew, bc_en, bc_epk, bc_eaaa, bc_pks_den, r_bc_pks_den;
     // van Genuchten exponents A/(A-1.), (A-1.)/A, 2.*(A-1.)/A (three-phase.cpp:153-181)
     double vg_a, vg_b, vg_c;
+    // 1: those exponents let the closures' powers go without a test per power
+    // (moderate ones, for which a vanishing base's power vanishes beside 1)
+    int pow_fast;
     // Newton constants: ro0_w*beta_w, ro0_n*beta_n (three-phase.cpp:315-316)
     double c_wb, c_nb;
     // three-phase Border_P top/bottom constants (three-phase.cpp:402-421)

@@ -189,7 +189,7 @@ int capaz_step(capaz_ctx* ctx, long first_step, long nsteps);
  *   "fused_kernel"  0: one thread per cell; 1: z-marching 64 x tile_y tiles
  *                   with two planes' coefficients staged in LDS (default);
  *                   2: as 1
- *   "tile_y"        0, 4 or 8 (default 0: 8 for the three-phase Corey-2 step, 4 otherwise)
+ *   "tile_y"        0, 4 or 8 (default 0: chosen by model and closure)
  *   "kchunk"        planes per workgroup along z (above 32: 32); 0 (default):
  *                   chosen from the grid (16 on large grids, fewer on small
  *                   ones)

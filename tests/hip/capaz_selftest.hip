@@ -7,6 +7,7 @@
 #include <cstdint>
 
 #include "capaz_cell.h"
+#include "capaz_derive.h"
 
 namespace {
 
@@ -87,9 +88,80 @@ __global__ void k_map(int which, const double* x, double* y, uint64_t n) {
     if (i < n) y[i] = which == 0 ? capaz::pow_half(x[i]) : capaz::pow_two(x[i]);
 }
 
+// A cell's closure and, for two phases, its Newton with the powers that go
+// without selects (p.pow_fast) and without: differing values (NaNs aside).
+__global__ void k_closures(capaz::DevParams p, const double* x, const double* y, uint64_t n, unsigned long long* bad) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const uint64_t l = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (l >= n) return;
+    auto differ = [](double a, double b) {
+        return __double_as_longlong(a) != __double_as_longlong(b) && !(a != a && b != b);
+    };
+    capaz::DevParams g = p;
+    g.pow_fast = 0;
+    double a[3] = {}, b[3] = {};
+    if (p.model == 3) {
+        capaz::relperm3(p, x[l], y[l], a[0], a[1], a[2]);
+        capaz::relperm3(g, x[l], y[l], b[0], b[1], b[2]);
+    } else {
+        capaz::relperm2(p, x[l], a[0], a[1], a[2]);
+        capaz::relperm2(g, x[l], b[0], b[1], b[2]);
+    }
+    bool d = differ(a[0], b[0]) || differ(a[1], b[1]) || differ(a[2], b[2]);
+    if (p.model == 2) {
+        double P[2] = {1.1e5, 1.1e5}, S[2] = {x[l], x[l]};
+        const double rw = 0.4 * p.ro0_w * (1 - y[l]), rn = 0.4 * p.ro0_n * y[l];
+        if (capaz::newton2_fast<0>(p, P[0], S[0], rw, rn)) {
+            capaz::newton2_ieee<0>(p, P[1], S[1], rw, rn);
+            d = d || differ(P[0], P[1]) || differ(S[0], S[1]);
+        }
+    }
+    if (d) atomicAdd(bad, 1ull);
+#else
+    (void)p, (void)x, (void)y, (void)n, (void)bad;
+#endif
+}
+
 }  // namespace
 
 extern "C" {
+
+// Number of the n states (two phases: S_n = x and, for Newton's right side,
+// y; three: S_w = x, S_n = y) whose reference closure, with the exponent
+// lambda, differs with and without its powers' selects; -1 on a HIP error, -2
+// if the exponent has no path without them.
+long long capaz_selftest_closures(int model, double lambda, const double* x, const double* y, unsigned long long n) {
+    capaz_params u = {};
+    u.model = model;
+    u.Nx = u.Ny = u.Nz = 3;
+    u.hx = u.hy = u.hz = u.dt = 1.;
+    u.newton_iterations = 3;
+    u.P_atm = 1e5;
+    u.mu_w = u.mu_n = u.mu_g = 1e-3;
+    u.ro0_w = 1000., u.ro0_n = 1460., u.ro0_g = 1.4;
+    u.beta_w = u.beta_n = 4.4e-10;
+    u.lambda = lambda;
+    u.S_wr = 0.09, u.S_nr = 0.05, u.S_gr = 0.01;
+    u.P_d = 755.;
+    const capaz::DevParams p = capaz::derive(u);
+    if (!p.pow_fast) return -2;
+    double *dx = nullptr, *dy = nullptr;
+    unsigned long long *d = nullptr, h = 0;
+    long long rc = -1;
+    const size_t b = n * sizeof(double);
+    if (hipMalloc(&dx, b) == hipSuccess && hipMalloc(&dy, b) == hipSuccess && hipMalloc(&d, sizeof(h)) == hipSuccess &&
+        hipMemcpy(dx, x, b, hipMemcpyHostToDevice) == hipSuccess &&
+        hipMemcpy(dy, y, b, hipMemcpyHostToDevice) == hipSuccess &&
+        hipMemcpy(d, &h, sizeof(h), hipMemcpyHostToDevice) == hipSuccess) {
+        hipLaunchKernelGGL(k_closures, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, p, dx, dy, (uint64_t)n, d);
+        if (hipGetLastError() == hipSuccess && hipMemcpy(&h, d, sizeof(h), hipMemcpyDeviceToHost) == hipSuccess)
+            rc = (long long)h;
+    }
+    if (dx) (void)hipFree(dx);
+    if (dy) (void)hipFree(dy);
+    if (d) (void)hipFree(d);
+    return rc;
+}
 
 // y = pow_half(x) (which = 0) or pow_two(x) (which = 1) on the device for n
 // host doubles; 0, or -1 on a HIP error.

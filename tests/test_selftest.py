@@ -158,3 +158,27 @@ def test_closure_log_is_within_two_ulp_of_log():
     ys = np.empty_like(special)
     assert L.capaz_selftest_log(special.ctypes.data, ys.ctypes.data, special.size) == 0
     assert ys[0] == -np.inf and ys[1] == -np.inf and ys[2] == np.inf and np.isnan(ys[3]) and np.isnan(ys[4])
+
+
+@pytest.mark.parametrize("model,lam", [(3, 3.25), (3, 2.25), (3, 40.0), (2, 2.7), (2, 0.4), (2, 8.0)])
+def test_closures_without_the_powers_selects_have_the_same_bits(model, lam):
+    """The reference closures' short path (a device test per cell, none per
+    power) against the general one, over states inside the saturations' range,
+    on its edges (effective saturations 0, 1, the 1e-3 cuts, residuals) and
+    outside it, infinities and NaN included."""
+    from capaz_amd import capaz
+    capaz.load()
+    L = ctypes.CDLL(LIB)
+    L.capaz_selftest_closures.restype = ctypes.c_longlong
+    L.capaz_selftest_closures.argtypes = [ctypes.c_int, ctypes.c_double, ctypes.c_void_p, ctypes.c_void_p,
+                                          ctypes.c_ulonglong]
+    rng = np.random.default_rng(11)
+    den = 1.0 - 0.09 - 0.05 - 0.01
+    edges = np.array([0.0, -0.0, 1e-3, 0.999, 1.0, 1.0 + 1e-16, 1e-9, -1e-9, 5e-324, 0.5, -0.5, 1.5])
+    sw = np.concatenate([0.09 + den * edges, edges, [np.inf, -np.inf, np.nan, 1e300, 0.91]])
+    sn = np.concatenate([0.05 + den * edges, edges, [np.inf, -np.inf, np.nan, 1e300, 0.91]])
+    ex, ey = (a.ravel() for a in np.meshgrid(sw, sn))
+    u = rng.uniform(0.0, 1.0, (2, 1 << 20))
+    x = np.ascontiguousarray(np.concatenate([ex, u[0], u[0] ** 6, 0.91 - u[0] ** 6, rng.uniform(-0.3, 1.3, 1 << 20)]))
+    y = np.ascontiguousarray(np.concatenate([ey, u[1] * (1 - u[0]), u[1], u[1] ** 6, rng.uniform(-0.3, 1.3, 1 << 20)]))
+    assert L.capaz_selftest_closures(model, lam, x.ctypes.data, y.ctypes.data, x.size) == 0
