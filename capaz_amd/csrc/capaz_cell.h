@@ -1026,6 +1026,70 @@ CAPAZ_HD bool newton_energy2_t(const DevParams& p, double& Sw, double& Sn, doubl
     return true;
 }
 
+// newton_energy2_t for a kernel's hot path, with no call and no branch per
+// iteration, H_* taken from T where an iteration begins: false (and any
+// values) if some pivot lay outside DivisorRange; newton_energy2_t<false> then
+// redoes the cell.  The inverse is reverse_matrix<4>'s operations on the
+// entries that the system's zeros and ones leave to be computed,
+//   row 0: 1 1 0 0 | row 1: rw 0 a b | row 2: 0 rn c d | row 3: e f g h:
+// the first pivot is 1; the second is -rw, and its row's -rw / -rw is 1; the
+// first two rows' entries right of there differ in sign, but for column 4.
+// The same bits up to the sign of entries that are exactly 0 (finite entries:
+// a rw or rn that is not makes a pivot that is not).
+CAPAZ_HD bool newton_energy2_fast(const DevParams& p, double& Sw, double& Sn, double& P, double& T, double m,
+                                  double roS_w, double roS_n, double E_new) {
+    DivisorRange range;
+    const double dwP = p.ro0_w * p.beta_w, dwT = (-1) * p.ro0_w * kAlfaW;
+    const double dnP = p.ro0_n * p.beta_n, dnT = (-1) * p.ro0_n * kAlfaN;
+    for (int w = 1; w <= p.iterations; w++) {
+        const double Hw = H_w_of(p, T), Hn = H_n_T(p, T), Hr = H_r_of(p, T);
+        const double rw = ro_w_T(p, P, T), rn = ro_n_T(p, P, T);
+        const double F0 = Sw + Sn - 1., F1 = rw * Sw - roS_w, F2 = rn * Sn - roS_n;
+        const double ew = rw * Hw - P, en = rn * Hn - P;
+        const double F3 = m * (Sw * ew + Sn * en) + (1. - m) * (p.ro_r * Hr - P) - E_new;
+        const double a = dwP * Sw, b = dwT * Sw, c = dnP * Sn, d = dnT * Sn, e = m * ew, f = m * en;
+        const double g = m * (Sw * (dwP * Hw - 1.) + Sn * (dnP * Hn - 1.)) + (1. - m) * (-1);
+        const double h = m * (Sw * (dwT * Hw + rw * c_w_T(T)) + Sn * (dnT * Hn + rn * c_n_T(T))) +
+                         (1. - m) * p.ro_r * c_r_of(p, T);
+        // pivot 1 (-rw)
+        const double nrw = -rw;
+        range.see(nrw);
+        const double r1 = rcp_in_range(nrw);
+        const double s2 = exact_div(a, nrw, r1), s3 = exact_div(b, nrw, r1);
+        const double v = f - e;
+        double m22 = c - s2 * rn, m23 = d - s3 * rn, m25 = -(r1 * rn);
+        double m32 = g - s2 * v, m33 = h - s3 * v, m34 = -e - v, m35 = -(r1 * v);
+        // pivot 2
+        range.see(m22);
+        const double r2 = rcp_in_range(m22);
+        const double t3 = exact_div(m23, m22, r2), t4 = exact_div(-rn, m22, r2), t5 = exact_div(m25, m22, r2);
+        double m04 = t4 * s2, m14 = 1. - m04;
+        const double m13 = s3 - t3 * s2;  // -m03
+        double m15 = r1 - t5 * s2;        // -m05
+        double m16 = -(r2 * s2);          // -m06
+        m33 = m33 - t3 * m32;
+        m34 = m34 - t4 * m32;
+        m35 = m35 - t5 * m32;
+        const double m36 = -(r2 * m32);
+        // pivot 3
+        range.see(m33);
+        const double r3 = rcp_in_range(m33);
+        const double u4 = exact_div(m34, m33, r3), u5 = exact_div(m35, m33, r3), u6 = exact_div(m36, m33, r3);
+        m04 = m04 + u4 * m13;
+        m14 = m14 - u4 * m13;
+        m15 = m15 - u5 * m13;
+        m16 = m16 - u6 * m13;
+        const double m17 = -(r3 * m13);
+        const double o24 = t4 - u4 * t3, o25 = t5 - u5 * t3, o26 = r2 - u6 * t3, o27 = -(r3 * t3);
+        const double q1 = m15 * F1, q2 = m16 * F2, q3 = m17 * F3;
+        Sw = Sw - (m04 * F0 - q1 - q2 - q3);
+        Sn = Sn - (m14 * F0 + q1 + q2 + q3);
+        P = P - (o24 * F0 + o25 * F1 + o26 * F2 + o27 * F3);
+        T = T - (u4 * F0 + u5 * F1 + u6 * F2 + r3 * F3);
+    }
+    return range.ok();
+}
+
 // ---- three-phase Border_P faces (three-phase.cpp:383-422) ---------------------------------
 
 // Sets (P_w, P_n, P_g) of a boundary cell in row j from the inward

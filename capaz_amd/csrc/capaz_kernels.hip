@@ -285,7 +285,7 @@ int resident_groups(int threads) {
     return cached;
 }
 
-int fused_kchunk(const DevParams& p, int kchunk, int ty, int resident) {
+int fused_kchunk(const DevParams& p, int kchunk, int ty, int resident, int tx) {
     if (kchunk >= 1) return std::min(kchunk, kMaxPlanes);
     // automatic: the planes per tile that minimise (rounds of resident
     // workgroups) x (planes per tile + the tile's extra coefficient planes).
@@ -293,7 +293,7 @@ int fused_kchunk(const DevParams& p, int kchunk, int ty, int resident) {
     // 24^3 three-phase step takes 12.7 us against 15.9 with two (40^3 two
     // phases: 7.4 against 8.5), each plane's latency being a quarter of that.
     const int64_t nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
-    const int64_t txy = ((nx + 63) / 64) * ((ny + ty - 1) / ty);
+    const int64_t txy = ((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
     int best = 16;
     double best_cost = -1.;
     for (int kc = 1; kc <= 16; ++kc) {

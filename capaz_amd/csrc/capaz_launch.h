@@ -75,7 +75,7 @@ hipError_t launch_energy2_step(const DevParams& p, const double* const* cur, dou
 // Planes per tile of the fused z kernels: kchunk if >= 1, else chosen from
 // the grid and the number of workgroups resident at once, so that small grids
 // fill the GPU without a nearly empty last round.
-int fused_kchunk(const DevParams& p, int kchunk, int ty, int resident);
+int fused_kchunk(const DevParams& p, int kchunk, int ty, int resident, int tx = 64);
 // One fused three-phase step (Corey closures, 64 x 8 tiles) that also writes
 // each interior cell's flux divergence of phase a to div[a*stride + l].
 hipError_t launch_fused_record(const DevParams& p, const StepIO& io, int kchunk, double* div, int64_t stride,

@@ -130,6 +130,38 @@ def test_pivot_search_cells_equal_the_oracle():
     b.close()
 
 
+@pytest.mark.parametrize("dims,tune", [((34, 18, 40), dict(kchunk=64)), ((66, 17, 6), dict(kchunk=2)),
+                                       ((33, 35, 3), dict()), ((35, 19, 1), dict()), ((3, 34, 5), dict(kchunk=1))],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else "")
+@pytest.mark.parametrize("closure", ["corey", "corey-n", "reference"])
+@pytest.mark.parametrize("beta", [1e-6, 0.0], ids=["", "pivot-search"])
+def test_tile_edges_equal_the_entry_points(dims, tune, closure, beta):
+    """Grids at the edges of the fused kernel's 32 x 16 tiles and chunks, each
+    closure, with every cell's Newton in the planes and (beta 0) every one left
+    for after them: the entry points' bits after one step and, where the state
+    stays finite, after three."""
+    keys = case("2phe", *dims, P_BOTTOM=0.0, SOURCE=1, BETA_W=beta, BETA_N=beta,
+                CLOSURE="corey" if closure != "reference" else closure)
+    if closure == "corey-n":
+        keys["COREY_N"] = 2.5
+    if closure == "reference":
+        keys.update(LAMBDA_0=2.7, P_D_0=755.0, S_WR_0=0.09)
+    st = random_state(keys, sum(dims))
+    a, b = capaz.Domain(keys, st), capaz.Domain(keys, st)
+    a.tune(energy_kernel=1, **tune)
+    b.tune(energy_kernel=0)
+    for first, count in ((1, 1),) + (((2, 2),) if beta else ()):
+        a.run(count, first_step=first)
+        b.run(count, first_step=first)
+        for f in a.names:
+            x, y = a.field(f), b.field(f)
+            fin = np.isfinite(y)
+            assert fin.all() or not beta, f
+            assert np.array_equal(np.isfinite(x), fin) and bit_equal(x[fin], y[fin]), (first, f)
+    a.close()
+    b.close()
+
+
 def test_whole_run_40_within_1e9():
     """The non-isothermal physics at the Buckley-Leverett workload's 40^3
     size over 1000 steps: every field within 1e-9 of the oracle."""
