@@ -10,6 +10,8 @@
 // interior P_n / P_g); they are marked stale and recomputed from the previous
 // state -- which the second arrays still hold -- before anything reads them,
 // so every field always reads as after the same number of reference steps.
+// Reading or writing the stored state itself (P_w, S_n, S_w of three phases, T)
+// leaves them stale.
 // The three-phase energy model's step (six passes) works in place like the
 // sequence; the two-phase energy model's fused step ping-pongs P_w, S_n and T
 // and re-runs the step's entry points from the previous state when a caller
@@ -124,6 +126,20 @@ int materialize(capaz_ctx* c) {
     c->stale = false;
     return CAPAZ_OK;
 }
+
+// The arrays that are the field's as they are after a fused step: the state it
+// writes whole.  (P_n and P_g of the three-phase model it writes on the
+// boundary only.)
+bool stored_whole(const capaz_ctx* c, int f) {
+    return c->primary[f] && !(c->user.model == 3 && (f == capaz::F_P_n || f == capaz::F_P_g));
+}
+
+// Before field f is read or written: the last step's intermediates, unless f is
+// a state field that step has stored.  Reading such a field needs none of them
+// -- five 256^3 three-phase steps and a read of P_w, S_w and S_n take 2.5 ms
+// where the intermediates took another 1.9 -- and writing it leaves what they
+// are recomputed from, the previous state, as it was.
+int prepare_field(capaz_ctx* c, int f) { return stored_whole(c, f) ? CAPAZ_OK : materialize(c); }
 
 int check_ctx(capaz_ctx* c) {
     if (!c) return CAPAZ_ERR_INVALID;
@@ -331,7 +347,7 @@ int capaz_set_field(capaz_ctx* c, int field, const double* host, size_t n) {
     if ((rc = check_ctx(c))) return rc;
     if ((rc = check_field(c, field, n))) return rc;
     if (!host) return fail(c, CAPAZ_ERR_INVALID, "NULL host pointer");
-    if ((rc = materialize(c))) return rc;
+    if ((rc = prepare_field(c, field))) return rc;
     CAPAZ_HIP(c, hipMemcpyAsync(c->cur[field], host, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
     CAPAZ_HIP(c, hipStreamSynchronize(c->stream));
     if (field == capaz::F_m) c->m_checked = false;
@@ -343,7 +359,7 @@ int capaz_set_field_device(capaz_ctx* c, int field, const double* dsrc, size_t n
     if ((rc = check_ctx(c))) return rc;
     if ((rc = check_field(c, field, n))) return rc;
     if (!dsrc) return fail(c, CAPAZ_ERR_INVALID, "NULL device pointer");
-    if ((rc = materialize(c))) return rc;
+    if ((rc = prepare_field(c, field))) return rc;
     CAPAZ_HIP(c, hipMemcpyAsync(c->cur[field], dsrc, n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
     if (field == capaz::F_m) c->m_checked = false;
     return CAPAZ_OK;
@@ -354,7 +370,7 @@ int capaz_get_field(capaz_ctx* c, int field, double* host, size_t n) {
     if ((rc = check_ctx(c))) return rc;
     if ((rc = check_field(c, field, n))) return rc;
     if (!host) return fail(c, CAPAZ_ERR_INVALID, "NULL host pointer");
-    if ((rc = materialize(c))) return rc;
+    if ((rc = prepare_field(c, field))) return rc;
     CAPAZ_HIP(c, hipMemcpyAsync(host, c->cur[field], n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     CAPAZ_HIP(c, hipStreamSynchronize(c->stream));
     return CAPAZ_OK;
@@ -365,7 +381,7 @@ int capaz_field_device_ptr(capaz_ctx* c, int field, double** dptr) {
     if ((rc = check_ctx(c))) return rc;
     if (!field_exists(c->user, field)) return fail(c, CAPAZ_ERR_INVALID, "field does not exist for this model");
     if (!dptr) return fail(c, CAPAZ_ERR_INVALID, "NULL dptr");
-    if ((rc = materialize(c))) return rc;
+    if ((rc = prepare_field(c, field))) return rc;
     *dptr = c->cur[field];
     if (field == capaz::F_m) c->m_checked = false;  // the caller may write through the pointer
     return CAPAZ_OK;

@@ -158,7 +158,10 @@ int capaz_set_field(capaz_ctx* ctx, int field, const double* host, size_t n);
 int capaz_get_field(capaz_ctx* ctx, int field, double* host, size_t n);
 
 /* Device address of a field's current array (valid until the next call on
- * the context), for callers that share device memory, e.g. torch tensors. */
+ * the context), for callers that share device memory, e.g. torch tensors.
+ * After capaz_step the state it stores (P_w, S_n, S_w of three phases, T) is
+ * there as it is; the first access to another field recomputes the last
+ * step's intermediates. */
 int capaz_field_device_ptr(capaz_ctx* ctx, int field, double** dptr);
 
 /* Device-to-device copy of n doubles into a field (stream-ordered). */

@@ -227,6 +227,42 @@ def test_tile_cells_done_after_the_planes(dims, tune, closure):
         assert np.isfinite(b["P_w"]).all()
 
 
+@pytest.mark.parametrize("model,state", [("2ph", ("P_w", "S_n")), ("3ph", ("P_w", "S_w", "S_n")),
+                                         ("2phe", ("P_w", "S_n", "T")), ("3phe", ("P_w", "S_w", "S_n", "T"))])
+@pytest.mark.parametrize("write", ["set_field", "device"])
+def test_state_read_and_written_before_the_intermediates(model, state, write):
+    """After fused steps the state fields are read and written as they stand,
+    the intermediates recomputed later: every field as where all of them were
+    read first, then after one more step, too."""
+    keys = case(model, 19, 11, 10)
+    st = random_state(keys, seed=3)
+    got = []
+    for first in (False, True):
+        d = capaz.Domain(keys, st)
+        d.run(3)
+        if first:
+            d.fields()
+        read = {f: d.field(f) for f in state}
+        for f in state:
+            v = np.ascontiguousarray(read[f] * 0.999)
+            if write == "set_field":
+                d.set_field(f, v)
+            else:  # device to device, from another domain's array
+                o = capaz.Domain(keys, dict(st, **{f: v}))
+                o.sync()
+                capaz.load().capaz_set_field_device(d._ctx, capaz.FIELD_ID[f], o.device_ptr(f), v.size)
+                d.sync()
+                o.close()
+            assert bit_equal(d.field(f), v)
+        one = d.fields()
+        d.run(1, first_step=4)
+        got.append((read, one, d.fields()))
+        d.close()
+    for a, b in zip(*got):
+        for f in b:
+            assert bit_equal(a[f], b[f]), f
+
+
 @pytest.mark.parametrize("model,tune", [("3ph", dict(tile_y=8)), ("3ph", dict(tile_y=4)), ("3phe", dict()),
                                         ("3phe", dict(energy_kernel=0))])
 @pytest.mark.parametrize("nx", [1 << 20, (1 << 20) + 1024])
