@@ -136,7 +136,7 @@ bool stored_whole(const capaz_ctx* c, int f) {
 
 // Before field f is read or written: the last step's intermediates, unless f is
 // a state field that step has stored.  Reading such a field needs none of them
-// -- five 256^3 three-phase steps and a read of P_w, S_w and S_n take 2.5 ms
+// -- ten 256^3 three-phase steps and a read of P_w, S_w and S_n take 4.8 ms
 // where the intermediates took another 1.9 -- and writing it leaves what they
 // are recomputed from, the previous state, as it was.
 int prepare_field(capaz_ctx* c, int f) { return stored_whole(c, f) ? CAPAZ_OK : materialize(c); }

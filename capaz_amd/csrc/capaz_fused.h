@@ -265,9 +265,9 @@ __device__ __forceinline__ void st(double* f, const CellAt& a, double v) {
 }
 
 // A tile's halo cell (hi, hj) of a plane: from the cell below and left of the
-// tile's first (i0, j0), whose index is uniform, a lane offset of up to 9 rows,
-// below 2^32 bytes for rows of at most kMaxRow32 cells (which leaves a factor
-// of 50); with(k, f) calls f with the cell of plane k, by its own 64-bit index
+// tile's first (i0, j0), whose index is uniform, a lane offset of up to 19
+// rows, below 2^32 bytes for rows of at most kMaxRow32 cells (which leaves a
+// factor of 25); with(k, f) calls f with the cell of plane k, by its own 64-bit index
 // in wider grids.
 constexpr int kMaxRow32 = 1 << 20;
 struct HaloAt {
@@ -1007,7 +1007,8 @@ __global__ void __launch_bounds__(TX * TY) k_roS_z(DevParams p, StepIO io, int k
 // Bound by memory (14 fields read and one written per cell): the next plane's
 // loads are issued before this plane's sums and one barrier ends a plane (two
 // LDS buffers).  160 x 128 x 96: 92 us against 115 for tiles that read the
-// fields again for the z neighbours.
+// fields again for the z neighbours (32 x 16 tiles, whose threads cover the 158
+// columns without the sixth that 64 x 8 leave idle: 88, and roS 98 against 95).
 //
 // LAM, where lambda_eff comes from: kLamStored, lam as the step's first pass
 // stored it; kLamEvaluated (the entry point), from m, S_w, S_n, S_g and T;
@@ -1194,22 +1195,30 @@ __global__ void __launch_bounds__(TX * TY) k_fused_z_record(DevParams p, StepIO 
                                                    FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE>{io}, div, stride});
 }
 
-// Waves per SIMD and the automatic tile height.  Measured on one MI355X, us per
-// step: three-phase Corey-2 (256^3) 64 x 8 at 4 waves (128 VGPRs, a few spilled)
-// 488, 64 x 4 (whose two LDS buffers leave 3 workgroups per CU) 515; two-phase
-// Corey-2 (256^3) 64 x 4 at 5 waves (95 VGPRs) 285, 64 x 8 at 4 296; the
-// closures that raise powers: van Genuchten (160 x 144 x 130) 64 x 8 at 4 waves
-// 241, 64 x 4 at 3 (whose ring re-evaluates 55% of the cells, not 29%) 269;
-// Brooks-Corey (190 x 150 x 110) 213 and 190, its Newton's powers outweighing the
-// ring's; a run-time Corey exponent, three phases (160 x 144 x 130) 187 and 198,
-// two (256^3) 394 and 400.
-template <int MODEL, int CLOSURE, int TY>
-constexpr int kFusedWaves = TY == 8 ? 4 : (MODEL == 2 && CLOSURE == 2 ? 5 : 3);
+// Waves per SIMD of the step's tiles, and their shapes per model and closure: a
+// wide one, 64 x kWideTY, and a narrow one, 32 x kNarrowTY, of which the launch
+// takes the one whose workgroups cover the grid's columns with fewer threads,
+// and 64 x 4 for grids so small that its workgroups all fit at once.  us per
+// step, wide / narrow, and per thread and plane of the covering workgroups (ps):
+//   three phases, Corey-2   256^3 498 / 498 (29.9 / 29.9), 203 x 117 x 83 76.1 / 67.7 (30.6 / 29.2)
+//     van Genuchten         160 x 144 x 130 237 / 195 (66.9 / 66.0)
+//     run-time exponent     160 x 144 x 130 185 / 152
+//   two phases, Corey-2     256^3 288 / 285, 96^3 26.5 / 21.4
+//     Brooks-Corey          190 x 150 x 110 192 / 209 (62.6 / 63.0), 160^3 290 / 243 (59.7 / 60.2)
+//     run-time exponent     256^3 398 / 391
+// the other shapes of 256 and 512 threads are slower or equal, but in small
+// grids, where a workgroup's latency counts: three phases 24^3 64 x 4 10.8,
+// 64 x 8 12.5, 32 x 16 12.1; 48^3 15.0, 18.2, 18.2.  Registers: 128 VGPRs at 4
+// waves (a few spilled for three phases), 95 at 5, 168 at 3.
+template <int MODEL, int CLOSURE, int TX, int TY>
+constexpr int kFusedWaves = TX * TY == 512 ? 4 : (MODEL == 2 && CLOSURE == 2 ? 5 : 3);
 template <int MODEL, int CLOSURE>
-constexpr int kFusedTileY = MODEL == 2 && CLOSURE != 1 ? 4 : 8;
+constexpr int kWideTY = MODEL == 2 && CLOSURE != 1 ? 4 : 8;
+template <int MODEL, int CLOSURE>
+constexpr int kNarrowTY = MODEL == 2 && CLOSURE == 2 ? 8 : 16;
 
 template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
-__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(kFusedWaves<MODEL, CLOSURE, TY>)))
+__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(kFusedWaves<MODEL, CLOSURE, TX, TY>)))
 k_fused_z(DevParams p, StepIO io, int kchunk) {
     __shared__ FusedLds<MODEL, CLOSURE, TX, TY> lds;
     int bx, by, bz;

@@ -327,15 +327,30 @@ hipError_t launch_pack_model(const DevParams& p, const StepIO& io, hipStream_t s
     return launch_pack<MODEL, 1>(p, io, s);
 }
 
-template <int MODEL, int CLOSURE, int TY, bool FULL>
+// Threads of the TX x TY workgroups that cover the interior columns.
+int64_t covering_threads(const DevParams& p, int TX, int TY) {
+    const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2;
+    return (int64_t)((nx + TX - 1) / TX) * TX * ((ny + TY - 1) / TY) * TY;
+}
+// f(TX, TY) (integral constants) with the better of a wide and a narrow shape
+// (the comment at kWideTY).
+template <int WIDE_TY, int NARROW_TY, class F>
+hipError_t with_tile(const DevParams& p, const F& f) {
+    using std::integral_constant;
+    if (covering_threads(p, 32, NARROW_TY) <= covering_threads(p, 64, WIDE_TY))
+        return f(integral_constant<int, 32>{}, integral_constant<int, NARROW_TY>{});
+    return f(integral_constant<int, 64>{}, integral_constant<int, WIDE_TY>{});
+}
+
+template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
 hipError_t launch_z(const DevParams& p, const StepIO& io, int kchunk, hipStream_t s, const KernelEvents* ev) {
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
-    constexpr auto kernel = k_fused_z<MODEL, CLOSURE, 64, TY, FULL>;
-    kchunk = fused_kchunk(p, kchunk, TY, resident_groups<kernel>(64 * TY));
-    dim3 grid((nx + 63) / 64, (ny + TY - 1) / TY, (nz + kchunk - 1) / kchunk);
+    constexpr auto kernel = k_fused_z<MODEL, CLOSURE, TX, TY, FULL>;
+    kchunk = fused_kchunk(p, kchunk, TY, resident_groups<kernel>(TX * TY), TX);
+    dim3 grid((nx + TX - 1) / TX, (ny + TY - 1) / TY, (nz + kchunk - 1) / kchunk);
     hipError_t e;
     if (ev && (e = hipEventRecord(ev->begin, s)) != hipSuccess) return e;
-    hipLaunchKernelGGL(kernel, grid, dim3(64, TY), 0, s, p, io, kchunk);
+    hipLaunchKernelGGL(kernel, grid, dim3(TX, TY), 0, s, p, io, kchunk);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (ev && (e = hipEventRecord(ev->end, s)) != hipSuccess) return e;
     if constexpr (!kFusedFaces<MODEL>) {
@@ -351,23 +366,28 @@ hipError_t launch_z(const DevParams& p, const StepIO& io, int kchunk, hipStream_
 }
 
 template <int MODEL, int CLOSURE>
-hipError_t launch_z_ty(const DevParams& p, const StepIO& io, const Tuning& t, hipStream_t s, const KernelEvents* ev) {
-    const bool full = p.Nx >= 3 && p.Nz >= 3;
-    const int ty = t.tile_y ? t.tile_y : kFusedTileY<MODEL, CLOSURE>;
-    if (ty == 8)
-        return full ? launch_z<MODEL, CLOSURE, 8, true>(p, io, t.kchunk, s, ev)
-                    : launch_z<MODEL, CLOSURE, 8, false>(p, io, t.kchunk, s, ev);
-    return full ? launch_z<MODEL, CLOSURE, 4, true>(p, io, t.kchunk, s, ev)
-                : launch_z<MODEL, CLOSURE, 4, false>(p, io, t.kchunk, s, ev);
+hipError_t launch_z_tile(const DevParams& p, const StepIO& io, const Tuning& t, hipStream_t s, const KernelEvents* ev) {
+    auto launch = [&](auto tx, auto ty) {
+        constexpr int TX = decltype(tx)::value, TY = decltype(ty)::value;
+        return p.Nx >= 3 && p.Nz >= 3 ? launch_z<MODEL, CLOSURE, TX, TY, true>(p, io, t.kchunk, s, ev)
+                                      : launch_z<MODEL, CLOSURE, TX, TY, false>(p, io, t.kchunk, s, ev);
+    };
+    using std::integral_constant;
+    const int64_t groups = covering_threads(p, 64, 4) / 256 * (p.Nz >= 3 ? p.Nz - 2 : 1);
+    const bool small = groups <= resident_groups<k_fused_z<MODEL, CLOSURE, 64, 4, true>>(256);
+    if (t.tile_y == 4 || (t.tile_y == 0 && small))
+        return launch(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+    if (t.tile_y == 8) return launch(integral_constant<int, 64>{}, integral_constant<int, 8>{});
+    return with_tile<kWideTY<MODEL, CLOSURE>, kNarrowTY<MODEL, CLOSURE>>(p, launch);
 }
 
 // CLOSURE ids of the fused kernels: 0 reference, 1 Corey with a run-time
 // exponent, 2 Corey with exponent 2 (no pow in the kernel).
 template <int MODEL>
 hipError_t launch_z_model(const DevParams& p, const StepIO& io, const Tuning& t, hipStream_t s, const KernelEvents* ev) {
-    if (p.closure == 0) return launch_z_ty<MODEL, 0>(p, io, t, s, ev);
-    if (p.corey_n == 2.) return launch_z_ty<MODEL, 2>(p, io, t, s, ev);
-    return launch_z_ty<MODEL, 1>(p, io, t, s, ev);
+    if (p.closure == 0) return launch_z_tile<MODEL, 0>(p, io, t, s, ev);
+    if (p.corey_n == 2.) return launch_z_tile<MODEL, 2>(p, io, t, s, ev);
+    return launch_z_tile<MODEL, 1>(p, io, t, s, ev);
 }
 
 hipError_t launch_fused(const DevParams& p, const StepIO& io, const Tuning& t, hipStream_t s, const KernelEvents* ev) {
@@ -381,37 +401,40 @@ hipError_t launch_fused(const DevParams& p, const StepIO& io, const Tuning& t, h
     return p.model == 3 ? launch_z_model<3>(p, io, t, s, ev) : launch_z_model<2>(p, io, t, s, ev);
 }
 
-template <int MODEL, int CLOSURE, bool FULL>
+template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
 hipError_t launch_record(const DevParams& p, const StepIO& io, int kchunk, double* div, int64_t stride,
                          hipStream_t s) {
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
-    constexpr auto kernel = k_fused_z_record<MODEL, CLOSURE, 64, 8, FULL>;
-    kchunk = fused_kchunk(p, kchunk, 8, resident_groups<kernel>(512));
-    dim3 grid((nx + 63) / 64, (ny + 7) / 8, (nz + kchunk - 1) / kchunk);
-    hipLaunchKernelGGL(kernel, grid, dim3(64, 8), 0, s, p, io, kchunk, div, stride);
+    constexpr auto kernel = k_fused_z_record<MODEL, CLOSURE, TX, TY, FULL>;
+    kchunk = fused_kchunk(p, kchunk, TY, resident_groups<kernel>(TX * TY), TX);
+    dim3 grid((nx + TX - 1) / TX, (ny + TY - 1) / TY, (nz + kchunk - 1) / kchunk);
+    hipLaunchKernelGGL(kernel, grid, dim3(TX, TY), 0, s, p, io, kchunk, div, stride);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || kFusedFaces<MODEL>) return e;  // two phases: the tiles write the boundary cells
     hipLaunchKernelGGL((k_fused_faces<MODEL, CLOSURE>), grid_for(fused_face_cells(p)), dim3(256), 0, s, p, io);
     return hipGetLastError();
 }
 template <int MODEL, int CLOSURE>
-hipError_t launch_record_full(const DevParams& p, const StepIO& io, int kchunk, double* div, int64_t stride,
+hipError_t launch_record_tile(const DevParams& p, const StepIO& io, int kchunk, double* div, int64_t stride,
                               hipStream_t s) {
-    return p.Nx >= 3 && p.Nz >= 3 ? launch_record<MODEL, CLOSURE, true>(p, io, kchunk, div, stride, s)
-                                  : launch_record<MODEL, CLOSURE, false>(p, io, kchunk, div, stride, s);
+    return with_tile<8, 16>(p, [&](auto tx, auto ty) {
+        constexpr int TX = decltype(tx)::value, TY = decltype(ty)::value;
+        return p.Nx >= 3 && p.Nz >= 3 ? launch_record<MODEL, CLOSURE, TX, TY, true>(p, io, kchunk, div, stride, s)
+                                      : launch_record<MODEL, CLOSURE, TX, TY, false>(p, io, kchunk, div, stride, s);
+    });
 }
 
 hipError_t launch_fused_record(const DevParams& p, const StepIO& io, int kchunk, double* div, int64_t stride,
                                hipStream_t s) {
     if (p.model == 2) {
         if (p.closure == 0) return hipErrorInvalidValue;  // the Corey closures
-        return p.corey_n == 2. ? launch_record_full<2, 2>(p, io, kchunk, div, stride, s)
-                               : launch_record_full<2, 1>(p, io, kchunk, div, stride, s);
+        return p.corey_n == 2. ? launch_record_tile<2, 2>(p, io, kchunk, div, stride, s)
+                               : launch_record_tile<2, 1>(p, io, kchunk, div, stride, s);
     }
     if (p.model != 3) return hipErrorInvalidValue;
-    if (p.closure == 0) return launch_record_full<3, 0>(p, io, kchunk, div, stride, s);
-    return p.corey_n == 2. ? launch_record_full<3, 2>(p, io, kchunk, div, stride, s)
-                           : launch_record_full<3, 1>(p, io, kchunk, div, stride, s);
+    if (p.closure == 0) return launch_record_tile<3, 0>(p, io, kchunk, div, stride, s);
+    return p.corey_n == 2. ? launch_record_tile<3, 2>(p, io, kchunk, div, stride, s)
+                           : launch_record_tile<3, 1>(p, io, kchunk, div, stride, s);
 }
 
 // roS (and, with U, u) of the interior cells on the z tiles, from the P, Xi
@@ -440,6 +463,7 @@ hipError_t launch_roS_tiles(const DevParams& p, const DevFields& F, const double
         for (int x = 0; x < 3; ++x) st.u[a][x] = U ? F.f[uf[a][x]] : nullptr;
     }
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
+    // bound by memory: the narrow tiles' smaller cover gains nothing here
     auto launch = [&](auto full) {
         constexpr auto kernel = k_roS_z<64, 8, decltype(full)::value, U>;
         const int kchunk = fused_kchunk(p, 0, 8, resident_groups<kernel>(512));

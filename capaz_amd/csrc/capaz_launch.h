@@ -30,7 +30,7 @@ enum class Entry { S, P_Xi_ro, U, RoS, HE, E, Newton, Boundary };
 struct Tuning {
     int check_every = 0;  // non-finite sentinel after every check_every-th step (0: off)
     int fused_kernel = 1;
-    int tile_y = 0;  // 0: automatic (kFusedTileY)
+    int tile_y = 0;  // 0: automatic (kWideTY, kNarrowTY)
     int kchunk = 0;
     int adjoint_kernel = 2;
     int adjoint_streams = 2;
@@ -76,7 +76,7 @@ hipError_t launch_energy2_step(const DevParams& p, const double* const* cur, dou
 // the grid and the number of workgroups resident at once, so that small grids
 // fill the GPU without a nearly empty last round.
 int fused_kchunk(const DevParams& p, int kchunk, int ty, int resident, int tx = 64);
-// One fused three-phase step (Corey closures, 64 x 8 tiles) that also writes
+// One fused step (two phases: Corey closures) that also writes
 // each interior cell's flux divergence of phase a to div[a*stride + l].
 hipError_t launch_fused_record(const DevParams& p, const StepIO& io, int kchunk, double* div, int64_t stride,
                                hipStream_t s);

@@ -189,10 +189,11 @@ int capaz_step_sequence(capaz_ctx* ctx, double t);
 int capaz_step(capaz_ctx* ctx, long first_step, long nsteps);
 
 /* Launch shape of capaz_step's kernels (does not change results):
- *   "fused_kernel"  0: one thread per cell; 1: z-marching 64 x tile_y tiles
- *                   with two planes' coefficients staged in LDS (default);
+ *   "fused_kernel"  0: one thread per cell; 1: z-marching tiles with two
+ *                   planes' coefficients staged in LDS (default);
  *                   2: as 1
- *   "tile_y"        0, 4 or 8 (default 0: chosen by model and closure)
+ *   "tile_y"        4 or 8: tiles of 64 x tile_y columns; 0 (default): their
+ *                   shape chosen by model, closure and grid
  *   "kchunk"        planes per workgroup along z (above 32: 32); 0 (default):
  *                   chosen from the grid (16 on large grids, fewer on small
  *                   ones)

@@ -227,6 +227,33 @@ def test_tile_cells_done_after_the_planes(dims, tune, closure):
         assert np.isfinite(b["P_w"]).all()
 
 
+# interior columns that 32 x 16 and 32 x 8 workgroups cover with fewer threads than
+# 64 x 8 and 64 x 4 ones (28 x 13, 32 x 16, 95 x 17), and not (62 x 19); planes
+# enough that the workgroups do not all fit at once; one plane
+@pytest.mark.parametrize("dims", [(30, 15, 402), (34, 18, 402), (97, 19, 135), (64, 21, 300), (3, 530, 9), (1, 4099, 5),
+                                  (3000, 40, 1)])
+@pytest.mark.parametrize("model,over", [("3ph", dict(CLOSURE="corey")), ("3ph", dict()), ("3ph", dict(CLOSURE="corey", COREY_N=2.5)),
+                                        ("2ph", dict(CLOSURE="corey")), ("2ph", dict()), ("2ph", dict(CLOSURE="corey", COREY_N=2.5)),
+                                        ("3phe", dict(CLOSURE="corey"))])
+def test_narrow_and_wide_tiles_equal_the_per_cell_step(model, over, dims):
+    """The tile shape that the launch chooses by the columns it covers: every
+    field as from one thread per cell (with the energy equation, as from the
+    entry points) after 2 steps."""
+    if model == "2ph" and dims[0] < 3:
+        pytest.skip("two phases need Nx >= 3")
+    keys = case(model, *dims, DT=1e-5, SOURCE=1, **over)
+    st = random_state(keys, seed=sum(dims))
+    got = []
+    for tune in (dict(), dict(energy_kernel=0) if model == "3phe" else dict(fused_kernel=0)):
+        d = capaz.Domain(keys, st)
+        d.tune(**tune)
+        d.run(2)
+        got.append(d.fields())
+        d.close()
+    for f in got[0]:
+        assert bit_equal(got[0][f], got[1][f]), f
+
+
 @pytest.mark.parametrize("model,state", [("2ph", ("P_w", "S_n")), ("3ph", ("P_w", "S_w", "S_n")),
                                          ("2phe", ("P_w", "S_n", "T")), ("3phe", ("P_w", "S_w", "S_n", "T"))])
 @pytest.mark.parametrize("write", ["set_field", "device"])
