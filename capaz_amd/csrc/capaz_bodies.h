@@ -265,13 +265,17 @@ CAPAZ_HD void body_E(const DevParams& p, const DevFields& F, int64_t l) { body_E
 // The energy model's Newton update of interior cell l without the pivot
 // search: writes the new state and returns true, or writes nothing and
 // returns false when a pivot needs the search (body_newton then does the cell).
+// STEP: S_g and H_* are those of the step's first pass, taken from S_w, S_n and
+// T again instead of from memory.
+template <bool STEP = false>
 CAPAZ_HD bool body_newton_energy_nopivot(const DevParams& p, const DevFields& F, int64_t l) {
-    double P = F.f[F_P_w][l], Sw = F.f[F_S_w][l], Sn = F.f[F_S_n][l];
-    double Sg = F.f[F_S_g][l], T = F.f[F_T][l];
-    double Hw = F.f[F_H_w][l], Hn = F.f[F_H_n][l], Hg = F.f[F_H_g][l], Hr = F.f[F_H_r][l];
+    double P = F.f[F_P_w][l], Sw = F.f[F_S_w][l], Sn = F.f[F_S_n][l], T = F.f[F_T][l];
+    double Sg = STEP ? 1. - Sw - Sn : F.f[F_S_g][l];
+    double Hw = STEP ? H_w_of(p, T) : F.f[F_H_w][l], Hn = STEP ? H_n_T(p, T) : F.f[F_H_n][l];
+    double Hg = STEP ? H_g_T(p, T) : F.f[F_H_g][l], Hr = STEP ? H_r_of(p, T) : F.f[F_H_r][l];
     const double E_new = F.f[F_E_new][l];
-    if (!newton_energy_t<true>(p, Sw, Sn, Sg, P, T, Hw, Hn, Hg, Hr, F.f[F_m][l], F.f[F_roS_w][l], F.f[F_roS_n][l],
-                               F.f[F_roS_g][l], E_new))
+    if (!newton_energy_fast(p, Sw, Sn, Sg, P, T, Hw, Hn, Hg, Hr, F.f[F_m][l], F.f[F_roS_w][l], F.f[F_roS_n][l],
+                            F.f[F_roS_g][l], E_new))
         return false;
     F.f[F_S_g][l] = Sg;
     F.f[F_T][l] = T;

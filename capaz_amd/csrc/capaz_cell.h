@@ -927,14 +927,10 @@ CAPAZ_HD bool reverse_nopivot(double* a) {
 }
 
 // Energy-model 5x5 Newton in (S_w, S_n, S_g, P_w, T) (energy.cpp:370-463);
-// H_* are refreshed after every iteration as assign_H does.  NOPIVOT: every
-// inverse by reverse_nopivot; returns false as soon as one needs the pivot
-// search (the arguments are then partly updated: the caller keeps copies and
-// reruns the cell with NOPIVOT false, which always returns true).
-template <bool NOPIVOT>
-CAPAZ_HD bool newton_energy_t(const DevParams& p, double& Sw, double& Sn, double& Sg, double& P, double& T, double& Hw,
-                              double& Hn, double& Hg, double& Hr, double m, double roS_w, double roS_n, double roS_g,
-                              double E_new) {
+// H_* are refreshed after every iteration as assign_H does
+CAPAZ_HD void newton_energy(const DevParams& p, double& Sw, double& Sn, double& Sg, double& P, double& T, double& Hw,
+                            double& Hn, double& Hg, double& Hr, double m, double roS_w, double roS_n, double roS_g,
+                            double E_new) {
     constexpr int n = 5;
     for (int w = 1; w <= p.iterations; w++) {
         double rw = ro_w_T(p, P, T), rn = ro_n_T(p, P, T), rg = ro_g_T(p, P, T);
@@ -959,11 +955,7 @@ CAPAZ_HD bool newton_energy_t(const DevParams& p, double& Sw, double& Sn, double
         dF[4 + n * 4] = m * (Sw * (dwT * Hw + rw * c_w_T(T)) + Sn * (dnT * Hn + rn * c_n_T(T)) +
                              Sg * (dgT * Hg + rg * c_g_T(T))) +
                         (1. - m) * p.ro_r * c_r_of(p, T);
-        if constexpr (NOPIVOT) {
-            if (!reverse_nopivot<5>(dF)) return false;
-        } else {
-            reverse_matrix<5>(dF);
-        }
+        reverse_matrix<5>(dF);
         mult_matrix_vector<5>(corr, dF, F);
         Sw = Sw - corr[0];
         Sn = Sn - corr[1];
@@ -975,19 +967,109 @@ CAPAZ_HD bool newton_energy_t(const DevParams& p, double& Sw, double& Sn, double
         Hg = H_g_T(p, T);
         Hr = H_r_of(p, T);
     }
-    return true;
 }
 
-CAPAZ_HD void newton_energy(const DevParams& p, double& Sw, double& Sn, double& Sg, double& P, double& T, double& Hw,
-                            double& Hn, double& Hg, double& Hr, double m, double roS_w, double roS_n, double roS_g,
-                            double E_new) {
-    newton_energy_t<false>(p, Sw, Sn, Sg, P, T, Hw, Hn, Hg, Hr, m, roS_w, roS_n, roS_g, E_new);
+// newton_energy without the pivot search, with no call and no branch per
+// iteration: false (and any values) if some pivot, or T, lay outside
+// DivisorRange; newton_energy then does the cell.  The inverse is
+// reverse_matrix<5>'s operations on the entries that the system's zeros and
+// ones leave to be computed,
+//   row 0: 1 1 1 0 0 | row 1: rw 0 0 a b | row 2: 0 rn 0 c d | row 3: 0 0 rg e f |
+//   row 4: g h i q s:
+// the first pivots are 1, -rw and -rn, and the rows' quotients by them -rw / -rw
+// and -rn / -rn are 1.  The same bits up to the sign of entries that are exactly
+// 0 (finite entries; one that is not makes a pivot that is not).
+CAPAZ_HD bool newton_energy_fast(const DevParams& p, double& Sw, double& Sn, double& Sg, double& P, double& T,
+                                 double& Hw, double& Hn, double& Hg, double& Hr, double m, double roS_w,
+                                 double roS_n, double roS_g, double E_new) {
+    DivisorRange range;
+    const double dwP = p.ro0_w * p.beta_w, dwT = (-1) * p.ro0_w * kAlfaW;
+    const double dnP = p.ro0_n * p.beta_n, dnT = (-1) * p.ro0_n * kAlfaN;
+    for (int w = 1; w <= p.iterations; w++) {
+        range.see(T);
+        const double rT = rcp_in_range(T), iT = exact_div(kT0, T, rT);  // kT0 / T
+        const double rP = exact_div(P, p.P_atm, p.r_P_atm);
+        const double rw = ro_w_T(p, P, T), rn = ro_n_T(p, P, T), rg = p.ro0_g * rP * iT;
+        const double dgP = exact_div(p.ro0_g, p.P_atm, p.r_P_atm) * iT;
+        const double dgT = exact_div(p.ro0_g * rP * (-1) * iT, T, rT);
+        const double F0 = Sg + Sw + Sn - 1., F1 = rw * Sw - roS_w, F2 = rn * Sn - roS_n, F3 = rg * Sg - roS_g;
+        const double ew = rw * Hw - P, en = rn * Hn - P, eg = rg * Hg - P;
+        const double F4 = m * (Sw * ew + Sn * en + Sg * eg) + (1. - m) * (p.ro_r * Hr - P) - E_new;
+        const double a = dwP * Sw, b = dwT * Sw, c = dnP * Sn, d = dnT * Sn, e = dgP * Sg, f = dgT * Sg;
+        const double g = m * ew, h = m * en, i = m * eg;
+        const double q = m * (Sw * (dwP * Hw - 1.) + Sn * (dnP * Hn - 1.) + Sg * (dgP * Hg - 1.)) + (1. - m) * (-1);
+        const double s = m * (Sw * (dwT * Hw + rw * c_w_T(T)) + Sn * (dnT * Hn + rn * c_n_T(T)) +
+                              Sg * (dgT * Hg + rg * c_g_T(T))) +
+                         (1. - m) * p.ro_r * c_r_of(p, T);
+        // pivot 1 (-rw)
+        const double nrw = -rw, v1 = h - g;
+        range.see(nrw);
+        const double r1 = rcp_in_range(nrw);
+        const double s3 = exact_div(a, nrw, r1), s4 = exact_div(b, nrw, r1);
+        const double m26 = -(r1 * rn);
+        const double v2 = (i - g) - v1;
+        double m43 = q - s3 * v1, m44 = s - s4 * v1, m45 = -g - v1, m46 = -(r1 * v1);
+        // pivot 2 (-rn)
+        const double nrn = -rn;
+        range.see(nrn);
+        const double r2 = rcp_in_range(nrn);
+        const double t3 = exact_div(c - s3 * rn, nrn, r2), t4 = exact_div(d - s4 * rn, nrn, r2);
+        const double t6 = exact_div(m26, nrn, r2);
+        const double m13 = s3 - t3;
+        double m14 = s4 - t4, m16 = r1 - t6, m17 = -r2;
+        const double m33 = e - t3 * rg, m34 = f - t4 * rg, m36 = -(t6 * rg), m37 = -(r2 * rg);
+        m43 = m43 - t3 * v2;
+        m44 = m44 - t4 * v2;
+        m45 = m45 - v2;
+        m46 = m46 - t6 * v2;
+        double m47 = -(r2 * v2);
+        // pivot 3
+        range.see(m33);
+        const double r3 = rcp_in_range(m33);
+        const double u4 = exact_div(m34, m33, r3), u5 = exact_div(-rg, m33, r3), u6 = exact_div(m36, m33, r3),
+                     u7 = exact_div(m37, m33, r3);
+        const double m04 = u4 * s3 - s4;
+        double m05 = u5 * s3, m06 = u6 * s3 - r1, m07 = u7 * s3, m08 = r3 * s3;
+        m14 = m14 - u4 * m13;
+        double m15 = -(u5 * m13), m18 = -(r3 * m13);
+        m16 = m16 - u6 * m13;
+        m17 = m17 - u7 * m13;
+        const double m24 = t4 - u4 * t3;
+        double m25 = 1. - u5 * t3, m26b = t6 - u6 * t3, m27 = r2 - u7 * t3, m28 = -(r3 * t3);
+        m44 = m44 - u4 * m43;
+        m45 = m45 - u5 * m43;
+        m46 = m46 - u6 * m43;
+        m47 = m47 - u7 * m43;
+        const double m48 = -(r3 * m43);
+        // pivot 4; row by row, the inverse's entries times F
+        range.see(m44);
+        const double r4 = rcp_in_range(m44);
+        const double x5 = exact_div(m45, m44, r4), x6 = exact_div(m46, m44, r4), x7 = exact_div(m47, m44, r4),
+                     x8 = exact_div(m48, m44, r4);
+        auto row = [&](double m5, double m6, double m7, double m8, double f1) {
+            return (m5 - x5 * f1) * F0 + (m6 - x6 * f1) * F1 + (m7 - x7 * f1) * F2 + (m8 - x8 * f1) * F3 +
+                   -(r4 * f1) * F4;
+        };
+        Sw = Sw - row(m05, m06, m07, m08, m04);
+        Sn = Sn - row(m15, m16, m17, m18, m14);
+        Sg = Sg - row(m25, m26b, m27, m28, m24);
+        P = P - row(u5, u6, u7, r3, u4);
+        T = T - (x5 * F0 + x6 * F1 + x7 * F2 + x8 * F3 + r4 * F4);
+        Hw = H_w_of(p, T);
+        Hn = H_n_T(p, T);
+        Hg = H_g_T(p, T);
+        Hr = H_r_of(p, T);
+    }
+    return range.ok();
 }
 
 // The two-phase energy model's Newton (configuration closure): energy.cpp:370-463's
 // system without the gas row and column, 4 x 4 in (S_w, S_n, P_w, T), the
 // densities at P_w for both phases as energy.cpp:388-394 has them, H_*
-// refreshed after every iteration.  NOPIVOT as newton_energy_t.
+// refreshed after every iteration.  NOPIVOT: every inverse by reverse_nopivot;
+// returns false as soon as one needs the pivot search (the arguments are then
+// partly updated: the caller keeps copies and reruns the cell with NOPIVOT
+// false, which always returns true).
 template <bool NOPIVOT>
 CAPAZ_HD bool newton_energy2_t(const DevParams& p, double& Sw, double& Sn, double& P, double& T, double& Hw,
                                double& Hn, double& Hr, double m, double roS_w, double roS_n, double E_new) {

@@ -62,18 +62,21 @@ __global__ void __launch_bounds__(kBlock) k_energy_u_faces(DevParams p, DevField
         body_u(p, F, (int64_t)i + (int64_t)j * p.sy + (int64_t)k * p.sz);
 }
 // The energy model's Newton update: every interior cell without the pivot
-// search (166 VGPRs, no scratch: 3 waves per SIMD against 2 for the general
-// routine); a cell whose matrices need the search is marked in `redo` and
-// recomputed from its untouched state by k_newton_energy_redo.
+// search; a cell whose matrices need the search is marked in `redo` and
+// recomputed from its untouched state by k_newton_energy_redo.  Three phases,
+// bound by memory (15 to 20 values in, 10 out) and VALU issue alike: 160 x 128 x
+// 96, 3 iterations, 90 us in the step (STEP, body_newton_energy_nopivot) where
+// the inverse with its zeros and ones computed, S_g and H_* read, took 103.
+template <bool STEP>
 __global__ void __launch_bounds__(kBlock) k_newton_energy(DevParams p, DevFields F, unsigned char* redo) {
     const int64_t l = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (l >= p.n) return;
     int i, j, k;
     decompose(p, l, i, j, k);
-    if (p.model == 2)
+    if (!STEP && p.model == 2)
         redo[l] = interior_newton2(p, i, j, k) && !body_newton_energy2_nopivot(p, F, l) ? 1 : 0;
     else
-        redo[l] = interior3(p, i, j, k) && !body_newton_energy_nopivot(p, F, l) ? 1 : 0;
+        redo[l] = interior3(p, i, j, k) && !body_newton_energy_nopivot<STEP>(p, F, l) ? 1 : 0;
 }
 // One thread per 16 marks (one 16-byte load; redo is allocated rounded up to
 // 16 bytes, the marks past Nx*Ny*Nz are never read as cells).
@@ -508,11 +511,16 @@ hipError_t launch_energy_e_tiles(const DevParams& p, const DevFields& F, const d
     return lam ? launch(std::integral_constant<int, kLamStored>{}) : launch(std::integral_constant<int, kLamEvaluated>{});
 }
 
-hipError_t launch_newton_energy(const DevParams& p, const DevFields& F, unsigned char* redo, hipStream_t s) {
+template <bool STEP>
+hipError_t launch_newton_energy_t(const DevParams& p, const DevFields& F, unsigned char* redo, hipStream_t s) {
     if (!redo) return launch_entry(Entry::Newton, p, F, s);
-    hipLaunchKernelGGL(k_newton_energy, grid_for(p.n), dim3(kBlock), 0, s, p, F, redo);
+    hipLaunchKernelGGL(k_newton_energy<STEP>, grid_for(p.n), dim3(kBlock), 0, s, p, F, redo);
     hipLaunchKernelGGL(k_newton_energy_redo, grid_for((p.n + 15) / 16), dim3(kBlock), 0, s, p, F, redo);
     return hipGetLastError();
+}
+
+hipError_t launch_newton_energy(const DevParams& p, const DevFields& F, unsigned char* redo, hipStream_t s) {
+    return launch_newton_energy_t<false>(p, F, redo, s);
 }
 
 hipError_t launch_roS_stored(const DevParams& p, const DevFields& F, const double* dtm, hipStream_t s) {
@@ -530,7 +538,7 @@ hipError_t launch_energy_step(const DevParams& p, const DevFields& F, double* la
     hipLaunchKernelGGL(k_energy_u_faces, grid_for(fused_face_cells(p)), b, 0, s, p, F);
     if ((e = launch_roS_tiles<true>(p, F, dtm, s)) != hipSuccess) return e;
     if ((e = launch_energy_e_tiles(p, F, lam, s)) != hipSuccess) return e;
-    if ((e = launch_newton_energy(p, F, redo, s)) != hipSuccess) return e;
+    if ((e = launch_newton_energy_t<true>(p, F, redo, s)) != hipSuccess) return e;
     hipLaunchKernelGGL(k_boundary_faces, grid_for(fused_face_cells(p)), b, 0, s, p, F);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     return ev ? hipEventRecord(ev->end, s) : hipSuccess;
