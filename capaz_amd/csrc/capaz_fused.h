@@ -537,8 +537,9 @@ struct CellState {
 // does every cell.
 //
 // Cells that the planes' code does not cover -- the epilogue left it undone (a
-// pivot search), or an x or z face neighbour has a P_n or P_g that is not its
-// P_w (values a caller set; Border_P gives those faces P_n = P_g = P_w) -- are
+// pivot search), or an x or z face neighbour (for the roS entry point: the cell
+// or any neighbour) has a P_n or P_g that is not its P_w (values a caller set;
+// Border_P gives those faces P_n = P_g = P_w, P_Xi_ro every interior cell) -- are
 // marked and done after the last plane from the state the step reads, which
 // it does not write: the planes' code then holds no call and no registers for
 // them (kchunk <= kMaxPlanes, one mark per plane).
@@ -553,6 +554,8 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
     constexpr int ROW = (TX + 2) * NV, PLANE = (TY + 2) * ROW;  // LDS pitch of a row, of a plane
     constexpr bool U = EpiWantsU<Epi>::value;
     constexpr bool EARLY = CLOSURE == 0 || CLOSURE == 1;
+    // the roS entry point: a P_n or P_g of its own in any cell, as a caller set it
+    constexpr bool OWN_P = CLOSURE == 3 && !U;
 
     const int tx = threadIdx.x, ty = threadIdx.y;
     const bool hasx = FULL || p.Nx >= 3, hasz = FULL || p.Nz >= 3;
@@ -567,7 +570,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
     // no active lane reads); jw: the wavefront's first row
     const int ic = min(i, p.Nx - 1), jc = min(j, p.Ny - 1);
     const int jw = __builtin_amdgcn_readfirstlane(jc);
-    const bool own_ij = inner_ij<MODEL>(p, ic, jc);
+    const bool own_ij = !OWN_P && inner_ij<MODEL>(p, ic, jc);
     CellAt own{(int64_t)i0 + (int64_t)jw * p.sy + (int64_t)k0 * p.sz, 8u * (uint32_t)(ic - i0)};
     if (TX < 64) own.off += 8u * (uint32_t)(jc - jw) * (uint32_t)p.sy;
 
@@ -579,7 +582,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
     else if (ty == 2 && tx < TY) { hi = i0 - 1; hj = j0 + tx; hx = 0; hy = tx + 1; }
     else if (ty == 2 && tx >= TY && tx < 2 * TY) { hi = i0 + TX; hj = j0 + tx - TY; hx = TX + 1; hy = tx - TY + 1; }
     const bool halo = hi >= 0 && hi < p.Nx && hj >= 0 && hj < p.Ny && (hasx || hi == i0 + tx);
-    const bool halo_ij = inner_ij<MODEL>(p, hi, hj);
+    const bool halo_ij = !OWN_P && inner_ij<MODEL>(p, hi, hj);
     const HaloAt hat(p, i0, j0, hi, hj);
 
     // LDS places in the buffer of plane 0: the own and the halo cell
@@ -794,7 +797,8 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
             bool done = true;
             if constexpr (MODEL == 3) {
                 const uint64_t lane = 1ull << ((ty * TX + tx) & 63);
-                const bool row_odd = lds.odd[k & 1][ty + 1] == k;
+                bool row_odd = lds.odd[k & 1][ty + 1] == k;
+                if constexpr (OWN_P) row_odd = row_odd || lds.odd[k & 1][ty] == k || lds.odd[k & 1][ty + 2] == k;
                 if (__builtin_expect((zodd | odd) != 0 || __ballot(row_odd) != 0, 0))
                     done = !row_odd && ((zodd | odd) & lane) == 0;
             }

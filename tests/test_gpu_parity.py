@@ -312,6 +312,38 @@ def test_rows_at_the_halo_offset_limit(model, tune, nx):
         assert np.isfinite(a).all()
 
 
+@pytest.mark.parametrize("dims", [(70, 13, 11), (66, 9, 1), (1, 21, 9), (3, 3, 3)])
+@pytest.mark.parametrize("share", [0.0, 0.02, 1.0])
+def test_roS_entry_point_with_phase_pressures_as_set(dims, share):
+    """capaz_roS after P_n and P_g were set in a share of the cells, interior ones
+    included, with no P_Xi_ro in between: the bits of the kernel with one thread
+    per cell, which runs where some interior cell has m = 0 (that cell aside)."""
+    keys = case("3ph", *dims)
+    st = random_state(keys, seed=sum(dims))
+    rng = np.random.default_rng(sum(dims))
+    zero = (dims[2] // 2, dims[1] // 2, dims[0] // 2)
+    got = []
+    own = rng.random(st["P_w"].shape) < share
+    put = {f: np.where(own, st["P_w"] + rng.uniform(-20, 20, own.shape), st["P_w"]) for f in ("P_n", "P_g")}
+    for m0 in (False, True):
+        m = st["m"].copy()
+        if m0:
+            m[zero] = 0.0
+        d = capaz.Domain(keys, dict(st, m=m))
+        L = capaz.load()
+        assert L.capaz_P_Xi_ro(d._ctx) == 0
+        for f, v in put.items():
+            d.set_field(f, v)
+        assert L.capaz_roS(d._ctx, 0.0) == 0
+        out = {f: d.field(f) for f in ("roS_w", "roS_n", "roS_g", "roS_g_old")}
+        for v in out.values():
+            v[zero] = 0.0
+        got.append(out)
+        d.close()
+    for f in got[0]:
+        assert bit_equal(got[0][f], got[1][f]), f
+
+
 def test_headline_physics_bitwise_at_96():
     """The benchmark physics (three-phase, Corey-2, lognormal K, top
     injection) at 96^3: one and three fused steps equal the oracle bit for bit."""
