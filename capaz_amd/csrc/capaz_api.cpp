@@ -469,8 +469,11 @@ int capaz_step(capaz_ctx* c, long first_step, long nsteps) {
         for (long s = 0; s < nsteps; ++s) {
             const KernelEvents* ev;
             if ((rc = next_events(c, &ev))) return rc;
+            // the intermediates of the steps after which a caller can read them
+            const bool keep = s == nsteps - 1 ||
+                              (c->tuning.check_every > 0 && (first_step + s) % c->tuning.check_every == 0);
             CAPAZ_HIP(c, launch_energy_step(c->p, fields_of(c), c->d_lam, c->d_dtm,
-                                            c->tuning.energy_newton ? c->d_redo : nullptr, c->stream, ev));
+                                            c->tuning.energy_newton ? c->d_redo : nullptr, keep, c->stream, ev));
             if ((rc = check_after_step(c, first_step + s))) return rc;
         }
         return CAPAZ_OK;

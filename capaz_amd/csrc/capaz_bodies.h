@@ -99,13 +99,9 @@ CAPAZ_HD void body_P_Xi_ro(const DevParams& p, const DevFields& F, int64_t l) {
 CAPAZ_HD double u_axis(const double* Xi, const double* P, const double* ro, int64_t l, int64_t s, int idx, int n,
                        double h, double rh, double h2, double rh2, bool grav, double g) {
     if (n <= 2) return 0.;
-    double d;
-    if (idx == 0)
-        d = exact_div(P[l + s] - P[l], h, rh);
-    else if (idx == n - 1)
-        d = exact_div(P[l] - P[l - s], h, rh);
-    else
-        d = exact_div(P[l + s] - P[l - s], h2, rh2);
+    const bool lo = idx == 0, hi = idx == n - 1;
+    const double dP = P[hi ? l : l + s] - P[lo ? l : l - s];
+    const double d = lo || hi ? exact_div(dP, h, rh) : exact_div(dP, h2, rh2);
     return grav ? Xi[l] * (d - ro[l] * g) : Xi[l] * d;
 }
 
@@ -115,11 +111,26 @@ CAPAZ_HD void body_u(const DevParams& p, const DevFields& F, int64_t l) {
     const int ph = p.model == 3 ? 3 : 2;
     const int xi[3] = {F_Xi_w, F_Xi_n, F_Xi_g}, pr[3] = {F_P_w, F_P_n, F_P_g}, ro[3] = {F_ro_w, F_ro_n, F_ro_g};
     const int ux[3] = {F_ux_w, F_ux_n, F_ux_g}, uy[3] = {F_uy_w, F_uy_n, F_uy_g}, uz[3] = {F_uz_w, F_uz_n, F_uz_g};
-    for (int a = 0; a < ph; ++a) {
+    // every load before the first store, which might alias it
+    double v[3][3];
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+    for (int a = 0; a < 3; ++a) {
+        if (a >= ph) break;
         const double *X = F.f[xi[a]], *P = F.f[pr[a]], *R = F.f[ro[a]];
-        F.f[ux[a]][l] = u_axis(X, P, R, l, 1, i, p.Nx, p.hx, p.r_hx, p.two_hx, p.r_two_hx, false, p.g);
-        F.f[uy[a]][l] = u_axis(X, P, R, l, p.sy, j, p.Ny, p.hy, p.r_hy, p.two_hy, p.r_two_hy, true, p.g);
-        F.f[uz[a]][l] = u_axis(X, P, R, l, p.sz, k, p.Nz, p.hz, p.r_hz, p.two_hz, p.r_two_hz, false, p.g);
+        v[a][0] = u_axis(X, P, R, l, 1, i, p.Nx, p.hx, p.r_hx, p.two_hx, p.r_two_hx, false, p.g);
+        v[a][1] = u_axis(X, P, R, l, p.sy, j, p.Ny, p.hy, p.r_hy, p.two_hy, p.r_two_hy, true, p.g);
+        v[a][2] = u_axis(X, P, R, l, p.sz, k, p.Nz, p.hz, p.r_hz, p.two_hz, p.r_two_hz, false, p.g);
+    }
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+    for (int a = 0; a < 3; ++a) {
+        if (a >= ph) break;
+        F.f[ux[a]][l] = v[a][0];
+        F.f[uy[a]][l] = v[a][1];
+        F.f[uz[a]][l] = v[a][2];
     }
 }
 
@@ -262,12 +273,13 @@ CAPAZ_HD void body_E_with(const DevParams& p, const DevFields& F, const Lam& lam
 CAPAZ_HD void body_E(const DevParams& p, const DevFields& F, int64_t l) { body_E_with(p, F, LamOfFields{p, F}, l); }
 
 // ---- P_S_calculation -> Newton (cpu.cpp:80-89), interior cells -------------------------
+CAPAZ_HD void body_newton(const DevParams& p, const DevFields& F, int64_t l);
 // The energy model's Newton update of interior cell l without the pivot
 // search: writes the new state and returns true, or writes nothing and
 // returns false when a pivot needs the search (body_newton then does the cell).
 // STEP: S_g and H_* are those of the step's first pass, taken from S_w, S_n and
-// T again instead of from memory.
-template <bool STEP = false>
+// T again instead of from memory.  KEEP: as body_energy_a.
+template <bool STEP = false, bool KEEP = true>
 CAPAZ_HD bool body_newton_energy_nopivot(const DevParams& p, const DevFields& F, int64_t l) {
     double P = F.f[F_P_w][l], Sw = F.f[F_S_w][l], Sn = F.f[F_S_n][l], T = F.f[F_T][l];
     double Sg = STEP ? 1. - Sw - Sn : F.f[F_S_g][l];
@@ -277,17 +289,29 @@ CAPAZ_HD bool body_newton_energy_nopivot(const DevParams& p, const DevFields& F,
     if (!newton_energy_fast(p, Sw, Sn, Sg, P, T, Hw, Hn, Hg, Hr, F.f[F_m][l], F.f[F_roS_w][l], F.f[F_roS_n][l],
                             F.f[F_roS_g][l], E_new))
         return false;
-    F.f[F_S_g][l] = Sg;
     F.f[F_T][l] = T;
-    F.f[F_H_w][l] = Hw;
-    F.f[F_H_n][l] = Hn;
-    F.f[F_H_g][l] = Hg;
-    F.f[F_H_r][l] = Hr;
-    F.f[F_E][l] = E_new;
     F.f[F_P_w][l] = P;
     F.f[F_S_w][l] = Sw;
     F.f[F_S_n][l] = Sn;
+    if constexpr (KEEP) {
+        F.f[F_S_g][l] = Sg;
+        F.f[F_H_w][l] = Hw;
+        F.f[F_H_n][l] = Hn;
+        F.f[F_H_g][l] = Hg;
+        F.f[F_H_r][l] = Hr;
+        F.f[F_E][l] = E_new;
+    }
     return true;
+}
+// The same cell with the pivot search, in a step.
+CAPAZ_HD void body_newton_energy_step(const DevParams& p, const DevFields& F, int64_t l) {
+    const double Sw = F.f[F_S_w][l], Sn = F.f[F_S_n][l], T = F.f[F_T][l];
+    F.f[F_S_g][l] = 1. - Sw - Sn;
+    F.f[F_H_w][l] = H_w_of(p, T);
+    F.f[F_H_n][l] = H_n_T(p, T);
+    F.f[F_H_g][l] = H_g_T(p, T);
+    F.f[F_H_r][l] = H_r_of(p, T);
+    body_newton(p, F, l);
 }
 
 // The two-phase energy model's Newton update of interior cell l without the
@@ -431,11 +455,59 @@ CAPAZ_HD void body_boundary(const DevParams& p, const DevFields& F, int64_t l) {
 // ran slower than apart; the Newton update holds ~200 registers, which would
 // cut the stencils' occupancy.
 
+// Intermediates that only a caller reads (S_g, interior P_n and P_g, ro, H, the
+// roS_old, E after the Newton, and u_z where the z term advects with u_y) are
+// stored by the steps whose fields can be read (KEEP): the last one of a run and
+// those checked for a non-finite state.  C, E and N take ro, H and S_g from the
+// state instead of from memory, which bounds them: 160 x 128 x 96, 285 us per step
+// without the stores, 335 with them, 401 with every pass reading them.
+
+// A cell's phase pressures in the energy step: the boundary cells' own ones.
+CAPAZ_HD void energy_P(const DevFields& F, int64_t l, double Pw, bool inner, double& Pn, double& Pg) {
+    Pn = inner ? Pw : F.f[F_P_n][l];
+    Pg = inner ? Pw : F.f[F_P_g][l];
+}
+
+template <bool KEEP>
 CAPAZ_HD void body_energy_a(const DevParams& p, const DevFields& F, double* lam, int64_t l) {
-    body_S(p, F, l);
-    body_P_Xi_ro(p, F, l);
-    body_HE(p, F, l);
-    lam[l] = lambda_eff_at(p, F, l);
+    if constexpr (KEEP) {
+        body_S(p, F, l);
+        body_P_Xi_ro(p, F, l);
+        body_HE(p, F, l);
+        lam[l] = lambda_eff_at(p, F, l);
+        return;
+    }
+    int i, j, k;
+    decompose(p, l, i, j, k);
+    const bool inner = interior3(p, i, j, k);
+    const double K = F.f[F_K][l], m = F.f[F_m][l], T = F.f[F_T][l];
+    const double Pw = F.f[F_P_w][l], Sw = F.f[F_S_w][l], Sn = F.f[F_S_n][l], Sg = 1. - Sw - Sn;
+    double Pn, Pg, kw, kn, kg, mw, mn, mg;
+    energy_P(F, l, Pw, inner, Pn, Pg);
+    relperm3(p, Sw, Sn, kw, kn, kg);
+    if (p.ecfg) {
+        mw = mu_cfg(p, p.mu_w, T);
+        mn = mu_cfg(p, p.mu_n, T);
+        mg = mu_cfg(p, p.mu_g, T);
+    } else {
+        mu_of_T(T, mw, mn, mg);
+    }
+    F.f[F_Xi_w][l] = xi_var(K, kw, mw);
+    F.f[F_Xi_n][l] = xi_var(K, kn, mn);
+    F.f[F_Xi_g][l] = xi_var(K, kg, mg);
+    const double rw = ro_w_T(p, Pw, T), rn = ro_n_T(p, Pn, T), rg = ro_g_T(p, Pg, T);
+    F.f[F_E][l] = (m * (Sw * (rw * H_w_of(p, T) - Pw) + Sn * (rn * H_n_T(p, T) - Pn) + Sg * (rg * H_g_T(p, T) - Pg)) +
+                   (1. - m) * (p.ro_r * H_r_of(p, T) - Pw));
+    if (!p.ecfg) lam[l] = lambda_eff(m, Sw, Sn, Sg, T);
+    // what u of the boundary cells reads: their ro, and P next to them
+    if (!inner) {
+        F.f[F_ro_w][l] = rw;
+        F.f[F_ro_n][l] = rn;
+        F.f[F_ro_g][l] = rg;
+    } else if (i == 1 || i == p.Nx - 2 || j == 1 || j == p.Ny - 2 || k == 1 || k == p.Nz - 2) {
+        F.f[F_P_n][l] = Pn;
+        F.f[F_P_g][l] = Pg;
+    }
 }
 
 // ---- fused step (two- and three-phase without energy) -------------------------------------
@@ -457,6 +529,7 @@ struct StepIO {
     // Xi and ro per phase as stored by P_Xi_ro (read by the fused z kernel's
     // stored-coefficient variant only, the energy step's roS pass)
     const double *Xi[3] = {}, *ro[3] = {};
+    const double* T = nullptr;  // the energy step's: densities from P and T
     // non-NULL: the step also writes the z exchange planes of its new state
     // here (fused_pack)
     double* pack = nullptr;

@@ -61,24 +61,29 @@ __device__ __forceinline__ double corey_t(const DevParams& p, double s) {
 
 // assign_P_Xi + assign_ro of one cell with the model and closure fixed at
 // compile time (cpu.cpp:143-169; two-phase.cpp:4-23; three-phase.cpp:198-240).
-// CLOSURE 3 (three phases): the values the closure pass of this step has
-// already stored (P_n, P_g, Xi, ro arrays).
+// CLOSURE 3 (three phases): the values in the P_n, P_g, Xi and ro arrays; 4, the
+// energy step: Xi as its first pass stored it, ro from P and T.
 template <int MODEL, int CLOSURE>
 __device__ __forceinline__ CoefT<MODEL> coef_at(const DevParams& p, const StepIO& io, int64_t l, bool inner) {
     CoefT<MODEL> c;
-    if constexpr (CLOSURE == 3) {
+    if constexpr (CLOSURE >= 3) {
         static_assert(MODEL == 3, "stored coefficients: three phases");
-        (void)p;
-        (void)inner;
+        inner = inner && CLOSURE == 4;
         c.Sw = io.Sw[l];
         c.Sn = io.Sn[l];
         c.P[0] = io.Pw[l];
-        c.P[1] = io.Pn[l];
-        c.P[2] = io.Pg[l];
+        c.P[1] = inner ? c.P[0] : io.Pn[l];
+        c.P[2] = inner ? c.P[0] : io.Pg[l];
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             c.Xi[a] = io.Xi[a][l];
-            c.ro[a] = io.ro[a][l];
+            if constexpr (CLOSURE == 3) c.ro[a] = io.ro[a][l];
+        }
+        if constexpr (CLOSURE == 4) {
+            const double T = io.T[l];
+            c.ro[0] = ro_w_T(p, c.P[0], T);
+            c.ro[1] = ro_n_T(p, c.P[1], T);
+            c.ro[2] = ro_g_T(p, c.P[2], T);
         }
         return c;
     }
@@ -308,6 +313,13 @@ template <int MODEL, int CLOSURE>
 __device__ __forceinline__ DevParams coef_params(ConstParams* q) {
     DevParams p;
     if constexpr (CLOSURE == 3) return p;
+    if constexpr (CLOSURE == 4) {
+        p.P_atm = q->P_atm, p.r_P_atm = q->r_P_atm;
+        p.ro0_w = q->ro0_w, p.beta_w = q->beta_w;
+        p.ro0_n = q->ro0_n, p.beta_n = q->beta_n;
+        p.ro0_g = q->ro0_g;
+        return p;
+    }
     p.closure = CLOSURE == 0 ? 0 : 1;
     if constexpr (CLOSURE == 0) p.pow_fast = q->pow_fast;
     p.P_atm = q->P_atm;
@@ -362,7 +374,7 @@ __device__ __forceinline__ DevParams newton_params(ConstParams* q) {
 // ahead of their use), and the coefficients themselves.
 template <int MODEL, int CLOSURE>
 struct CellRaw {
-    double Pw, Sw, Sn, K, Pn, Pg, Xi[MODEL], ro[MODEL];
+    double Pw, Sw, Sn, K, Pn, Pg, Xi[MODEL], ro[MODEL], T;
 };
 template <int MODEL, int CLOSURE>
 struct CellCoef {
@@ -374,12 +386,13 @@ __device__ __forceinline__ void load_raw(const StepIO& io, const At& at, bool in
     r.Pw = ld(io.Pw, at);
     r.Sn = ld(io.Sn, at);
     if constexpr (MODEL == 3) r.Sw = ld(io.Sw, at);
-    if constexpr (CLOSURE == 3) {
+    if constexpr (CLOSURE >= 3) {
 #pragma unroll
         for (int a = 0; a < MODEL; ++a) {
             r.Xi[a] = ld(io.Xi[a], at);
-            r.ro[a] = ld(io.ro[a], at);
+            if constexpr (CLOSURE == 3) r.ro[a] = ld(io.ro[a], at);
         }
+        if constexpr (CLOSURE == 4) r.T = ld(io.T, at);
     } else {
         r.K = ld(io.K, at);
     }
@@ -397,11 +410,16 @@ template <int MODEL, int CLOSURE>
 __device__ __forceinline__ bool coef_of(const DevParams& p, const CellRaw<MODEL, CLOSURE>& r, bool inner,
                                         CellCoef<MODEL, CLOSURE>& c) {
     c.P[0] = r.Pw;
-    if constexpr (CLOSURE == 3) {
+    if constexpr (CLOSURE >= 3) {
 #pragma unroll
         for (int a = 0; a < MODEL; ++a) {
             c.Xi[a] = r.Xi[a];
-            c.ro[a] = r.ro[a];
+            if constexpr (CLOSURE == 3) c.ro[a] = r.ro[a];
+        }
+        if constexpr (CLOSURE == 4) {
+            c.ro[0] = ro_w_T(p, r.Pw, r.T);
+            c.ro[1] = ro_n_T(p, inner ? r.Pw : r.Pn, r.T);
+            c.ro[2] = ro_g_T(p, inner ? r.Pw : r.Pg, r.T);
         }
     } else if constexpr (MODEL == 2) {
         double mKw, mKn;  // -K k_r
@@ -445,7 +463,7 @@ __device__ __forceinline__ bool coef_of(const DevParams& p, const CellRaw<MODEL,
     }
     if constexpr (MODEL == 3) {
         if (!inner) {
-            if constexpr (CLOSURE != 3) {
+            if constexpr (CLOSURE < 3) {
                 c.ro[1] = ro_n_of(p, r.Pn);
                 c.ro[2] = ro_g_of(p, r.Pg);
             }
@@ -555,7 +573,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
     constexpr bool U = EpiWantsU<Epi>::value;
     constexpr bool EARLY = CLOSURE == 0 || CLOSURE == 1;
     // the roS entry point: a P_n or P_g of its own in any cell, as a caller set it
-    constexpr bool OWN_P = CLOSURE == 3 && !U;
+    constexpr bool OWN_P = CLOSURE == 3;
 
     const int tx = threadIdx.x, ty = threadIdx.y;
     const bool hasx = FULL || p.Nx >= 3, hasz = FULL || p.Nz >= 3;
@@ -956,10 +974,10 @@ struct FusedStoreRecord {
     }
 };
 
-// assign_roS_nr (cpu.cpp:619-731) on the z tiles from the stored
-// coefficients (CLOSURE 3, three phases): roS_old and roS of the cell and,
-// with U, its velocities (assign_u) from the same neighbours -- the roS entry
-// point, and the energy step's roS + u pass.
+// assign_roS_nr (cpu.cpp:619-731) on the z tiles (three phases): roS_old and
+// roS of the cell from the stored coefficients (CLOSURE 3, the roS entry point),
+// or (U, CLOSURE 4) the energy step's roS + u pass, with the cell's velocities
+// (assign_u) from the same neighbours.  Arrays that are NULL are not stored.
 template <bool U>
 struct RoSStore {
     static constexpr bool kWantsU = U;
@@ -975,7 +993,8 @@ struct RoSStore {
 #pragma unroll
         for (int a = 0; a < 3; ++a)
 #pragma unroll
-            for (int x = 0; x < 3; ++x) st(u[a][x], to, v[a][x]);
+            for (int x = 0; x < 3; ++x)
+                if (x < 2 || u[a][2]) st(u[a][x], to, v[a][x]);
     }
     template <bool GENERAL, class At>
     __device__ __forceinline__ bool cell(const DevParams& p, const DevParams& pn, int i, int j, int k, const At& at,
@@ -986,7 +1005,7 @@ struct RoSStore {
         renew(to);
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            st(roS_old[a], to, old[a]);
+            if (!U || roS_old[a]) st(roS_old[a], to, old[a]);
             st(roS[a], to, old[a] - d * div[a]);
         }
         return true;
@@ -995,10 +1014,10 @@ struct RoSStore {
 
 template <int TX, int TY, bool FULL, bool U>
 __global__ void __launch_bounds__(TX * TY) k_roS_z(DevParams p, StepIO io, int kchunk, RoSStore<U> st) {
-    __shared__ FusedLds<3, 3, TX, TY> lds;
+    __shared__ FusedLds<3, U ? 4 : 3, TX, TY> lds;
     int bx, by, bz;
     xcd_tile(bx, by, bz);
-    fused_z_tile<3, 3, TX, TY, FULL>(p, kernel_params(), io, kchunk, bx, by, bz, lds, st);
+    fused_z_tile<3, U ? 4 : 3, TX, TY, FULL>(p, kernel_params(), io, kchunk, bx, by, bz, lds, st);
 }
 
 // The energy step's E pass (assign_E_new, energy.cpp:235-340, as body_E_with)
@@ -1008,15 +1027,16 @@ __global__ void __launch_bounds__(TX * TY) k_roS_z(DevParams p, StepIO io, int k
 // x and y neighbours and carried in registers for the z ones.  Each term is
 // the product the per-cell body forms, so E_new has its bits.
 //
-// Bound by memory (14 fields read and one written per cell): the next plane's
+// Bound by memory (14 fields read and one written per cell; with STEP 10 and one): the next plane's
 // loads are issued before this plane's sums and one barrier ends a plane (two
 // LDS buffers).  160 x 128 x 96: 92 us against 115 for tiles that read the
 // fields again for the z neighbours (32 x 16 tiles, whose threads cover the 158
 // columns without the sixth that 64 x 8 leave idle: 88, and roS 98 against 95).
 //
-// LAM, where lambda_eff comes from: kLamStored, lam as the step's first pass
-// stored it; kLamEvaluated (the entry point), from m, S_w, S_n, S_g and T;
-// kLamConstant, lam_cfg: the configurations' energy closure, whose z term
+// STEP: ro and H from P and T, as the step's first pass has them, instead of
+// from their arrays.  LAM, where lambda_eff comes from: kLamStored (STEP), lam as
+// that pass stored it; kLamEvaluated (the entry point), from m, S_w, S_n, S_g and
+// T; kLamConstant, lam_cfg: the configurations' energy closure, whose z term
 // advects with uz (the reference's with uy, energy.cpp:300-305) and whose z
 // conduction adds to the x and y terms.
 enum { kLamStored, kLamEvaluated, kLamConstant };
@@ -1024,16 +1044,17 @@ struct EnergyEIO {
     const double *lam, *T, *E;
     const double *m, *Sw, *Sn, *Sg;
     const double *ro[3], *H[3], *ux[3], *uy[3], *uz[3];
+    const double *P[3];
     double* E_new;
     double lam_cfg;
 };
 
-template <int LAM>
+template <bool STEP, int LAM>
 struct EnergyRaw {
-    double lam, m, Sw, Sn, Sg, T, ro[3], H[3], ux[3], uy[3], uz[3];
+    double lam, m, Sw, Sn, Sg, T, P[3], ro[3], H[3], ux[3], uy[3], uz[3];
 };
-template <int LAM, class At>
-__device__ __forceinline__ void load_energy(const EnergyEIO& a, const At& at, EnergyRaw<LAM>& r) {
+template <bool STEP, int LAM, class At>
+__device__ __forceinline__ void load_energy(const EnergyEIO& a, const At& at, bool inner, EnergyRaw<STEP, LAM>& r) {
     r.T = ld(a.T, at);
     if constexpr (LAM == kLamStored) r.lam = ld(a.lam, at);
     if constexpr (LAM == kLamEvaluated) {
@@ -1042,10 +1063,19 @@ __device__ __forceinline__ void load_energy(const EnergyEIO& a, const At& at, En
         r.Sn = ld(a.Sn, at);
         r.Sg = ld(a.Sg, at);
     }
+    if constexpr (STEP) {
+        r.P[0] = ld(a.P[0], at);
+        if (!inner) {
+            r.P[1] = ld(a.P[1], at);
+            r.P[2] = ld(a.P[2], at);
+        }
+    }
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-        r.ro[q] = ld(a.ro[q], at);
-        r.H[q] = ld(a.H[q], at);
+        if constexpr (!STEP) {
+            r.ro[q] = ld(a.ro[q], at);
+            r.H[q] = ld(a.H[q], at);
+        }
         r.ux[q] = ld(a.ux[q], at);
         r.uy[q] = ld(a.uy[q], at);
         if constexpr (LAM == kLamConstant) r.uz[q] = ld(a.uz[q], at);
@@ -1053,19 +1083,26 @@ __device__ __forceinline__ void load_energy(const EnergyEIO& a, const At& at, En
 }
 // v[0] = lambda_eff * T, v[1 + a] = (ro_a H_a) ux_a, v[4 + a] = (ro_a H_a) uy_a;
 // z[a]: the product that the z term advects
-template <int LAM>
-__device__ __forceinline__ void energy_vals(const EnergyEIO& a, const EnergyRaw<LAM>& r, double* v, double* z) {
+template <bool STEP, int LAM>
+__device__ __forceinline__ void energy_vals(const DevParams& p, const EnergyEIO& a, const EnergyRaw<STEP, LAM>& r,
+                                            bool inner, double* v, double* z) {
     double lam;
     if constexpr (LAM == kLamStored) lam = r.lam;
     if constexpr (LAM == kLamEvaluated) lam = lambda_eff(r.m, r.Sw, r.Sn, r.Sg, r.T);
     if constexpr (LAM == kLamConstant) lam = a.lam_cfg;
     v[0] = lam * r.T;
+    double rh[3];
+    if constexpr (STEP) {
+        rh[0] = ro_w_T(p, r.P[0], r.T) * H_w_of(p, r.T);
+        rh[1] = ro_n_T(p, inner ? r.P[0] : r.P[1], r.T) * H_n_T(p, r.T);
+        rh[2] = ro_g_T(p, inner ? r.P[0] : r.P[2], r.T) * H_g_T(p, r.T);
+    }
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-        const double rh = r.ro[q] * r.H[q];
-        v[1 + q] = rh * r.ux[q];
-        v[4 + q] = rh * r.uy[q];
-        z[q] = LAM == kLamConstant ? rh * r.uz[q] : v[4 + q];
+        if constexpr (!STEP) rh[q] = r.ro[q] * r.H[q];
+        v[1 + q] = rh[q] * r.ux[q];
+        v[4 + q] = rh[q] * r.uy[q];
+        z[q] = LAM == kLamConstant ? rh[q] * r.uz[q] : v[4 + q];
     }
 }
 
@@ -1074,7 +1111,7 @@ __device__ __forceinline__ double energy_adv(double wp, double wm, double np_, d
     return wp - wm + np_ - nm + gp - gm;
 }
 
-template <int LAM, int TX, int TY>
+template <bool STEP, int LAM, int TX, int TY>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(4)))
 k_energy_e_z(DevParams p, EnergyEIO a, int kchunk) {
     static_assert(TY >= 3 && TX == 64, "halo ring and whole rows per wavefront");
@@ -1100,6 +1137,7 @@ k_energy_e_z(DevParams p, EnergyEIO a, int kchunk) {
     else if (ty == 2 && tx < TY) { hi = i0 - 1; hj = j0 + tx; hx = 0; hy = tx + 1; }
     else if (ty == 2 && tx >= TY && tx < 2 * TY) { hi = i0 + TX; hj = j0 + tx - TY; hx = TX + 1; hy = tx - TY + 1; }
     const bool halo = hi >= 0 && hi < p.Nx && hj >= 0 && hj < p.Ny && (hasx || hi == i0 + tx);
+    const bool own_ij = inner_ij<3>(p, ic, min(j, p.Ny - 1)), halo_ij = inner_ij<3>(p, hi, hj);
     const HaloAt hat(p, i0, j0, hi, hj);
     const LdsDouble v0 = (LdsDouble)&lds[0][ty + 1][tx + 1][0], vh = (LdsDouble)&lds[0][hy][hx][0];
     auto stage = [&](LdsDouble w, const double* v) {
@@ -1110,21 +1148,23 @@ k_energy_e_z(DevParams p, EnergyEIO a, int kchunk) {
     // lambda_eff * T and the z products of the planes k - 1 and k
     double lm = 0., zm[3] = {}, lc, zc[3];
     {
-        EnergyRaw<LAM> r, rh;
+        EnergyRaw<STEP, LAM> r, rh;
         double v[NV], z[3];
         if (hasz) {
-            load_energy(a, CellAt{own.base - p.sz, own.off}, r);
-            energy_vals(a, r, v, zm);
+            const bool inner = own_ij && inner_k(p, k0 - 1);
+            load_energy(a, CellAt{own.base - p.sz, own.off}, inner, r);
+            energy_vals(p, a, r, inner, v, zm);
             lm = v[0];
         }
         asm volatile("" ::: "memory");  // one plane's values in registers at a time
-        load_energy(a, own, r);
-        if (halo) hat.with(p, k0, [&](const auto& at) { load_energy(a, at, rh); });
-        energy_vals(a, r, v, zc);
+        const bool inner = own_ij && inner_k(p, k0), inner_h = halo_ij && inner_k(p, k0);
+        load_energy(a, own, inner, r);
+        if (halo) hat.with(p, k0, [&](const auto& at) { load_energy(a, at, inner_h, rh); });
+        energy_vals(p, a, r, inner, v, zc);
         lc = v[0];
         stage(v0 + (k0 & 1) * PLANE, v);
         if (halo) {
-            energy_vals(a, rh, v, z);
+            energy_vals(p, a, rh, inner_h, v, z);
             stage(vh + (k0 & 1) * PLANE, v);
         }
     }
@@ -1132,9 +1172,10 @@ k_energy_e_z(DevParams p, EnergyEIO a, int kchunk) {
     for (int k = k0; k <= k1; ++k) {
         const bool next = k < k1;
         renew(own);
-        EnergyRaw<LAM> r, rh;
-        if (hasz) load_energy(a, CellAt{own.base + p.sz, own.off}, r);
-        if (next && halo) hat.with(p, k + 1, [&](const auto& at) { load_energy(a, at, rh); });
+        EnergyRaw<STEP, LAM> r, rh;
+        const bool inner = own_ij && inner_k(p, k + 1), inner_h = halo_ij && inner_k(p, k + 1);
+        if (hasz) load_energy(a, CellAt{own.base + p.sz, own.off}, inner, r);
+        if (next && halo) hat.with(p, k + 1, [&](const auto& at) { load_energy(a, at, inner_h, rh); });
         const double E = ld(a.E, own);
         const LdsDouble c = v0 + (k & 1) * PLANE;
         double T_flow = 0, E_flow = 0;
@@ -1151,13 +1192,13 @@ k_energy_e_z(DevParams p, EnergyEIO a, int kchunk) {
         double zp[3], lp = 0.;
         if (hasz) {
             double v[NV];
-            energy_vals(a, r, v, zp);
+            energy_vals(p, a, r, inner, v, zp);
             lp = v[0];
             if (next) stage(v0 + ((k + 1) & 1) * PLANE, v);
         }
         if (next && halo) {
             double v[NV], z[3];
-            energy_vals(a, rh, v, z);
+            energy_vals(p, a, rh, inner_h, v, z);
             stage(vh + ((k + 1) & 1) * PLANE, v);
         }
         if (hasz) {

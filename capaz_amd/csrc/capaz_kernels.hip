@@ -52,9 +52,10 @@ __global__ void __launch_bounds__(kBlock) k_fused_step(DevParams p, StepIO io) {
 // Energy step passes of their own: A and u of the boundary cells (face_cell's
 // numbering); roS with the interior u, and E, run on z tiles (capaz_fused.h);
 // Newton and the boundary are the entry points.
+template <bool KEEP>
 __global__ void __launch_bounds__(kBlock) k_energy_a(DevParams p, DevFields F, double* lam) {
     int64_t l = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (l < p.n) body_energy_a(p, F, lam, l);
+    if (l < p.n) body_energy_a<KEEP>(p, F, lam, l);
 }
 __global__ void __launch_bounds__(kBlock) k_energy_u_faces(DevParams p, DevFields F) {
     int i, j, k;
@@ -67,7 +68,7 @@ __global__ void __launch_bounds__(kBlock) k_energy_u_faces(DevParams p, DevField
 // bound by memory (15 to 20 values in, 10 out) and VALU issue alike: 160 x 128 x
 // 96, 3 iterations, 90 us in the step (STEP, body_newton_energy_nopivot) where
 // the inverse with its zeros and ones computed, S_g and H_* read, took 103.
-template <bool STEP>
+template <bool STEP, bool KEEP>
 __global__ void __launch_bounds__(kBlock) k_newton_energy(DevParams p, DevFields F, unsigned char* redo) {
     const int64_t l = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (l >= p.n) return;
@@ -76,10 +77,11 @@ __global__ void __launch_bounds__(kBlock) k_newton_energy(DevParams p, DevFields
     if (!STEP && p.model == 2)
         redo[l] = interior_newton2(p, i, j, k) && !body_newton_energy2_nopivot(p, F, l) ? 1 : 0;
     else
-        redo[l] = interior3(p, i, j, k) && !body_newton_energy_nopivot<STEP>(p, F, l) ? 1 : 0;
+        redo[l] = interior3(p, i, j, k) && !body_newton_energy_nopivot<STEP, KEEP>(p, F, l) ? 1 : 0;
 }
 // One thread per 16 marks (one 16-byte load; redo is allocated rounded up to
 // 16 bytes, the marks past Nx*Ny*Nz are never read as cells).
+template <bool STEP>
 __global__ void __launch_bounds__(kBlock) k_newton_energy_redo(DevParams p, DevFields F, const unsigned char* redo) {
     const int64_t l0 = ((int64_t)blockIdx.x * kBlock + threadIdx.x) * 16;
     if (l0 >= p.n) return;
@@ -87,7 +89,10 @@ __global__ void __launch_bounds__(kBlock) k_newton_energy_redo(DevParams p, DevF
     if ((w.x | w.y | w.z | w.w) == 0u) return;
     const int64_t end = l0 + 16 < p.n ? l0 + 16 : p.n;
     for (int64_t l = l0; l < end; ++l)
-        if (redo[l]) body_newton(p, F, l);
+        if (redo[l]) {
+            if constexpr (STEP) body_newton_energy_step(p, F, l);
+            else body_newton(p, F, l);
+        }
 }
 
 // boundary_conditions over the boundary cells only (the entry point and the
@@ -440,10 +445,10 @@ hipError_t launch_fused_record(const DevParams& p, const StepIO& io, int kchunk,
                            : launch_record_tile<3, 1>(p, io, kchunk, div, stride, s);
 }
 
-// roS (and, with U, u) of the interior cells on the z tiles, from the P, Xi
-// and ro arrays of this step (three phases).
+// roS (and, with U, u) of the interior cells on the z tiles (three phases);
+// without `keep` not the roS_old, nor the u_z that nothing in the step reads.
 template <bool U>
-hipError_t launch_roS_tiles(const DevParams& p, const DevFields& F, const double* dtm, hipStream_t s) {
+hipError_t launch_roS_tiles(const DevParams& p, const DevFields& F, const double* dtm, bool keep, hipStream_t s) {
     StepIO io{};
     io.Pw = F.f[F_P_w];
     io.Sw = F.f[F_S_w];
@@ -453,6 +458,7 @@ hipError_t launch_roS_tiles(const DevParams& p, const DevFields& F, const double
     io.m = F.f[F_m];
     io.K = F.f[F_K];
     io.dtm = dtm;
+    io.T = U ? F.f[F_T] : nullptr;
     const int xi[3] = {F_Xi_w, F_Xi_n, F_Xi_g}, ro[3] = {F_ro_w, F_ro_n, F_ro_g};
     const int rs[3] = {F_roS_w, F_roS_n, F_roS_g}, ro_old[3] = {F_roS_w_old, F_roS_n_old, F_roS_g_old};
     const int uf[3][3] = {{F_ux_w, F_uy_w, F_uz_w}, {F_ux_n, F_uy_n, F_uz_n}, {F_ux_g, F_uy_g, F_uz_g}};
@@ -462,23 +468,25 @@ hipError_t launch_roS_tiles(const DevParams& p, const DevFields& F, const double
         io.Xi[a] = F.f[xi[a]];
         io.ro[a] = F.f[ro[a]];
         st.roS[a] = F.f[rs[a]];
-        st.roS_old[a] = F.f[ro_old[a]];
-        for (int x = 0; x < 3; ++x) st.u[a][x] = U ? F.f[uf[a][x]] : nullptr;
+        st.roS_old[a] = keep ? F.f[ro_old[a]] : nullptr;
+        for (int x = 0; x < 3; ++x) st.u[a][x] = U && (x < 2 || keep || p.ecfg) ? F.f[uf[a][x]] : nullptr;
     }
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
-    // bound by memory: the narrow tiles' smaller cover gains nothing here
+    // 148 to 160 VGPRs: 32 x 8 workgroups, three per CU (160 x 128 x 96: 84 us),
+    // where a CU holds one of 64 x 8 (91; 101 at 4 waves, whose 128 VGPRs spill)
     auto launch = [&](auto full) {
-        constexpr auto kernel = k_roS_z<64, 8, decltype(full)::value, U>;
-        const int kchunk = fused_kchunk(p, 0, 8, resident_groups<kernel>(512));
-        dim3 grid((nx + 63) / 64, (ny + 7) / 8, (nz + kchunk - 1) / kchunk);
-        hipLaunchKernelGGL(kernel, grid, dim3(64, 8), 0, s, p, io, kchunk, st);
+        constexpr auto kernel = k_roS_z<32, 8, decltype(full)::value, U>;
+        const int kchunk = fused_kchunk(p, 0, 8, resident_groups<kernel>(256), 32);
+        dim3 grid((nx + 31) / 32, (ny + 7) / 8, (nz + kchunk - 1) / kchunk);
+        hipLaunchKernelGGL(kernel, grid, dim3(32, 8), 0, s, p, io, kchunk, st);
         return hipGetLastError();
     };
     return p.Nx >= 3 && p.Nz >= 3 ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
-// E_new of the interior cells on the z tiles; lam: the step's stored
-// lambda_eff, or NULL to evaluate it per staged cell (the entry point).
+// E_new of the interior cells on the z tiles; lam: the step's work array of
+// lambda_eff, or NULL for the entry point, which evaluates it per staged cell
+// and reads ro and H.
 hipError_t launch_energy_e_tiles(const DevParams& p, const DevFields& F, const double* lam, hipStream_t s) {
     EnergyEIO ea{};
     ea.lam = lam;
@@ -498,47 +506,58 @@ hipError_t launch_energy_e_tiles(const DevParams& p, const DevFields& F, const d
         ea.uy[a] = F.f[uy[a]];
         ea.uz[a] = F.f[uz[a]];
     }
+    const int pr[3] = {F_P_w, F_P_n, F_P_g};
+    for (int a = 0; a < 3; ++a) ea.P[a] = F.f[pr[a]];
     ea.lam_cfg = p.lam_eff;
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
-    auto launch = [&](auto lam_id) {
-        constexpr auto kernel = k_energy_e_z<decltype(lam_id)::value, 64, 8>;
+    auto launch = [&](auto step, auto lam_id) {
+        constexpr auto kernel = k_energy_e_z<decltype(step)::value, decltype(lam_id)::value, 64, 8>;
         const int kc = fused_kchunk(p, 0, 8, resident_groups<kernel>(512));
         dim3 ge((nx + 63) / 64, (ny + 7) / 8, (nz + kc - 1) / kc);
         hipLaunchKernelGGL(kernel, ge, dim3(64, 8), 0, s, p, ea, kc);
         return hipGetLastError();
     };
-    if (p.ecfg) return launch(std::integral_constant<int, kLamConstant>{});
-    return lam ? launch(std::integral_constant<int, kLamStored>{}) : launch(std::integral_constant<int, kLamEvaluated>{});
+    using std::integral_constant;
+    if (lam)
+        return p.ecfg ? launch(std::true_type{}, integral_constant<int, kLamConstant>{})
+                      : launch(std::true_type{}, integral_constant<int, kLamStored>{});
+    return p.ecfg ? launch(std::false_type{}, integral_constant<int, kLamConstant>{})
+                  : launch(std::false_type{}, integral_constant<int, kLamEvaluated>{});
 }
 
-template <bool STEP>
+template <bool STEP, bool KEEP>
 hipError_t launch_newton_energy_t(const DevParams& p, const DevFields& F, unsigned char* redo, hipStream_t s) {
     if (!redo) return launch_entry(Entry::Newton, p, F, s);
-    hipLaunchKernelGGL(k_newton_energy<STEP>, grid_for(p.n), dim3(kBlock), 0, s, p, F, redo);
-    hipLaunchKernelGGL(k_newton_energy_redo, grid_for((p.n + 15) / 16), dim3(kBlock), 0, s, p, F, redo);
+    hipLaunchKernelGGL((k_newton_energy<STEP, KEEP>), grid_for(p.n), dim3(kBlock), 0, s, p, F, redo);
+    hipLaunchKernelGGL(k_newton_energy_redo<STEP>, grid_for((p.n + 15) / 16), dim3(kBlock), 0, s, p, F, redo);
     return hipGetLastError();
 }
 
 hipError_t launch_newton_energy(const DevParams& p, const DevFields& F, unsigned char* redo, hipStream_t s) {
-    return launch_newton_energy_t<false>(p, F, redo, s);
+    return launch_newton_energy_t<false, true>(p, F, redo, s);
 }
 
 hipError_t launch_roS_stored(const DevParams& p, const DevFields& F, const double* dtm, hipStream_t s) {
     if (p.model != 3) return hipErrorInvalidValue;
-    return launch_roS_tiles<false>(p, F, dtm, s);
+    return launch_roS_tiles<false>(p, F, dtm, true, s);
 }
 
 hipError_t launch_energy_step(const DevParams& p, const DevFields& F, double* lam, const double* dtm,
-                              unsigned char* redo, hipStream_t s, const KernelEvents* ev) {
+                              unsigned char* redo, bool keep, hipStream_t s, const KernelEvents* ev) {
     hipError_t e;
     const dim3 g = grid_for(p.n), b(kBlock);
+    keep = keep || !redo;  // the general Newton alone reads S_g and H
     if (ev && (e = hipEventRecord(ev->begin, s)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_energy_a, g, b, 0, s, p, F, lam);
+    if (keep)
+        hipLaunchKernelGGL(k_energy_a<true>, g, b, 0, s, p, F, lam);
+    else
+        hipLaunchKernelGGL(k_energy_a<false>, g, b, 0, s, p, F, lam);
     // u of the boundary cells here, of the interior cells in the roS tiles
     hipLaunchKernelGGL(k_energy_u_faces, grid_for(fused_face_cells(p)), b, 0, s, p, F);
-    if ((e = launch_roS_tiles<true>(p, F, dtm, s)) != hipSuccess) return e;
+    if ((e = launch_roS_tiles<true>(p, F, dtm, keep, s)) != hipSuccess) return e;
     if ((e = launch_energy_e_tiles(p, F, lam, s)) != hipSuccess) return e;
-    if ((e = launch_newton_energy_t<true>(p, F, redo, s)) != hipSuccess) return e;
+    e = keep ? launch_newton_energy_t<true, true>(p, F, redo, s) : launch_newton_energy_t<true, false>(p, F, redo, s);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_boundary_faces, grid_for(fused_face_cells(p)), b, 0, s, p, F);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     return ev ? hipEventRecord(ev->end, s) : hipSuccess;

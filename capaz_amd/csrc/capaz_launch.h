@@ -59,9 +59,10 @@ hipError_t launch_energy_e_tiles(const DevParams& p, const DevFields& F, const d
 // One step of the energy model in six passes, in place on F; lam is a work
 // array of Nx*Ny*Nz doubles, dtm holds dt / m per cell, redo Nx*Ny*Nz bytes
 // (rounded up to 16) for the Newton pass (NULL: the Newton in one pass, as
-// launch_newton_energy); ev brackets the whole step.
+// launch_newton_energy); keep: store every intermediate (else those that the
+// step itself needs, see body_energy_a); ev brackets the whole step.
 hipError_t launch_energy_step(const DevParams& p, const DevFields& F, double* lam, const double* dtm,
-                              unsigned char* redo, hipStream_t s, const KernelEvents* ev = nullptr);
+                              unsigned char* redo, bool keep, hipStream_t s, const KernelEvents* ev = nullptr);
 // The energy model's Newton entry point: interior cells without the pivot
 // search, then the cells that need it (marked in redo, Nx*Ny*Nz bytes rounded
 // up to 16) with the general routine; redo NULL: the general routine on every

@@ -502,6 +502,35 @@ def test_energy_passes_equal_the_sequence(dims, closure):
     d.close()
 
 
+@pytest.mark.parametrize("tune", [dict(), dict(energy_newton=0)])
+def test_energy_step_fields_where_a_run_stops(tune):
+    """The steps of a run after which nothing can be read store fewer fields:
+    every field as from the sequence where a run of 1, 2 or 4 steps ends, and
+    where the sentinel ends one early."""
+    keys = case("3phe", 20, 11, 9, DT=1e-4, SOURCE=1)
+    st = random_state(keys, seed=8)
+    for steps, bad in ((1, False), (2, False), (4, False), (4, True)):
+        s = {f: v.copy() for f, v in st.items()}
+        if bad:
+            s["T"][4, 5, 10] = np.nan
+        seq, d = capaz.Domain(keys, s), capaz.Domain(keys, s)
+        seq.tune(energy_kernel=0)
+        seq.run(2 if bad else steps)
+        d.tune(**tune)
+        if bad:
+            d.tune(check_every=2)
+            with pytest.raises(capaz.NonFiniteState):
+                d.run(steps)
+        else:
+            d.run(steps)
+        for f in seq.names:
+            x, y = d.field(f), seq.field(f)
+            fin = np.isfinite(y)
+            assert np.array_equal(np.isfinite(x), fin) and bit_equal(x[fin], y[fin]), (steps, bad, f)
+        seq.close()
+        d.close()
+
+
 def test_energy_full_size_six_passes_equal_the_sequence():
     """The energy workload at 256 x 256 x 128: two steps of the six-pass
     energy step and two entry-point sequences give identical bits in every
