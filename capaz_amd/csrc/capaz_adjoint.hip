@@ -1,12 +1,14 @@
 // Adjoint kernels for gfx950: the two passes of the discrete adjoint step
 // (capaz_adjoint.h) and the observation gathers of the history-matching
-// objective.  One thread per cell, x fastest: a 64-wide wavefront reads 64
-// consecutive doubles of every field it touches, as the forward kernels do.
+// objective.  One thread per cell, x fastest: a wavefront reads rows of 64 (the
+// tiles of pass 2: 32) consecutive doubles of every field it touches, as the
+// forward kernels do.
 #include <hip/hip_runtime.h>
 
 #include "capaz_adjoint.h"
 #include "capaz_adjoint_launch.h"
 #include "capaz_fused.h"
+#include "capaz_launch.h"
 
 namespace capaz {
 
@@ -139,108 +141,227 @@ __global__ void __launch_bounds__(kTX * kTY) k_adj_newton_z(DevParams p, StepIO 
                                               (int)blockIdx.z, lds, AdjNewtonStore<IT>{a});
 }
 
-// Pass 2 over tiles of kTX x kTY columns (every cell, boundary included)
-// marching kchunk planes: each plane's coefficients and mu, with a one-cell
-// halo ring, are staged in LDS once and read by the x / y neighbours; the
-// z neighbours are carried in registers.
-struct AdjCoefLds {
-    double v[12][kTY + 2][kTX + 2];  // P[3], Xi[3], ro[3], mu[3]
+// Pass 2 on tiles of 32 x 8 columns (every cell, boundary included) marching
+// kchunk planes: each cell's pressures, L = -Xi ro, ro and mu are formed once
+// (and once more where another tile's ring holds it) and staged in LDS with a
+// one-cell ring for the x and y neighbours; a z face's driving force and upwind L
+// are carried from the plane below.  The values of adj_coef_cell, with its terms
+// in its order: a neighbour that is not interior, or does not exist, counts with
+// mu = 0 (the cells past the grid repeat the one before them).
+//
+// Bound by VALU issue and, at three waves per SIMD, by latency; the cell-by-cell
+// pass forms each cell's coefficients seven times (1608 instructions per cell):
+// 96^3, Corey-2, 42 us against 54.  159 VGPRs; four waves spill 31 of them (58
+// us), 32 x 16 workgroups, one per CU, 116.  One plane's LDS and two barriers per
+// plane; the next plane's loads are issued before this plane's terms.
+struct AdjRaw {
+    double Pw[1], Sw[1], Sn[1], K[1], Pn[1], Pg[1], mu[3];  // arrays of one, as coef_v reads them
 };
-
+struct AdjCell {
+    double P[3], L[3], ro[3], mu[3];
+};
+template <class At>
+__device__ __forceinline__ void adj_load(const AdjIO& a, const At& at, bool inner, AdjRaw& r) {
+    r.Pw[0] = ld(a.Pw, at);
+    r.Sw[0] = ld(a.Sw, at);
+    r.Sn[0] = ld(a.Sn, at);
+    r.K[0] = ld(a.K, at);
+    if (inner) {
+        r.mu[0] = ld(a.mu_w, at);
+        r.mu[1] = ld(a.mu_n, at);
+        r.mu[2] = ld(a.mu_g, at);
+    } else {
+        r.Pn[0] = ld(a.Pn, at);
+        r.Pg[0] = ld(a.Pg, at);
+        r.mu[0] = r.mu[1] = r.mu[2] = 0.;
+    }
+}
 template <int CL>
-__device__ __forceinline__ AdjNb adj_stage(const DevParams& p, const AdjIO& a, int i, int j, int k, bool in_grid) {
-    AdjNb n;
-    n.exists = in_grid;
-    n.interior = false;
-    n.mu[0] = n.mu[1] = n.mu[2] = 0.;
-    n.c = Coef{};
-    if (!in_grid) return n;
-    const int64_t q = (int64_t)i + (int64_t)j * p.sy + (int64_t)k * p.sz;
-    n.interior = interior3(p, i, j, k);
-    n.c = coef_v<CL>(p, a, q, n.interior);
-    if (n.interior) {
-        n.mu[0] = a.mu_w[q];
-        n.mu[1] = a.mu_n[q];
-        n.mu[2] = a.mu_g[q];
-    }
-    return n;
-}
-
-__device__ __forceinline__ void lds_put(AdjCoefLds& lds, int y, int x, const AdjNb& n) {
+__device__ __forceinline__ void adj_cell(const DevParams& p, const AdjRaw& r, bool inner, AdjCell& c) {
+    const Coef v = coef_v<CL>(p, r, 0, inner);
 #pragma unroll
-    for (int ph = 0; ph < 3; ++ph) {
-        lds.v[ph][y][x] = n.c.P[ph];
-        lds.v[3 + ph][y][x] = n.c.Xi[ph];
-        lds.v[6 + ph][y][x] = n.c.ro[ph];
-        lds.v[9 + ph][y][x] = n.mu[ph];
+    for (int a = 0; a < 3; ++a) {
+        c.P[a] = v.P[a];
+        c.L[a] = -v.Xi[a] * v.ro[a];
+        c.ro[a] = v.ro[a];
+        c.mu[a] = r.mu[a];
     }
 }
-
-__device__ __forceinline__ AdjNb lds_get(const DevParams& p, const AdjCoefLds& lds, int y, int x, int i, int j,
-                                         int k) {
-    AdjNb n;
-    n.exists = i >= 0 && i < p.Nx && j >= 0 && j < p.Ny;
-    n.interior = n.exists && interior3(p, i, j, k);
-#pragma unroll
-    for (int ph = 0; ph < 3; ++ph) {
-        n.c.P[ph] = lds.v[ph][y][x];
-        n.c.Xi[ph] = lds.v[3 + ph][y][x];
-        n.c.ro[ph] = lds.v[6 + ph][y][x];
-        n.mu[ph] = lds.v[9 + ph][y][x];
-    }
-    return n;
+// The upwind L of a face whose driving force is x: Lm of its minus side for x >
+// 0, Lp of its plus side for x < 0, their mean else (upwind_w).
+__device__ __forceinline__ double upwind_L(double x, double Lm, double Lp) {
+    const double t = 0.5 * Lm + 0.5 * Lp;
+    return x > 0. ? Lm : (x < 0. ? Lp : t);
+}
+// adj_coef_axis's terms of one phase from the driving forces and upwind Ls of the
+// own flux's faces (x1, T1, x2, T2) and of the two neighbours' fluxes there.
+__device__ __forceinline__ void adj_terms(double x1, double T1, double x2, double T2, double xm, double Tm, double xq,
+                                          double Tq, double mu, double mum, double muq, double rh, double& lP,
+                                          double& lL) {
+    const double d1 = -(T1 * rh), d2 = T2 * rh;
+    lP += mu * (d2 - d1) * rh;
+    lL += mu * ((pos_part(x2) - neg_part(x1)) * rh);
+    lP += muq * -(Tq * rh) * rh;
+    lL += muq * (-pos_part(xq) * rh);
+    lP += mum * (-(Tm * rh) * rh);
+    lL += mum * (neg_part(xm) * rh);
 }
 
-template <int CL>
-__global__ void __launch_bounds__(kTX * kTY) k_adj_coef_z(DevParams p, AdjIO a, int kchunk) {
-    __shared__ AdjCoefLds lds;
+template <int CL, int TX, int TY>
+__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(CL == 0 ? 2 : 3)))
+k_adj_coef_z(DevParams p, AdjIO a, int kchunk) {
+    static_assert((TX == 32 || TX == 64) && TX >= 2 * TY && TY >= 3, "whole rows per wavefront; ring cells of three rows");
+    constexpr int NV = 13, ROW = (TX + 2) * NV;  // an odd count: a row's reads of one value on distinct banks
+    __shared__ double lds[TY + 2][TX + 2][NV];
+    int bx, by, bz;
+    xcd_tile(bx, by, bz);
     const int tx = threadIdx.x, ty = threadIdx.y;
-    const int i0 = kTX * (int)blockIdx.x, j0 = kTY * (int)blockIdx.y, k0 = kchunk * (int)blockIdx.z;
-    const int k1 = min(p.Nz - 1, k0 + kchunk - 1);
+    const int i0 = TX * bx, j0 = TY * by, k0 = kchunk * bz, k1 = min(p.Nz - 1, k0 + kchunk - 1);
     const int i = i0 + tx, j = j0 + ty;
-    const bool own = i < p.Nx && j < p.Ny;
-    // halo cell of this thread, as in the fused step's tiles
-    int hi = -1, hj = -1, hx = 0, hy = 0;
+    const bool own = i < p.Nx && j < p.Ny, hasx = p.Nx >= 2, hasz = p.Nz >= 2;
+    const int ic = min(i, p.Nx - 1), jc = min(j, p.Ny - 1);
+    const int jw = __builtin_amdgcn_readfirstlane(jc);
+    CellAt at{(int64_t)i0 + (int64_t)jw * p.sy + (int64_t)k0 * p.sz, 8u * (uint32_t)(ic - i0)};
+    if (TX < 64) at.off += 8u * (uint32_t)(jc - jw) * (uint32_t)p.sy;
+    const bool own_ij = own && inner_ij<3>(p, ic, jc);
+    // ring cell of this thread, clamped into the grid
+    int hi = 0, hj = 0, hx = 0, hy = 0;
     if (ty == 0) { hi = i; hj = j0 - 1; hx = tx + 1; hy = 0; }
-    else if (ty == 1) { hi = i; hj = j0 + kTY; hx = tx + 1; hy = kTY + 1; }
-    else if (ty == 2 && tx < kTY) { hi = i0 - 1; hj = j0 + tx; hx = 0; hy = tx + 1; }
-    else if (ty == 2 && tx >= kTY && tx < 2 * kTY) { hi = i0 + kTX; hj = j0 + tx - kTY; hx = kTX + 1; hy = tx - kTY + 1; }
-    const bool halo = hi >= 0 && hi < p.Nx && hj >= 0 && hj < p.Ny;
-    const bool hasz = !(p.Nz < 2);
+    else if (ty == 1) { hi = i; hj = j0 + TY; hx = tx + 1; hy = TY + 1; }
+    else { hi = tx < TY ? i0 - 1 : i0 + TX; hj = j0 + (tx & (TY - 1)); hx = tx < TY ? 0 : TX + 1; hy = (tx & (TY - 1)) + 1; }
+    const bool halo = ty < 2 || (ty == 2 && tx < 2 * TY);
+    const bool halo_ij = hi >= 0 && hi < p.Nx && hj >= 0 && hj < p.Ny && inner_ij<3>(p, hi, hj);
+    hi = min(max(hi, 0), p.Nx - 1);
+    hj = min(max(hj, 0), p.Ny - 1);
+    const int64_t hcol = (int64_t)hi + (int64_t)hj * p.sy;
 
-    AdjNb zm = adj_stage<CL>(p, a, i, j, k0 - 1, own && hasz && k0 >= 1);
-    AdjNb c = adj_stage<CL>(p, a, i, j, k0, own);
-    for (int k = k0; k <= k1; ++k) {
-        if (own) lds_put(lds, ty + 1, tx + 1, c);
-        if (halo) lds_put(lds, hy, hx, adj_stage<CL>(p, a, hi, hj, k, true));
-        __syncthreads();
-        const AdjNb zp = adj_stage<CL>(p, a, i, j, k + 1, own && hasz && k + 1 < p.Nz);
-        if (own) {
-            const int64_t l = (int64_t)i + (int64_t)j * p.sy + (int64_t)k * p.sz;
-            const CoefD cd = coef_d<CL>(p, a, l, c.interior);
-            double lP[3] = {0., 0., 0.}, lL[3] = {0., 0., 0.}, lro[3] = {0., 0., 0.};
-            if (!(p.Nx < 2))
-                adj_coef_axis(p, cd, c.mu, lds_get(p, lds, ty + 1, tx, i - 1, j, k),
-                              lds_get(p, lds, ty + 1, tx + 2, i + 1, j, k), p.r_hx, false, lP, lL, lro);
-            adj_coef_axis(p, cd, c.mu, lds_get(p, lds, ty, tx + 1, i, j - 1, k),
-                          lds_get(p, lds, ty + 2, tx + 1, i, j + 1, k), p.r_hy, true, lP, lL, lro);
-            if (hasz) adj_coef_axis(p, cd, c.mu, zm, zp, p.r_hz, false, lP, lL, lro);
-            adj_coef_finish(p, a, l, cd, lP, lL, lro);
+    const LdsDouble v0 = (LdsDouble)&lds[ty + 1][tx + 1][0], vh = (LdsDouble)&lds[hy][hx][0];
+    auto stage = [&](LdsDouble w, const AdjCell& c) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            w[q] = c.P[q];
+            w[3 + q] = c.L[q];
+            w[6 + q] = c.ro[q];
+            w[9 + q] = c.mu[q];
         }
-        __syncthreads();
-        zm = c;
-        c = zp;
+    };
+
+    AdjRaw r;
+    // the face between this plane and the one below: its driving force and
+    // upwind L, and the mu below
+    double x1[3] = {0., 0., 0.}, T1[3] = {0., 0., 0.}, mum[3] = {0., 0., 0.};
+    bool inner = own_ij && inner_k(p, k0);
+    adj_load(a, at, inner, r);
+    {
+        AdjRaw rm, rh;
+        AdjCell c, m;
+        const bool inner_m = own_ij && k0 >= 1 && inner_k(p, k0 - 1), inner_h = halo_ij && inner_k(p, k0);
+        if (k0 >= 1) adj_load(a, CellAt{at.base - p.sz, at.off}, inner_m, rm);
+        if (halo) adj_load(a, CellIndex{hcol + (int64_t)k0 * p.sz}, inner_h, rh);
+        adj_cell<CL>(p, r, inner, c);
+        stage(v0, c);
+        if (k0 >= 1) {
+            adj_cell<CL>(p, rm, inner_m, m);
+#pragma unroll
+            for (int ph = 0; ph < 3; ++ph) {
+                x1[ph] = -((c.P[ph] - m.P[ph]) * p.r_hz);
+                T1[ph] = upwind_L(x1[ph], m.L[ph], c.L[ph]);
+                mum[ph] = m.mu[ph];
+            }
+        }
+        if (halo) {
+            adj_cell<CL>(p, rh, inner_h, m);
+            stage(vh, m);
+        }
+    }
+    __syncthreads();
+    for (int k = k0; k <= k1; ++k) {
+        const bool next = k < k1, zp = hasz && k + 1 < p.Nz;
+        const bool inner_q = own_ij && zp && inner_k(p, k + 1), inner_h = halo_ij && inner_k(p, k + 1);
+        renew(at);
+        AdjRaw rq, rh;
+        if (zp) adj_load(a, CellAt{at.base + p.sz, at.off}, inner_q, rq);
+        double lP[3], lL[3], lro[3];
+        // the own cell's row of values and the rows below and above it, from x - 1 on
+        LdsDouble row[3];
+#pragma unroll
+        for (int y = 0; y < 3; ++y) {
+            row[y] = v0 + (y - 1) * ROW - NV;
+            asm("" : "+v"(row[y]));
+        }
+        auto nb = [&](int q, int y, int x) { return row[y][x * NV + q]; };
+#pragma unroll
+        for (int ph = 0; ph < 3; ++ph) {
+            lP[ph] = lL[ph] = lro[ph] = 0.;
+            const double P = nb(ph, 1, 1), L = nb(3 + ph, 1, 1), mu = nb(9 + ph, 1, 1);
+            if (hasx) {
+                const double xa = -((P - nb(ph, 1, 0)) * p.r_hx), xb = -((nb(ph, 1, 2) - P) * p.r_hx);
+                const double Ta = upwind_L(xa, nb(3 + ph, 1, 0), L), Tb = upwind_L(xb, L, nb(3 + ph, 1, 2));
+                adj_terms(xa, Ta, xb, Tb, xa, Ta, xb, Tb, mu, nb(9 + ph, 1, 0), nb(9 + ph, 1, 2), p.r_hx, lP[ph], lL[ph]);
+            }
+            const double da = -((P - nb(ph, 0, 1)) * p.r_hy), db = -((nb(ph, 2, 1) - P) * p.r_hy);
+            const double La = nb(3 + ph, 0, 1), Lb = nb(3 + ph, 2, 1), gc = p.g * nb(6 + ph, 1, 1);
+            const double xa = da + gc, xb = db + gc, xm = da + p.g * nb(6 + ph, 0, 1), xq = db + p.g * nb(6 + ph, 2, 1);
+            const double Ta = upwind_L(xa, La, L), Tb = upwind_L(xb, L, Lb);
+            adj_terms(xa, Ta, xb, Tb, xm, upwind_L(xm, La, L), xq, upwind_L(xq, L, Lb), mu, nb(9 + ph, 0, 1),
+                      nb(9 + ph, 2, 1), p.r_hy, lP[ph], lL[ph]);
+            lro[ph] += mu * (-(Ta * p.r_hy) + Tb * p.r_hy) * p.g;
+            // one phase's values in registers at a time: its sums are done here
+            asm volatile("" : "+v"(lP[ph]), "+v"(lL[ph]), "+v"(lro[ph])::"memory");
+        }
+        if (next && halo) adj_load(a, CellIndex{hcol + (int64_t)(k + 1) * p.sz}, inner_h, rh);
+        AdjCell q;
+        if (zp) adj_cell<CL>(p, rq, inner_q, q);
+        if (hasz) {
+#pragma unroll
+            for (int ph = 0; ph < 3; ++ph) {
+                const double mu = nb(9 + ph, 1, 1);
+                double x2 = 0., T2 = 0.;
+                if (zp) {
+                    x2 = -((q.P[ph] - nb(ph, 1, 1)) * p.r_hz);
+                    T2 = upwind_L(x2, nb(3 + ph, 1, 1), q.L[ph]);
+                }
+                adj_terms(x1[ph], T1[ph], x2, T2, x1[ph], T1[ph], x2, T2, mu, mum[ph], zp ? q.mu[ph] : 0., p.r_hz,
+                          lP[ph], lL[ph]);
+                x1[ph] = x2;
+                T1[ph] = T2;
+                mum[ph] = mu;
+            }
+        }
+        if (own) {
+            const CoefD cd = coef_d<CL>(p, r, 0, inner);
+            CellAt to = at;
+            renew(to);
+            adj_coef_finish(p, a, to.l(), cd, lP, lL, lro);
+        }
+        if (next) {
+            r = rq;
+            inner = inner_q;
+            at.base += p.sz;
+            __syncthreads();
+            stage(v0, q);
+            if (halo) {
+                AdjCell h;
+                adj_cell<CL>(p, rh, inner_h, h);
+                stage(vh, h);
+            }
+            __syncthreads();
+        }
     }
 }
 
-hipError_t launch_adj_coef_z(const DevParams& p, const AdjIO& a, dim3 g, int kchunk, hipStream_t s) {
-    if (p.closure == 0)
-        hipLaunchKernelGGL(k_adj_coef_z<0>, g, dim3(kTX, kTY), 0, s, p, a, kchunk);
-    else if (p.corey_n == 2.)
-        hipLaunchKernelGGL(k_adj_coef_z<2>, g, dim3(kTX, kTY), 0, s, p, a, kchunk);
-    else
-        hipLaunchKernelGGL(k_adj_coef_z<1>, g, dim3(kTX, kTY), 0, s, p, a, kchunk);
+template <int CL>
+hipError_t launch_adj_coef_tile(const DevParams& p, const AdjIO& a, hipStream_t s) {
+    constexpr int TX = 32, TY = 8;
+    constexpr auto kernel = k_adj_coef_z<CL, TX, TY>;
+    const int kchunk = fused_kchunk(p, 0, TY, resident_groups<kernel>(TX * TY), TX);
+    const dim3 grid((p.Nx + TX - 1) / TX, (p.Ny + TY - 1) / TY, (p.Nz + kchunk - 1) / kchunk);
+    hipLaunchKernelGGL(kernel, grid, dim3(TX, TY), 0, s, p, a, kchunk);
     return hipGetLastError();
+}
+hipError_t launch_adj_coef_z(const DevParams& p, const AdjIO& a, hipStream_t s) {
+    if (p.closure == 0) return launch_adj_coef_tile<0>(p, a, s);
+    return p.corey_n == 2. ? launch_adj_coef_tile<2>(p, a, s) : launch_adj_coef_tile<1>(p, a, s);
 }
 
 // Planes per tile: enough workgroups to fill the GPU several times over,
@@ -286,11 +407,7 @@ hipError_t launch_adjoint_step_tiled(const DevParams& p, const AdjIO& a, hipStre
 #undef CAPAZ_ADJ1
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const int64_t txy2 = (int64_t)((p.Nx + kTX - 1) / kTX) * ((p.Ny + kTY - 1) / kTY);
-    const int kc2 = adj_kchunk(p.Nz, txy2);
-    const dim3 g2((unsigned)((p.Nx + kTX - 1) / kTX), (unsigned)((p.Ny + kTY - 1) / kTY),
-                  (unsigned)((p.Nz + kc2 - 1) / kc2));
-    return launch_adj_coef_z(p, a, g2, kc2, s);
+    return launch_adj_coef_z(p, a, s);
 }
 
 hipError_t launch_adjoint_coef(const DevParams& p, const AdjIO& a, hipStream_t s) {
@@ -326,7 +443,7 @@ hipError_t launch_adjoint_step_recorded(const DevParams& p, const AdjIO& a, cons
                        total);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_adjoint_coef(p, a, s);
+    return launch_adj_coef_z(p, a, s);
 }
 
 hipError_t launch_adjoint_step(const DevParams& p, const AdjIO& a, hipStream_t s) {

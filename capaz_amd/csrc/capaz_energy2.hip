@@ -543,25 +543,12 @@ k_energy2_z(DevParams p, E2IO io, int kchunk) {
     e2_tile<CLOSURE, TX, TY, HASZ>(p, kernel_params(), io, kchunk, lds);
 }
 
-template <auto Kernel>
-int resident(int threads) {
-    static int cached = 0;
-    if (cached) return cached;
-    int dev = 0, cus = 0, per_cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, Kernel, threads, 0) != hipSuccess || per_cu < 1)
-        return 512;
-    cached = cus * per_cu;
-    return cached;
-}
-
 template <int CLOSURE, bool HASZ>
 hipError_t launch_e2(const DevParams& p, const E2IO& io, int kchunk, hipStream_t s, const KernelEvents* ev) {
     constexpr int TX = 32, TY = 512 / TX;
     const int nx = p.Nx - 2, ny = p.Ny - 2, nz = HASZ ? p.Nz - 2 : 1;
     constexpr auto kernel = k_energy2_z<CLOSURE, TX, TY, HASZ>;
-    kchunk = fused_kchunk(p, kchunk, TY, resident<kernel>(TX * TY), TX);
+    kchunk = fused_kchunk(p, kchunk, TY, resident_groups<kernel>(TX * TY), TX);
     const dim3 grid((nx + TX - 1) / TX, (ny + TY - 1) / TY, (nz + kchunk - 1) / kchunk);
     hipError_t e;
     if (ev && (e = hipEventRecord(ev->begin, s)) != hipSuccess) return e;

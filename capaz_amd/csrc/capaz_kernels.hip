@@ -278,21 +278,6 @@ hipError_t launch_fused_step(const DevParams& p, const StepIO& io, hipStream_t s
     return hipGetLastError();
 }
 
-// Workgroups of a kernel resident at once on the device (cached per kernel;
-// one device type per process).
-template <auto Kernel>
-int resident_groups(int threads) {
-    static int cached = 0;
-    if (cached) return cached;
-    int dev = 0, cus = 0, per_cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, Kernel, threads, 0) != hipSuccess || per_cu < 1)
-        return 512;
-    cached = cus * per_cu;
-    return cached;
-}
-
 int fused_kchunk(const DevParams& p, int kchunk, int ty, int resident, int tx) {
     if (kchunk >= 1) return std::min(kchunk, kMaxPlanes);
     // automatic: the planes per tile that minimise (rounds of resident

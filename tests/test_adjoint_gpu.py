@@ -86,6 +86,26 @@ def test_adjoint_matches_host_build_and_checkpointing_is_exact(kernel, dims, clo
     ref.close()
 
 
+@pytest.mark.parametrize("dims", [(32, 8, 5), (33, 9, 40), (64, 17, 3), (3, 3, 3), (31, 25, 1), (1, 33, 6)])
+@pytest.mark.parametrize("closure,over", [("corey", dict()), ("corey", dict(COREY_N=2.5)), ("reference", dict())])
+def test_tiled_gather_equals_the_cell_by_cell_one(dims, closure, over):
+    """Pass 2 on its 32 x 8 tiles (adjoint_kernel 2, 1) at the edges of tiles and
+    chunks against one thread per cell (0): the same J, and gradients equal but
+    for the roundings in which their first passes differ."""
+    keys, st, lnK, obs, rng = problem(*dims, 7, 3, closure)
+    keys = dict(keys, **over)
+    grads = []
+    for kernel in (2, 1, 0):
+        d = capaz.Domain(keys, st)
+        d.tune(adjoint_kernel=kernel)
+        grads.append(d.adjoint(3, obs))
+        d.close()
+    for J, gK, gm in grads[1:]:
+        assert J == grads[0][0]
+        assert rel(gK, grads[0][1]) < 1e-12 and rel(gm, grads[0][2]) < 1e-12
+        assert np.isfinite(gK).all()
+
+
 @pytest.mark.parametrize("closure", ["corey", "reference"])
 def test_adjoint_directional_derivatives_match_central_differences(closure):
     keys, st, lnK, obs, rng = problem(24, 20, 16, 41, 12, closure)
