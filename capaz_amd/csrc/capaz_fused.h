@@ -905,7 +905,7 @@ __device__ __forceinline__ void store_faces(const DevParams& p, const StepIO& io
 // k_fused_faces writes them after the kernel).  The two-phase kernels write
 // their faces here (the strided x faces cost a separate pass more than the
 // epilogue costs); in the three-phase kernels the extra registers would cost
-// a wave per SIMD, so they keep the face pass.  CLOSURE: the kernel's
+// a wave per SIMD, so but for small grids they keep the face pass.  CLOSURE: the kernel's
 // (the two-phase Newton then carries only its closure's code).
 template <int MODEL, bool FACES = false, int CLOSURE = -1>
 struct FusedStore {
@@ -950,7 +950,7 @@ struct FusedStore {
 };
 
 // Two phases: boundary cells included (kFusedFaces); three phases: followed
-// by k_fused_faces.
+// by k_fused_faces (but for small grids, k_fused_z).
 template <int MODEL>
 constexpr bool kFusedFaces = MODEL == 2;
 
@@ -1265,14 +1265,18 @@ constexpr int kWideTY = MODEL == 2 && CLOSURE != 1 ? 4 : 8;
 template <int MODEL, int CLOSURE>
 constexpr int kNarrowTY = MODEL == 2 && CLOSURE == 2 ? 8 : 16;
 
-template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
+// FACES: the boundary cells too, for three phases in grids that take the 64 x 4
+// tiles for being small: there a launch counts, not the registers (24^3 9.6 us per
+// step against 11.1 with k_fused_faces, 48^3 13.4 against 15.0; 256^3 574 against
+// 538 with these tiles).
+template <int MODEL, int CLOSURE, int TX, int TY, bool FULL, bool FACES>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(kFusedWaves<MODEL, CLOSURE, TX, TY>)))
 k_fused_z(DevParams p, StepIO io, int kchunk) {
     __shared__ FusedLds<MODEL, CLOSURE, TX, TY> lds;
     int bx, by, bz;
     xcd_tile(bx, by, bz);
     fused_z_tile<MODEL, CLOSURE, TX, TY, FULL>(p, kernel_params(), io, kchunk, bx, by, bz, lds,
-                                               FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE>{io});
+                                               FusedStore<MODEL, FACES, CLOSURE>{io});
 }
 
 // Cell number t of a box of ni x nj cells per plane starting at (i0, j0, k0),

@@ -335,10 +335,10 @@ hipError_t with_tile(const DevParams& p, const F& f) {
     return f(integral_constant<int, 64>{}, integral_constant<int, WIDE_TY>{});
 }
 
-template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
+template <int MODEL, int CLOSURE, int TX, int TY, bool FULL, bool FACES>
 hipError_t launch_z(const DevParams& p, const StepIO& io, int kchunk, hipStream_t s, const KernelEvents* ev) {
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
-    constexpr auto kernel = k_fused_z<MODEL, CLOSURE, TX, TY, FULL>;
+    constexpr auto kernel = k_fused_z<MODEL, CLOSURE, TX, TY, FULL, FACES>;
     kchunk = fused_kchunk(p, kchunk, TY, resident_groups<kernel>(TX * TY), TX);
     dim3 grid((nx + TX - 1) / TX, (ny + TY - 1) / TY, (nz + kchunk - 1) / kchunk);
     hipError_t e;
@@ -346,7 +346,7 @@ hipError_t launch_z(const DevParams& p, const StepIO& io, int kchunk, hipStream_
     hipLaunchKernelGGL(kernel, grid, dim3(TX, TY), 0, s, p, io, kchunk);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (ev && (e = hipEventRecord(ev->end, s)) != hipSuccess) return e;
-    if constexpr (!kFusedFaces<MODEL>) {
+    if constexpr (!FACES) {
         const int64_t nfaces = fused_face_cells(p);
         if (io.pack)
             hipLaunchKernelGGL((k_fused_faces_pack<MODEL, CLOSURE>), grid_for(nfaces + 2LL * p.Nx * p.Ny), dim3(256),
@@ -360,16 +360,21 @@ hipError_t launch_z(const DevParams& p, const StepIO& io, int kchunk, hipStream_
 
 template <int MODEL, int CLOSURE>
 hipError_t launch_z_tile(const DevParams& p, const StepIO& io, const Tuning& t, hipStream_t s, const KernelEvents* ev) {
-    auto launch = [&](auto tx, auto ty) {
-        constexpr int TX = decltype(tx)::value, TY = decltype(ty)::value;
-        return p.Nx >= 3 && p.Nz >= 3 ? launch_z<MODEL, CLOSURE, TX, TY, true>(p, io, t.kchunk, s, ev)
-                                      : launch_z<MODEL, CLOSURE, TX, TY, false>(p, io, t.kchunk, s, ev);
-    };
     using std::integral_constant;
+    auto launch_faces = [&](auto tx, auto ty, auto faces) {
+        constexpr int TX = decltype(tx)::value, TY = decltype(ty)::value;
+        constexpr bool FACES = decltype(faces)::value;
+        return p.Nx >= 3 && p.Nz >= 3 ? launch_z<MODEL, CLOSURE, TX, TY, true, FACES>(p, io, t.kchunk, s, ev)
+                                      : launch_z<MODEL, CLOSURE, TX, TY, false, FACES>(p, io, t.kchunk, s, ev);
+    };
+    auto launch = [&](auto tx, auto ty) {
+        return launch_faces(tx, ty, integral_constant<bool, kFusedFaces<MODEL>>{});
+    };
     const int64_t groups = covering_threads(p, 64, 4) / 256 * (p.Nz >= 3 ? p.Nz - 2 : 1);
-    const bool small = groups <= resident_groups<k_fused_z<MODEL, CLOSURE, 64, 4, true>>(256);
-    if (t.tile_y == 4 || (t.tile_y == 0 && small))
-        return launch(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+    const bool small = groups <= resident_groups<k_fused_z<MODEL, CLOSURE, 64, 4, true, true>>(256);
+    if (t.tile_y == 0 && small)
+        return launch_faces(integral_constant<int, 64>{}, integral_constant<int, 4>{}, std::true_type{});
+    if (t.tile_y == 4) return launch(integral_constant<int, 64>{}, integral_constant<int, 4>{});
     if (t.tile_y == 8) return launch(integral_constant<int, 64>{}, integral_constant<int, 8>{});
     return with_tile<kWideTY<MODEL, CLOSURE>, kNarrowTY<MODEL, CLOSURE>>(p, launch);
 }
