@@ -38,8 +38,8 @@ ALGO_BYTES_PER_CELL = 64
 # the counters read a device-to-device copy of known size correctly) and FP64
 # flops (64 lanes x (ADD + MUL + TRANS + 2 FMA) of SQ_INSTS_VALU_*_F64).
 # profiles/fused_step_3ph_256.md holds the runs and their commands.
-TRAFFIC_BYTES_PER_CELL = 74.7
-FP64_FLOPS_PER_CELL = 873.1
+TRAFFIC_BYTES_PER_CELL = 78.5
+FP64_FLOPS_PER_CELL = 788.6
 
 
 def _cpu_model() -> str:
@@ -295,8 +295,8 @@ ENERGY2_ALGO_BYTES_PER_CELL = 56
 # Measured per interior cell of one k_energy2_z launch at 256 x 256 x 128, as
 # for the three-phase step: HBM bytes (FETCH_SIZE x 2.0 + WRITE_SIZE) and FP64
 # flops; profiles/energy2_2ph_256x256x128.md holds the runs and their commands.
-ENERGY2_TRAFFIC_BYTES_PER_CELL = 71.7
-ENERGY2_FP64_FLOPS_PER_CELL = 1640.8
+ENERGY2_TRAFFIC_BYTES_PER_CELL = 130.7
+ENERGY2_FP64_FLOPS_PER_CELL = 1335.6
 
 
 def bench_energy(nx: int = 256, ny: int = 256, nz: int = 128, steps: int = 20) -> dict:
