@@ -193,8 +193,9 @@ struct E2Lds {
 };
 
 // One tile.  Bound by VALU issue (FP64), 1330 instructions per cell at 4 Newton
-// iterations, 850 of them the Newton's.  256 x 256 x 128, Corey-2: 408 us per
-// step against 866 for one workgroup per CU with 215 VGPRs, a called Newton
+// iterations, 850 of them the Newton's.  256 x 256 x 128, Corey-2: 381 us per
+// step (408 with S_n, T and lambda_eff * T kept across the Newton, whose loop
+// then spilled) against 866 for one workgroup per CU with 215 VGPRs, a called Newton
 // and parameters in vector-register lanes (2510 instructions).  Blocks of
 // 32 x 16: their two planes' LDS (80 KB) lets two workgroups share a CU and
 // their rings re-evaluate 20% of the cells; 64 x 8 (87 KB, 29%) takes 499 us.
@@ -276,10 +277,11 @@ __device__ __forceinline__ void e2_tile(const DevParams& p, ConstParams* cp, con
         return exact_div(Pp - Pm, pf.two_hz, pf.r_two_hz);
     };
 
-    // carried along z: the minus face (directed()'s neg_part(x1) and t2),
-    // lambda_eff * T of plane k - 1, the (ro H) u_z products of planes k - 1
-    // (gm) and k (gc), and the own S_n and T
-    double zneg[NP], zt2[2] = {0., 0.}, zLT = 0., gm[2] = {0., 0.}, gc[2] = {0., 0.}, Sn_c, T_c;
+    // carried along z: the minus face (directed()'s neg_part(x1) and t2) and the
+    // (ro H) u_z products of planes k - 1 (gm) and k (gc); lambda_eff * T of plane
+    // k - 1 stands in the own cell's place of the other buffer until plane k + 1
+    // is staged there
+    double zneg[NP], zt2[2] = {0., 0.}, gm[2] = {0., 0.}, gc[2] = {0., 0.};
 #pragma unroll
     for (int a = 0; a < NP; ++a) zneg[a] = 0.;
     uint32_t undone = 0;
@@ -300,11 +302,9 @@ __device__ __forceinline__ void e2_tile(const DevParams& p, ConstParams* cp, con
         E2Coef<CLOSURE> c, m;
         e2_coef(pc, r, c);
         stage(k0, c0, p0, c);
-        Sn_c = r.Sn;
-        T_c = r.T;
         if (HASZ) {
             e2_coef(pc, rm, m);
-            zLT = m.LT;
+            (c0 + ((k0 + 1) & 1) * PLANE)[6] = m.LT;
 #pragma unroll
             for (int q = 0; q < NP; ++q) {
                 const double d = exact_div(c.P[q] - m.P[q], pf.hz, pf.r_hz);
@@ -351,7 +351,8 @@ __device__ __forceinline__ void e2_tile(const DevParams& p, ConstParams* cp, con
                 }
             });
         }
-        const double m_c = ld(io.m, own);
+        // read again rather than kept from the plane before: registers
+        const double m_c = ld(io.m, own), Sn_c = ld(io.Sn, own), T_c = ld(io.T, own);
 
         const DevParams pf = e2_flux_params(fresh(cp));
         // the own cell's row of coefficients and the rows below and above it, from
@@ -365,6 +366,7 @@ __device__ __forceinline__ void e2_tile(const DevParams& p, ConstParams* cp, con
         asm("" : "+v"(pp));
         auto C_at = [&](int q, int y, int x) { return row[y][x * 7 + q]; };
         double div[2], T_flow = 0., E_flow = 0.;
+        const double zLT = HASZ ? (c0 + ((k + 1) & 1) * PLANE)[6] : 0.;
         if (active) {
             double e[2][2];  // (ro H) u of the minus and plus neighbours
             const double LT2 = 2. * C_at(6, 1, 1);
@@ -440,7 +442,7 @@ __device__ __forceinline__ void e2_tile(const DevParams& p, ConstParams* cp, con
             }
         }
         asm volatile("" ::: "memory");
-        double gp[2] = {0., 0.}, LT_c = 0.;
+        double gp[2] = {0., 0.};
         if (active) {
             double Xi[2], ro[2];
 #pragma unroll
@@ -449,7 +451,7 @@ __device__ __forceinline__ void e2_tile(const DevParams& p, ConstParams* cp, con
                 ro[a] = C_at(2 + a, 1, 1);
             }
             if (HASZ) {
-                LT_c = C_at(6, 1, 1);
+                const double LT_c = C_at(6, 1, 1);
 #pragma unroll
                 for (int q = 0; q < NP; ++q) {
                     const double P = pp[q];
@@ -499,14 +501,11 @@ __device__ __forceinline__ void e2_tile(const DevParams& p, ConstParams* cp, con
             st(io.T1, to, T);
         }
         if (next) {
-            zLT = LT_c;
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
                 gm[a] = gc[a];
                 gc[a] = gp[a];
             }
-            Sn_c = r.Sn;
-            T_c = r.T;
             own.base += p.sz;
             __syncthreads();
         }
