@@ -295,7 +295,7 @@ ENERGY2_ALGO_BYTES_PER_CELL = 56
 # Measured per interior cell of one k_energy2_z launch at 256 x 256 x 128, as
 # for the three-phase step: HBM bytes (FETCH_SIZE x 2.0 + WRITE_SIZE) and FP64
 # flops; profiles/energy2_2ph_256x256x128.md holds the runs and their commands.
-ENERGY2_TRAFFIC_BYTES_PER_CELL = 130.7
+ENERGY2_TRAFFIC_BYTES_PER_CELL = 86.3
 ENERGY2_FP64_FLOPS_PER_CELL = 1335.6
 
 

@@ -192,8 +192,8 @@ struct E2Lds {
     double C[2][TY + 2][TX + 2][7];  // Xi_w, Xi_n, ro_w, ro_n, roH_w, roH_n, lambda_eff * T
 };
 
-// One tile.  Bound by VALU issue (FP64), 1330 instructions per cell at 4 Newton
-// iterations, 850 of them the Newton's.  256 x 256 x 128, Corey-2: 381 us per
+// One tile.  Bound by VALU issue (FP64), 1290 instructions per cell at 4 Newton
+// iterations, 840 of them the Newton's.  256 x 256 x 128, Corey-2: 381 us per
 // step (408 with S_n, T and lambda_eff * T kept across the Newton, whose loop
 // then spilled) against 866 for one workgroup per CU with 215 VGPRs, a called Newton
 // and parameters in vector-register lanes (2510 instructions).  Blocks of
