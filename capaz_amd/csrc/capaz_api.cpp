@@ -433,7 +433,7 @@ int capaz_roS(capaz_ctx* c, double t) {
         // three phases: on the z tiles unless some interior cell has m == 0
         if ((rc = scan_m(c))) return rc;
         if (!c->m_has_zero) {
-            CAPAZ_HIP(c, capaz::launch_roS_stored(c->p, fields_of(c), c->d_dtm, c->stream));
+            CAPAZ_HIP(c, capaz::launch_roS_stored(c->p, fields_of(c), c->d_dtm, c->tuning.kchunk, c->stream));
             return CAPAZ_OK;
         }
     }

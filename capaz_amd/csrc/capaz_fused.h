@@ -213,26 +213,30 @@ template <class E>
 struct EpiWantsU<E, std::void_t<decltype(E::kWantsU)>> : std::bool_constant<E::kWantsU> {};
 
 // Pressures staged per cell: the phases' pressures are one value except where
-// a closure has a capillary pressure (two phases, Brooks-Corey).  Three
-// phases: P_n = P_g = P_w in the interior and, once Border_P has run, on the
-// x and z faces; the top and bottom rows' own P_n and P_g are staged apart.
+// a closure has a capillary pressure (two phases, Brooks-Corey) and in the roS
+// entry point (CLOSURE 3), which takes P_n and P_g of every cell as a caller set
+// them.  Three phases otherwise: P_n = P_g = P_w in the interior and, once
+// Border_P has run, on the x and z faces; the top and bottom rows' own P_n and
+// P_g are staged apart.
 template <int MODEL, int CLOSURE>
-constexpr int kStagedP = MODEL == 2 && CLOSURE == 0 ? 2 : 1;
+constexpr int kStagedP = MODEL == 2 ? (CLOSURE == 0 ? 2 : 1) : (CLOSURE == 3 ? 3 : 1);
 
 // LDS of a tile: two planes' coefficients (P, Xi, ro) of the tile and its
 // one-cell ring, the plane being read and the one being staged.  A cell's
 // values lie together, so that a neighbour's are one address and constant
 // offsets that a paired read reaches (an array per value needed ~20 address
 // additions per cell); their number is odd, which puts 64 lanes' reads of one
-// value on distinct banks.  Three phases: edge[.][0 / 1] = P_n, P_g of the top / bottom row (j = 0 / Ny - 1)
-// where the tile touches it, odd[.][row] = the plane k in which a staged x
-// face cell of that row has a P_n or P_g of its own (any other value: none).
+// value on distinct banks.  Three phases with one staged pressure: edge[.][0 / 1]
+// = P_n, P_g of the top / bottom row (j = 0 / Ny - 1) where the tile touches it,
+// odd[.][row] = the plane k in which a staged x face cell of that row has a P_n or
+// P_g of its own (any other value: none).
 template <int MODEL, int CLOSURE, int TX, int TY>
 struct FusedLds {
-    static constexpr int kNV = (kStagedP<MODEL, CLOSURE> + 2 * MODEL) | 1;
+    static constexpr int kNP = kStagedP<MODEL, CLOSURE>, kNV = (kNP + 2 * MODEL) | 1;
+    static constexpr bool kApart = MODEL == 3 && kNP == 1;
     double v[2][TY + 2][TX + 2][kNV];
-    double edge[2][MODEL == 3 ? 2 : 0][2][TX + 2];
-    int odd[2][MODEL == 3 ? TY + 2 : 0];
+    double edge[2][kApart ? 2 : 0][2][TX + 2];
+    int odd[2][kApart ? TY + 2 : 0];
 };
 
 // A cell of a field array: a wave-uniform index (scalar registers) and the
@@ -405,12 +409,17 @@ __device__ __forceinline__ void load_raw(const StepIO& io, const At& at, bool in
 }
 
 // coef_at's values from what load_raw read; the return value tells a cell
-// whose P_n or P_g is not its P_w (three phases, boundary cells).
+// whose P_n or P_g is not its P_w (three phases with one staged pressure,
+// boundary cells).
 template <int MODEL, int CLOSURE>
 __device__ __forceinline__ bool coef_of(const DevParams& p, const CellRaw<MODEL, CLOSURE>& r, bool inner,
                                         CellCoef<MODEL, CLOSURE>& c) {
     c.P[0] = r.Pw;
     if constexpr (CLOSURE >= 3) {
+        if constexpr (CLOSURE == 3) {
+            c.P[1] = r.Pn;
+            c.P[2] = r.Pg;
+        }
 #pragma unroll
         for (int a = 0; a < MODEL; ++a) {
             c.Xi[a] = r.Xi[a];
@@ -461,7 +470,7 @@ __device__ __forceinline__ bool coef_of(const DevParams& p, const CellRaw<MODEL,
         c.ro[1] = ro_n_of(p, r.Pw);
         c.ro[2] = ro_g_of(p, r.Pw);
     }
-    if constexpr (MODEL == 3) {
+    if constexpr (MODEL == 3 && CLOSURE != 3) {
         if (!inner) {
             if constexpr (CLOSURE < 3) {
                 c.ro[1] = ro_n_of(p, r.Pn);
@@ -555,10 +564,9 @@ struct CellState {
 // does every cell.
 //
 // Cells that the planes' code does not cover -- the epilogue left it undone (a
-// pivot search), or an x or z face neighbour (for the roS entry point: the cell
-// or any neighbour) has a P_n or P_g that is not its P_w (values a caller set;
-// Border_P gives those faces P_n = P_g = P_w, P_Xi_ro every interior cell) -- are
-// marked and done after the last plane from the state the step reads, which
+// pivot search), or, where one pressure is staged, an x or z face neighbour has a
+// P_n or P_g that is not its P_w (values a caller set; Border_P gives those faces
+// P_n = P_g = P_w, P_Xi_ro every interior cell) -- are marked and done after the last plane from the state the step reads, which
 // it does not write: the planes' code then holds no call and no registers for
 // them (kchunk <= kMaxPlanes, one mark per plane).
 // cp: p in constant memory (fresh()).
@@ -572,8 +580,8 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
     constexpr int ROW = (TX + 2) * NV, PLANE = (TY + 2) * ROW;  // LDS pitch of a row, of a plane
     constexpr bool U = EpiWantsU<Epi>::value;
     constexpr bool EARLY = CLOSURE == 0 || CLOSURE == 1;
-    // the roS entry point: a P_n or P_g of its own in any cell, as a caller set it
-    constexpr bool OWN_P = CLOSURE == 3;
+    // three phases: P_n and P_g apart from the staged pressure, where they differ
+    constexpr bool APART = FusedLds<MODEL, CLOSURE, TX, TY>::kApart;
 
     const int tx = threadIdx.x, ty = threadIdx.y;
     const bool hasx = FULL || p.Nx >= 3, hasz = FULL || p.Nz >= 3;
@@ -588,7 +596,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
     // no active lane reads); jw: the wavefront's first row
     const int ic = min(i, p.Nx - 1), jc = min(j, p.Ny - 1);
     const int jw = __builtin_amdgcn_readfirstlane(jc);
-    const bool own_ij = !OWN_P && inner_ij<MODEL>(p, ic, jc);
+    const bool own_ij = CLOSURE != 3 && inner_ij<MODEL>(p, ic, jc);
     CellAt own{(int64_t)i0 + (int64_t)jw * p.sy + (int64_t)k0 * p.sz, 8u * (uint32_t)(ic - i0)};
     if (TX < 64) own.off += 8u * (uint32_t)(jc - jw) * (uint32_t)p.sy;
 
@@ -600,7 +608,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
     else if (ty == 2 && tx < TY) { hi = i0 - 1; hj = j0 + tx; hx = 0; hy = tx + 1; }
     else if (ty == 2 && tx >= TY && tx < 2 * TY) { hi = i0 + TX; hj = j0 + tx - TY; hx = TX + 1; hy = tx - TY + 1; }
     const bool halo = hi >= 0 && hi < p.Nx && hj >= 0 && hj < p.Ny && (hasx || hi == i0 + tx);
-    const bool halo_ij = !OWN_P && inner_ij<MODEL>(p, hi, hj);
+    const bool halo_ij = CLOSURE != 3 && inner_ij<MODEL>(p, hi, hj);
     const HaloAt hat(p, i0, j0, hi, hj);
 
     // LDS places in the buffer of plane 0: the own and the halo cell
@@ -615,7 +623,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
             w[NPR + a] = c.Xi[a];
             w[NPR + NPH + a] = c.ro[a];
         }
-        if constexpr (MODEL == 3) {
+        if constexpr (APART) {
             if (!inner) {
                 if (jj == 0 || jj == p.Ny - 1) {
                     lds.edge[k & 1][jj == 0 ? 0 : 1][0][x] = r.Pn;
@@ -630,7 +638,9 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
     // the minus z face (directed()'s neg_part(x1) and t2) and the own
     // saturations, carried from plane to plane
     double zneg[NPR], zt2[NPH], zmP[NPR], Sw = 0., Sn = 0.;
-    uint64_t zodd = 0;  // the lanes whose cell below (k - 1) has a P_n or P_g of its own
+    // the lanes whose cell below (k - 1) has a P_n or P_g of its own: a boundary
+    // plane's, below the tile's first one
+    uint64_t zodd = 0;
     uint32_t undone = 0;
 #pragma unroll
     for (int a = 0; a < NPR; ++a) zneg[a] = zmP[a] = 0.;
@@ -682,7 +692,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
             const DevParams pc = coef_params<MODEL, CLOSURE>(fresh(cp));
             if (hasz) {
                 const bool mine = coef_of(pc, r, inner, zp);
-                if constexpr (MODEL == 3) odd = __ballot(mine);
+                if constexpr (APART) odd = __ballot(mine);
                 if (next || EARLY) stage(k + 1, v0 + buffer(k + 1), ty + 1, tx + 1, jc, r, inner, zp, mine);
             }
             if (next && halo) {
@@ -749,11 +759,11 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
             };
             // three phases, next to the top and bottom rows: their own P_n and P_g
             const int jr = TX == 64 ? jw : j;
-            if (MODEL == 3 && (jr == 1 || jr == p.Ny - 2)) {
+            if (APART && (jr == 1 || jr == p.Ny - 2)) {
 #pragma unroll
                 for (int a = 0; a < NPH; ++a) {
                     double Pm = P_at(0, 0, 1), Pp = P_at(0, 2, 1);
-                    if constexpr (MODEL == 3) {
+                    if constexpr (APART) {
                         if (a > 0 && jr == 1) Pm = lds.edge[k & 1][0][a - 1][tx + 1];
                         if (a > 0 && jr == p.Ny - 2) Pp = lds.edge[k & 1][1][a - 1][tx + 1];
                     }
@@ -813,10 +823,9 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
 #pragma unroll
             for (int a = 0; a < NPH; ++a) s.ro[a] = c.ro[a];
             bool done = true;
-            if constexpr (MODEL == 3) {
+            if constexpr (APART) {
                 const uint64_t lane = 1ull << ((ty * TX + tx) & 63);
-                bool row_odd = lds.odd[k & 1][ty + 1] == k;
-                if constexpr (OWN_P) row_odd = row_odd || lds.odd[k & 1][ty] == k || lds.odd[k & 1][ty + 2] == k;
+                const bool row_odd = lds.odd[k & 1][ty + 1] == k;
                 if (__builtin_expect((zodd | odd) != 0 || __ballot(row_odd) != 0, 0))
                     done = !row_odd && ((zodd | odd) & lane) == 0;
             }
@@ -829,7 +838,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
             }
         }
         if (next) {
-            zodd = odd;
+            zodd = 0;
             Sn = r.Sn;
             if constexpr (MODEL == 3) Sw = r.Sw;
             own.base += p.sz;
@@ -975,9 +984,10 @@ struct FusedStoreRecord {
 };
 
 // assign_roS_nr (cpu.cpp:619-731) on the z tiles (three phases): roS_old and
-// roS of the cell from the stored coefficients (CLOSURE 3, the roS entry point),
-// or (U, CLOSURE 4) the energy step's roS + u pass, with the cell's velocities
-// (assign_u) from the same neighbours.  Arrays that are NULL are not stored.
+// roS of the cell from the stored coefficients (CLOSURE 3, the roS entry point,
+// every cell's P_n and P_g as they stand) or (U, CLOSURE 4) the energy step's roS +
+// u pass, with the cell's velocities (assign_u) from the same neighbours.  Arrays
+// that are NULL are not stored.
 template <bool U>
 struct RoSStore {
     static constexpr bool kWantsU = U;

@@ -438,7 +438,8 @@ hipError_t launch_fused_record(const DevParams& p, const StepIO& io, int kchunk,
 // roS (and, with U, u) of the interior cells on the z tiles (three phases);
 // without `keep` not the roS_old, nor the u_z that nothing in the step reads.
 template <bool U>
-hipError_t launch_roS_tiles(const DevParams& p, const DevFields& F, const double* dtm, bool keep, hipStream_t s) {
+hipError_t launch_roS_tiles(const DevParams& p, const DevFields& F, const double* dtm, bool keep, int planes,
+                            hipStream_t s) {
     StepIO io{};
     io.Pw = F.f[F_P_w];
     io.Sw = F.f[F_S_w];
@@ -462,16 +463,28 @@ hipError_t launch_roS_tiles(const DevParams& p, const DevFields& F, const double
         for (int x = 0; x < 3; ++x) st.u[a][x] = U && (x < 2 || keep || p.ecfg) ? F.f[uf[a][x]] : nullptr;
     }
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
-    // 148 to 160 VGPRs: 32 x 8 workgroups, three per CU (160 x 128 x 96: 84 us),
-    // where a CU holds one of 64 x 8 (91; 101 at 4 waves, whose 128 VGPRs spill)
-    auto launch = [&](auto full) {
-        constexpr auto kernel = k_roS_z<32, 8, decltype(full)::value, U>;
-        const int kchunk = fused_kchunk(p, 0, 8, resident_groups<kernel>(256), 32);
-        dim3 grid((nx + 31) / 32, (ny + 7) / 8, (nz + kchunk - 1) / kchunk);
-        hipLaunchKernelGGL(kernel, grid, dim3(32, 8), 0, s, p, io, kchunk, st);
+    auto launch = [&](auto tx, auto full) {
+        constexpr int TX = decltype(tx)::value, TY = 8;
+        constexpr auto kernel = k_roS_z<TX, TY, decltype(full)::value, U>;
+        const int kchunk = fused_kchunk(p, planes, TY, resident_groups<kernel>(TX * TY), TX);
+        dim3 grid((nx + TX - 1) / TX, (ny + TY - 1) / TY, (nz + kchunk - 1) / kchunk);
+        hipLaunchKernelGGL(kernel, grid, dim3(TX, TY), 0, s, p, io, kchunk, st);
         return hipGetLastError();
     };
-    return p.Nx >= 3 && p.Nz >= 3 ? launch(std::true_type{}) : launch(std::false_type{});
+    auto launch_wide = [&](auto tx) {
+        return p.Nx >= 3 && p.Nz >= 3 ? launch(tx, std::true_type{}) : launch(tx, std::false_type{});
+    };
+    // With u, 142 to 154 VGPRs: 32 x 8 workgroups, three per CU (160 x 128 x 96: 84
+    // us), where a CU holds one of 64 x 8 (91; 101 at 4 waves, whose 128 VGPRs
+    // spill).  The entry point, which stages three pressures (95 KB of LDS for 64 x
+    // 8, 49 for 32 x 8) and is bound by memory: 256^3 583 us on 64 x 8, 743 on 32 x
+    // 8; 200 x 180 x 150 216 and 227; narrow grids, whose 64-wide rows would stay
+    // half empty, on 32 x 8 (34 x 120 x 200 27.4, 31.5 on 64
+    // x 8; 1 x 256 x 256 27.3 and 63).
+    using std::integral_constant;
+    if constexpr (!U)
+        if (nx > 32) return launch_wide(integral_constant<int, 64>{});
+    return launch_wide(integral_constant<int, 32>{});
 }
 
 // E_new of the interior cells on the z tiles; lam: the step's work array of
@@ -527,9 +540,9 @@ hipError_t launch_newton_energy(const DevParams& p, const DevFields& F, unsigned
     return launch_newton_energy_t<false, true>(p, F, redo, s);
 }
 
-hipError_t launch_roS_stored(const DevParams& p, const DevFields& F, const double* dtm, hipStream_t s) {
+hipError_t launch_roS_stored(const DevParams& p, const DevFields& F, const double* dtm, int kchunk, hipStream_t s) {
     if (p.model != 3) return hipErrorInvalidValue;
-    return launch_roS_tiles<false>(p, F, dtm, true, s);
+    return launch_roS_tiles<false>(p, F, dtm, true, kchunk, s);
 }
 
 hipError_t launch_energy_step(const DevParams& p, const DevFields& F, double* lam, const double* dtm,
@@ -544,7 +557,7 @@ hipError_t launch_energy_step(const DevParams& p, const DevFields& F, double* la
         hipLaunchKernelGGL(k_energy_a<false>, g, b, 0, s, p, F, lam);
     // u of the boundary cells here, of the interior cells in the roS tiles
     hipLaunchKernelGGL(k_energy_u_faces, grid_for(fused_face_cells(p)), b, 0, s, p, F);
-    if ((e = launch_roS_tiles<true>(p, F, dtm, keep, s)) != hipSuccess) return e;
+    if ((e = launch_roS_tiles<true>(p, F, dtm, keep, 0, s)) != hipSuccess) return e;
     if ((e = launch_energy_e_tiles(p, F, lam, s)) != hipSuccess) return e;
     e = keep ? launch_newton_energy_t<true, true>(p, F, redo, s) : launch_newton_energy_t<true, false>(p, F, redo, s);
     if (e != hipSuccess) return e;

@@ -51,8 +51,9 @@ hipError_t launch_fused(const DevParams& p, const StepIO& io, const Tuning& t, h
                         const KernelEvents* ev = nullptr);
 // The roS entry point of the three-phase model on the fused kernel's z tiles,
 // from the P, Xi and ro arrays P_Xi_ro wrote (no cell may have m == 0: the
-// per-cell entry point keeps their stale roS); dtm holds dt / m per cell.
-hipError_t launch_roS_stored(const DevParams& p, const DevFields& F, const double* dtm, hipStream_t s);
+// per-cell entry point keeps their stale roS); dtm holds dt / m per cell;
+// kchunk: planes per tile (fused_kchunk).
+hipError_t launch_roS_stored(const DevParams& p, const DevFields& F, const double* dtm, int kchunk, hipStream_t s);
 // E_new of the interior cells on z tiles (energy model); lam: lambda_eff per
 // cell computed earlier in the step, or NULL to evaluate it from the fields.
 hipError_t launch_energy_e_tiles(const DevParams& p, const DevFields& F, const double* lam, hipStream_t s);

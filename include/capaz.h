@@ -194,9 +194,9 @@ int capaz_step(capaz_ctx* ctx, long first_step, long nsteps);
  *                   2: as 1
  *   "tile_y"        4 or 8: tiles of 64 x tile_y columns; 0 (default): their
  *                   shape chosen by model, closure and grid
- *   "kchunk"        planes per workgroup along z (above 32: 32); 0 (default):
- *                   chosen from the grid (16 on large grids, fewer on small
- *                   ones)
+ *   "kchunk"        planes per workgroup along z (above 32: 32), of
+ *                   capaz_roS's tiles too; 0 (default): chosen from the grid
+ *                   (16 on large grids, fewer on small ones)
  *   "adjoint_kernel" capaz_adjoint's passes: 2 (default) the backward
  *                   Newton from the flux divergence recorded while each
  *                   segment is recomputed; 1 both passes on z-marching LDS

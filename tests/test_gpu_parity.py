@@ -344,6 +344,48 @@ def test_roS_entry_point_with_phase_pressures_as_set(dims, share):
         assert bit_equal(got[0][f], got[1][f]), f
 
 
+@pytest.mark.parametrize("dims,planes", [((34, 11, 24), 2), ((35, 19, 19), 5), ((66, 9, 40), 16), ((96, 96, 96), 0)])
+@pytest.mark.parametrize("set_cells", ["few", "column", "box"])
+def test_roS_entry_point_over_several_planes(dims, planes, set_cells):
+    """capaz_roS on tiles of several planes (96^3: as many as it takes by itself)
+    where P_n and P_g were set in a few scattered cells, in one column of every
+    third plane or in a box that ends inside a tile's planes, so that a cell's only
+    neighbour with phase pressures of its own may be any of the six: the bits of
+    the kernel with one thread per cell."""
+    keys = case("3ph", *dims)
+    st = random_state(keys, seed=sum(dims))
+    rng = np.random.default_rng(sum(dims))
+    nx, ny, nz = dims
+    own = np.zeros(st["P_w"].shape, bool)
+    if set_cells == "few":
+        own = rng.random(own.shape) < 0.004
+    elif set_cells == "column":
+        own[1:-1:3, ny // 2, nx // 2] = True
+    else:
+        own[nz // 4:nz // 4 + 7, 2:-2, 3:-3] = True
+    assert own.any()
+    put = {f: np.where(own, st["P_w"] + rng.uniform(-20, 20, own.shape), st["P_w"]) for f in ("P_n", "P_g")}
+    zero = (nz // 2, ny // 2, nx // 2)
+    got = []
+    for m0 in (False, True):
+        m = st["m"].copy()
+        if m0:
+            m[zero] = 0.0
+        d = capaz.Domain(keys, dict(st, m=m))
+        d.tune(kchunk=planes)
+        d.ro_P_Xi_calculation()
+        for f, v in put.items():
+            d.set_field(f, v)
+        d.roS_calculation()
+        out = {f: d.field(f) for f in ("roS_w", "roS_n", "roS_g", "roS_g_old")}
+        for v in out.values():
+            v[zero] = 0.0
+        got.append(out)
+        d.close()
+    for f in got[0]:
+        assert bit_equal(got[0][f], got[1][f]), f
+
+
 def test_headline_physics_bitwise_at_96():
     """The benchmark physics (three-phase, Corey-2, lognormal K, top
     injection) at 96^3: one and three fused steps equal the oracle bit for bit."""
