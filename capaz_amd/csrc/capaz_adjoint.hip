@@ -122,9 +122,10 @@ __global__ void k_obs_adjoint(double* lSw, double* lSn, const int64_t* cells, in
 template <int IT>
 struct AdjNewtonStore {
     AdjIO a;
+    static constexpr bool kLeaves = false;
     template <class At>
     __device__ __forceinline__ int prefetch(const At&) const { return 0; }
-    template <bool GENERAL, class At>
+    template <class At>
     __device__ __forceinline__ bool cell(const DevParams& p, const DevParams&, int i, int j, int k, const At& at,
                                          const CellState<3>& s, const double* div, int) const {
         adj_newton_tail<IT>(p, a, i, j, k, at.l(), s.ro, s.P, s.Sw, s.Sn, div);

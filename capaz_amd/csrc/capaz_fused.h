@@ -29,12 +29,6 @@
 
 namespace capaz {
 
-template <int NPH>
-struct CoefT {
-    double P[NPH], Xi[NPH], ro[NPH];
-    double Sw, Sn;  // the cell's saturations, as read
-};
-
 // -K k_r of a phase with the Corey closure: exponent 2 (CLOSURE 2) or read
 // from p (1).  For exponent 2 the clip to [0, 1] is one instruction (the clamp
 // modifier, which makes a NaN 0), and a NaN s comes back through K: 0 * s + K
@@ -49,103 +43,23 @@ __device__ __forceinline__ double corey_mK(const DevParams& p, double K, double 
     }
 }
 
+// The two phases' densities of a cell in the state a step reads (body_P_Xi_ro).
 template <int CLOSURE>
-__device__ __forceinline__ double corey_t(const DevParams& p, double s) {
-    if constexpr (CLOSURE == 2) {
-        s = clamp01(s);
-        return s * s;
-    } else {
-        return corey_kr(p, s);
-    }
-}
-
-// assign_P_Xi + assign_ro of one cell with the model and closure fixed at
-// compile time (cpu.cpp:143-169; two-phase.cpp:4-23; three-phase.cpp:198-240).
-// CLOSURE 3 (three phases): the values in the P_n, P_g, Xi and ro arrays; 4, the
-// energy step: Xi as its first pass stored it, ro from P and T.
-template <int MODEL, int CLOSURE>
-__device__ __forceinline__ CoefT<MODEL> coef_at(const DevParams& p, const StepIO& io, int64_t l, bool inner) {
-    CoefT<MODEL> c;
-    if constexpr (CLOSURE >= 3) {
-        static_assert(MODEL == 3, "stored coefficients: three phases");
-        inner = inner && CLOSURE == 4;
-        c.Sw = io.Sw[l];
-        c.Sn = io.Sn[l];
-        c.P[0] = io.Pw[l];
-        c.P[1] = inner ? c.P[0] : io.Pn[l];
-        c.P[2] = inner ? c.P[0] : io.Pg[l];
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            c.Xi[a] = io.Xi[a][l];
-            if constexpr (CLOSURE == 3) c.ro[a] = io.ro[a][l];
-        }
-        if constexpr (CLOSURE == 4) {
-            const double T = io.T[l];
-            c.ro[0] = ro_w_T(p, c.P[0], T);
-            c.ro[1] = ro_n_T(p, c.P[1], T);
-            c.ro[2] = ro_g_T(p, c.P[2], T);
-        }
-        return c;
-    }
-    const double Pw = io.Pw[l], K = io.K[l];
-    if constexpr (MODEL == 2) {
+__device__ __forceinline__ void densities2(const DevParams& p, const StepIO& io, int64_t l, double* ro) {
+    const double Pw = io.Pw[l];
+    double Pn = Pw;
+    if constexpr (CLOSURE == 0) {
         double kw, kn, Pk;
-        const double Sn = io.Sn[l];
-        c.Sn = Sn;
-        c.Sw = 0.;
-        if constexpr (CLOSURE >= 1) {
-            double se = exact_div(1. - Sn - p.S_wr, p.den2c, p.r_den2c);
-            kw = corey_t<CLOSURE>(p, se);
-            kn = corey_t<CLOSURE>(p, 1. - se);
-            Pk = 0.;
-        } else {
-            relperm2(p, Sn, kw, kn, Pk);
-        }
-        const double Pn = Pw + Pk;
-        c.P[0] = Pw;
-        c.P[1] = Pn;
-        c.Xi[0] = xi_const(K, kw, p.mu_w, p.r_mu_w);
-        c.Xi[1] = xi_const(K, kn, p.mu_n, p.r_mu_n);
-        c.ro[0] = ro_w_of(p, Pw);
-        c.ro[1] = ro_n_of(p, Pn);
-    } else {
-        double kw, kn, kg;
-        const double Sw = io.Sw[l], Sn = io.Sn[l];
-        c.Sw = Sw;
-        c.Sn = Sn;
-        if constexpr (CLOSURE >= 1) {
-            const double Swe = exact_div(Sw - p.S_wr, p.den3, p.r_den3);
-            const double Sne = exact_div(Sn - p.S_nr, p.den3, p.r_den3);
-            const double Sge = 1. - Swe - Sne;
-            kw = corey_t<CLOSURE>(p, Swe);
-            kn = corey_t<CLOSURE>(p, Sne);
-            kg = corey_t<CLOSURE>(p, Sge);
-        } else {
-            relperm3(p, Sw, Sn, kw, kn, kg);
-        }
-        const double Pn = inner ? Pw : io.Pn[l];
-        const double Pg = inner ? Pw : io.Pg[l];
-        c.P[0] = Pw;
-        c.P[1] = Pn;
-        c.P[2] = Pg;
-        c.Xi[0] = xi_const(K, kw, p.mu_w, p.r_mu_w);
-        c.Xi[1] = xi_const(K, kn, p.mu_n, p.r_mu_n);
-        c.Xi[2] = xi_const(K, kg, p.mu_g, p.r_mu_g);
-        c.ro[0] = ro_w_of(p, Pw);
-        c.ro[1] = ro_n_of(p, Pn);
-        c.ro[2] = ro_g_of(p, Pg);
+        relperm2(p, io.Sn[l], kw, kn, Pk);
+        Pn = Pw + Pk;
     }
-    return c;
+    ro[0] = ro_w_of(p, Pw);
+    ro[1] = ro_n_of(p, Pn);
 }
 
-template <int MODEL>
-__device__ __forceinline__ bool inner_cell(const DevParams& p, int i, int j, int k) {
-    return MODEL == 2 ? interior_newton2(p, i, j, k) : interior3(p, i, j, k);
-}
-
-// inner_cell split into its (i, j) and k factors: inner_cell(p, i, j, k) ==
-// inner_ij(p, i, j) && inner_k(p, k).  A tile column evaluates the (i, j)
-// factor once, so only one lane mask per column stays live across the planes.
+// Whether a cell is interior (interior_newton2, interior3), split into its (i, j)
+// and k factors: a tile column evaluates the (i, j) factor once, so only one lane
+// mask per column stays live across the planes.
 template <int MODEL>
 __device__ __forceinline__ bool inner_ij(const DevParams& p, int i, int j) {
     const bool ii = (i != 0) && (i != p.Nx - 1);
@@ -228,14 +142,15 @@ constexpr int kStagedP = MODEL == 2 ? (CLOSURE == 0 ? 2 : 1) : (CLOSURE == 3 ? 3
 // additions per cell); their number is odd, which puts 64 lanes' reads of one
 // value on distinct banks.  Three phases with one staged pressure: edge[.][0 / 1]
 // = P_n, P_g of the top / bottom row (j = 0 / Ny - 1) where the tile touches it,
-// odd[.][row] = the plane k in which a staged x face cell of that row has a P_n or
-// P_g of its own (any other value: none).
+// side[.][0 / 1] of the x face cells (i = 0 / Nx - 1), odd[.][row] = the plane k in
+// which such a cell of that row has a P_n or P_g that is not its P_w (else any
+// value, k too: side holds them whether they differ or not).
 template <int MODEL, int CLOSURE, int TX, int TY>
 struct FusedLds {
     static constexpr int kNP = kStagedP<MODEL, CLOSURE>, kNV = (kNP + 2 * MODEL) | 1;
     static constexpr bool kApart = MODEL == 3 && kNP == 1;
     double v[2][TY + 2][TX + 2][kNV];
-    double edge[2][kApart ? 2 : 0][2][TX + 2];
+    double edge[2][kApart ? 2 : 0][2][TX + 2], side[2][kApart ? 2 : 0][2][TY + 2];
     int odd[2][kApart ? TY + 2 : 0];
 };
 
@@ -408,8 +323,11 @@ __device__ __forceinline__ void load_raw(const StepIO& io, const At& at, bool in
     }
 }
 
-// coef_at's values from what load_raw read; the return value tells a cell
-// whose P_n or P_g is not its P_w (three phases with one staged pressure,
+// assign_P_Xi + assign_ro of one cell with the model and closure fixed at compile
+// time (cpu.cpp:143-169; two-phase.cpp:4-23; three-phase.cpp:198-240) from what
+// load_raw read.  CLOSURE 3 (three phases): the values of the P_n, P_g, Xi and ro
+// arrays; 4, the energy step: Xi as its first pass stored it, ro from P and T.  The
+// return value tells a cell whose P_n or P_g is not its P_w (three phases with one staged pressure,
 // boundary cells).
 template <int MODEL, int CLOSURE>
 __device__ __forceinline__ bool coef_of(const DevParams& p, const CellRaw<MODEL, CLOSURE>& r, bool inner,
@@ -482,51 +400,6 @@ __device__ __forceinline__ bool coef_of(const DevParams& p, const CellRaw<MODEL,
     return false;
 }
 
-// The state, the divergence (and, for U, the velocities u[phase][axis]) of an
-// interior cell from memory, every neighbour with its own phase pressures;
-// one axis at a time, for few registers.
-template <int MODEL, int CLOSURE, bool U>
-__device__ __forceinline__ void general_cell(const DevParams& p, const StepIO& io, int i, int j, int k, double* ro,
-                                             double* div, double (&u)[MODEL][3]) {
-    auto at = [&](int ii, int jj, int kk) {
-        return coef_at<MODEL, CLOSURE>(p, io, (int64_t)ii + (int64_t)jj * p.sy + (int64_t)kk * p.sz,
-                                       inner_cell<MODEL>(p, ii, jj, kk));
-    };
-    const CoefT<MODEL> c = at(i, j, k);
-#pragma unroll
-    for (int a = 0; a < MODEL; ++a) ro[a] = c.ro[a];
-    auto axis = [&](bool has, int dx, int dy, int dz, int x, double h, double rh, double h2, double rh2) {
-        if (!has) {
-#pragma unroll
-            for (int a = 0; a < MODEL; ++a) {
-                if (x != 0) div[a] = div[a] + 0.;
-                else div[a] = 0.;
-                u[a][x] = 0.;
-            }
-            return;
-        }
-        const CoefT<MODEL> m = at(i - dx, j - dy, k - dz), q = at(i + dx, j + dy, k + dz);
-#pragma unroll
-        for (int a = 0; a < MODEL; ++a) {
-            double x1 = -1. * exact_div(c.P[a] - m.P[a], h, rh), x2 = -1. * exact_div(q.P[a] - c.P[a], h, rh);
-            if (x == 1) {
-                x1 = x1 + p.g * c.ro[a];
-                x2 = x2 + p.g * c.ro[a];
-            }
-            const double f = directed(x1, x2, c.Xi[a], c.ro[a], m.Xi[a], m.ro[a], q.Xi[a], q.ro[a], h, rh);
-            div[a] = x == 0 ? (a == 2 ? 0. + f : f) : div[a] + f;
-            if (U) {
-                const double d = exact_div(q.P[a] - m.P[a], h2, rh2);
-                u[a][x] = c.Xi[a] * (x == 1 ? d - c.ro[a] * p.g : d);
-            }
-        }
-    };
-    // x, y, z in turn: the order of the sum (cpu.cpp:707-708)
-    axis(p.Nx >= 3, 1, 0, 0, 0, p.hx, p.r_hx, p.two_hx, p.r_two_hx);
-    axis(true, 0, 1, 0, 1, p.hy, p.r_hy, p.two_hy, p.r_two_hy);
-    axis(p.Nz >= 3, 0, 0, 1, 2, p.hz, p.r_hz, p.two_hz, p.r_two_hz);
-}
-
 using LdsDouble = __attribute__((address_space(3))) double*;
 
 // What an epilogue reads of the cell it finishes.
@@ -560,15 +433,16 @@ struct CellState {
 // Epi: what happens at an interior cell once its state and flux divergence
 // are known -- the Newton solve and store of the step (FusedStore) or the
 // adjoint's backward Newton (AdjNewtonStore).  prefetch() loads what it needs;
-// epi.cell<false> may leave the cell undone and say so (false), epi.cell<true>
-// does every cell.
+// with kLeaves, cell() may leave the cell undone and say so (false), its right
+// side in the cell's place of the next state, which nothing else in the launch
+// reads: late() does it after the last plane, so that the planes' code holds no
+// call and no registers for it (kchunk <= kMaxPlanes, one mark per plane).
 //
-// Cells that the planes' code does not cover -- the epilogue left it undone (a
-// pivot search), or, where one pressure is staged, an x or z face neighbour has a
-// P_n or P_g that is not its P_w (values a caller set; Border_P gives those faces
-// P_n = P_g = P_w, P_Xi_ro every interior cell) -- are marked and done after the last plane from the state the step reads, which
-// it does not write: the planes' code then holds no call and no registers for
-// them (kchunk <= kMaxPlanes, one mark per plane).
+// P_n or P_g apart from P_w in an x or z face cell (values a caller set, or an
+// exchange of faces: Border_P gives those faces P_n = P_g = P_w, P_Xi_ro every
+// interior cell): the x face's stand in LDS as the top and bottom rows' do, the z
+// face's are read again; the wavefronts next to such a cell take each phase's own
+// differences in that plane.
 // cp: p in constant memory (fresh()).
 constexpr int kMaxPlanes = 32;
 template <int MODEL, int CLOSURE, int TX, int TY, bool FULL, class Epi>
@@ -614,7 +488,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
     // LDS places in the buffer of plane 0: the own and the halo cell
     auto buffer = [](int k) { return (k & 1) * PLANE; };
     const LdsDouble v0 = (LdsDouble)&lds.v[0][ty + 1][tx + 1][0], vh = (LdsDouble)&lds.v[0][hy][hx][0];
-    auto stage = [&](int k, LdsDouble w, int row, int x, int jj, const CellRaw<MODEL, CLOSURE>& r, bool inner,
+    auto stage = [&](int k, LdsDouble w, int row, int x, int ii, int jj, const CellRaw<MODEL, CLOSURE>& r, bool inner,
                      const CellCoef<MODEL, CLOSURE>& c, bool odd) {
 #pragma unroll
         for (int a = 0; a < NPR; ++a) w[a] = c.P[a];
@@ -628,8 +502,10 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
                 if (jj == 0 || jj == p.Ny - 1) {
                     lds.edge[k & 1][jj == 0 ? 0 : 1][0][x] = r.Pn;
                     lds.edge[k & 1][jj == 0 ? 0 : 1][1][x] = r.Pg;
-                } else if (odd) {
-                    lds.odd[k & 1][row] = k;
+                } else if (hasx && (ii == 0 || ii == p.Nx - 1)) {
+                    lds.side[k & 1][ii == 0 ? 0 : 1][0][row] = r.Pn;
+                    lds.side[k & 1][ii == 0 ? 0 : 1][1][row] = r.Pg;
+                    if (odd) lds.odd[k & 1][row] = k;
                 }
             }
         }
@@ -656,11 +532,12 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
         CellCoef<MODEL, CLOSURE> c, m;
         const DevParams pc = coef_params<MODEL, CLOSURE>(cp);
         const bool odd = coef_of(pc, r, inner, c);
-        stage(k0, v0 + buffer(k0), ty + 1, tx + 1, jc, r, inner, c, odd);
+        stage(k0, v0 + buffer(k0), ty + 1, tx + 1, ic, jc, r, inner, c, odd);
         Sn = r.Sn;
         if constexpr (MODEL == 3) Sw = r.Sw;
         if (hasz) {
-            zodd = __ballot(coef_of(pc, rm, inner_m, m));
+            const bool apart = coef_of(pc, rm, inner_m, m);
+            if constexpr (APART) zodd = __ballot(apart);
 #pragma unroll
             for (int a = 0; a < NPR; ++a) {
                 zmP[a] = m.P[a];
@@ -669,10 +546,16 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
 #pragma unroll
                 for (int b = a; b < (NPR == 1 ? NPH : a + 1); ++b) zt2[b] = directed_t2(-1. * d, m.Xi[b], m.ro[b]);
             }
+            if constexpr (APART) {
+                if (apart) {
+                    zt2[1] = directed_t2(-1. * exact_div(c.P[0] - rm.Pn, p.hz, p.r_hz), m.Xi[1], m.ro[1]);
+                    zt2[2] = directed_t2(-1. * exact_div(c.P[0] - rm.Pg, p.hz, p.r_hz), m.Xi[2], m.ro[2]);
+                }
+            }
         }
         if (halo) {
             const bool oddh = coef_of(pc, rh, inner_h, c);
-            stage(k0, vh + buffer(k0), hy, hx, hj, rh, inner_h, c, oddh);
+            stage(k0, vh + buffer(k0), hy, hx, hi, hj, rh, inner_h, c, oddh);
         }
     }
     __syncthreads();
@@ -693,12 +576,12 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
             if (hasz) {
                 const bool mine = coef_of(pc, r, inner, zp);
                 if constexpr (APART) odd = __ballot(mine);
-                if (next || EARLY) stage(k + 1, v0 + buffer(k + 1), ty + 1, tx + 1, jc, r, inner, zp, mine);
+                if (next || EARLY) stage(k + 1, v0 + buffer(k + 1), ty + 1, tx + 1, ic, jc, r, inner, zp, mine);
             }
             if (next && halo) {
                 CellCoef<MODEL, CLOSURE> h;
                 const bool oddh = coef_of(pc, rh, inner_h, h);
-                stage(k + 1, vh + buffer(k + 1), hy, hx, hj, rh, inner_h, h, oddh);
+                stage(k + 1, vh + buffer(k + 1), hy, hx, hi, hj, rh, inner_h, h, oddh);
             }
         };
         if constexpr (EARLY) next_plane();
@@ -728,15 +611,14 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
                 div[a] = 0.;
             }
             if (hasx) {
-#pragma unroll
-                for (int q = 0; q < NPR; ++q) {
-                    const double Pm = P_at(q, 1, 0), Pp = P_at(q, 1, 2);
-                    const double x1 = -1. * exact_div(c.P[q] - Pm, pf.hx, pf.r_hx);
-                    const double x2 = -1. * exact_div(Pp - c.P[q], pf.hx, pf.r_hx);
+                // the phases from a0 to a1, whose pressure is one
+                auto x_flux = [&](double P, double Pm, double Pp, int a0, int a1) {
+                    const double x1 = -1. * exact_div(P - Pm, pf.hx, pf.r_hx);
+                    const double x2 = -1. * exact_div(Pp - P, pf.hx, pf.r_hx);
                     const double s1 = (pos_part(x2) - neg_part(x1)) * (-1.), s2 = pos_part(x1) * (-1.),
                                  s3 = neg_part(x2) * (-1.);
 #pragma unroll
-                    for (int a = q; a < (NPR == 1 ? NPH : q + 1); ++a) {
+                    for (int a = a0; a < a1; ++a) {
                         const double t1 = s1 * c.Xi[a] * c.ro[a];
                         const double t2 = s2 * Xi_at(a, 1, 0) * ro_at(a, 1, 0);
                         const double t3 = s3 * Xi_at(a, 1, 2) * ro_at(a, 1, 2);
@@ -744,6 +626,23 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
                         div[a] = a == 2 ? 0. + fx : fx;
                         if constexpr (U) u[a][0] = c.Xi[a] * exact_div(Pp - Pm, pf.two_hx, pf.r_two_hx);
                     }
+                };
+                bool apart = false;
+                if constexpr (APART) apart = __ballot(lds.odd[k & 1][ty + 1] == k) != 0;
+                if (__builtin_expect(apart, 0)) {
+#pragma unroll
+                    for (int a = 0; a < NPH; ++a) {
+                        double Pm = P_at(0, 1, 0), Pp = P_at(0, 1, 2);
+                        if constexpr (APART) {
+                            if (a > 0 && i == 1) Pm = lds.side[k & 1][0][a - 1][ty + 1];
+                            if (a > 0 && i == p.Nx - 2) Pp = lds.side[k & 1][1][a - 1][ty + 1];
+                        }
+                        x_flux(c.P[0], Pm, Pp, a, a + 1);
+                    }
+                } else {
+#pragma unroll
+                    for (int q = 0; q < NPR; ++q)
+                        x_flux(c.P[q], P_at(q, 1, 0), P_at(q, 1, 2), q, NPR == 1 ? NPH : q + 1);
                 }
             } else if constexpr (U) {
 #pragma unroll
@@ -793,21 +692,44 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
         }
         if (active) {
             if (hasz) {
-#pragma unroll
-                for (int q = 0; q < NPR; ++q) {
-                    const double x2 = -1. * exact_div(zp.P[q] - c.P[q], pf.hz, pf.r_hz);
+                // the phases from a0 to a1, of one pressure; the plus face's neg_part
+                auto z_flux = [&](double zn, double Pm, double P, double Pp, int a0, int a1) {
+                    const double x2 = -1. * exact_div(Pp - P, pf.hz, pf.r_hz);
                     const double n2 = neg_part(x2), p2 = pos_part(x2);
-                    const double s1 = (p2 - zneg[q]) * (-1.), s3 = n2 * (-1.), s2 = p2 * (-1.);
+                    const double s1 = (p2 - zn) * (-1.), s3 = n2 * (-1.), s2 = p2 * (-1.);
 #pragma unroll
-                    for (int a = q; a < (NPR == 1 ? NPH : q + 1); ++a) {
+                    for (int a = a0; a < a1; ++a) {
                         const double t1 = s1 * c.Xi[a] * c.ro[a];
                         const double t3 = s3 * zp.Xi[a] * zp.ro[a];
                         div[a] = div[a] + exact_div(t1 - zt2[a] + t3, pf.hz, pf.r_hz);
                         zt2[a] = s2 * c.Xi[a] * c.ro[a];  // the next plane's minus face
-                        if constexpr (U) u[a][2] = c.Xi[a] * exact_div(zp.P[q] - zmP[q], pf.two_hz, pf.r_two_hz);
+                        if constexpr (U) u[a][2] = c.Xi[a] * exact_div(Pp - Pm, pf.two_hz, pf.r_two_hz);
                     }
-                    zneg[q] = n2;
-                    if constexpr (U) zmP[q] = c.P[q];
+                    return n2;
+                };
+                if (APART && __builtin_expect((zodd | odd) != 0, 0)) {
+                    const uint64_t lane = 1ull << ((ty * TX + tx) & 63);
+                    const double zn = zneg[0];
+                    zneg[0] = z_flux(zn, zmP[0], c.P[0], zp.P[0], 0, 1);
+#pragma unroll
+                    for (int a = 1; a < NPH; ++a) {
+                        const double* P = a == 1 ? io.Pn : io.Pg;
+                        double zna = zn, Pm = zmP[0], Pp = zp.P[0];
+                        if (zodd & lane) {
+                            Pm = ld(P, CellAt{own.base - p.sz, own.off});
+                            zna = neg_part(-1. * exact_div(c.P[0] - Pm, pf.hz, pf.r_hz));
+                        }
+                        if (odd & lane) Pp = ld(P, CellAt{own.base + p.sz, own.off});
+                        z_flux(zna, Pm, c.P[0], Pp, a, a + 1);
+                    }
+                } else {
+#pragma unroll
+                    for (int q = 0; q < NPR; ++q)
+                        zneg[q] = z_flux(zneg[q], zmP[q], c.P[q], zp.P[q], q, NPR == 1 ? NPH : q + 1);
+                }
+                if constexpr (U) {
+#pragma unroll
+                    for (int q = 0; q < NPR; ++q) zmP[q] = c.P[q];
                 }
             } else {
 #pragma unroll
@@ -822,18 +744,9 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
             s.Sn = Sn;
 #pragma unroll
             for (int a = 0; a < NPH; ++a) s.ro[a] = c.ro[a];
-            bool done = true;
-            if constexpr (APART) {
-                const uint64_t lane = 1ull << ((ty * TX + tx) & 63);
-                const bool row_odd = lds.odd[k & 1][ty + 1] == k;
-                if (__builtin_expect((zodd | odd) != 0 || __ballot(row_odd) != 0, 0))
-                    done = !row_odd && ((zodd | odd) & lane) == 0;
-            }
-            if (done) {
-                if constexpr (U) epi.store_u(own, u);
-                done = epi.template cell<false>(p, newton_params<MODEL, CLOSURE>(fresh(cp)), i, j, k, own, s, div, pre);
-            }
-            if (__builtin_expect(__ballot(!done) != 0, 0)) {
+            if constexpr (U) epi.store_u(own, u);
+            const bool done = epi.cell(p, newton_params<MODEL, CLOSURE>(fresh(cp)), i, j, k, own, s, div, pre);
+            if constexpr (Epi::kLeaves) {
                 if (!done) undone |= 1u << (k - k0);
             }
         }
@@ -846,18 +759,11 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
         }
     }
 
-    while (__builtin_expect(undone != 0, 0)) {
-        const int k = k0 + __ffs(undone) - 1;
-        undone &= undone - 1;
-        const CellIndex at{(int64_t)i + (int64_t)j * p.sy + (int64_t)k * p.sz};
-        CellState<MODEL> s;
-        s.P = ld(io.Pw, at);
-        s.Sn = ld(io.Sn, at);
-        s.Sw = MODEL == 3 ? ld(io.Sw, at) : 0.;
-        double div[NPH], u[NPH][3];
-        general_cell<MODEL, CLOSURE, U>(p, io, i, j, k, s.ro, div, u);
-        if constexpr (U) epi.store_u(at, u);
-        epi.template cell<true>(p, p, i, j, k, at, s, div, epi.prefetch(at));
+    if constexpr (Epi::kLeaves) {
+        while (__builtin_expect(undone != 0, 0)) {
+            epi.late(p, i, j, k0 + __ffs(undone) - 1);
+            undone &= undone - 1;
+        }
     }
 }
 
@@ -922,39 +828,59 @@ struct FusedStore {
     // dt / m, computed once per porosity field
     template <class At>
     __device__ __forceinline__ double prefetch(const At& at) const { return ld(io.dtm, at); }
-    template <bool GENERAL, class At>
+    static constexpr bool kLeaves = true;
+    // false: the right side stored for late()
+    template <class At>
     __device__ __forceinline__ bool cell(const DevParams& p, const DevParams& pn, int i, int j, int k, const At& at,
                                          const CellState<MODEL>& s, const double* div, double dtm) const {
         (void)i; (void)j; (void)k;
         double Pw = s.P, Sn = s.Sn, Sw = s.Sw;
+        bool done;
         if constexpr (MODEL == 2) {
             const double A1 = s.ro[0] * (1. - Sn) - dtm * div[0];
             const double A2 = s.ro[1] * Sn - dtm * div[1];
-            if constexpr (GENERAL)
-                newton2_ieee<CLOSURE>(pn, Pw, Sn, A1, A2);
-            else if (!newton2_fast<CLOSURE>(pn, Pw, Sn, A1, A2))
-                return false;
-            At to = at;
-            renew(to);
-            st(io.Pw1, to, Pw);
-            st(io.Sn1, to, Sn);
-            if constexpr (FACES) store_faces<2>(p, io, i, j, k, at.l(), s.ro, Pw, 0., Sn);
+            done = newton2_fast<CLOSURE>(pn, Pw, Sn, A1, A2);
+            if (__builtin_expect(!done, 0)) {
+                Pw = A1;
+                Sn = A2;
+            }
         } else {
             const double A1 = s.ro[0] * Sw - dtm * div[0];
             const double A2 = s.ro[1] * Sn - dtm * div[1];
             const double A3 = s.ro[2] * (1. - Sw - Sn) - dtm * div[2];
-            if constexpr (GENERAL)
-                newton3_general(pn, Pw, Sw, Sn, A1, A2, A3);
-            else if (!newton3_fast(pn, Pw, Sw, Sn, A1, A2, A3))
-                return false;
-            At to = at;
-            renew(to);
-            st(io.Pw1, to, Pw);
-            st(io.Sw1, to, Sw);
-            st(io.Sn1, to, Sn);
-            if constexpr (FACES) store_faces<3>(p, io, i, j, k, at.l(), s.ro, Pw, Sw, Sn);
+            done = newton3_fast(pn, Pw, Sw, Sn, A1, A2, A3);
+            if (__builtin_expect(!done, 0)) {
+                Pw = A1;
+                Sw = A3;
+                Sn = A2;
+            }
         }
-        return true;
+        At to = at;
+        renew(to);
+        st(io.Pw1, to, Pw);
+        if constexpr (MODEL == 3) st(io.Sw1, to, Sw);
+        st(io.Sn1, to, Sn);
+        if constexpr (FACES)
+            if (done) store_faces<MODEL>(p, io, i, j, k, at.l(), s.ro, Pw, Sw, Sn);
+        return done;
+    }
+    // The cell from its state and the right side that cell() left.
+    __device__ __forceinline__ void late(const DevParams& p, int i, int j, int k) const {
+        const int64_t l = (int64_t)i + (int64_t)j * p.sy + (int64_t)k * p.sz;
+        const double A1 = io.Pw1[l], A2 = io.Sn1[l];
+        double Pw = io.Pw[l], Sn = io.Sn[l], Sw = 0., ro[MODEL] = {};
+        if constexpr (MODEL == 2) {
+            if constexpr (FACES) densities2<CLOSURE>(p, io, l, ro);
+            newton2_ieee<CLOSURE>(p, Pw, Sn, A1, A2);
+        } else {
+            const double A3 = io.Sw1[l];
+            Sw = io.Sw[l];
+            newton3_general(p, Pw, Sw, Sn, A1, A2, A3);
+            io.Sw1[l] = Sw;
+        }
+        io.Pw1[l] = Pw;
+        io.Sn1[l] = Sn;
+        if constexpr (FACES) store_faces<MODEL>(p, io, i, j, k, l, ro, Pw, Sw, Sn);
     }
 };
 
@@ -972,15 +898,17 @@ struct FusedStoreRecord {
     int64_t stride;
     template <class At>
     __device__ __forceinline__ double prefetch(const At& at) const { return step.prefetch(at); }
-    template <bool GENERAL, class At>
+    static constexpr bool kLeaves = true;
+    template <class At>
     __device__ __forceinline__ bool cell(const DevParams& p, const DevParams& pn, int i, int j, int k, const At& at,
                                          const CellState<MODEL>& s, const double* d, double dtm) const {
         At to = at;
         renew(to);
 #pragma unroll
         for (int a = 0; a < MODEL; ++a) st(div + a * stride, to, d[a]);
-        return step.template cell<GENERAL>(p, pn, i, j, k, at, s, d, dtm);
+        return step.cell(p, pn, i, j, k, at, s, d, dtm);
     }
+    __device__ __forceinline__ void late(const DevParams& p, int i, int j, int k) const { step.late(p, i, j, k); }
 };
 
 // assign_roS_nr (cpu.cpp:619-731) on the z tiles (three phases): roS_old and
@@ -990,7 +918,7 @@ struct FusedStoreRecord {
 // that are NULL are not stored.
 template <bool U>
 struct RoSStore {
-    static constexpr bool kWantsU = U;
+    static constexpr bool kWantsU = U, kLeaves = false;
     const double* dtm;
     double *roS[3], *roS_old[3];
     double* u[3][3];  // [phase][axis]: ux_w, uy_w, uz_w, ux_n, ... (U only)
@@ -1006,7 +934,7 @@ struct RoSStore {
             for (int x = 0; x < 3; ++x)
                 if (x < 2 || u[a][2]) st(u[a][x], to, v[a][x]);
     }
-    template <bool GENERAL, class At>
+    template <class At>
     __device__ __forceinline__ bool cell(const DevParams& p, const DevParams& pn, int i, int j, int k, const At& at,
                                          const CellState<3>& s, const double* div, double d) const {
         (void)p; (void)pn; (void)i; (void)j; (void)k;
@@ -1350,8 +1278,9 @@ __device__ __forceinline__ void fused_face(const DevParams& p, const StepIO& io,
         // step's densities of the inward cell (from its previous state) with
         // its new saturation
         if (j == p.Ny - 1) {
-            const CoefT<2> c1 = coef_at<2, CLOSURE>(p, io, l1, true);
-            ro_eff = (c1.ro[1] * Sn + c1.ro[0] * (1 - Sn)) * io.m[l1] * p.g * p.hy;
+            double ro[2];
+            densities2<CLOSURE>(p, io, l1, ro);
+            ro_eff = (ro[1] * Sn + ro[0] * (1 - Sn)) * io.m[l1] * p.g * p.hy;
         }
     }
     write_boundary<MODEL>(p, io, i, j, k, Pw, Sw, Sn, ro_eff);
@@ -1401,8 +1330,9 @@ __device__ __forceinline__ void fused_pack(const DevParams& p, const StepIO& io,
         double ro_eff = 0.;
         if constexpr (MODEL == 2) {
             if (j == p.Ny - 1) {
-                const CoefT<2> c1 = coef_at<2, CLOSURE>(p, io, l1, true);
-                ro_eff = (c1.ro[1] * Sn + c1.ro[0] * (1 - Sn)) * io.m[l1] * p.g * p.hy;
+                double ro[2];
+                densities2<CLOSURE>(p, io, l1, ro);
+                ro_eff = (ro[1] * Sn + ro[0] * (1 - Sn)) * io.m[l1] * p.g * p.hy;
             }
         }
         boundary_values<MODEL>(p, i, j, k, Pw, Sw, Sn, ro_eff, v);

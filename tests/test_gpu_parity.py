@@ -11,13 +11,14 @@ the state fields P_w, S_w, S_n, which never approach zero:
   * the fused step and the entry-point sequence run the same device
     arithmetic and must agree bit for bit, every field.
 """
+import ctypes
 import glob
 import os
 
 import numpy as np
 import pytest
 
-from capaz_amd import capaz, workloads
+from capaz_amd import capaz, hip, workloads
 from capaz_cases import bit_equal, case, max_rel, norm_rel, random_state
 from golden.make_golden import ENTRIES, load
 from oracle import oracle
@@ -225,6 +226,49 @@ def test_tile_cells_done_after_the_planes(dims, tune, closure):
         for f in b:
             assert bit_equal(a[f], b[f]), f
         assert np.isfinite(b["P_w"]).all()
+
+
+@pytest.mark.parametrize("dims", [(34, 18, 12), (66, 11, 9), (35, 20, 3), (3, 9, 40), (70, 9, 1)])
+@pytest.mark.parametrize("axis", [0, 2])
+@pytest.mark.parametrize("model,over", [("3ph", dict(CLOSURE="corey")), ("3ph", dict()),
+                                        ("3ph", dict(CLOSURE="corey", COREY_N=2.5)), ("3phe", dict())])
+def test_steps_between_face_exchanges(model, over, axis, dims):
+    """Steps with an exchange of faces (capaz_load_faces, capaz_save_faces with the
+    sides swapped) after each: the ghost cells' P_n and P_g are the neighbour's
+    previous P_w, so every cell next to them has fluxes with each phase's own
+    difference.  Every field as from one thread per cell (with the energy equation,
+    as from the entry points)."""
+    if dims[axis] < 3:
+        pytest.skip("no planes to exchange")
+    keys = case(model, *dims, DT=1e-5, SOURCE=1, **over)
+    st = random_state(keys, seed=sum(dims))
+    names = ("P_w", "S_w", "S_n", "P_n", "P_g") + (("T",) if model == "3phe" else ())
+    ids = (ctypes.c_int * len(names))(*[capaz.FIELD_ID[f] for f in names])
+    plane = int(np.prod(dims)) // dims[axis]
+    L = capaz.load()
+    got = []
+    for tune in (dict(), dict(kchunk=2), dict(tile_y=4), dict(energy_kernel=0) if model == "3phe" else dict(fused_kernel=0)):
+        d = capaz.Domain(keys, st)
+        d.tune(**tune)
+        buf = hip.DeviceBuffer(8 * plane * 2 * len(names))
+        b = ctypes.c_void_p(buf.address)
+        for step in range(1, 4):
+            d.run(1, first_step=step)
+            assert L.capaz_load_faces(d._ctx, ids, len(names), axis, b) == 0
+            d.sync()
+            v = buf.download(plane * 2 * len(names)).reshape(len(names), 2, plane)
+            buf.upload(np.ascontiguousarray(v[:, ::-1]))
+            assert L.capaz_save_faces(d._ctx, ids, len(names), axis, b) == 0
+            d.sync()
+        d.run(1, first_step=4)
+        got.append(d.fields())
+        d.close()
+        buf.close()
+    own = np.abs(v[names.index("P_n")] - v[0]).max()
+    assert own > 0 and np.isfinite(got[-1]["P_w"]).all()
+    for g in got[:-1]:
+        for f in g:
+            assert bit_equal(g[f], got[-1][f]), f
 
 
 # interior columns that 32 x 16 and 32 x 8 workgroups cover with fewer threads than
