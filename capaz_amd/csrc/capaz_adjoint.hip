@@ -123,6 +123,7 @@ template <int IT>
 struct AdjNewtonStore {
     AdjIO a;
     static constexpr bool kLeaves = false;
+    __device__ __forceinline__ int none() const { return 0; }
     template <class At>
     __device__ __forceinline__ int prefetch(const At&) const { return 0; }
     template <class At>
@@ -137,8 +138,8 @@ constexpr int kTX = 64, kTY = 8;
 
 template <int CLOSURE, int IT>
 __global__ void __launch_bounds__(kTX * kTY) k_adj_newton_z(DevParams p, StepIO io, AdjIO a, int kchunk) {
-    __shared__ FusedLds<3, CLOSURE, kTX, kTY> lds;
-    fused_z_tile<3, CLOSURE, kTX, kTY, false>(p, kernel_params(), io, kchunk, (int)blockIdx.x, (int)blockIdx.y,
+    __shared__ FusedLds<3, CLOSURE, kTX, kTY, kAxesAny> lds;
+    fused_z_tile<3, CLOSURE, kTX, kTY, kAxesAny>(p, kernel_params(), io, kchunk, (int)blockIdx.x, (int)blockIdx.y,
                                               (int)blockIdx.z, lds, AdjNewtonStore<IT>{a});
 }
 

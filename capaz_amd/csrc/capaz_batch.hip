@@ -30,11 +30,11 @@ constexpr int kBatchWaves =
 
 using ConstDomain = const __attribute__((address_space(4))) BatchDomain;
 
-template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
+template <int MODEL, int CLOSURE, int TX, int TY, int AXES>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(kBatchWaves<MODEL, CLOSURE, TX, TY>)))
     k_batch_z(const BatchDomain* __restrict__ doms, const int* __restrict__ owner, int ntiles, int parity,
               int kchunk, int* counter) {
-    __shared__ FusedLds<MODEL, CLOSURE, TX, TY> lds;
+    __shared__ FusedLds<MODEL, CLOSURE, TX, TY, AXES> lds;
     __shared__ int claimed;
     // one workgroup per tile: each XCD (workgroups go to the 8 XCDs round
     // robin) takes a contiguous run of the tile list, so a realization's
@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(kB
         const StepIO io = *(const StepIO*)&d->io[parity];
         const int lt = t - d->tile_begin;
         const int bx = lt % d->tiles_x, r = lt / d->tiles_x;
-        fused_z_tile<MODEL, CLOSURE, TX, TY, FULL>(p, &d->p, io, kchunk, bx, r % d->tiles_y, r / d->tiles_y, lds,
+        fused_z_tile<MODEL, CLOSURE, TX, TY, AXES>(p, &d->p, io, kchunk, bx, r % d->tiles_y, r / d->tiles_y, lds,
                                                     FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE>{io});
         if (!counter) return;
     }
@@ -76,14 +76,14 @@ __global__ void k_zero_ints(int* p, int n) {
     if (i < n) p[i] = 0;
 }
 
-template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
-hipError_t step_full(const BatchShape& sh, const BatchDomain* doms, const int* tile_owner, int ntiles,
+template <int MODEL, int CLOSURE, int TX, int TY, int AXES>
+hipError_t step_axes(const BatchShape& sh, const BatchDomain* doms, const int* tile_owner, int ntiles,
                       const int* face_owner, int nface_blocks, int parity, int* counter, int grid, hipStream_t s) {
     if (ntiles > 0) {
         // (the one-per-tile grid is rounded up to a multiple of the 8 XCDs;
         // the extra workgroups find no tile and exit)
         const int g = sh.persistent ? grid : (ntiles + 7) / 8 * 8;
-        hipLaunchKernelGGL((k_batch_z<MODEL, CLOSURE, TX, TY, FULL>), dim3(g), dim3(TX, TY), 0, s, doms, tile_owner, ntiles,
+        hipLaunchKernelGGL((k_batch_z<MODEL, CLOSURE, TX, TY, AXES>), dim3(g), dim3(TX, TY), 0, s, doms, tile_owner, ntiles,
                            parity, tile_planes(sh), sh.persistent ? counter : nullptr);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -98,9 +98,9 @@ hipError_t step_full(const BatchShape& sh, const BatchDomain* doms, const int* t
 template <int MODEL, int CLOSURE, int TX, int TY>
 hipError_t step_shape(const BatchShape& sh, const BatchDomain* doms, const int* tile_owner, int ntiles,
                       const int* face_owner, int nface_blocks, int parity, int* counter, int grid, hipStream_t s) {
-    return sh.full ? step_full<MODEL, CLOSURE, TX, TY, true>(sh, doms, tile_owner, ntiles, face_owner, nface_blocks,
+    return sh.full ? step_axes<MODEL, CLOSURE, TX, TY, kAxesAll>(sh, doms, tile_owner, ntiles, face_owner, nface_blocks,
                                                              parity, counter, grid, s)
-                   : step_full<MODEL, CLOSURE, TX, TY, false>(sh, doms, tile_owner, ntiles, face_owner, nface_blocks,
+                   : step_axes<MODEL, CLOSURE, TX, TY, kAxesAny>(sh, doms, tile_owner, ntiles, face_owner, nface_blocks,
                                                               parity, counter, grid, s);
 }
 
@@ -117,17 +117,17 @@ hipError_t step_closure(const BatchShape& sh, const BatchDomain* doms, const int
                                              grid, s);
 }
 
-template <int MODEL, int CLOSURE, bool FULL>
-hipError_t occupancy_full(const BatchShape& sh, int* n) {
+template <int MODEL, int CLOSURE, int AXES>
+hipError_t occupancy_axes(const BatchShape& sh, int* n) {
     if (sh.tx == 64 && sh.ty == 8)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, k_batch_z<MODEL, CLOSURE, 64, 8, FULL>, 512, 0);
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, k_batch_z<MODEL, CLOSURE, 64, 8, AXES>, 512, 0);
     if (sh.tx == 64 && sh.ty == 4)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, k_batch_z<MODEL, CLOSURE, 64, 4, FULL>, 256, 0);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, k_batch_z<MODEL, CLOSURE, 32, 8, FULL>, 256, 0);
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, k_batch_z<MODEL, CLOSURE, 64, 4, AXES>, 256, 0);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, k_batch_z<MODEL, CLOSURE, 32, 8, AXES>, 256, 0);
 }
 template <int MODEL, int CLOSURE>
 hipError_t occupancy_closure(const BatchShape& sh, int* n) {
-    return sh.full ? occupancy_full<MODEL, CLOSURE, true>(sh, n) : occupancy_full<MODEL, CLOSURE, false>(sh, n);
+    return sh.full ? occupancy_axes<MODEL, CLOSURE, kAxesAll>(sh, n) : occupancy_axes<MODEL, CLOSURE, kAxesAny>(sh, n);
 }
 
 }  // namespace

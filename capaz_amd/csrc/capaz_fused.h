@@ -145,13 +145,21 @@ constexpr int kStagedP = MODEL == 2 ? (CLOSURE == 0 ? 2 : 1) : (CLOSURE == 3 ? 3
 // side[.][0 / 1] of the x face cells (i = 0 / Nx - 1), odd[.][row] = the plane k in
 // which such a cell of that row has a P_n or P_g that is not its P_w (else any
 // value, k too: side holds them whether they differ or not).
-template <int MODEL, int CLOSURE, int TX, int TY>
+// The axes of the grids a kernel is compiled for: any; Nx, Ny, Nz >= 3 (no axis
+// tests in the plane's code); one plane (Nz = 1: nothing carried along z, one
+// plane's LDS, 52 to 88 VGPRs and no spills instead of 94 to 150, and what the
+// epilogue reads is loaded before the barrier, whose latency is all such a grid
+// waits for: us per step, one plane / any axes, 512 x 512 x 1 three phases Corey-2
+// 13.0 / 18.2, van Genuchten 21.1 / 27.0, two phases Corey-2 6.8 / 9.3).
+enum Axes { kAxesAny, kAxesAll, kAxesOnePlane };
+template <int MODEL, int CLOSURE, int TX, int TY, int AXES>
 struct FusedLds {
     static constexpr int kNP = kStagedP<MODEL, CLOSURE>, kNV = (kNP + 2 * MODEL) | 1;
     static constexpr bool kApart = MODEL == 3 && kNP == 1;
-    double v[2][TY + 2][TX + 2][kNV];
-    double edge[2][kApart ? 2 : 0][2][TX + 2], side[2][kApart ? 2 : 0][2][TY + 2];
-    int odd[2][kApart ? TY + 2 : 0];
+    static constexpr int kPlanes = AXES == kAxesOnePlane ? 1 : 2;
+    double v[kPlanes][TY + 2][TX + 2][kNV];
+    double edge[kPlanes][kApart ? 2 : 0][2][TX + 2], side[kPlanes][kApart ? 2 : 0][2][TY + 2];
+    int odd[kPlanes][kApart ? TY + 2 : 0];
 };
 
 // A cell of a field array: a wave-uniform index (scalar registers) and the
@@ -429,7 +437,6 @@ struct CellState {
 // thread keeps two pressure parts, the minus z face's flux terms and its
 // saturations; its own coefficients come back from LDS.
 //
-// FULL: Nx, Ny, Nz >= 3 (no axis tests in the plane's code).
 // Epi: what happens at an interior cell once its state and flux divergence
 // are known -- the Newton solve and store of the step (FusedStore) or the
 // adjoint's backward Newton (AdjNewtonStore).  prefetch() loads what it needs;
@@ -445,25 +452,26 @@ struct CellState {
 // differences in that plane.
 // cp: p in constant memory (fresh()).
 constexpr int kMaxPlanes = 32;
-template <int MODEL, int CLOSURE, int TX, int TY, bool FULL, class Epi>
+template <int MODEL, int CLOSURE, int TX, int TY, int AXES, class Epi>
 __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp, const StepIO& io, int kchunk, int bx, int by, int bz,
-                                             FusedLds<MODEL, CLOSURE, TX, TY>& lds, const Epi& epi) {
+                                             FusedLds<MODEL, CLOSURE, TX, TY, AXES>& lds, const Epi& epi) {
     static_assert(TY >= 3 && TX >= 2 * TY, "halo ring needs TY >= 3 and TX >= 2*TY");
     static_assert(TX == 32 || TX == 64, "whole rows per wavefront");
-    constexpr int NPH = MODEL, NPR = kStagedP<MODEL, CLOSURE>, NV = FusedLds<MODEL, CLOSURE, TX, TY>::kNV;
+    constexpr int NPH = MODEL, NPR = kStagedP<MODEL, CLOSURE>, NV = FusedLds<MODEL, CLOSURE, TX, TY, AXES>::kNV;
     constexpr int ROW = (TX + 2) * NV, PLANE = (TY + 2) * ROW;  // LDS pitch of a row, of a plane
     constexpr bool U = EpiWantsU<Epi>::value;
     constexpr bool EARLY = CLOSURE == 0 || CLOSURE == 1;
     // three phases: P_n and P_g apart from the staged pressure, where they differ
-    constexpr bool APART = FusedLds<MODEL, CLOSURE, TX, TY>::kApart;
+    constexpr bool APART = FusedLds<MODEL, CLOSURE, TX, TY, AXES>::kApart;
 
     const int tx = threadIdx.x, ty = threadIdx.y;
-    const bool hasx = FULL || p.Nx >= 3, hasz = FULL || p.Nz >= 3;
+    constexpr bool FLAT = AXES == kAxesOnePlane;
+    const bool hasx = AXES == kAxesAll || p.Nx >= 3, hasz = AXES == kAxesAll || (!FLAT && p.Nz >= 3);
     const int ilo = hasx ? 1 : 0, ihi = hasx ? p.Nx - 2 : 0;
     const int klo = hasz ? 1 : 0, khi = hasz ? p.Nz - 2 : 0;
     const int i0 = ilo + TX * bx, j0 = 1 + TY * by;
-    const int k0 = klo + kchunk * bz;
-    const int k1 = min(khi, k0 + kchunk - 1);
+    const int k0 = FLAT ? 0 : klo + kchunk * bz;
+    const int k1 = FLAT ? 0 : min(khi, k0 + kchunk - 1);
     const int i = i0 + tx, j = j0 + ty;
     const bool active = i <= ihi && j <= p.Ny - 2;
     // the own column, clamped into the grid (lanes past it stage values that
@@ -486,7 +494,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
     const HaloAt hat(p, i0, j0, hi, hj);
 
     // LDS places in the buffer of plane 0: the own and the halo cell
-    auto buffer = [](int k) { return (k & 1) * PLANE; };
+    auto buffer = [](int k) { return FLAT ? 0 : (k & 1) * PLANE; };
     const LdsDouble v0 = (LdsDouble)&lds.v[0][ty + 1][tx + 1][0], vh = (LdsDouble)&lds.v[0][hy][hx][0];
     auto stage = [&](int k, LdsDouble w, int row, int x, int ii, int jj, const CellRaw<MODEL, CLOSURE>& r, bool inner,
                      const CellCoef<MODEL, CLOSURE>& c, bool odd) {
@@ -522,6 +530,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
     for (int a = 0; a < NPR; ++a) zneg[a] = zmP[a] = 0.;
 #pragma unroll
     for (int a = 0; a < NPH; ++a) zt2[a] = 0.;
+    auto pre = epi.none();
     {
         CellRaw<MODEL, CLOSURE> r, rm, rh;
         const bool inner = own_ij && inner_k(p, k0), inner_m = own_ij && inner_k(p, k0 - 1);
@@ -529,6 +538,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
         load_raw(io, own, inner, r);
         if (hasz) load_raw(io, CellAt{own.base - p.sz, own.off}, inner_m, rm);
         if (halo) hat.with(p, k0, [&](const auto& at) { load_raw(io, at, inner_h, rh); });
+        if constexpr (FLAT) pre = epi.prefetch(own);
         CellCoef<MODEL, CLOSURE> c, m;
         const DevParams pc = coef_params<MODEL, CLOSURE>(cp);
         const bool odd = coef_of(pc, r, inner, c);
@@ -567,7 +577,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
         const bool inner = own_ij && inner_k(p, k + 1), inner_h = halo_ij && inner_k(p, k + 1);
         if (hasz) load_raw(io, CellAt{own.base + p.sz, own.off}, inner, r);
         if (next && halo) hat.with(p, k + 1, [&](const auto& at) { load_raw(io, at, inner_h, rh); });
-        const auto pre = epi.prefetch(own);
+        if constexpr (!FLAT) pre = epi.prefetch(own);
         // the next plane: coefficients, staged in the other buffer
         CellCoef<MODEL, CLOSURE> zp;
         uint64_t odd = 0;
@@ -826,6 +836,7 @@ template <int MODEL, bool FACES = false, int CLOSURE = -1>
 struct FusedStore {
     StepIO io;
     // dt / m, computed once per porosity field
+    __device__ __forceinline__ double none() const { return 0.; }
     template <class At>
     __device__ __forceinline__ double prefetch(const At& at) const { return ld(io.dtm, at); }
     static constexpr bool kLeaves = true;
@@ -896,6 +907,7 @@ struct FusedStoreRecord {
     FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE> step;
     double* div;
     int64_t stride;
+    __device__ __forceinline__ double none() const { return 0.; }
     template <class At>
     __device__ __forceinline__ double prefetch(const At& at) const { return step.prefetch(at); }
     static constexpr bool kLeaves = true;
@@ -922,6 +934,7 @@ struct RoSStore {
     const double* dtm;
     double *roS[3], *roS_old[3];
     double* u[3][3];  // [phase][axis]: ux_w, uy_w, uz_w, ux_n, ... (U only)
+    __device__ __forceinline__ double none() const { return 0.; }
     template <class At>
     __device__ __forceinline__ double prefetch(const At& at) const { return ld(dtm, at); }
     template <class At>
@@ -950,12 +963,12 @@ struct RoSStore {
     }
 };
 
-template <int TX, int TY, bool FULL, bool U>
+template <int TX, int TY, int AXES, bool U>
 __global__ void __launch_bounds__(TX * TY) k_roS_z(DevParams p, StepIO io, int kchunk, RoSStore<U> st) {
-    __shared__ FusedLds<3, U ? 4 : 3, TX, TY> lds;
+    __shared__ FusedLds<3, U ? 4 : 3, TX, TY, AXES> lds;
     int bx, by, bz;
     xcd_tile(bx, by, bz);
-    fused_z_tile<3, U ? 4 : 3, TX, TY, FULL>(p, kernel_params(), io, kchunk, bx, by, bz, lds, st);
+    fused_z_tile<3, U ? 4 : 3, TX, TY, AXES>(p, kernel_params(), io, kchunk, bx, by, bz, lds, st);
 }
 
 // The energy step's E pass (assign_E_new, energy.cpp:235-340, as body_E_with)
@@ -1170,13 +1183,13 @@ k_energy_e_z(DevParams p, EnergyEIO a, int kchunk) {
 // The step that also records each interior cell's flux divergence.  Four waves
 // per SIMD, two workgroups per CU: 96^3 three phases 38 us, 45 with the 142 VGPRs
 // the compiler takes by itself.
-template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
+template <int MODEL, int CLOSURE, int TX, int TY, int AXES>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(4))) k_fused_z_record(DevParams p, StepIO io, int kchunk, double* div,
                                                            int64_t stride) {
-    __shared__ FusedLds<MODEL, CLOSURE, TX, TY> lds;
+    __shared__ FusedLds<MODEL, CLOSURE, TX, TY, AXES> lds;
     int bx, by, bz;
     xcd_tile(bx, by, bz);
-    fused_z_tile<MODEL, CLOSURE, TX, TY, FULL>(p, kernel_params(), io, kchunk, bx, by, bz, lds,
+    fused_z_tile<MODEL, CLOSURE, TX, TY, AXES>(p, kernel_params(), io, kchunk, bx, by, bz, lds,
                                                FusedStoreRecord<MODEL, CLOSURE>{
                                                    FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE>{io}, div, stride});
 }
@@ -1207,13 +1220,13 @@ constexpr int kNarrowTY = MODEL == 2 && CLOSURE == 2 ? 8 : 16;
 // tiles for being small: there a launch counts, not the registers (24^3 9.6 us per
 // step against 11.1 with k_fused_faces, 48^3 13.4 against 15.0; 256^3 574 against
 // 538 with these tiles).
-template <int MODEL, int CLOSURE, int TX, int TY, bool FULL, bool FACES>
+template <int MODEL, int CLOSURE, int TX, int TY, int AXES, bool FACES>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(kFusedWaves<MODEL, CLOSURE, TX, TY>)))
 k_fused_z(DevParams p, StepIO io, int kchunk) {
-    __shared__ FusedLds<MODEL, CLOSURE, TX, TY> lds;
+    __shared__ FusedLds<MODEL, CLOSURE, TX, TY, AXES> lds;
     int bx, by, bz;
     xcd_tile(bx, by, bz);
-    fused_z_tile<MODEL, CLOSURE, TX, TY, FULL>(p, kernel_params(), io, kchunk, bx, by, bz, lds,
+    fused_z_tile<MODEL, CLOSURE, TX, TY, AXES>(p, kernel_params(), io, kchunk, bx, by, bz, lds,
                                                FusedStore<MODEL, FACES, CLOSURE>{io});
 }
 

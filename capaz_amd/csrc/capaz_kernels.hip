@@ -320,6 +320,14 @@ hipError_t launch_pack_model(const DevParams& p, const StepIO& io, hipStream_t s
     return launch_pack<MODEL, 1>(p, io, s);
 }
 
+// f(AXES) with the kernels for the grid's axes.
+template <class F>
+hipError_t with_axes(const DevParams& p, const F& f) {
+    using std::integral_constant;
+    if (p.Nz < 3) return f(integral_constant<int, kAxesOnePlane>{});
+    return p.Nx >= 3 ? f(integral_constant<int, kAxesAll>{}) : f(integral_constant<int, kAxesAny>{});
+}
+
 // Threads of the TX x TY workgroups that cover the interior columns.
 int64_t covering_threads(const DevParams& p, int TX, int TY) {
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2;
@@ -335,10 +343,10 @@ hipError_t with_tile(const DevParams& p, const F& f) {
     return f(integral_constant<int, 64>{}, integral_constant<int, WIDE_TY>{});
 }
 
-template <int MODEL, int CLOSURE, int TX, int TY, bool FULL, bool FACES>
+template <int MODEL, int CLOSURE, int TX, int TY, int AXES, bool FACES>
 hipError_t launch_z(const DevParams& p, const StepIO& io, int kchunk, hipStream_t s, const KernelEvents* ev) {
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
-    constexpr auto kernel = k_fused_z<MODEL, CLOSURE, TX, TY, FULL, FACES>;
+    constexpr auto kernel = k_fused_z<MODEL, CLOSURE, TX, TY, AXES, FACES>;
     kchunk = fused_kchunk(p, kchunk, TY, resident_groups<kernel>(TX * TY), TX);
     dim3 grid((nx + TX - 1) / TX, (ny + TY - 1) / TY, (nz + kchunk - 1) / kchunk);
     hipError_t e;
@@ -364,14 +372,15 @@ hipError_t launch_z_tile(const DevParams& p, const StepIO& io, const Tuning& t, 
     auto launch_faces = [&](auto tx, auto ty, auto faces) {
         constexpr int TX = decltype(tx)::value, TY = decltype(ty)::value;
         constexpr bool FACES = decltype(faces)::value;
-        return p.Nx >= 3 && p.Nz >= 3 ? launch_z<MODEL, CLOSURE, TX, TY, true, FACES>(p, io, t.kchunk, s, ev)
-                                      : launch_z<MODEL, CLOSURE, TX, TY, false, FACES>(p, io, t.kchunk, s, ev);
+        return with_axes(p, [&](auto axes) {
+            return launch_z<MODEL, CLOSURE, TX, TY, decltype(axes)::value, FACES>(p, io, t.kchunk, s, ev);
+        });
     };
     auto launch = [&](auto tx, auto ty) {
         return launch_faces(tx, ty, integral_constant<bool, kFusedFaces<MODEL>>{});
     };
     const int64_t groups = covering_threads(p, 64, 4) / 256 * (p.Nz >= 3 ? p.Nz - 2 : 1);
-    const bool small = groups <= resident_groups<k_fused_z<MODEL, CLOSURE, 64, 4, true, true>>(256);
+    const bool small = groups <= resident_groups<k_fused_z<MODEL, CLOSURE, 64, 4, kAxesAll, true>>(256);
     if (t.tile_y == 0 && small)
         return launch_faces(integral_constant<int, 64>{}, integral_constant<int, 4>{}, std::true_type{});
     if (t.tile_y == 4) return launch(integral_constant<int, 64>{}, integral_constant<int, 4>{});
@@ -399,11 +408,11 @@ hipError_t launch_fused(const DevParams& p, const StepIO& io, const Tuning& t, h
     return p.model == 3 ? launch_z_model<3>(p, io, t, s, ev) : launch_z_model<2>(p, io, t, s, ev);
 }
 
-template <int MODEL, int CLOSURE, int TX, int TY, bool FULL>
+template <int MODEL, int CLOSURE, int TX, int TY, int AXES>
 hipError_t launch_record(const DevParams& p, const StepIO& io, int kchunk, double* div, int64_t stride,
                          hipStream_t s) {
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
-    constexpr auto kernel = k_fused_z_record<MODEL, CLOSURE, TX, TY, FULL>;
+    constexpr auto kernel = k_fused_z_record<MODEL, CLOSURE, TX, TY, AXES>;
     kchunk = fused_kchunk(p, kchunk, TY, resident_groups<kernel>(TX * TY), TX);
     dim3 grid((nx + TX - 1) / TX, (ny + TY - 1) / TY, (nz + kchunk - 1) / kchunk);
     hipLaunchKernelGGL(kernel, grid, dim3(TX, TY), 0, s, p, io, kchunk, div, stride);
@@ -417,8 +426,9 @@ hipError_t launch_record_tile(const DevParams& p, const StepIO& io, int kchunk, 
                               hipStream_t s) {
     return with_tile<8, 16>(p, [&](auto tx, auto ty) {
         constexpr int TX = decltype(tx)::value, TY = decltype(ty)::value;
-        return p.Nx >= 3 && p.Nz >= 3 ? launch_record<MODEL, CLOSURE, TX, TY, true>(p, io, kchunk, div, stride, s)
-                                      : launch_record<MODEL, CLOSURE, TX, TY, false>(p, io, kchunk, div, stride, s);
+        return with_axes(p, [&](auto axes) {
+            return launch_record<MODEL, CLOSURE, TX, TY, decltype(axes)::value>(p, io, kchunk, div, stride, s);
+        });
     });
 }
 
@@ -463,16 +473,16 @@ hipError_t launch_roS_tiles(const DevParams& p, const DevFields& F, const double
         for (int x = 0; x < 3; ++x) st.u[a][x] = U && (x < 2 || keep || p.ecfg) ? F.f[uf[a][x]] : nullptr;
     }
     const int nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
-    auto launch = [&](auto tx, auto full) {
+    auto launch = [&](auto tx, auto axes) {
         constexpr int TX = decltype(tx)::value, TY = 8;
-        constexpr auto kernel = k_roS_z<TX, TY, decltype(full)::value, U>;
+        constexpr auto kernel = k_roS_z<TX, TY, decltype(axes)::value, U>;
         const int kchunk = fused_kchunk(p, planes, TY, resident_groups<kernel>(TX * TY), TX);
         dim3 grid((nx + TX - 1) / TX, (ny + TY - 1) / TY, (nz + kchunk - 1) / kchunk);
         hipLaunchKernelGGL(kernel, grid, dim3(TX, TY), 0, s, p, io, kchunk, st);
         return hipGetLastError();
     };
     auto launch_wide = [&](auto tx) {
-        return p.Nx >= 3 && p.Nz >= 3 ? launch(tx, std::true_type{}) : launch(tx, std::false_type{});
+        return with_axes(p, [&](auto axes) { return launch(tx, axes); });
     };
     // With u, 142 to 154 VGPRs: 32 x 8 workgroups, three per CU (160 x 128 x 96: 84
     // us), where a CU holds one of 64 x 8 (91; 101 at 4 waves, whose 128 VGPRs

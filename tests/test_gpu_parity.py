@@ -271,6 +271,35 @@ def test_steps_between_face_exchanges(model, over, axis, dims):
             assert bit_equal(g[f], got[-1][f]), f
 
 
+@pytest.mark.parametrize("dims", [(3, 3, 1), (1, 21, 1), (34, 18, 1), (35, 19, 1), (66, 10, 1), (67, 11, 1), (520, 700, 1)])
+@pytest.mark.parametrize("model,over", [("3ph", dict(CLOSURE="corey", BETA_W=4.5e-10)), ("3ph", dict()),
+                                        ("3ph", dict(CLOSURE="corey", COREY_N=2.5)), ("2ph", dict(CLOSURE="corey")),
+                                        ("2ph", dict()), ("2ph", dict(CLOSURE="corey", COREY_N=2.5)), ("3phe", dict())])
+def test_grids_of_one_plane(model, over, dims):
+    """The tiles of grids with Nz = 1, at the edges of each tile shape, with phase
+    pressures of their own in the x faces and cells that need the pivot search:
+    every field as from one thread per cell (with the energy equation, as from the
+    entry points)."""
+    if model == "2ph" and dims[0] < 3:
+        pytest.skip("two phases need Nx >= 3")
+    keys = case(model, *dims, DT=1e-5, SOURCE=1, **over)
+    st = random_state(keys, seed=sum(dims))
+    rng = np.random.default_rng(sum(dims) + 2)
+    if "BETA_W" in over:
+        st["S_w"] = np.where(rng.random(st["S_w"].shape) < 0.1, 0.01, st["S_w"])
+    got = []
+    for tune in (dict(), dict(tile_y=8), dict(tile_y=4), dict(energy_kernel=0) if model == "3phe" else dict(fused_kernel=0)):
+        d = capaz.Domain(keys, st)
+        d.tune(**tune)
+        d.run(2)
+        got.append(d.fields())
+        d.close()
+    for g in got[:-1]:
+        for f in g:
+            assert bit_equal(g[f], got[-1][f]), f
+    assert np.isfinite(got[-1]["P_w"]).all()
+
+
 # interior columns that 32 x 16 and 32 x 8 workgroups cover with fewer threads than
 # 64 x 8 and 64 x 4 ones (28 x 13, 32 x 16, 95 x 17), and not (62 x 19); planes
 # enough that the workgroups do not all fit at once; one plane
