@@ -127,10 +127,9 @@ struct AdjNewtonStore {
     template <class At>
     __device__ __forceinline__ int prefetch(const At&) const { return 0; }
     template <class At>
-    __device__ __forceinline__ bool cell(const DevParams& p, const DevParams&, int i, int j, int k, const At& at,
-                                         const CellState<3>& s, const double* div, int) const {
+    __device__ __forceinline__ void cell(const DevParams& p, const DevParams&, int i, int j, int k, const At& at,
+                                         const CellState<3>& s, const double* div, int, uint32_t&, uint32_t) const {
         adj_newton_tail<IT>(p, a, i, j, k, at.l(), s.ro, s.P, s.Sw, s.Sn, div);
-        return true;
     }
 };
 

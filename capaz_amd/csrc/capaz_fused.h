@@ -196,6 +196,15 @@ __device__ __forceinline__ void st(double* f, const CellAt& a, double v) {
     *(__attribute__((address_space(1))) double*)(row_of(f, a.base) + a.off) = v;
 }
 
+// A value compared in rarely taken code: the compiler otherwise makes the
+// comparison's lane mask outside the plane loop and keeps it there, in scalar
+// registers that the closures' constants need (van Genuchten: 8 more lane reads per
+// closure evaluation, 1.2% of the step's VALU instructions).
+__device__ __forceinline__ int seldom(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // A tile's halo cell (hi, hj) of a plane: from the cell below and left of the
 // tile's first (i0, j0), whose index is uniform, a lane offset of up to 19
 // rows, below 2^32 bytes for rows of at most kMaxRow32 cells (which leaves a
@@ -440,10 +449,11 @@ struct CellState {
 // Epi: what happens at an interior cell once its state and flux divergence
 // are known -- the Newton solve and store of the step (FusedStore) or the
 // adjoint's backward Newton (AdjNewtonStore).  prefetch() loads what it needs;
-// with kLeaves, cell() may leave the cell undone and say so (false), its right
-// side in the cell's place of the next state, which nothing else in the launch
-// reads: late() does it after the last plane, so that the planes' code holds no
-// call and no registers for it (kchunk <= kMaxPlanes, one mark per plane).
+// with kLeaves, cell() may leave the cell undone, with its plane's bit set in
+// `undone` and its right side in the cell's place of the next state, which nothing
+// else in the launch reads: late() does it after the last plane, so that the
+// planes' code holds no call and no registers for it (kchunk <= kMaxPlanes, one
+// bit per plane).
 //
 // P_n or P_g apart from P_w in an x or z face cell (values a caller set, or an
 // exchange of faces: Border_P gives those faces P_n = P_g = P_w, P_Xi_ro every
@@ -510,9 +520,11 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
                 if (jj == 0 || jj == p.Ny - 1) {
                     lds.edge[k & 1][jj == 0 ? 0 : 1][0][x] = r.Pn;
                     lds.edge[k & 1][jj == 0 ? 0 : 1][1][x] = r.Pg;
-                } else if (hasx && (ii == 0 || ii == p.Nx - 1)) {
-                    lds.side[k & 1][ii == 0 ? 0 : 1][0][row] = r.Pn;
-                    lds.side[k & 1][ii == 0 ? 0 : 1][1][row] = r.Pg;
+                } else {
+                    // an x face cell (a z face's plane is not read from LDS)
+                    const int s = seldom(ii) == 0 ? 0 : 1;
+                    lds.side[k & 1][s][0][row] = r.Pn;
+                    lds.side[k & 1][s][1][row] = r.Pg;
                     if (odd) lds.odd[k & 1][row] = k;
                 }
             }
@@ -637,22 +649,18 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
                         if constexpr (U) u[a][0] = c.Xi[a] * exact_div(Pp - Pm, pf.two_hx, pf.r_two_hx);
                     }
                 };
-                bool apart = false;
-                if constexpr (APART) apart = __ballot(lds.odd[k & 1][ty + 1] == k) != 0;
-                if (__builtin_expect(apart, 0)) {
 #pragma unroll
-                    for (int a = 0; a < NPH; ++a) {
-                        double Pm = P_at(0, 1, 0), Pp = P_at(0, 1, 2);
-                        if constexpr (APART) {
-                            if (a > 0 && i == 1) Pm = lds.side[k & 1][0][a - 1][ty + 1];
-                            if (a > 0 && i == p.Nx - 2) Pp = lds.side[k & 1][1][a - 1][ty + 1];
-                        }
-                        x_flux(c.P[0], Pm, Pp, a, a + 1);
+                for (int q = 0; q < NPR; ++q)
+                    x_flux(c.P[q], P_at(q, 1, 0), P_at(q, 1, 2), q, NPR == 1 ? NPH : q + 1);
+                if constexpr (APART) {
+                    // n and g again, each from its own pressures
+                    if (__builtin_expect(__ballot(lds.odd[k & 1][ty + 1] == k) != 0, 0)) {
+                        const int is = seldom(i);
+#pragma unroll
+                        for (int a = 1; a < NPH; ++a)
+                            x_flux(c.P[0], is == 1 ? lds.side[k & 1][0][a - 1][ty + 1] : P_at(0, 1, 0),
+                                   is == p.Nx - 2 ? lds.side[k & 1][1][a - 1][ty + 1] : P_at(0, 1, 2), a, a + 1);
                     }
-                } else {
-#pragma unroll
-                    for (int q = 0; q < NPR; ++q)
-                        x_flux(c.P[q], P_at(q, 1, 0), P_at(q, 1, 2), q, NPR == 1 ? NPH : q + 1);
                 }
             } else if constexpr (U) {
 #pragma unroll
@@ -755,10 +763,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
 #pragma unroll
             for (int a = 0; a < NPH; ++a) s.ro[a] = c.ro[a];
             if constexpr (U) epi.store_u(own, u);
-            const bool done = epi.cell(p, newton_params<MODEL, CLOSURE>(fresh(cp)), i, j, k, own, s, div, pre);
-            if constexpr (Epi::kLeaves) {
-                if (!done) undone |= 1u << (k - k0);
-            }
+            epi.cell(p, newton_params<MODEL, CLOSURE>(fresh(cp)), i, j, k, own, s, div, pre, undone, 1u << (k - k0));
         }
         if (next) {
             zodd = 0;
@@ -771,7 +776,7 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
 
     if constexpr (Epi::kLeaves) {
         while (__builtin_expect(undone != 0, 0)) {
-            epi.late(p, i, j, k0 + __ffs(undone) - 1);
+            epi.late(p, newton_params<MODEL, CLOSURE>(fresh(cp)), i, j, k0 + __ffs(undone) - 1);
             undone &= undone - 1;
         }
     }
@@ -840,10 +845,10 @@ struct FusedStore {
     template <class At>
     __device__ __forceinline__ double prefetch(const At& at) const { return ld(io.dtm, at); }
     static constexpr bool kLeaves = true;
-    // false: the right side stored for late()
     template <class At>
-    __device__ __forceinline__ bool cell(const DevParams& p, const DevParams& pn, int i, int j, int k, const At& at,
-                                         const CellState<MODEL>& s, const double* div, double dtm) const {
+    __device__ __forceinline__ void cell(const DevParams& p, const DevParams& pn, int i, int j, int k, const At& at,
+                                         const CellState<MODEL>& s, const double* div, double dtm, uint32_t& undone,
+                                         uint32_t bit) const {
         (void)i; (void)j; (void)k;
         double Pw = s.P, Sn = s.Sn, Sw = s.Sw;
         bool done;
@@ -854,6 +859,7 @@ struct FusedStore {
             if (__builtin_expect(!done, 0)) {
                 Pw = A1;
                 Sn = A2;
+                undone |= bit;
             }
         } else {
             const double A1 = s.ro[0] * Sw - dtm * div[0];
@@ -864,6 +870,7 @@ struct FusedStore {
                 Pw = A1;
                 Sw = A3;
                 Sn = A2;
+                undone |= bit;
             }
         }
         At to = at;
@@ -873,20 +880,19 @@ struct FusedStore {
         st(io.Sn1, to, Sn);
         if constexpr (FACES)
             if (done) store_faces<MODEL>(p, io, i, j, k, at.l(), s.ro, Pw, Sw, Sn);
-        return done;
     }
     // The cell from its state and the right side that cell() left.
-    __device__ __forceinline__ void late(const DevParams& p, int i, int j, int k) const {
+    __device__ __forceinline__ void late(const DevParams& p, const DevParams& pn, int i, int j, int k) const {
         const int64_t l = (int64_t)i + (int64_t)j * p.sy + (int64_t)k * p.sz;
         const double A1 = io.Pw1[l], A2 = io.Sn1[l];
         double Pw = io.Pw[l], Sn = io.Sn[l], Sw = 0., ro[MODEL] = {};
         if constexpr (MODEL == 2) {
             if constexpr (FACES) densities2<CLOSURE>(p, io, l, ro);
-            newton2_ieee<CLOSURE>(p, Pw, Sn, A1, A2);
+            newton2_ieee<CLOSURE>(pn, Pw, Sn, A1, A2);
         } else {
             const double A3 = io.Sw1[l];
             Sw = io.Sw[l];
-            newton3_general(p, Pw, Sw, Sn, A1, A2, A3);
+            newton3_general(pn, Pw, Sw, Sn, A1, A2, A3);
             io.Sw1[l] = Sw;
         }
         io.Pw1[l] = Pw;
@@ -912,15 +918,16 @@ struct FusedStoreRecord {
     __device__ __forceinline__ double prefetch(const At& at) const { return step.prefetch(at); }
     static constexpr bool kLeaves = true;
     template <class At>
-    __device__ __forceinline__ bool cell(const DevParams& p, const DevParams& pn, int i, int j, int k, const At& at,
-                                         const CellState<MODEL>& s, const double* d, double dtm) const {
+    __device__ __forceinline__ void cell(const DevParams& p, const DevParams& pn, int i, int j, int k, const At& at,
+                                         const CellState<MODEL>& s, const double* d, double dtm, uint32_t& undone,
+                                         uint32_t bit) const {
         At to = at;
         renew(to);
 #pragma unroll
         for (int a = 0; a < MODEL; ++a) st(div + a * stride, to, d[a]);
-        return step.cell(p, pn, i, j, k, at, s, d, dtm);
+        step.cell(p, pn, i, j, k, at, s, d, dtm, undone, bit);
     }
-    __device__ __forceinline__ void late(const DevParams& p, int i, int j, int k) const { step.late(p, i, j, k); }
+    __device__ __forceinline__ void late(const DevParams& p, const DevParams& pn, int i, int j, int k) const { step.late(p, pn, i, j, k); }
 };
 
 // assign_roS_nr (cpu.cpp:619-731) on the z tiles (three phases): roS_old and
@@ -948,8 +955,8 @@ struct RoSStore {
                 if (x < 2 || u[a][2]) st(u[a][x], to, v[a][x]);
     }
     template <class At>
-    __device__ __forceinline__ bool cell(const DevParams& p, const DevParams& pn, int i, int j, int k, const At& at,
-                                         const CellState<3>& s, const double* div, double d) const {
+    __device__ __forceinline__ void cell(const DevParams& p, const DevParams& pn, int i, int j, int k, const At& at,
+                                         const CellState<3>& s, const double* div, double d, uint32_t&, uint32_t) const {
         (void)p; (void)pn; (void)i; (void)j; (void)k;
         const double old[3] = {s.ro[0] * s.Sw, s.ro[1] * s.Sn, s.ro[2] * (1. - s.Sw - s.Sn)};
         At to = at;
@@ -959,7 +966,6 @@ struct RoSStore {
             if (!U || roS_old[a]) st(roS_old[a], to, old[a]);
             st(roS[a], to, old[a] - d * div[a]);
         }
-        return true;
     }
 };
 
