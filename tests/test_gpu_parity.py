@@ -646,6 +646,33 @@ def test_energy_step_fields_where_a_run_stops(tune):
         d.close()
 
 
+@pytest.mark.parametrize("dims", [(20, 11, 9), (34, 19, 40), (68, 9, 3), (19, 12, 1), (1, 21, 9), (1, 9, 1)])
+@pytest.mark.parametrize("closure", ["corey", "reference"])
+def test_energy_step_with_the_configurations_closure(dims, closure):
+    """Three phases with the configurations' energy closure (constant conductivity
+    and rock, exponential viscosities, the z term advected by u_z): every field of
+    a run of 1, 2 and 4 steps as from the sequence, and the oracle's within the
+    one-step bar after one."""
+    keys = case("3phe", *dims, DT=1e-4, SOURCE=1, CLOSURE=closure, ENERGY_CLOSURE="config", LAMBDA_EFF=1.5, C_R=800.0,
+                RO_R=2000.0, T_TOP=300.0, T_BOTTOM=0.0, MU_T_A=0.02, MU_T_REF=285.0)
+    st = random_state(keys, seed=sum(dims) + 4)
+    for steps in (1, 2, 4):
+        seq, d = capaz.Domain(keys, st), capaz.Domain(keys, st)
+        seq.tune(energy_kernel=0)
+        seq.run(steps)
+        d.run(steps)
+        got = d.fields()
+        for f in seq.names:
+            assert bit_equal(got[f], seq.field(f)), (steps, f)
+        assert np.isfinite(got["T"]).all()
+        if steps == 1:
+            od = oracle.OracleDomain(keys, st)
+            od.run(1)
+            check_fields({f: got[f] for f in d.names}, {f: od.field(f) for f in d.names}, TOL_STEP1, str(dims))
+        seq.close()
+        d.close()
+
+
 def test_energy_full_size_six_passes_equal_the_sequence():
     """The energy workload at 256 x 256 x 128: two steps of the six-pass
     energy step and two entry-point sequences give identical bits in every
