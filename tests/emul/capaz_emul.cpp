@@ -159,6 +159,17 @@ int capaz_emul_coef_d(const capaz_params* u, const double* x, int inner, double*
     return 0;
 }
 
+// The three-phase Newton of one cell: x = {P_w, S_w, S_n} (updated) from the right
+// side A = {roS_w, roS_n, roS_g}.  fast: the tiles' form, 1 where it leaves the
+// cell undone; else gauss.cpp's routine.
+int capaz_emul_newton3(const capaz_params* u, double* x, const double* A, int fast) {
+    if (!capaz::validate(*u).empty()) return -1;
+    const capaz::DevParams p = capaz::derive(*u);
+    if (fast) return capaz::newton3_fast(p, x[0], x[1], x[2], A[0], A[1], A[2]) ? 0 : 1;
+    capaz::newton3_general(p, x[0], x[1], x[2], A[0], A[1], A[2]);
+    return 0;
+}
+
 int capaz_emul_reverse_matrix(double* a, int n) {
     if (n == -3) return capaz::reverse3(a);  // the no-pivot fast path with fallback
     if (n == -4) return capaz::reverse3<true>(a);  // the same for a[2] == +0

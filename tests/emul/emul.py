@@ -74,6 +74,17 @@ def coef_d(keys: dict, Pw: float, Sw: float, Sn: float, K: float):
     return v[0:3], v[3:6], v[6:9]
 
 
+def newton3(keys: dict, x, A, fast: bool):
+    """(done, (P_w, S_w, S_n)) of the three-phase Newton of one cell from its state x
+    and right side A; fast: the tiles' form, which may leave it undone."""
+    p = params_from_keys(keys)
+    v, r = (ctypes.c_double * 3)(*x), (ctypes.c_double * 3)(*A)
+    rc = lib().capaz_emul_newton3(ctypes.byref(p), v, r, int(fast))
+    if rc < 0:
+        raise ValueError("invalid parameters")
+    return rc == 0, np.array(v)
+
+
 def reverse_matrix(a: np.ndarray, fast: bool = False, a02zero: bool = False) -> tuple[int, np.ndarray]:
     """The kernels' reverse_matrix<n>; fast=True runs the 3x3 no-pivot path
     with its fallback (for n = 4, 5 the no-pivot routine alone, rc 1 when it

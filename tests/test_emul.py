@@ -4,7 +4,7 @@ bodies are covered by tests/test_golden.py)."""
 import numpy as np
 import pytest
 
-from capaz_cases import bit_equal
+from capaz_cases import bit_equal, case
 from emul import emul
 from oracle import oracle
 
@@ -78,6 +78,33 @@ def test_reverse_nopivot_matches_oracle_or_refuses(n):
             assert rc_o == 0 and bit_equal(out_o, out_e), a
             hits += 1
     assert hits > 2000 and refused > 1000
+
+
+@pytest.mark.parametrize("beta", [4.4e-7, 4.5e-10, 0.0])
+def test_three_phase_newton_without_the_search_or_undone(beta):
+    """The tiles' three-phase Newton: the general routine's bits, or undone where a
+    pivot is below 1e-8 (water of a saturation near zero, no compressibility) or
+    not finite."""
+    keys = case("3ph", 3, 3, 3, BETA_W=beta, BETA_N=beta)
+    rng = np.random.default_rng(int(beta * 1e12) + 3)
+    done = undone = 0
+    for q in range(4000):
+        Sw = rng.uniform(0.0, 0.05) if q % 2 else rng.uniform(0.1, 0.6)
+        x = (1e5 + rng.uniform(-200, 200), Sw, rng.uniform(0.05, 0.35))
+        A = [1000 * x[1], 850 * x[2], 1.4 * (1 - x[1] - x[2])] + rng.normal(0, 1e-3, 3)
+        if q % 97 == 0:
+            A[q % 3] = (np.nan, np.inf)[q % 2]
+        ok, got = emul.newton3(keys, x, A, True)
+        _, want = emul.newton3(keys, x, A, False)
+        if ok:
+            assert bit_equal(got, want), (x, A)
+        done, undone = done + ok, undone + (not ok)
+    if beta == 4.4e-7:
+        assert done > 3800 and undone > 10
+    elif beta:
+        assert done > 1800 and undone > 500
+    else:
+        assert done == 0
 
 
 @pytest.mark.parametrize("closure,gas_free", [("reference", False), ("corey", False), ("reference", True)])
