@@ -14,9 +14,22 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (runs through the C ABI on device 0)")
 
 
+REFERENCE_SOURCE = "/root/reference/cpu.cpp"
+
+
 def pytest_collection_modifyitems(config, items):
-    # GPU tests announce their case before running so that a failing run names it.
-    pass
+    # The drop-in drivers hold the reference's own main.cpp: without its sources
+    # build() leaves them out, and their tests cannot run.  Where the sources are,
+    # a missing driver stays a failure.
+    drivers = os.path.join(ROOT, "capaz_amd", "adapter", "_bin")
+    if os.path.isfile(REFERENCE_SOURCE):
+        return
+    for item in items:
+        if item.path.name == "test_dropin.py":
+            model = item.callspec.params["model"]
+            if not os.path.exists(os.path.join(drivers, f"capaz_dropin_{model}")):
+                item.add_marker(pytest.mark.skip(reason="the drop-in driver is built from the reference's sources, "
+                                                        f"which are not here ({REFERENCE_SOURCE})"))
 
 
 @pytest.fixture(autouse=True)
