@@ -138,7 +138,7 @@ constexpr int kTX = 64, kTY = 8;
 template <int CLOSURE, int IT>
 __global__ void __launch_bounds__(kTX * kTY) k_adj_newton_z(DevParams p, StepIO io, AdjIO a, int kchunk) {
     __shared__ FusedLds<3, CLOSURE, kTX, kTY, kAxesAny> lds;
-    fused_z_tile<3, CLOSURE, kTX, kTY, kAxesAny>(p, kernel_params(), io, kchunk, (int)blockIdx.x, (int)blockIdx.y,
+    fused_z_tile<3, CLOSURE, kTX, kTY, kAxesAny>(p, kernel_params(), kernel_io(), io, kchunk, (int)blockIdx.x, (int)blockIdx.y,
                                               (int)blockIdx.z, lds, AdjNewtonStore<IT>{a});
 }
 

@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(kB
         const StepIO io = *(const StepIO*)&d->io[parity];
         const int lt = t - d->tile_begin;
         const int bx = lt % d->tiles_x, r = lt / d->tiles_x;
-        fused_z_tile<MODEL, CLOSURE, TX, TY, AXES>(p, &d->p, io, kchunk, bx, r % d->tiles_y, r / d->tiles_y, lds,
+        fused_z_tile<MODEL, CLOSURE, TX, TY, AXES>(p, &d->p, &d->io[parity], io, kchunk, bx, r % d->tiles_y, r / d->tiles_y, lds,
                                                     FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE>{io});
         if (!counter) return;
     }

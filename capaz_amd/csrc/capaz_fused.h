@@ -244,6 +244,26 @@ __device__ __forceinline__ ConstParams* fresh(ConstParams* p) {
 __device__ __forceinline__ ConstParams* kernel_params() {
     return (ConstParams*)__builtin_amdgcn_kernarg_segment_ptr();
 }
+// The field pointers in constant memory (the kernel's second argument), read again
+// in every plane by the reference's closures, whose constants need the scalar
+// registers: van Genuchten 256^3 455 M -> 449 M VALU instructions, 160 x 144 x 130
+// 195.3 -> 193.3 us.
+using ConstIO = const __attribute__((address_space(4))) StepIO;
+__device__ __forceinline__ ConstIO* fresh(ConstIO* q) {
+    asm volatile("" : "+s"(q));
+    return q;
+}
+static_assert(sizeof(DevParams) % alignof(StepIO) == 0, "the second argument follows the first");
+__device__ __forceinline__ ConstIO* kernel_io() { return (ConstIO*)(kernel_params() + 1); }
+template <int CLOSURE>
+__device__ __forceinline__ StepIO state_arrays(const StepIO& io, ConstIO* q) {
+    StepIO now = io;
+    if constexpr (CLOSURE == 0) {
+        q = fresh(q);
+        now.Pw = q->Pw, now.Sw = q->Sw, now.Sn = q->Sn, now.Pn = q->Pn, now.Pg = q->Pg, now.K = q->K;
+    }
+    return now;
+}
 // The parameters that coef_of / the fluxes / the Newton solves read.
 template <int MODEL, int CLOSURE>
 __device__ __forceinline__ DevParams coef_params(ConstParams* q) {
@@ -460,10 +480,10 @@ struct CellState {
 // interior cell): the x face's stand in LDS as the top and bottom rows' do, the z
 // face's are read again; the wavefronts next to such a cell take each phase's own
 // differences in that plane.
-// cp: p in constant memory (fresh()).
+// cp, ci: p and io in constant memory (fresh()).
 constexpr int kMaxPlanes = 32;
 template <int MODEL, int CLOSURE, int TX, int TY, int AXES, class Epi>
-__device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp, const StepIO& io, int kchunk, int bx, int by, int bz,
+__device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp, ConstIO* ci, const StepIO& io, int kchunk, int bx, int by, int bz,
                                              FusedLds<MODEL, CLOSURE, TX, TY, AXES>& lds, const Epi& epi) {
     static_assert(TY >= 3 && TX >= 2 * TY, "halo ring needs TY >= 3 and TX >= 2*TY");
     static_assert(TX == 32 || TX == 64, "whole rows per wavefront");
@@ -587,8 +607,9 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
         renew(own);
         CellRaw<MODEL, CLOSURE> r, rh;
         const bool inner = own_ij && inner_k(p, k + 1), inner_h = halo_ij && inner_k(p, k + 1);
-        if (hasz) load_raw(io, CellAt{own.base + p.sz, own.off}, inner, r);
-        if (next && halo) hat.with(p, k + 1, [&](const auto& at) { load_raw(io, at, inner_h, rh); });
+        const StepIO now = state_arrays<CLOSURE>(io, ci);
+        if (hasz) load_raw(now, CellAt{own.base + p.sz, own.off}, inner, r);
+        if (next && halo) hat.with(p, k + 1, [&](const auto& at) { load_raw(now, at, inner_h, rh); });
         if constexpr (!FLAT) pre = epi.prefetch(own);
         // the next plane: coefficients, staged in the other buffer
         CellCoef<MODEL, CLOSURE> zp;
@@ -728,10 +749,11 @@ __device__ __forceinline__ void fused_z_tile(const DevParams& p, ConstParams* cp
                 if (APART && __builtin_expect((zodd | odd) != 0, 0)) {
                     const uint64_t lane = 1ull << ((ty * TX + tx) & 63);
                     const double zn = zneg[0];
+                    const StepIO now = state_arrays<CLOSURE>(io, ci);
                     zneg[0] = z_flux(zn, zmP[0], c.P[0], zp.P[0], 0, 1);
 #pragma unroll
                     for (int a = 1; a < NPH; ++a) {
-                        const double* P = a == 1 ? io.Pn : io.Pg;
+                        const double* P = a == 1 ? now.Pn : now.Pg;
                         double zna = zn, Pm = zmP[0], Pp = zp.P[0];
                         if (zodd & lane) {
                             Pm = ld(P, CellAt{own.base - p.sz, own.off});
@@ -974,7 +996,7 @@ __global__ void __launch_bounds__(TX * TY) k_roS_z(DevParams p, StepIO io, int k
     __shared__ FusedLds<3, U ? 4 : 3, TX, TY, AXES> lds;
     int bx, by, bz;
     xcd_tile(bx, by, bz);
-    fused_z_tile<3, U ? 4 : 3, TX, TY, AXES>(p, kernel_params(), io, kchunk, bx, by, bz, lds, st);
+    fused_z_tile<3, U ? 4 : 3, TX, TY, AXES>(p, kernel_params(), kernel_io(), io, kchunk, bx, by, bz, lds, st);
 }
 
 // The energy step's E pass (assign_E_new, energy.cpp:235-340, as body_E_with)
@@ -1195,7 +1217,7 @@ __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(4)
     __shared__ FusedLds<MODEL, CLOSURE, TX, TY, AXES> lds;
     int bx, by, bz;
     xcd_tile(bx, by, bz);
-    fused_z_tile<MODEL, CLOSURE, TX, TY, AXES>(p, kernel_params(), io, kchunk, bx, by, bz, lds,
+    fused_z_tile<MODEL, CLOSURE, TX, TY, AXES>(p, kernel_params(), kernel_io(), io, kchunk, bx, by, bz, lds,
                                                FusedStoreRecord<MODEL, CLOSURE>{
                                                    FusedStore<MODEL, kFusedFaces<MODEL>, CLOSURE>{io}, div, stride});
 }
@@ -1232,7 +1254,7 @@ k_fused_z(DevParams p, StepIO io, int kchunk) {
     __shared__ FusedLds<MODEL, CLOSURE, TX, TY, AXES> lds;
     int bx, by, bz;
     xcd_tile(bx, by, bz);
-    fused_z_tile<MODEL, CLOSURE, TX, TY, AXES>(p, kernel_params(), io, kchunk, bx, by, bz, lds,
+    fused_z_tile<MODEL, CLOSURE, TX, TY, AXES>(p, kernel_params(), kernel_io(), io, kchunk, bx, by, bz, lds,
                                                FusedStore<MODEL, FACES, CLOSURE>{io});
 }
 
