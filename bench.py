@@ -38,8 +38,10 @@ ALGO_BYTES_PER_CELL = 64
 # the counters read a device-to-device copy of known size correctly) and FP64
 # flops (64 lanes x (ADD + MUL + TRANS + 2 FMA) of SQ_INSTS_VALU_*_F64).
 # profiles/fused_step_3ph_256.md holds the runs and their commands.
-TRAFFIC_BYTES_PER_CELL = 78.5
+TRAFFIC_BYTES_PER_CELL = 76.5
 FP64_FLOPS_PER_CELL = 788.6
+# The main kernel of that grid: three phases, Corey-2, 32 x 16 tiles, all axes.
+MAIN_KERNEL = "k_fused_z<3,2,32,16,1,false>"
 
 
 def _cpu_model() -> str:
@@ -693,7 +695,7 @@ def main() -> int:
     roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": round(TRAFFIC_BYTES_PER_CELL * interior),
-            "kernel": "k_fused_z<3,2,64,8,true>", "algorithmic_bytes_per_cell": ALGO_BYTES_PER_CELL,
+            "kernel": MAIN_KERNEL if args.n == 256 else "k_fused_z<3,2>", "algorithmic_bytes_per_cell": ALGO_BYTES_PER_CELL,
             "cells_per_launch": interior, "avg_launch_us": round(launch_s * 1e6, 2),
             "step_us": round(gpu_ms * 1e3 / args.steps, 2)}
     fp64 = None

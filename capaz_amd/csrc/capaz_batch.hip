@@ -22,8 +22,8 @@ namespace {
 // Occupancy bounds: the two-phase Corey-2 tiles of 256 threads (the 32 x 8
 // and 64 x 4 shapes) at 5 waves per SIMD (96 VGPRs, few spilled), the
 // three-phase Corey-2 ones at 4 (128 VGPRs).  32 two-phase realizations of edges
-// 32-96 step in 186 us on 32 x 8 tiles of 8 planes, one workgroup each,
-// against 218 with the tiles before (capaz_fused.h).
+// 32-96 step in 192 us with the shape that the autotuner takes (32 x 8 tiles),
+// against 269 with tiles of two barriers per plane.
 template <int MODEL, int CLOSURE, int TX, int TY>
 constexpr int kBatchWaves =
     MODEL == 2 && CLOSURE == 2 && TX * TY == 256 ? 5 : (MODEL == 3 && CLOSURE == 2 ? 4 : 1);

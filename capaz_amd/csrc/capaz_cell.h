@@ -478,16 +478,9 @@ CAPAZ_HD double directed(double x1, double x2, double Xic, double roc, double Xi
     return exact_div(t1 - t2 + t3, h, rh);
 }
 
-// directed() from its minus face's parts computed beforehand: nx1 =
-// neg_part(x1) and t2 = directed_t2(x1, Xim, rom); the same operations in
-// the same order, so the same result.
+// directed()'s t2, the minus neighbour's term: the tiles carry it from plane to
+// plane.
 CAPAZ_HD double directed_t2(double x1, double Xim, double rom) { return pos_part(x1) * (-1.) * Xim * rom; }
-CAPAZ_HD double directed_parts(double nx1, double t2, double x2, double Xic, double roc, double Xip, double rop,
-                               double h, double rh) {
-    double t1 = (pos_part(x2) - nx1) * (-1.) * Xic * roc;
-    double t3 = neg_part(x2) * (-1.) * Xip * rop;
-    return exact_div(t1 - t2 + t3, h, rh);
-}
 
 // The upwind flux of one phase along one axis, from the face differences
 // dm = (P_c - P_m)/h and dp = (P_p - P_c)/h; in y the driving force carries

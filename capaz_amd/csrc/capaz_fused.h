@@ -7,14 +7,14 @@
 // plane the closure coefficients of each cell -- phase pressures, Xi and
 // densities, the values the upwind flux reads from a neighbour -- are computed
 // once and staged in LDS together with a one-cell halo ring, so the x and y
-// neighbours come from LDS; the z neighbours stay in registers from the
-// previous and next plane, and the z face differences (P_c - P_zm)/h are
-// carried over from the previous plane (the same bits as recomputing them).
+// neighbours come from LDS; the z face's flux terms are carried over from the
+// previous plane (the same bits as recomputing them).
 // After the divergence each thread solves its cell's Newton system in
-// registers and writes the new state.  The boundary cells are written
-// afterwards by k_fused_faces from their inward neighbours' new state
-// (Border_S/Border_P, two-phase.cpp:163-215, three-phase.cpp:345-427): an
-// O(N^2) pass that keeps the face logic out of the interior kernel's
+// registers and writes the new state.  The boundary cells take theirs from
+// their inward neighbours' new state (Border_S/Border_P, two-phase.cpp:163-215,
+// three-phase.cpp:345-427): in the tiles for two phases and for three-phase
+// grids whose workgroups all fit at once, else in an O(N^2) pass afterwards
+// (k_fused_faces), which keeps the face logic out of the interior kernel's
 // registers.
 //
 // Arithmetic is that of capaz_cell.h / capaz_bodies.h, so the kernel gives
@@ -452,10 +452,10 @@ struct CellState {
 // so that a wavefront holds whole rows).
 //
 // What bounds it: VALU issue (FP64).  The 256^3 three-phase Corey-2 step went
-// from 850 to some 660 VALU instructions per cell and from 571 to 488 us, the
-// two-phase one from 336 to 285 us, against the tiles before (two barriers
-// and one LDS buffer per plane, every phase's pressure staged, calls and
-// branches in the Newton, parameters in vector-register lanes).
+// from 850 to 715 VALU instructions per cell and from 571 to 475 us, the
+// two-phase one from 336 to 266 us, against tiles with two barriers and one LDS
+// buffer per plane, every phase's pressure staged, calls and branches in the
+// Newton and parameters in vector-register lanes.
 //
 // A plane's turn: issue the loads of the next plane (own cell and ring) and
 // of what the epilogue reads; the x and y fluxes of this plane from LDS,
@@ -1209,8 +1209,8 @@ k_energy_e_z(DevParams p, EnergyEIO a, int kchunk) {
 }
 
 // The step that also records each interior cell's flux divergence.  Four waves
-// per SIMD, two workgroups per CU: 96^3 three phases 38 us, 45 with the 142 VGPRs
-// the compiler takes by itself.
+// per SIMD, two workgroups per CU: 96^3 three phases 38 us where the 142 VGPRs that
+// the compiler takes by itself gave 45; 36.5 now.
 template <int MODEL, int CLOSURE, int TX, int TY, int AXES>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(4))) k_fused_z_record(DevParams p, StepIO io, int kchunk, double* div,
                                                            int64_t stride) {
@@ -1227,16 +1227,17 @@ __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(4)
 // takes the one whose workgroups cover the grid's columns with fewer threads,
 // and 64 x 4 for grids so small that its workgroups all fit at once.  us per
 // step, wide / narrow, and per thread and plane of the covering workgroups (ps):
-//   three phases, Corey-2   256^3 498 / 498 (29.9 / 29.9), 203 x 117 x 83 76.1 / 67.7 (30.6 / 29.2)
-//     van Genuchten         160 x 144 x 130 237 / 195 (66.9 / 66.0)
-//     run-time exponent     160 x 144 x 130 185 / 152
-//   two phases, Corey-2     256^3 288 / 285, 96^3 26.5 / 21.4
-//     Brooks-Corey          190 x 150 x 110 192 / 209 (62.6 / 63.0), 160^3 290 / 243 (59.7 / 60.2)
-//     run-time exponent     256^3 398 / 391
+//   three phases, Corey-2   256^3 479 / 475 (28.8 / 28.5), 203 x 117 x 83 72.5 / 65.6 (29.1 / 28.2)
+//     van Genuchten         160 x 144 x 130 236 / 193 (66.6 / 65.3)
+//     run-time exponent     160 x 144 x 130 144 / 120
+//   two phases, Corey-2     256^3 273 / 266, 96^3 25.4 / 20.0
+//     Brooks-Corey          190 x 150 x 110 186 / 206, 160^3 282 / 240
+//     run-time exponent     256^3 386 / 378
 // the other shapes of 256 and 512 threads are slower or equal, but in small
-// grids, where a workgroup's latency counts: three phases 24^3 64 x 4 10.8,
-// 64 x 8 12.5, 32 x 16 12.1; 48^3 15.0, 18.2, 18.2.  Registers: 128 VGPRs at 4
-// waves (a few spilled for three phases), 95 at 5, 168 at 3.
+// grids, where a workgroup's latency counts: three phases (with k_fused_faces)
+// 24^3 64 x 4 9.7, 64 x 8 11.3, 32 x 16 11.3; 48^3 13.9, 16.8, 16.3.  Registers:
+// 128 VGPRs at 4 waves (32 to 64 B spilled for three phases, in code taken seldom),
+// 88 at 5, 168 at 3.
 template <int MODEL, int CLOSURE, int TX, int TY>
 constexpr int kFusedWaves = TX * TY == 512 ? 4 : (MODEL == 2 && CLOSURE == 2 ? 5 : 3);
 template <int MODEL, int CLOSURE>
@@ -1245,9 +1246,9 @@ template <int MODEL, int CLOSURE>
 constexpr int kNarrowTY = MODEL == 2 && CLOSURE == 2 ? 8 : 16;
 
 // FACES: the boundary cells too, for three phases in grids that take the 64 x 4
-// tiles for being small: there a launch counts, not the registers (24^3 9.6 us per
-// step against 11.1 with k_fused_faces, 48^3 13.4 against 15.0; 256^3 574 against
-// 538 with these tiles).
+// tiles for being small: there a launch counts, not the registers (24^3 8.4 us per
+// step against 9.7 with k_fused_faces, 48^3 12.2 against 13.9; 256^3 579 against
+// 475 with the tiles and pass that large grids take).
 template <int MODEL, int CLOSURE, int TX, int TY, int AXES, bool FACES>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(kFusedWaves<MODEL, CLOSURE, TX, TY>)))
 k_fused_z(DevParams p, StepIO io, int kchunk) {

@@ -283,8 +283,8 @@ int fused_kchunk(const DevParams& p, int kchunk, int ty, int resident, int tx) {
     // automatic: the planes per tile that minimise (rounds of resident
     // workgroups) x (planes per tile + the tile's extra coefficient planes).
     // One plane is worth it where the workgroups then still fit at once: a
-    // 24^3 three-phase step takes 12.7 us against 15.9 with two (40^3 two
-    // phases: 7.4 against 8.5), each plane's latency being a quarter of that.
+    // 24^3 three-phase step takes 8.4 us against 12.8 with two (40^3 two
+    // phases: 6.4 against 7.8).
     const int64_t nx = p.Nx >= 3 ? p.Nx - 2 : 1, ny = p.Ny - 2, nz = p.Nz >= 3 ? p.Nz - 2 : 1;
     const int64_t txy = ((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
     int best = 16;

@@ -11,11 +11,12 @@ enum class Entry { S, P_Xi_ro, U, RoS, HE, E, Newton, Boundary };
 
 // Launch shape of the fused step: fused_kernel 0 = one thread per cell
 // (k_fused_step), 1 and 2 = z-marching tiles (k_fused_z) of 64 x tile_y
-// columns and kchunk planes per workgroup (0: chosen from the grid).
+// columns (0: a shape chosen by model, closure and grid) and kchunk planes per
+// workgroup (0: chosen from the grid).
 // adjoint_kernel: 2 = the backward Newton per cell from the flux divergence
-// recorded by the segment's forward recompute, then the coefficient pass per
-// cell; 1 = both passes on the z-marching LDS tiles; 0 = both per cell,
-// recomputing the neighbours' coefficients.
+// recorded by the segment's forward recompute, then the coefficient pass (three
+// phases: on LDS tiles); 1 = both passes on the z-marching LDS tiles; 0 = both per
+// cell, recomputing the neighbours' coefficients.
 // adjoint_streams: 2 = the reverse sweep recomputes segment q-1 on a second
 // stream while the adjoint passes run over segment q (two segment buffers),
 // 1 = one stream, recompute then passes.

@@ -209,7 +209,7 @@ int capaz_step(capaz_ctx* ctx, long first_step, long nsteps);
  *                   six passes (per cell S, P_Xi_ro, HE and the
  *                   conductivity; u; roS; E from the stored conductivity;
  *                   Newton; the boundary faces), for two phases one fused
- *                   kernel on z-marching 64 x 8 tiles (P_w, S_n, T read
+ *                   kernel on z-marching 32 x 16 tiles (P_w, S_n, T read
  *                   once and written once per step, the Newton in
  *                   registers); 0 the eight entry-point kernels
  *   "energy_newton" the energy model's Newton (its entry point and step):
