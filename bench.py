@@ -38,7 +38,7 @@ ALGO_BYTES_PER_CELL = 64
 # the counters read a device-to-device copy of known size correctly) and FP64
 # flops (64 lanes x (ADD + MUL + TRANS + 2 FMA) of SQ_INSTS_VALU_*_F64).
 # profiles/fused_step_3ph_256.md holds the runs and their commands.
-TRAFFIC_BYTES_PER_CELL = 76.5
+TRAFFIC_BYTES_PER_CELL = 76.6
 FP64_FLOPS_PER_CELL = 788.6
 # The main kernel of that grid: three phases, Corey-2, 32 x 16 tiles, all axes.
 MAIN_KERNEL = "k_fused_z<3,2,32,16,1,false>"

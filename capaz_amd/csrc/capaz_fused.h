@@ -1236,8 +1236,8 @@ __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(4)
 // the other shapes of 256 and 512 threads are slower or equal, but in small
 // grids, where a workgroup's latency counts: three phases (with k_fused_faces)
 // 24^3 64 x 4 9.7, 64 x 8 11.3, 32 x 16 11.3; 48^3 13.9, 16.8, 16.3.  Registers:
-// 128 VGPRs at 4 waves (32 to 64 B spilled for three phases, in code taken seldom),
-// 88 at 5, 168 at 3.
+// 128 VGPRs at 4 waves (32 to 64 B spilled for three phases, nearly all of it
+// outside the plane loop's usual path), 88 at 5, 168 at 3.
 template <int MODEL, int CLOSURE, int TX, int TY>
 constexpr int kFusedWaves = TX * TY == 512 ? 4 : (MODEL == 2 && CLOSURE == 2 ? 5 : 3);
 template <int MODEL, int CLOSURE>
